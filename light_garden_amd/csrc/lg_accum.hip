@@ -6,9 +6,10 @@
 // so the raster + blend becomes three stages:
 //   1. binning: every segment is enumerated against the square screen tiles (64 or 32
 //      pixels a side, one size per frame) its deposits can touch. A workgroup owns a chunk
-//      of segments and counts pairs per (tile, major axis) in an LDS histogram; the
-//      [tile][axis][chunk] count matrix is scanned, and a second pass writes segment indices
-//      into per-tile lists, y-major pairs first (no global atomics).
+//      of segments, counts its pairs per row (tile, major axis) in an LDS histogram and adds
+//      them to the rows' totals; what the adds return is the chunk's place in each row. The
+//      row totals are scanned, and a second pass writes segment indices into per-tile lists,
+//      y-major pairs first.
 //   2. tiles: a persistent workgroup takes a (tile, pair range) work item, walks each of
 //      its segments' column (x-major) or row (y-major) samples that fall in the tile, one
 //      sample per lane (the samples of 64 pairs laid end to end, 64 per step, in two-channel
@@ -178,18 +179,17 @@ __device__ __forceinline__ uint64_t scene_segments(const SceneDesc& D) {
 }
 
 // Segments per bin chunk of a scene: the frame's chunk size, and at least kBinSegsPerCounter
-// per counter of the scene's [tile][axis] histogram, which every chunk initialises and writes
-// back with one strided access per counter (short chunks of a large image would spend their
-// time there) -- unless that would leave the scene fewer chunks than the frame has bin
-// workgroups. A scene with more chunks than workgroups gets a whole multiple of their number
+// per counter of the scene's [tile][axis] histogram, which every chunk initialises, adds to the
+// row totals and writes back (short chunks of a large image would spend their time there) --
+// unless that would leave the frame fewer chunks than it has bin workgroups (`spread` segments
+// each). A scene with more chunks than workgroups gets a whole multiple of their number
 // (a count just above it leaves most workgroups idle while the rest take one more chunk).
 // Never more chunks than the frame's chunk size gives, so the count matrix keeps its capacity.
 constexpr uint32_t kBinSegsPerCounter = 2;
-__device__ __forceinline__ uint32_t scene_chunk(uint32_t chunk, uint32_t groups, const SceneDesc& D) {
+__device__ __forceinline__ uint32_t scene_chunk(uint32_t chunk, uint32_t groups, uint32_t spread, const SceneDesc& D) {
   const uint64_t n = scene_segments(D);
   const uint64_t g = groups ? groups : 1u;
   uint64_t m = (uint64_t)kBinSegsPerCounter * 2u * (uint64_t)(D.view.tiles_x * D.view.tiles_y);
-  const uint64_t spread = (n + g - 1) / g;
   m = m < spread ? m : spread;
   uint64_t sc = m > chunk ? m : chunk;
   const uint64_t nch = (n + sc - 1) / sc;
@@ -202,13 +202,11 @@ __device__ __forceinline__ uint32_t scene_chunk(uint32_t chunk, uint32_t groups,
 
 // Bin layout of one frame, from the segment counts the trace just produced: the chunk size
 // gives about `target` chunks over the whole batch (at least `chunk_min` segments each);
-// chunk_pre[s] = first chunk of scene s, cbase[s] = first entry of scene s's [tile][axis][chunk]
-// count matrix (2 x tiles x its chunk count). Resets the accumulation part of the control block.
-// One block of 1024.
+// chunk_pre[s] = first chunk of scene s, cbase[s] = first entry of scene s's [chunk][tile][axis]
+// matrix (2 x tiles x its chunk count). One block of 1024.
 __global__ __launch_bounds__(1024) void build_chunks_kernel(const SceneDesc* __restrict__ descs, int n_scenes,
                                                            uint32_t chunk_min, uint32_t target, uint32_t groups,
-                                                           uint32_t* chunk_pre, uint32_t* cbase, uint32_t* counts,
-                                                           BatchCtl* ctl) {
+                                                           uint32_t* chunk_pre, uint32_t* cbase, BatchCtl* ctl) {
   __shared__ unsigned long long s_tot[16];
   __shared__ uint32_t s_wa[16], s_wb[16];
   __shared__ uint32_t s_ca, s_cb;
@@ -224,12 +222,14 @@ __global__ __launch_bounds__(1024) void build_chunks_kernel(const SceneDesc* __r
   for (int w = 0; w < 16; w++) total += s_tot[w];
   unsigned long long ch = (total + target - 1) / target;
   const uint32_t chunk = (uint32_t)(ch > chunk_min ? (ch < 0x80000000ull ? ch : 0x80000000ull) : chunk_min);
+  const unsigned long long sp = groups ? (total + groups - 1) / groups : total;
+  const uint32_t spread = (uint32_t)(sp < 0x80000000ull ? sp : 0x80000000ull);
   for (int base = 0; base < n_scenes; base += 1024) {
     const int sid = base + threadIdx.x;
     uint32_t nch = 0, ncnt = 0;
     if (sid < n_scenes) {
       const SceneDesc& D = descs[sid];
-      const uint32_t sc = scene_chunk(chunk, groups, D);
+      const uint32_t sc = scene_chunk(chunk, groups, spread, D);
       nch = (uint32_t)((scene_segments(D) + sc - 1) / sc);
       ncnt = 2u * nch * (uint32_t)(D.view.tiles_x * D.view.tiles_y);
     }
@@ -266,31 +266,36 @@ __global__ __launch_bounds__(1024) void build_chunks_kernel(const SceneDesc* __r
   if (threadIdx.x == 0) {
     chunk_pre[n_scenes] = s_ca;
     cbase[n_scenes] = s_cb;
-    // the count matrix's end entry; the counting pass writes every entry before it
-    counts[s_cb] = 0u;
     ctl->chunk = chunk;
+    ctl->spread = spread;
     ctl->bin_groups = groups;
     ctl->n_chunks = s_ca;
-    ctl->n_counts = s_cb;
-    ctl->chunk_cursor[0] = 0;
-    ctl->chunk_cursor[1] = 0;
-    ctl->total_pairs = 0;
-    ctl->n_work = 0;
-    ctl->work_cursor = 0;
   }
 }
 
-// Persistent over bin chunks. PASS 0 counts pairs per (tile, major axis) into the scene's
-// [tile][axis][chunk] matrix (axis 0: y-major, 1: x-major); PASS 1 writes segment indices at
-// the scanned offsets, so every tile's list holds its y-major pairs first, then its x-major
-// ones, and each phase of the tile walk reads one contiguous run.
+// Persistent over bin chunks. PASS 0 counts a chunk's pairs per row (2 tile + major axis; axis
+// 0: y-major, 1: x-major) in LDS, adds them to the row totals and keeps, in the chunk's row of
+// the [chunk][tile][axis] matrix, the totals from before its own adds: the chunk's first place
+// in each row's list. PASS 1 writes segment indices from row_start + that place on, so every
+// tile's list holds its y-major pairs first, then its x-major ones, and each phase of the tile
+// walk reads one contiguous run. (Which chunk comes first within a row changes from run to run;
+// the tile sums do not depend on it.) The two rows of a tile share one 64-bit add: a row holds
+// fewer than 2^31 pairs.
+//
+// What the chunks' places cost: one atomic per touched tile and chunk here, against a scan of
+// the whole [tile][axis][chunk] matrix, written and read with strides of the chunk count, which
+// this replaced (both passes and the scan, us: 1M-ray frame at 2048x2048 262 -> 204; 20 uneven
+// scenes in one frame 1210 -> 394, part of it from `spread` being the frame's and not the
+// scene's; 1.6M segments at 4096x4096 754 -> 630; 20k-ray frame at 1024x1024 45 -> 25).
 template <int PASS>
 __global__ __launch_bounds__(256) void bin_kernel(const SceneDesc* __restrict__ descs, int n_scenes,
                                                   const uint32_t* __restrict__ chunk_pre,
                                                   const uint32_t* __restrict__ cbase, BatchCtl* ctl,
-                                                  uint32_t* counts_or_offsets, uint32_t* pairs,
+                                                  uint32_t* places, uint32_t* rows, uint32_t* pairs,
                                                   uint64_t pairs_cap) {
-  extern __shared__ uint32_t s_hist[];
+  // rows: PASS 0 the row totals (zeroed before the frame), PASS 1 the rows' starts; both
+  // 2 per tile of the frame
+  extern __shared__ __align__(16) uint32_t s_hist[];
   __shared__ uint32_t s_chunk;
   __shared__ ColumnRec s_rec[4][64];
   __shared__ unsigned long long s_mask[4][kBinMaskWords];
@@ -312,13 +317,20 @@ __global__ __launch_bounds__(256) void bin_kernel(const SceneDesc* __restrict__ 
     const AccumView v = D.view;
     const int n_tiles = v.tiles_x * v.tiles_y;
     const uint32_t local = ci - chunk_pre[sid];
-    const uint32_t nch = chunk_pre[sid + 1] - chunk_pre[sid];
-    uint32_t* mat = counts_or_offsets + cbase[sid];
-    for (int t = threadIdx.x; t < 2 * n_tiles; t += blockDim.x)
-      s_hist[t] = PASS == 0 ? 0u : mat[(uint64_t)t * nch + local];
+    uint2* const mat = reinterpret_cast<uint2*>(places + cbase[sid]) + (uint64_t)local * n_tiles;
+    uint2* const tile_rows = reinterpret_cast<uint2*>(rows) + D.tile_base;
+    uint2* const hist2 = reinterpret_cast<uint2*>(s_hist);
+    for (int t = threadIdx.x; t < n_tiles; t += blockDim.x) {
+      if (PASS == 0) {
+        hist2[t] = make_uint2(0u, 0u);
+      } else {
+        const uint2 a = tile_rows[t], b = mat[t];
+        hist2[t] = make_uint2(a.x + b.x, a.y + b.y);
+      }
+    }
     __syncthreads();
     const uint64_t n = scene_segments(D);
-    const uint32_t sc = scene_chunk(chunk, ctl->bin_groups, D);
+    const uint32_t sc = scene_chunk(chunk, ctl->bin_groups, ctl->spread, D);
     const uint64_t s0 = (uint64_t)local * sc;
     const uint64_t s1 = s0 + sc < n ? s0 + sc : n;
     const int sh = v.tile_shift;
@@ -410,80 +422,203 @@ __global__ __launch_bounds__(256) void bin_kernel(const SceneDesc* __restrict__ 
       }
     }
     __syncthreads();
-    if (PASS == 0)
-      for (int t = threadIdx.x; t < 2 * n_tiles; t += blockDim.x) mat[(uint64_t)t * nch + local] = s_hist[t];
+    if (PASS == 0) {
+      for (int t = threadIdx.x; t < n_tiles; t += blockDim.x) {
+        const uint2 h = hist2[t];
+        if (h.x | h.y) {  // (a tile the chunk does not touch has no pairs to place)
+          const unsigned long long before = atomicAdd(reinterpret_cast<unsigned long long*>(tile_rows + t),
+                                                      (unsigned long long)h.y << 32 | h.x);
+          mat[t] = make_uint2((uint32_t)before, (uint32_t)(before >> 32));
+        }
+      }
+    }
     __syncthreads();
   }
 }
 
-// tile_start[g] for every global tile, tile_mid[g] = its first x-major pair, tile_start[T] =
-// total pairs; the work-item size (every thread derives the same one from the total) and
-// pieces[g], the tile's work items, counted per size class. With `whole_images` (the frame
-// clears, accumulates and resolves every image) a tile without pairs gets one empty item (size
-// class 0), which writes its cleared pixels. A workgroup sums its tiles' classes in LDS and adds
-// each non-zero class to the global count once (one global atomic per tile on a handful of class
-// counters serialises in the L2 when a frame has 1e5 tiles).
-__global__ __launch_bounds__(256) void tile_starts_kernel(const SceneDesc* __restrict__ descs,
-                                                          const uint32_t* __restrict__ tile_scene, int n_tiles_total,
-                                                          const uint32_t* __restrict__ chunk_pre,
-                                                          const uint32_t* __restrict__ cbase,
-                                                          const uint32_t* __restrict__ offsets, BatchCtl* ctl,
-                                                          uint32_t* tile_start, uint32_t* tile_mid, uint32_t* pieces,
-                                                          uint64_t pairs_cap, uint32_t min_piece, uint32_t max_piece,
-                                                          uint32_t grid, uint32_t whole_images) {
+// ---- tile work items ------------------------------------------------------------------------
+// Tile g's list is pairs [rows[2 g], rows[2 g + 2]) of the scanned row totals, its x-major part
+// from rows[2 g + 1] on. A tile is cut into full pieces and at most one remainder; the items are
+// ordered by size class (floor(log2(pairs))), largest class first. With `whole` (the frame clears,
+// accumulates and resolves every image) a tile without pairs gets one empty item (size class 0),
+// which writes its cleared pixels.
+struct PlanLimits {
+  uint64_t pairs_cap;
+  uint32_t items_cap, split_cap;
+  uint32_t min_piece, max_piece;
+  uint32_t grid;   // tile workgroups
+  uint32_t whole;
+};
+
+__device__ __forceinline__ uint32_t piece_size(unsigned long long total, const PlanLimits& L) {
+  unsigned long long pc = total / (2ull * L.grid) + 1;
+  pc = pc < L.min_piece ? L.min_piece : pc;
+  pc = pc > L.max_piece ? L.max_piece : pc;
+  return (uint32_t)pc;
+}
+
+// A tile of cnt pairs: its full pieces, whether one more item follows (the remainder, or the empty
+// item), and that item's class.
+struct TileCut {
+  uint32_t full, items;
+  int cls_rem;
+};
+__device__ __forceinline__ TileCut cut_tile(uint32_t cnt, uint32_t piece, uint32_t whole) {
+  TileCut c;
+  c.full = cnt / piece;
+  const uint32_t rem = cnt - c.full * piece;
+  c.items = cnt ? c.full + (rem ? 1u : 0u) : (whole ? 1u : 0u);
+  c.cls_rem = rem ? 31 - __clz(rem) : 0;
+  return c;
+}
+
+// Writes the items of tile g (list [b, e), x-major from mid); full_slot / rem_slot: the slots of
+// its full pieces and of its last item.
+__device__ __forceinline__ void put_items(WorkItem* items, uint32_t items_cap, uint32_t sid, uint32_t tile, uint32_t b,
+                                          uint32_t e, uint32_t mid, uint32_t piece, const TileCut& c,
+                                          uint32_t split_slot, uint32_t full_slot, uint32_t rem_slot) {
+  const uint32_t cnt = e - b;
+  for (uint32_t p = 0; p < c.items; p++) {
+    WorkItem w;
+    w.scene = sid | (c.items > 1 ? kSplitBit : 0u);
+    w.tile = tile;
+    w.begin = b + p * piece;
+    w.end = e - w.begin > piece ? w.begin + piece : e;
+    w.mid = mid;
+    w.tile_pairs = cnt < kPackedPiece ? cnt : kPackedPiece;
+    w.slot = split_slot;
+    w.pad = 0u;
+    const uint32_t slot = p < c.full ? full_slot + p : rem_slot;
+    if (slot < items_cap) items[slot] = w;
+  }
+}
+
+// Scan of the row totals and the work items in one workgroup, for frames of at most kPlanTiles
+// tiles: thread t owns consecutive tiles. What it takes is the latency of its few dependent steps,
+// so one launch in place of the five to seven of a multi-block scan, a piece count and an item
+// writer is what counts here (us, with the launches it replaces: 256 tiles 34 -> 6, 1024 tiles
+// 61 -> 18, 4096 tiles 122 -> 33, 6k tiles of 20 images 61 -> 30). One workgroup's time grows with
+// its tiles, so frames of more take the multi-block scan.
+constexpr int kPlanTiles = 8192;
+__global__ __launch_bounds__(1024) void plan_items_kernel(const SceneDesc* __restrict__ descs,
+                                                          const uint32_t* __restrict__ tile_scene, int n_tiles,
+                                                          const uint32_t* __restrict__ row_count, BatchCtl* ctl,
+                                                          uint32_t* row_start, WorkItem* items, uint32_t* split_tiles,
+                                                          PlanLimits L) {
+  __shared__ unsigned long long s_w[16];
+  __shared__ uint32_t s_cls[32], s_cur[32];
+  __shared__ uint32_t s_nsplit;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int per = (n_tiles + 1023) / 1024;
+  const int t0 = (int)threadIdx.x * per < n_tiles ? (int)threadIdx.x * per : n_tiles;
+  const int t1 = t0 + per < n_tiles ? t0 + per : n_tiles;
+  const uint2* counts = reinterpret_cast<const uint2*>(row_count);
+  uint2* starts = reinterpret_cast<uint2*>(row_start);
+  if (threadIdx.x < 32) s_cls[threadIdx.x] = 0u;
+  if (threadIdx.x == 0) s_nsplit = 0u;
+  unsigned long long own = 0;
+  for (int t = t0; t < t1; t++) {
+    const uint2 c = counts[t];
+    own += (unsigned long long)c.x + c.y;
+  }
+  unsigned long long incl = own;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const unsigned long long y = __shfl_up(incl, d, 64);
+    if (lane >= d) incl += y;
+  }
+  if (lane == 63) s_w[wave] = incl;
+  __syncthreads();
+  unsigned long long before = 0, total = 0;
+  for (int w = 0; w < 16; w++) {
+    before += w < wave ? s_w[w] : 0ull;
+    total += s_w[w];
+  }
+  const uint32_t first = (uint32_t)(before + incl - own);  // (wraps only past pairs_cap: flagged below)
+  const uint32_t piece = piece_size(total, L);
+  const int cls_full = 31 - __clz(piece);
+  uint32_t b = first;
+  for (int t = t0; t < t1; t++) {
+    const uint2 c = counts[t];
+    starts[t] = make_uint2(b, b + c.x);
+    const TileCut k = cut_tile(c.x + c.y, piece, L.whole);
+    if (k.full) atomicAdd(&s_cls[cls_full], k.full);
+    if (k.items > k.full) atomicAdd(&s_cls[k.cls_rem], 1u);
+    b += c.x + c.y;
+  }
+  __syncthreads();
+  if (threadIdx.x < 32) {  // first slot of each size class, largest class first
+    uint32_t base = 0;
+    for (int c = 31; c > (int)threadIdx.x; c--) base += s_cls[c];
+    s_cur[threadIdx.x] = base;
+    if (threadIdx.x == 0) {
+      const uint32_t n_items = base + s_cls[0];
+      row_start[2 * n_tiles] = (uint32_t)total;
+      ctl->total_pairs = total;
+      ctl->n_work = n_items < L.items_cap ? n_items : L.items_cap;
+      uint32_t f = 0;
+      if (total > L.pairs_cap) f |= CTL_PAIRS_OVERFLOW;
+      if (n_items > L.items_cap) f |= CTL_ITEMS_OVERFLOW;
+      if (f) atomicOr(&ctl->flags, f);
+    }
+  }
+  __syncthreads();
+  b = first;
+  for (int t = t0; t < t1; t++) {
+    const uint2 c = counts[t];
+    const uint32_t cnt = c.x + c.y;
+    const TileCut k = cut_tile(cnt, piece, L.whole);
+    if (k.items) {
+      uint32_t split_slot = 0, full_slot = 0, rem_slot = 0;
+      if (k.items > 1) {  // the tile's items merge their sums in a slot of the fixed-point merge buffer
+        split_slot = atomicAdd(&s_nsplit, 1u);
+        if (split_slot < L.split_cap) split_tiles[split_slot] = (uint32_t)t;
+      }
+      if (k.full) full_slot = atomicAdd(&s_cur[cls_full], k.full);
+      if (k.items > k.full) rem_slot = atomicAdd(&s_cur[k.cls_rem], 1u);
+      const uint32_t sid = tile_scene[t];
+      put_items(items, L.items_cap, sid, (uint32_t)(t - descs[sid].tile_base), b, b + cnt, b + c.x, piece, k,
+                split_slot, full_slot, rem_slot);
+    }
+    b += cnt;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    ctl->n_split = s_nsplit;
+    if (s_nsplit > L.split_cap) atomicOr(&ctl->flags, (uint32_t)CTL_SPLIT_OVERFLOW);
+  }
+}
+
+// Frames of more tiles: the row totals were scanned into row_start by a multi-block scan. Counts
+// the items per size class. A workgroup sums its tiles' classes in LDS and adds each non-zero
+// class to the global count once (one global atomic per tile on a handful of class counters
+// serialises in the L2 when a frame has 1e5 tiles).
+__global__ __launch_bounds__(256) void tile_classes_kernel(int n_tiles, const uint32_t* __restrict__ row_start,
+                                                           BatchCtl* ctl, PlanLimits L) {
   __shared__ uint32_t s_cls[32];
   if (threadIdx.x < 32) s_cls[threadIdx.x] = 0u;
   __syncthreads();
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   const unsigned long long total = ctl->total_pairs;
-  unsigned long long pc = total / (2ull * grid) + 1;
-  pc = pc < min_piece ? min_piece : pc;
-  pc = pc > max_piece ? max_piece : pc;
-  const uint32_t piece = (uint32_t)pc;
-  // entry of tile h's y-major (axis 0) or x-major (axis 1) pairs in the scanned matrix; a scene
-  // without chunks owns no entries: its tiles start where the next scene does
-  auto entry = [&](int h, int axis) {
-    const uint32_t sid = tile_scene[h];
-    const int t = h - descs[sid].tile_base;
-    const uint32_t nch = chunk_pre[sid + 1] - chunk_pre[sid];
-    return offsets[cbase[sid] + (uint64_t)(2 * t + axis) * nch];
-  };
-  if (g < n_tiles_total) {
-    const uint32_t b = entry(g, 0);
-    const uint32_t e = g + 1 < n_tiles_total ? entry(g + 1, 0) : (uint32_t)total;
-    tile_start[g] = b;
-    tile_mid[g] = entry(g, 1);
-    const uint32_t cnt = e - b;
-    if (cnt == 0) {
-      pieces[g] = whole_images ? 1u : 0u;
-      if (whole_images) atomicAdd(&s_cls[0], 1u);
-    } else {
-      const uint32_t full = cnt / piece, rem = cnt - full * piece;
-      pieces[g] = full + (rem ? 1u : 0u);
-      if (full) atomicAdd(&s_cls[31 - __clz(piece)], full);
-      if (rem) atomicAdd(&s_cls[31 - __clz(rem)], 1u);
-    }
+  const uint32_t piece = piece_size(total, L);
+  if (g < n_tiles) {
+    const TileCut k = cut_tile(row_start[2 * g + 2] - row_start[2 * g], piece, L.whole);
+    if (k.full) atomicAdd(&s_cls[31 - __clz(piece)], k.full);
+    if (k.items > k.full) atomicAdd(&s_cls[k.cls_rem], 1u);
   }
-  if (g == n_tiles_total) {
-    tile_start[g] = (uint32_t)total;
-    if (total > pairs_cap) atomicOr(&ctl->flags, (uint32_t)CTL_PAIRS_OVERFLOW);
-    ctl->piece = piece;
-  }
+  if (g == 0 && total > L.pairs_cap) atomicOr(&ctl->flags, (uint32_t)CTL_PAIRS_OVERFLOW);
   __syncthreads();
   if (threadIdx.x < 32 && s_cls[threadIdx.x]) atomicAdd(&ctl->class_count[threadIdx.x], s_cls[threadIdx.x]);
 }
 
-// Writes the work items of every tile into the slots of their size classes. A tile's items are
-// its full pieces (class of `piece`) and at most one remainder (class of its length; the empty
-// item of a pair-less tile in a whole-image frame is class 0). The workgroup reserves its slots
-// of each class, and its split-tile slots, with one global atomic each; a tile's items then take
-// consecutive slots from the offsets its LDS atomics returned.
+// Writes the work items of every tile into the slots of their size classes. The workgroup
+// reserves its slots of each class, and its split-tile slots, with one global atomic each; a
+// tile's items then take consecutive slots from the offsets its LDS atomics returned.
 __global__ __launch_bounds__(256) void write_items_kernel(const SceneDesc* __restrict__ descs,
                                                           const uint32_t* __restrict__ tile_scene,
-                                                          const uint32_t* __restrict__ tile_start,
-                                                          const uint32_t* __restrict__ pieces, int n_tiles_total,
-                                                          BatchCtl* ctl, WorkItem* items, uint32_t items_cap,
-                                                          uint32_t* split_tiles, uint32_t split_cap) {
+                                                          const uint32_t* __restrict__ row_start, int n_tiles,
+                                                          BatchCtl* ctl, WorkItem* items, uint32_t* split_tiles,
+                                                          PlanLimits L) {
   __shared__ uint32_t s_cnt[32], s_base[32], s_cls_base[32];
   __shared__ uint32_t s_nsplit, s_split_base;
   if (threadIdx.x < 32) {
@@ -497,58 +632,42 @@ __global__ __launch_bounds__(256) void write_items_kernel(const SceneDesc* __res
   if (blockIdx.x == 0 && threadIdx.x == 0) {  // the number of work items
     uint32_t n_items = 0;
     for (int c = 0; c < 32; c++) n_items += ctl->class_count[c];
-    if (n_items > items_cap) atomicOr(&ctl->flags, (uint32_t)CTL_ITEMS_OVERFLOW);
-    ctl->n_work = n_items < items_cap ? n_items : items_cap;
+    if (n_items > L.items_cap) atomicOr(&ctl->flags, (uint32_t)CTL_ITEMS_OVERFLOW);
+    ctl->n_work = n_items < L.items_cap ? n_items : L.items_cap;
   }
   __syncthreads();
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t piece = ctl->piece;
-  uint32_t np = 0, b = 0, e = 0, mid = 0;
-  if (g < n_tiles_total) {
-    np = pieces[g];
-    b = tile_start[g];
-    e = tile_start[g + 1];
-    mid = tile_start[n_tiles_total + 1 + g];  // tile_mid follows the n_tiles_total + 1 starts
+  const uint32_t piece = piece_size(ctl->total_pairs, L);
+  uint32_t b = 0, e = 0, mid = 0;
+  TileCut k{0u, 0u, 0};
+  if (g < n_tiles) {
+    b = row_start[2 * g];
+    mid = row_start[2 * g + 1];
+    e = row_start[2 * g + 2];
+    k = cut_tile(e - b, piece, L.whole);
   }
-  const uint32_t cnt = e - b;
-  const uint32_t n_full = cnt / piece;          // items of class cls_full
-  const bool has_rem = np > n_full;             // one more item: the remainder or the empty item
   const int cls_full = 31 - __clz(piece);
-  const int cls_rem = cnt - n_full * piece ? 31 - __clz(cnt - n_full * piece) : 0;
   uint32_t off_full = 0, off_rem = 0, off_split = 0;
-  if (n_full) off_full = atomicAdd(&s_cnt[cls_full], n_full);
-  if (has_rem) off_rem = atomicAdd(&s_cnt[cls_rem], 1u);
-  if (np > 1) off_split = atomicAdd(&s_nsplit, 1u);
+  if (k.full) off_full = atomicAdd(&s_cnt[cls_full], k.full);
+  if (k.items > k.full) off_rem = atomicAdd(&s_cnt[k.cls_rem], 1u);
+  if (k.items > 1) off_split = atomicAdd(&s_nsplit, 1u);
   __syncthreads();
   if (threadIdx.x < 32 && s_cnt[threadIdx.x])
     s_base[threadIdx.x] = s_cls_base[threadIdx.x] + atomicAdd(&ctl->class_cursor[threadIdx.x], s_cnt[threadIdx.x]);
   if (threadIdx.x == 32 && s_nsplit) s_split_base = atomicAdd(&ctl->n_split, s_nsplit);
   __syncthreads();
-  if (np == 0) return;
+  if (k.items == 0) return;
   const uint32_t sid = tile_scene[g];
-  const uint32_t t = (uint32_t)(g - descs[sid].tile_base);
   uint32_t split_slot = 0;
-  if (np > 1) {  // the tile's items merge their sums in a slot of the fixed-point merge buffer
+  if (k.items > 1) {  // the tile's items merge their sums in a slot of the fixed-point merge buffer
     split_slot = s_split_base + off_split;
-    if (split_slot < split_cap)
+    if (split_slot < L.split_cap)
       split_tiles[split_slot] = (uint32_t)g;
     else
       atomicOr(&ctl->flags, (uint32_t)CTL_SPLIT_OVERFLOW);
   }
-  const uint32_t base_full = n_full ? s_base[cls_full] + off_full : 0u;
-  for (uint32_t p = 0; p < np; p++) {
-    WorkItem w;
-    w.scene = sid | (np > 1 ? kSplitBit : 0u);
-    w.tile = t;
-    w.begin = b + p * piece;
-    w.end = (w.begin + piece < e) ? w.begin + piece : e;
-    w.mid = mid;
-    w.tile_pairs = cnt < kPackedPiece ? cnt : kPackedPiece;
-    w.slot = split_slot;
-    w.pad = 0u;
-    const uint32_t slot = p < n_full ? base_full + p : s_base[cls_rem] + off_rem;
-    if (slot < items_cap) items[slot] = w;
-  }
+  put_items(items, L.items_cap, sid, (uint32_t)(g - descs[sid].tile_base), b, e, mid, piece, k, split_slot,
+            k.full ? s_base[cls_full] + off_full : 0u, k.items > k.full ? s_base[k.cls_rem] + off_rem : 0u);
 }
 
 // ---- exclusive scan of u32 (block sums kept in u32; totals are checked on the host) ------
@@ -566,25 +685,15 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x) {
   return x;
 }
 
-// Elements of a capacity-sized buffer that are in use: n, or *n_used + 1 when given (a count
-// matrix holds *n_used entries and one more for its end).
-__device__ __forceinline__ uint64_t used_elems(uint64_t n, const uint32_t* n_used) {
-  if (!n_used) return n;
-  const uint64_t u = (uint64_t)*n_used + 1;
-  return u < n ? u : n;
-}
-
 // Block-level exclusive scan of kScanBlock elements; writes block total to sums[b]. With
 // `total`: a block whose elements sum to 2^32 or more (its u32 total wrapped) sets bit 63 of
 // *total, and the launch of a single block (the scan's top level, whose elements are the exact
 // block totals of the level below) adds their 64-bit sum to *total.
 __global__ __launch_bounds__(kScanThreads) void scan_block_kernel(const uint32_t* in, uint32_t* out,
                                                                   uint64_t n, uint32_t* sums,
-                                                                  const uint32_t* n_used,
                                                                   unsigned long long* total) {
   __shared__ uint32_t s_w[kScanThreads / 64];
   __shared__ unsigned long long s_w64[kScanThreads / 64];
-  n = used_elems(n, n_used);
   uint64_t base = (uint64_t)blockIdx.x * kScanBlock + (uint64_t)threadIdx.x * kScanPer;
   uint32_t v[kScanPer];
   uint32_t tot = 0;
@@ -621,8 +730,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_block_kernel(const uint32_t
 }
 
 __global__ __launch_bounds__(kScanThreads) void scan_add_kernel(uint32_t* out, uint64_t n,
-                                                                const uint32_t* block_ofs, const uint32_t* n_used) {
-  n = used_elems(n, n_used);
+                                                                const uint32_t* block_ofs) {
   uint64_t base = (uint64_t)blockIdx.x * kScanBlock;
   uint32_t add = block_ofs[blockIdx.x];
   for (int i = threadIdx.x; i < kScanBlock; i += kScanThreads)
@@ -702,8 +810,8 @@ __device__ __forceinline__ int packed_fixed_bits(const SceneDesc& D, int c, uint
 }
 
 // The pair count that bounds a packed tile's fields (see packed_fixed_bits).
-__device__ __forceinline__ uint32_t packed_pairs(const uint32_t* tile_start, uint32_t g) {
-  const uint32_t nt = tile_start[g + 1] - tile_start[g];
+__device__ __forceinline__ uint32_t packed_pairs(const uint32_t* row_start, uint32_t g) {
+  const uint32_t nt = row_start[2 * g + 2] - row_start[2 * g];
   return nt < kPackedPiece ? nt : kPackedPiece;
 }
 
@@ -1352,7 +1460,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
 // the unsplit flush) and leaves the slots zeroed for the next frame. Persistent over slots.
 __global__ __launch_bounds__(256) void tile_merge_kernel(const SceneDesc* __restrict__ descs,
                                                         const uint32_t* __restrict__ tile_scene,
-                                                        const uint32_t* __restrict__ tile_start,
+                                                        const uint32_t* __restrict__ row_start,
                                                         const uint32_t* __restrict__ split_tiles,
                                                         const BatchCtl* ctl, unsigned long long* split_fx,
                                                         uint32_t split_cap) {
@@ -1368,7 +1476,7 @@ __global__ __launch_bounds__(256) void tile_merge_kernel(const SceneDesc* __rest
     const int x0 = (int)(t % (uint32_t)v.tiles_x) * T, y0 = (int)(t / (uint32_t)v.tiles_x) * T;
     double un[4];
     if (D.flags & SCENE_PACKED) {
-      const uint32_t np = packed_pairs(tile_start, g);
+      const uint32_t np = packed_pairs(row_start, g);
 #pragma unroll
       for (int c = 0; c < 4; c++) un[c] = __builtin_ldexp(1.0, -packed_fixed_bits(D, c, np));
     } else {
@@ -1449,8 +1557,7 @@ hipError_t launch_lds_atomic_rate(int n_cu, uint32_t iters, unsigned long long* 
   return hipGetLastError();
 }
 
-__global__ void fill_u32_kernel(uint32_t* p, uint64_t n, uint32_t v, const uint32_t* n_used) {
-  n = used_elems(n, n_used);
+__global__ void fill_u32_kernel(uint32_t* p, uint64_t n, uint32_t v) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
     p[i] = v;
 }
@@ -1459,7 +1566,7 @@ __global__ void fill_u32_kernel(uint32_t* p, uint64_t n, uint32_t v, const uint3
 bool tile_size_supported(int tile) { return tile == 32 || tile == 64; }
 uint64_t merge_slot_u64() { return kSlotU64; }
 
-uint64_t scan_scratch_elems(uint64_t n) {
+static uint64_t scan_scratch_elems(uint64_t n) {
   uint64_t total = 0;
   while (n > 1) {
     uint64_t nb = (n + kScanBlock - 1) / kScanBlock;
@@ -1470,66 +1577,70 @@ uint64_t scan_scratch_elems(uint64_t n) {
 }
 
 // Exclusive scan of n u32 (out may not alias in). scratch holds scan_scratch_elems(n) u32.
-// With n_used (device memory), only the first *n_used + 1 elements are scanned.
-hipError_t launch_scan_exclusive(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* scratch,
-                                 hipStream_t st, const uint32_t* n_used, unsigned long long* total) {
+static hipError_t launch_scan_exclusive(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* scratch,
+                                        hipStream_t st, unsigned long long* total) {
   if (n == 0) return hipSuccess;
   uint64_t nb = (n + kScanBlock - 1) / kScanBlock;
   uint32_t* sums = scratch;
-  hipLaunchKernelGGL(scan_block_kernel, dim3((unsigned)nb), dim3(kScanThreads), 0, st, in, out, n, sums, n_used,
-                     total);
+  hipLaunchKernelGGL(scan_block_kernel, dim3((unsigned)nb), dim3(kScanThreads), 0, st, in, out, n, sums, total);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || nb == 1) return e;
-  e = launch_scan_exclusive(sums, sums, nb, scratch + nb, st, nullptr, total);
+  e = launch_scan_exclusive(sums, sums, nb, scratch + nb, st, total);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(scan_add_kernel, dim3((unsigned)nb), dim3(kScanThreads), 0, st, out, n, sums, n_used);
+  hipLaunchKernelGGL(scan_add_kernel, dim3((unsigned)nb), dim3(kScanThreads), 0, st, out, n, sums);
   return hipGetLastError();
 }
 
-hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t st, const uint32_t* n_used) {
+hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t st) {
   if (n == 0) return hipSuccess;
   uint64_t blocks = (n + 255) / 256;
   if (blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL(fill_u32_kernel, dim3((unsigned)blocks), dim3(256), 0, st, p, n, v, n_used);
+  hipLaunchKernelGGL(fill_u32_kernel, dim3((unsigned)blocks), dim3(256), 0, st, p, n, v);
   return hipGetLastError();
 }
 
 hipError_t launch_build_chunks(const SceneDesc* descs, int n_scenes, uint32_t chunk_min, uint32_t target,
-                               uint32_t groups, uint32_t* chunk_pre, uint32_t* cbase, uint32_t* counts,
-                               BatchCtl* ctl, hipStream_t st) {
+                               uint32_t groups, uint32_t* chunk_pre, uint32_t* cbase, BatchCtl* ctl, hipStream_t st) {
   hipLaunchKernelGGL(build_chunks_kernel, dim3(1), dim3(1024), 0, st, descs, n_scenes, chunk_min, target, groups,
-                     chunk_pre, cbase, counts, ctl);
+                     chunk_pre, cbase, ctl);
   return hipGetLastError();
 }
 
 hipError_t launch_bin(int pass, const SceneDesc* descs, int n_scenes, const uint32_t* chunk_pre,
-                      const uint32_t* cbase, BatchCtl* ctl, uint32_t* mat, uint32_t* pairs, uint64_t pairs_cap,
-                      int max_tiles, int grid, hipStream_t st) {
+                      const uint32_t* cbase, BatchCtl* ctl, uint32_t* places, uint32_t* rows, uint32_t* pairs,
+                      uint64_t pairs_cap, int max_tiles, int grid, hipStream_t st) {
   size_t lds = (size_t)max_tiles * 2 * sizeof(uint32_t);
   if (pass == 0)
-    hipLaunchKernelGGL(bin_kernel<0>, dim3(grid), dim3(256), lds, st, descs, n_scenes, chunk_pre, cbase, ctl, mat,
-                       pairs, pairs_cap);
+    hipLaunchKernelGGL(bin_kernel<0>, dim3(grid), dim3(256), lds, st, descs, n_scenes, chunk_pre, cbase, ctl, places,
+                       rows, pairs, pairs_cap);
   else
-    hipLaunchKernelGGL(bin_kernel<1>, dim3(grid), dim3(256), lds, st, descs, n_scenes, chunk_pre, cbase, ctl, mat,
-                       pairs, pairs_cap);
+    hipLaunchKernelGGL(bin_kernel<1>, dim3(grid), dim3(256), lds, st, descs, n_scenes, chunk_pre, cbase, ctl, places,
+                       rows, pairs, pairs_cap);
   return hipGetLastError();
 }
 
+uint64_t work_items_scratch_elems(int n_tiles_total) {
+  return n_tiles_total <= kPlanTiles ? 1 : scan_scratch_elems(2 * (uint64_t)n_tiles_total + 1);
+}
+
 hipError_t launch_work_items(const SceneDesc* descs, const uint32_t* tile_scene, int n_tiles_total,
-                             const uint32_t* chunk_pre, const uint32_t* cbase, const uint32_t* offsets,
-                             BatchCtl* ctl, uint32_t* tile_start, uint32_t* pieces,
-                             WorkItem* items, uint32_t items_cap, uint32_t* split_tiles,
-                             uint32_t split_cap, uint64_t pairs_cap, uint32_t min_piece, uint32_t max_piece,
-                             uint32_t grid, bool whole_images, hipStream_t st) {
-  // tile_start holds n_tiles_total + 1 tile starts, then the n_tiles_total tile_mid entries
-  int n = n_tiles_total + 1;
-  hipLaunchKernelGGL(tile_starts_kernel, dim3((n + 255) / 256), dim3(256), 0, st, descs, tile_scene, n_tiles_total,
-                     chunk_pre, cbase, offsets, ctl, tile_start, tile_start + n, pieces, pairs_cap, min_piece,
-                     max_piece, grid, whole_images ? 1u : 0u);
-  hipError_t e = hipGetLastError();
+                             const uint32_t* row_count, uint32_t* row_start, uint32_t* scan_scratch, BatchCtl* ctl,
+                             WorkItem* items, uint32_t items_cap, uint32_t* split_tiles, uint32_t split_cap,
+                             uint64_t pairs_cap, uint32_t min_piece, uint32_t max_piece, uint32_t grid,
+                             bool whole_images, hipStream_t st) {
+  const PlanLimits L{pairs_cap, items_cap, split_cap, min_piece, max_piece, grid, whole_images ? 1u : 0u};
+  const int n = n_tiles_total;
+  if (n <= kPlanTiles) {
+    hipLaunchKernelGGL(plan_items_kernel, dim3(1), dim3(1024), 0, st, descs, tile_scene, n, row_count, ctl, row_start,
+                       items, split_tiles, L);
+    return hipGetLastError();
+  }
+  hipError_t e = launch_scan_exclusive(row_count, row_start, 2 * (uint64_t)n + 1, scan_scratch, st, &ctl->total_pairs);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(write_items_kernel, dim3((n_tiles_total + 255) / 256), dim3(256), 0, st, descs, tile_scene,
-                     tile_start, pieces, n_tiles_total, ctl, items, items_cap, split_tiles, split_cap);
+  hipLaunchKernelGGL(tile_classes_kernel, dim3((n + 255) / 256), dim3(256), 0, st, n, row_start, ctl, L);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  hipLaunchKernelGGL(write_items_kernel, dim3((n + 255) / 256), dim3(256), 0, st, descs, tile_scene, row_start, n, ctl,
+                     items, split_tiles, L);
   return hipGetLastError();
 }
 
@@ -1561,10 +1672,10 @@ hipError_t launch_tile_accum(const SceneDesc* descs, const uint32_t* pairs, cons
   return hipGetLastError();
 }
 
-hipError_t launch_tile_merge(const SceneDesc* descs, const uint32_t* tile_scene, const uint32_t* tile_start,
+hipError_t launch_tile_merge(const SceneDesc* descs, const uint32_t* tile_scene, const uint32_t* row_start,
                              const uint32_t* split_tiles, const BatchCtl* ctl, unsigned long long* split_fx,
                              uint32_t split_cap, int grid, hipStream_t st) {
-  hipLaunchKernelGGL(tile_merge_kernel, dim3(grid), dim3(256), 0, st, descs, tile_scene, tile_start, split_tiles, ctl,
+  hipLaunchKernelGGL(tile_merge_kernel, dim3(grid), dim3(256), 0, st, descs, tile_scene, row_start, split_tiles, ctl,
                      split_fx, split_cap);
   return hipGetLastError();
 }

@@ -81,41 +81,31 @@ template <typename T>
 hipError_t launch_trace(const SceneDesc* descs, int n_scenes, uint32_t gen, uint32_t chunk, uint32_t launch_ix,
                         const uint32_t* item_pre, BatchCtl* ctl, uint32_t rpi, int cap_recs, int cap_objs,
                         int cap_verts, uint32_t* item_pre_next, int grid, hipStream_t stream);
-hipError_t launch_build_trace_items(const SceneDesc* descs, int n_scenes, uint32_t gen, uint32_t rpi,
-                                    uint32_t* item_pre, BatchCtl* ctl, hipStream_t stream);
 int trace_block();
 bool tile_size_supported(int tile);
-uint64_t scan_scratch_elems(uint64_t n);
-// n is a capacity; with n_used (a count in device memory, written by an earlier kernel of the
-// stream) only its first *n_used + 1 elements are touched. With total (zeroed by an earlier
-// kernel): *total += the 64-bit sum of the elements, or bit 63 set when 2048 consecutive
-// elements sum to 2^32 or more (the 32-bit offsets wrapped).
-hipError_t launch_scan_exclusive(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* scratch,
-                                 hipStream_t st, const uint32_t* n_used = nullptr,
-                                 unsigned long long* total = nullptr);
-hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t st, const uint32_t* n_used = nullptr);
-// Also zeroes counts[total entries], the end entry of the count matrix (the counting pass of
-// launch_bin writes every entry before it).
+hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t st);
 hipError_t launch_build_chunks(const SceneDesc* descs, int n_scenes, uint32_t chunk_min, uint32_t target,
-                               uint32_t groups, uint32_t* chunk_pre, uint32_t* cbase, uint32_t* counts,
-                               BatchCtl* ctl, hipStream_t st);
+                               uint32_t groups, uint32_t* chunk_pre, uint32_t* cbase, BatchCtl* ctl, hipStream_t st);
 // bin workgroups per compute unit (as many as the LDS allows run at once)
 constexpr uint32_t kBinWaves = 6;
+// rows: pass 0 the row totals (2 per tile, zeroed by the caller), pass 1 the rows' starts; places:
+// the [scene][chunk][tile][axis] matrix
 hipError_t launch_bin(int pass, const SceneDesc* descs, int n_scenes, const uint32_t* chunk_pre,
-                      const uint32_t* cbase, BatchCtl* ctl, uint32_t* mat, uint32_t* pairs, uint64_t pairs_cap,
-                      int max_tiles, int grid, hipStream_t st);
-// tile_start holds 2 * n_tiles_total + 1 entries: the tile starts (and the end), then each tile's
-// first x-major pair (tile_mid, which the work items carry).
+                      const uint32_t* cbase, BatchCtl* ctl, uint32_t* places, uint32_t* rows, uint32_t* pairs,
+                      uint64_t pairs_cap, int max_tiles, int grid, hipStream_t st);
+// row_count and row_start hold 2 * n_tiles_total + 1 entries (row_count's last is zero): per tile
+// its y-major and x-major pairs, and where they start; scan_scratch holds
+// work_items_scratch_elems(n_tiles_total) u32.
+uint64_t work_items_scratch_elems(int n_tiles_total);
 hipError_t launch_work_items(const SceneDesc* descs, const uint32_t* tile_scene, int n_tiles_total,
-                             const uint32_t* chunk_pre, const uint32_t* cbase, const uint32_t* offsets,
-                             BatchCtl* ctl, uint32_t* tile_start, uint32_t* pieces,
-                             WorkItem* items, uint32_t items_cap, uint32_t* split_tiles,
-                             uint32_t split_cap, uint64_t pairs_cap, uint32_t min_piece, uint32_t max_piece,
-                             uint32_t grid, bool whole_images, hipStream_t st);
+                             const uint32_t* row_count, uint32_t* row_start, uint32_t* scan_scratch, BatchCtl* ctl,
+                             WorkItem* items, uint32_t items_cap, uint32_t* split_tiles, uint32_t split_cap,
+                             uint64_t pairs_cap, uint32_t min_piece, uint32_t max_piece, uint32_t grid,
+                             bool whole_images, hipStream_t st);
 hipError_t launch_tile_accum(const SceneDesc* descs, const uint32_t* pairs, const WorkItem* items,
                              unsigned long long* split_fx, BatchCtl* ctl, int tile, bool packed_only, int block,
                              int n_cu, hipStream_t st);
-hipError_t launch_tile_merge(const SceneDesc* descs, const uint32_t* tile_scene, const uint32_t* tile_start,
+hipError_t launch_tile_merge(const SceneDesc* descs, const uint32_t* tile_scene, const uint32_t* row_start,
                              const uint32_t* split_tiles, const BatchCtl* ctl, unsigned long long* split_fx,
                              uint32_t split_cap, int grid, hipStream_t st);
 uint64_t merge_slot_u64();

@@ -286,7 +286,7 @@ struct BatchCtl {
   uint32_t n_chunks;
   uint32_t chunk;                  // segments per bin chunk (at least; see scene_chunk)
   uint32_t bin_groups;             // bin workgroups of the frame
-  uint32_t n_counts;               // entries of the [scene][tile][axis][chunk] count matrix
+  uint32_t spread;                 // segments per bin workgroup of the frame (see scene_chunk)
   uint32_t chunk_cursor[2];        // bin_count, bin_fill
   uint32_t piece;                  // pairs per work item
   unsigned long long total_pairs;

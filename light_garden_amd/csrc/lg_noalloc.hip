@@ -31,8 +31,9 @@ constexpr uint32_t kNaSplit = 128;          // tiles split over several work ite
 constexpr uint32_t kNaBinTarget = 128;      // bin chunks of one call
 constexpr uint32_t kNaChunkMin = 256;       // segments per bin chunk, at least
 constexpr uint32_t kNaMinPiece = 4096;      // smallest tile work item (bounds the item count)
-constexpr uint64_t kNaCounts = 2 * (uint64_t)kNaMaxTiles * (kNaBinTarget + 1) + 1;  // [tile][axis][chunk]
-constexpr uint64_t kNaScan = kNaCounts / 1024 + 64;  // >= scan_scratch_elems(kNaCounts)
+constexpr uint64_t kNaCounts = 2 * (uint64_t)kNaMaxTiles * (kNaBinTarget + 1);  // [chunk][tile][axis]
+constexpr uint64_t kNaRows = 2 * (uint64_t)kNaMaxTiles + 1;
+constexpr uint64_t kNaScan = 64;  // >= work_items_scratch_elems(kNaMaxTiles)
 constexpr uint64_t kNaItems = kNaMaxTiles + kNaPairs / kNaMinPiece + 1024;
 
 constexpr uint64_t na_align(uint64_t x) { return (x + 255) & ~uint64_t(255); }
@@ -42,12 +43,11 @@ constexpr uint64_t kOffCtl = na_align(kOffDesc + sizeof(SceneDesc));
 constexpr uint64_t kOffChunkPre = na_align(kOffCtl + sizeof(BatchCtl));
 constexpr uint64_t kOffCbase = na_align(kOffChunkPre + 2 * 4);
 constexpr uint64_t kOffCounts = na_align(kOffCbase + 2 * 4);
-constexpr uint64_t kOffOffsets = na_align(kOffCounts + kNaCounts * 4);
-constexpr uint64_t kOffScan = na_align(kOffOffsets + kNaCounts * 4);
+constexpr uint64_t kOffRowCount = na_align(kOffCounts + kNaCounts * 4);
+constexpr uint64_t kOffRowStart = na_align(kOffRowCount + kNaRows * 4);
+constexpr uint64_t kOffScan = na_align(kOffRowStart + kNaRows * 4);
 constexpr uint64_t kOffTileScene = na_align(kOffScan + kNaScan * 4);
-constexpr uint64_t kOffTileStart = na_align(kOffTileScene + (uint64_t)kNaMaxTiles * 4);
-constexpr uint64_t kOffPieces = na_align(kOffTileStart + (2 * (uint64_t)kNaMaxTiles + 1) * 4);
-constexpr uint64_t kOffSplitTiles = na_align(kOffPieces + (uint64_t)kNaMaxTiles * 4);
+constexpr uint64_t kOffSplitTiles = na_align(kOffTileScene + (uint64_t)kNaMaxTiles * 4);
 constexpr uint64_t kOffItems = na_align(kOffSplitTiles + (uint64_t)kNaSplit * 4);
 constexpr uint64_t kOffPairs = na_align(kOffItems + kNaItems * sizeof(WorkItem));
 constexpr uint64_t kOffSplitFx = na_align(kOffPairs + kNaPairs * 4);
@@ -134,7 +134,6 @@ int lg_accumulate_noalloc(lg_ctx* ctx, const lg_segments* segs, lg_image* img) {
   if (packed) D.flags |= SCENE_PACKED;
   const uint32_t min_piece = std::max(kNaMinPiece, std::min(ctx->tune.min_piece, kPackedPiece));
   const uint32_t max_piece = std::max(min_piece, std::min(ctx->tune.max_piece, kPackedPiece));
-  const uint64_t n_counts = 2 * (uint64_t)n_tiles * (kNaBinTarget + 1) + 1;
 
   unsigned char* b = static_cast<unsigned char*>(dev);
   SceneDesc* d_desc = reinterpret_cast<SceneDesc*>(b + kOffDesc);
@@ -142,11 +141,10 @@ int lg_accumulate_noalloc(lg_ctx* ctx, const lg_segments* segs, lg_image* img) {
   uint32_t* chunk_pre = reinterpret_cast<uint32_t*>(b + kOffChunkPre);
   uint32_t* cbase = reinterpret_cast<uint32_t*>(b + kOffCbase);
   uint32_t* counts = reinterpret_cast<uint32_t*>(b + kOffCounts);
-  uint32_t* offsets = reinterpret_cast<uint32_t*>(b + kOffOffsets);
+  uint32_t* row_count = reinterpret_cast<uint32_t*>(b + kOffRowCount);
+  uint32_t* row_start = reinterpret_cast<uint32_t*>(b + kOffRowStart);
   uint32_t* scan = reinterpret_cast<uint32_t*>(b + kOffScan);
   uint32_t* tile_scene = reinterpret_cast<uint32_t*>(b + kOffTileScene);
-  uint32_t* tile_start = reinterpret_cast<uint32_t*>(b + kOffTileStart);
-  uint32_t* pieces = reinterpret_cast<uint32_t*>(b + kOffPieces);
   uint32_t* split_tiles = reinterpret_cast<uint32_t*>(b + kOffSplitTiles);
   WorkItem* items = reinterpret_cast<WorkItem*>(b + kOffItems);
   uint32_t* pairs = reinterpret_cast<uint32_t*>(b + kOffPairs);
@@ -160,18 +158,16 @@ int lg_accumulate_noalloc(lg_ctx* ctx, const lg_segments* segs, lg_image* img) {
     LG_HIP(hipGetLastError());
     LG_HIP(launch_fill_u32(reinterpret_cast<uint32_t*>(d_ctl), sizeof(BatchCtl) / 4, 0u, st));
     LG_HIP(launch_fill_u32(tile_scene, (uint64_t)n_tiles, 0u, st));
+    LG_HIP(launch_fill_u32(row_count, 2 * (uint64_t)n_tiles + 1, 0u, st));
     const int bin_grid = ctx->n_cu * (int)kBinWaves;
-    LG_HIP(launch_build_chunks(d_desc, 1, kNaChunkMin, kNaBinTarget, (uint32_t)bin_grid, chunk_pre, cbase, counts,
-                               d_ctl, st));
-    LG_HIP(launch_bin(0, d_desc, 1, chunk_pre, cbase, d_ctl, counts, nullptr, 0, n_tiles, bin_grid, st));
-    LG_HIP(launch_scan_exclusive(counts, offsets, n_counts, scan, st, &d_ctl->n_counts, &d_ctl->total_pairs));
-    LG_HIP(launch_work_items(d_desc, tile_scene, n_tiles, chunk_pre, cbase, offsets, d_ctl, tile_start, pieces, items,
-                             (uint32_t)kNaItems, split_tiles, kNaSplit, kNaPairs, min_piece, max_piece,
-                             (uint32_t)ctx->n_cu, false, st));
-    LG_HIP(launch_bin(1, d_desc, 1, chunk_pre, cbase, d_ctl, offsets, pairs, kNaPairs, n_tiles, bin_grid, st));
+    LG_HIP(launch_build_chunks(d_desc, 1, kNaChunkMin, kNaBinTarget, (uint32_t)bin_grid, chunk_pre, cbase, d_ctl, st));
+    LG_HIP(launch_bin(0, d_desc, 1, chunk_pre, cbase, d_ctl, counts, row_count, nullptr, 0, n_tiles, bin_grid, st));
+    LG_HIP(launch_work_items(d_desc, tile_scene, n_tiles, row_count, row_start, scan, d_ctl, items, (uint32_t)kNaItems,
+                             split_tiles, kNaSplit, kNaPairs, min_piece, max_piece, (uint32_t)ctx->n_cu, false, st));
+    LG_HIP(launch_bin(1, d_desc, 1, chunk_pre, cbase, d_ctl, counts, row_start, pairs, kNaPairs, n_tiles, bin_grid, st));
     LG_HIP(launch_tile_accum(d_desc, pairs, items, split_fx, d_ctl,
                              tile, packed, (int)ctx->tune.tile_block, ctx->n_cu, st));
-    LG_HIP(launch_tile_merge(d_desc, tile_scene, tile_start, split_tiles, d_ctl, split_fx, kNaSplit, ctx->n_cu, st));
+    LG_HIP(launch_tile_merge(d_desc, tile_scene, row_start, split_tiles, d_ctl, split_fx, kNaSplit, ctx->n_cu, st));
     LG_HIP(hipMemcpyAsync(&hc, d_ctl, sizeof(BatchCtl), hipMemcpyDeviceToHost, st));
     LG_HIP(hipStreamSynchronize(st));
   }

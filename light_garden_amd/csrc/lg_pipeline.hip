@@ -40,21 +40,35 @@ struct DevView {
   }
 };
 
-// Bytes of a frame's tile-to-scene table in frame_in (16-byte multiple: px_pre follows).
-static size_t tile_scene_bytes(int n_tiles) { return ((size_t)n_tiles * 4 + 15) & ~size_t(15); }
+// Byte offsets of a frame's parts in frame_in and stage_in, each a multiple of 16.
+struct FrameLayout {
+  size_t tile_scene, px_pre, item_pre0, counters, ctl, row_count, total;
+  FrameLayout(int n, int n_tiles) {
+    auto up = [](size_t b) { return (b + 15) & ~size_t(15); };
+    tile_scene = up((size_t)n * sizeof(SceneDesc));
+    px_pre = tile_scene + up((size_t)n_tiles * 4);
+    item_pre0 = px_pre + up((size_t)n * 8);
+    counters = item_pre0 + up((size_t)(n + 1) * 4);
+    ctl = counters + (size_t)n * kCounterStride;
+    row_count = ctl + up(sizeof(BatchCtl));
+    total = row_count + up((size_t)(2 * n_tiles + 1) * 4);
+  }
+  size_t out_bytes() const { return row_count - counters; }
+};
 
 struct Pipeline {
-  // One allocation per direction, so that a frame uploads and reads back with one copy each:
-  // frame_in = descs | tile_scene | px_pre (the layout of stage_in), frame_out = counters | ctl.
-  DevBuf frame_in, frame_out;
-  DevView descs, tile_scene, px_pre, counters, ctl;
-  DevBuf item_pre, chunk_pre, cbase, counts, offsets, scan_scratch;
-  DevBuf tile_start, pieces, pairs, items;
+  // One allocation that a frame uploads with one copy: descs | tile_scene | px_pre | item_pre0 |
+  // counters | ctl | row_count (FrameLayout; the layout of stage_in, whose counters, control block
+  // and row totals are the frame's zeros). One copy reads counters | ctl back.
+  DevBuf frame_in;
+  DevView descs, tile_scene, px_pre, item_pre0, counters, ctl, row_count;
+  DevBuf item_pre, chunk_pre, cbase, places, row_start, scan_scratch;
+  DevBuf pairs, items;
   DevBuf split_tiles, split_fx;  // merge slots of tiles split over several items
   uint64_t pairs_cap = 1u << 20;
   uint32_t items_cap = 0;
   uint32_t split_cap = 0, split_min = 0;
-  PinnedBuf stage_in;   // descs | tile_scene | px_pre
+  PinnedBuf stage_in;   // as frame_in
   PinnedBuf stage_out;  // counters | ctl
   // Captured frames keyed on their shape (sizes, knobs and every buffer address they bake
   // in), least recently used evicted first.
@@ -112,7 +126,7 @@ struct Layout {
   int n_tiles = 0, max_tiles = 0;
   int tile = 64;                     // screen tile edge of the frame
   bool packed_only = false;          // every accumulated scene keeps two channels per LDS word
-  uint64_t n_counts = 0, n_px = 0;  // n_counts: capacity of the per-frame bin count matrix
+  uint64_t n_counts = 0, n_px = 0;  // n_counts: capacity of the per-frame [chunk][tile][axis] matrix
   uint32_t bin_target = 0;           // bin chunks per frame
   std::vector<int> tile_base;
   std::vector<uint64_t> px_base;
@@ -133,10 +147,8 @@ static int enqueue(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, const
   const bool whole = whole_images(stages);
   SceneDesc* d_descs = P.descs.as<SceneDesc>();
   BatchCtl* d_ctl = P.ctl.as<BatchCtl>();
-  const size_t in_bytes = n * sizeof(SceneDesc) + tile_scene_bytes(L.n_tiles) + (size_t)n * 8;
-  const size_t out_bytes = n * kCounterStride + sizeof(BatchCtl);
-  LG_HIP(hipMemcpyAsync(P.frame_in.p, P.stage_in.p, in_bytes, hipMemcpyHostToDevice, st));
-  LG_HIP(launch_fill_u32(P.frame_out.as<uint32_t>(), out_bytes / 4, 0u, st));  // counters and ctl
+  const FrameLayout F(n, L.n_tiles);
+  LG_HIP(hipMemcpyAsync(P.frame_in.p, P.stage_in.p, F.total, hipMemcpyHostToDevice, st));
   if ((stages & ST_CLEAR) && !whole) {
     Scope s(ctx, profile, "clear", L.n_px);
     LG_HIP(launch_pixels(0, d_descs, P.px_pre.as<uint64_t>(), n, L.n_px, st));
@@ -144,13 +156,13 @@ static int enqueue(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, const
   if (stages & ST_TRACE) {
     Scope s(ctx, profile, L.fp64 ? "trace_fp64" : "trace", L.max_bounce);
     const int grid = ctx->n_cu * (int)ctx->tune.trace_waves;
-    // generation 0's work list by its own launch; each later one by the last workgroup of the
-    // previous generation's trace
-    LG_HIP(launch_build_trace_items(d_descs, n, 0, ctx->tune.rays_per_item, P.item_pre.as<uint32_t>(), d_ctl, st));
+    // generation 0's work list comes with the frame's upload; each later one is built by the last
+    // workgroup of the previous launch
     uint32_t li = 0;  // launch index: `chunk` generations per launch
     for (uint32_t g = 0; g < L.max_bounce; g += L.chunk, li++) {
-      uint32_t* pre = P.item_pre.as<uint32_t>() + (size_t)li * (n + 1);
-      uint32_t* next = g + L.chunk < L.max_bounce ? pre + (n + 1) : nullptr;
+      uint32_t* const next_pre = P.item_pre.as<uint32_t>() + (size_t)li * (n + 1);
+      const uint32_t* pre = li ? next_pre - (n + 1) : P.item_pre0.as<uint32_t>();
+      uint32_t* next = g + L.chunk < L.max_bounce ? next_pre : nullptr;
       if (L.fp64)
         LG_HIP(launch_trace<double>(d_descs, n, g, L.chunk, li, pre, d_ctl, ctx->tune.rays_per_item, L.cap_recs,
                                     L.cap_objs, L.cap_verts, next, grid, st));
@@ -164,25 +176,23 @@ static int enqueue(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, const
     {
       Scope s(ctx, profile, "bin_count", 0);
       LG_HIP(launch_build_chunks(d_descs, n, kChunkMin, L.bin_target, (uint32_t)grid, P.chunk_pre.as<uint32_t>(),
-                                 P.cbase.as<uint32_t>(), P.counts.as<uint32_t>(), d_ctl, st));
+                                 P.cbase.as<uint32_t>(), d_ctl, st));
       LG_HIP(launch_bin(0, d_descs, n, P.chunk_pre.as<uint32_t>(), P.cbase.as<uint32_t>(), d_ctl,
-                        P.counts.as<uint32_t>(), nullptr, 0, L.max_tiles, grid, st));
+                        P.places.as<uint32_t>(), P.row_count.as<uint32_t>(), nullptr, 0, L.max_tiles, grid, st));
     }
     {
-      Scope s(ctx, profile, "bin_scan", L.n_counts);
-      LG_HIP(launch_scan_exclusive(P.counts.as<uint32_t>(), P.offsets.as<uint32_t>(), L.n_counts,
-                                   P.scan_scratch.as<uint32_t>(), st, &d_ctl->n_counts, &d_ctl->total_pairs));
-      LG_HIP(launch_work_items(d_descs, P.tile_scene.as<uint32_t>(), L.n_tiles, P.chunk_pre.as<uint32_t>(),
-                               P.cbase.as<uint32_t>(), P.offsets.as<uint32_t>(), d_ctl,
-                               P.tile_start.as<uint32_t>(), P.pieces.as<uint32_t>(), P.items.as<WorkItem>(),
-                               P.items_cap, P.split_tiles.as<uint32_t>(), P.split_cap,
+      Scope s(ctx, profile, "bin_scan", 2 * (uint64_t)L.n_tiles);
+      LG_HIP(launch_work_items(d_descs, P.tile_scene.as<uint32_t>(), L.n_tiles, P.row_count.as<uint32_t>(),
+                               P.row_start.as<uint32_t>(), P.scan_scratch.as<uint32_t>(), d_ctl,
+                               P.items.as<WorkItem>(), P.items_cap, P.split_tiles.as<uint32_t>(), P.split_cap,
                                P.pairs_cap, std::min(ctx->tune.min_piece, kPackedPiece),
                                std::min(ctx->tune.max_piece, kPackedPiece), (uint32_t)ctx->n_cu, whole, st));
     }
     {
       Scope s(ctx, profile, "bin_fill", 0);
       LG_HIP(launch_bin(1, d_descs, n, P.chunk_pre.as<uint32_t>(), P.cbase.as<uint32_t>(), d_ctl,
-                        P.offsets.as<uint32_t>(), P.pairs.as<uint32_t>(), P.pairs_cap, L.max_tiles, grid, st));
+                        P.places.as<uint32_t>(), P.row_start.as<uint32_t>(), P.pairs.as<uint32_t>(), P.pairs_cap,
+                        L.max_tiles, grid, st));
     }
     {
       Scope s(ctx, profile, "tile_accum", 0);
@@ -192,7 +202,7 @@ static int enqueue(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, const
     }
     {
       Scope s(ctx, profile, "tile_merge", 0);
-      LG_HIP(launch_tile_merge(d_descs, P.tile_scene.as<uint32_t>(), P.tile_start.as<uint32_t>(),
+      LG_HIP(launch_tile_merge(d_descs, P.tile_scene.as<uint32_t>(), P.row_start.as<uint32_t>(),
                                P.split_tiles.as<uint32_t>(), d_ctl, P.split_fx.as<unsigned long long>(), P.split_cap,
                                ctx->n_cu, st));
     }
@@ -201,7 +211,7 @@ static int enqueue(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, const
     Scope s(ctx, profile, "resolve", L.n_px);
     LG_HIP(launch_pixels(1, d_descs, P.px_pre.as<uint64_t>(), n, L.n_px, st));
   }
-  LG_HIP(hipMemcpyAsync(P.stage_out.p, P.frame_out.p, out_bytes, hipMemcpyDeviceToHost, st));
+  LG_HIP(hipMemcpyAsync(P.stage_out.p, P.counters.p, F.out_bytes(), hipMemcpyDeviceToHost, st));
   return LG_OK;
 }
 
@@ -320,9 +330,8 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
     L.bin_target = (uint32_t)std::max<uint64_t>(t, 2 * groups);
   }
   // chunks hold at least total / bin_target segments, so a scene has at most
-  // n_s * bin_target / total + 1 of them and the batch fewer than bin_target + n; the matrix
-  // has one more entry so that offsets[count] (the end) is always inside it
-  if (accum) L.n_counts = 2 * (uint64_t)L.max_tiles * (L.bin_target + (uint64_t)n) + 1;
+  // n_s * bin_target / total + 1 of them and the batch fewer than bin_target + n
+  if (accum) L.n_counts = 2 * (uint64_t)L.max_tiles * (L.bin_target + (uint64_t)n);
   if (L.n_counts > 0xffffffffull) return fail(LG_E_UNSUPPORTED, "batch too large for one frame");
   // ---- scratch ----
   // pieces hold at least min_piece pairs, so a frame without pair overflow has fewer than
@@ -330,26 +339,24 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
   const uint32_t items_need =
       (uint32_t)std::min<uint64_t>(0xffffffffull, (uint64_t)L.n_tiles + P.pairs_cap / ctx->tune.min_piece + 1024);
   P.items_cap = std::max(P.items_cap, items_need);
+  const FrameLayout F(n, L.n_tiles);
   {
-    const size_t desc_bytes = n * sizeof(SceneDesc), tile_bytes = tile_scene_bytes(L.n_tiles);
-    if ((rc = P.frame_in.ensure(desc_bytes + tile_bytes + (size_t)n * 8))) return rc;
-    if ((rc = P.frame_out.ensure(n * kCounterStride + sizeof(BatchCtl)))) return rc;
+    if ((rc = P.frame_in.ensure(F.total))) return rc;
     char* fi = P.frame_in.as<char>();
     P.descs.p = fi;
-    P.tile_scene.p = fi + desc_bytes;
-    P.px_pre.p = fi + desc_bytes + tile_bytes;
-    P.counters.p = P.frame_out.p;
-    P.ctl.p = P.frame_out.as<char>() + n * kCounterStride;
+    P.tile_scene.p = fi + F.tile_scene;
+    P.px_pre.p = fi + F.px_pre;
+    P.item_pre0.p = fi + F.item_pre0;
+    P.counters.p = fi + F.counters;
+    P.ctl.p = fi + F.ctl;
+    P.row_count.p = fi + F.row_count;
   }
   if ((rc = P.item_pre.ensure((size_t)kMaxGen * (n + 1) * 4))) return rc;
   if ((rc = P.chunk_pre.ensure((size_t)(n + 1) * 4))) return rc;
   if ((rc = P.cbase.ensure((size_t)(n + 1) * 4))) return rc;
-  if ((rc = P.counts.ensure(std::max<uint64_t>(L.n_counts, 1) * 4))) return rc;
-  if ((rc = P.offsets.ensure(std::max<uint64_t>(L.n_counts, 1) * 4))) return rc;
-  uint64_t ss = scan_scratch_elems(L.n_counts);
-  if ((rc = P.scan_scratch.ensure(ss * 4))) return rc;
-  if ((rc = P.tile_start.ensure((size_t)(2 * L.n_tiles + 1) * 4))) return rc;
-  if ((rc = P.pieces.ensure((size_t)std::max(L.n_tiles, 1) * 4))) return rc;
+  if ((rc = P.places.ensure(std::max<uint64_t>(L.n_counts, 1) * 4))) return rc;
+  if ((rc = P.scan_scratch.ensure(work_items_scratch_elems(L.n_tiles) * 4))) return rc;
+  if ((rc = P.row_start.ensure((size_t)(2 * L.n_tiles + 1) * 4))) return rc;
   if ((rc = P.pairs.ensure(P.pairs_cap * 4))) return rc;
   if ((rc = P.items.ensure((size_t)P.items_cap * sizeof(WorkItem)))) return rc;
   {
@@ -365,15 +372,17 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
       LG_HIP(hipStreamSynchronize(st));
     }
   }
-  const size_t desc_bytes = n * sizeof(SceneDesc), tile_bytes = tile_scene_bytes(L.n_tiles);
-  if ((rc = P.stage_in.ensure(desc_bytes + tile_bytes + (size_t)n * 8))) return rc;
-  if ((rc = P.stage_out.ensure(n * kCounterStride + sizeof(BatchCtl)))) return rc;
+  if ((rc = P.stage_in.ensure(F.total))) return rc;
+  if ((rc = P.stage_out.ensure(F.out_bytes()))) return rc;
   // ---- descriptors ----
   L.packed_only = accum;
   char* in = P.stage_in.as<char>();
   SceneDesc* hd = reinterpret_cast<SceneDesc*>(in);
-  uint32_t* h_tile_scene = reinterpret_cast<uint32_t*>(in + desc_bytes);
-  uint64_t* h_px = reinterpret_cast<uint64_t*>(in + desc_bytes + tile_bytes);
+  uint32_t* h_tile_scene = reinterpret_cast<uint32_t*>(in + F.tile_scene);
+  uint64_t* h_px = reinterpret_cast<uint64_t*>(in + F.px_pre);
+  uint32_t* h_pre = reinterpret_cast<uint32_t*>(in + F.item_pre0);
+  std::memset(in + F.counters, 0, F.total - F.counters);
+  h_pre[0] = 0;
   for (int i = 0; i < n; i++) {
     const Entry& e = E[i];
     SceneDesc& D = hd[i];
@@ -403,6 +412,9 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
       D.n_verts = sc->n_verts;
       D.n_lights = (int32_t)sc->lights.size();
       D.n_primary = sc->n_primary;
+      // trace items of the first launch
+      const uint64_t rpi = ctx->tune.rays_per_item;
+      h_pre[i + 1] = h_pre[i] + (e.params.max_bounce ? (uint32_t)((sc->n_primary + rpi - 1) / rpi) : 0u);
       D.max_bounce = e.params.max_bounce;
       for (int c = 0; c < 4; c++) D.cutoff[c] = e.params.cutoff_color[c];
       for (int c = 0; c < 4; c++) D.canvas[c] = e.params.canvas[c];
@@ -452,6 +464,7 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
       for (int k = 0; k < t; k++) h_tile_scene[L.tile_base[i] + k] = (uint32_t)i;
     }
   }
+  if (trace) reinterpret_cast<BatchCtl*>(in + F.ctl)->n_items_gen[0] = h_pre[n];
   // ---- launch (graph replay when the shape is unchanged) ----
   std::vector<uint64_t> shape = {(uint64_t)n, stages, L.fp64, L.max_bounce, (uint64_t)L.cap_recs,
                                  (uint64_t)L.cap_objs, (uint64_t)L.cap_verts, (uint64_t)L.n_tiles,
@@ -459,8 +472,8 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
                                  P.split_cap, ctx->tune.rays_per_item, ctx->tune.min_piece, ctx->tune.max_piece,
                                  ctx->tune.trace_waves, ctx->tune.bvh_min_objects,
                                  (uint64_t)L.tile, (uint64_t)L.packed_only, L.chunk, ctx->tune.tile_block};
-  for (DevBuf* b : {&P.frame_in, &P.frame_out, &P.item_pre, &P.chunk_pre, &P.cbase, &P.counts, &P.offsets,
-                    &P.scan_scratch, &P.tile_start, &P.pieces, &P.pairs, &P.items, &P.split_tiles, &P.split_fx})
+  for (DevBuf* b : {&P.frame_in, &P.item_pre, &P.chunk_pre, &P.cbase, &P.places, &P.scan_scratch, &P.row_start,
+                    &P.pairs, &P.items, &P.split_tiles, &P.split_fx})
     shape.push_back((uint64_t)b->p);
   shape.push_back((uint64_t)P.stage_in.p);
   shape.push_back((uint64_t)P.stage_out.p);
@@ -671,9 +684,8 @@ const std::vector<Entry>& frame_job_entries(const FrameJob* j) { return j->B.E; 
 size_t frame_job_scratch_bytes(const FrameJob* j) {
   const Pipeline& P = j->P;
   size_t b = 0;
-  for (const DevBuf* d : {&P.frame_in, &P.frame_out, &P.item_pre, &P.chunk_pre, &P.cbase, &P.counts, &P.offsets,
-                          &P.scan_scratch, &P.tile_start, &P.pieces, &P.pairs, &P.items,
-                          &P.split_tiles, &P.split_fx})
+  for (const DevBuf* d : {&P.frame_in, &P.item_pre, &P.chunk_pre, &P.cbase, &P.places, &P.scan_scratch, &P.row_start,
+                          &P.pairs, &P.items, &P.split_tiles, &P.split_fx})
     b += d->bytes;
   return b;
 }

@@ -1042,11 +1042,11 @@ __device__ __forceinline__ int find_scene(const uint32_t* pre, int n, uint32_t x
   return lo;
 }
 
-// item_pre[s] = first item of scene s for generation `gen_ix`; item_pre[n] = total, run by
-// one workgroup of BLOCK threads. COHERENT: the previous generation's child counts were
-// written by other workgroups of the running kernel, so they are read with device-scope
-// atomic loads (not through this CU's cache).
-template <int BLOCK, bool COHERENT>
+// item_pre[s] = first item of scene s for generation `gen_ix` > 0; item_pre[n] = total, run by
+// one workgroup of BLOCK threads (generation 0's comes from the host, which knows the primary
+// rays). The previous generation's child counts were written by other workgroups of the running
+// kernel, so they are read with device-scope atomic loads (not through this CU's cache).
+template <int BLOCK>
 __device__ __forceinline__ void build_items_block(const SceneDesc* __restrict__ descs, int n_scenes,
                                                   uint32_t gen_ix, uint32_t rpi, uint32_t* item_pre,
                                                   BatchCtl* ctl) {
@@ -1061,14 +1061,9 @@ __device__ __forceinline__ void build_items_block(const SceneDesc* __restrict__ 
     if (sid < n_scenes) {
       const SceneDesc& D = descs[sid];
       if (gen_ix < D.max_bounce) {
-        uint64_t c;
-        if (COHERENT && gen_ix > 0) {
-          const uint32_t g = __hip_atomic_load(gen(D.gen_count) + gen_ix - 1, __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_AGENT);
-          c = g < D.q_cap ? g : D.q_cap;
-        } else {
-          c = gen_input_count(D, gen_ix);
-        }
+        const uint32_t g = __hip_atomic_load(gen(D.gen_count) + gen_ix - 1, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+        const uint64_t c = g < D.q_cap ? g : D.q_cap;
         n_it = (uint32_t)((c + rpi - 1) / rpi);
       }
     }
@@ -1428,15 +1423,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
     __syncthreads();
     if (s_last) {
       __threadfence();
-      build_items_block<BLOCK, true>(descs, n_scenes, gen_ix + chunk, rpi, item_pre_next, ctl);
+      build_items_block<BLOCK>(descs, n_scenes, gen_ix + chunk, rpi, item_pre_next, ctl);
     }
   }
-}
-
-__global__ __launch_bounds__(1024) void build_trace_items_kernel(const SceneDesc* __restrict__ descs,
-                                                                 int n_scenes, uint32_t gen_ix, uint32_t rpi,
-                                                                 uint32_t* item_pre, BatchCtl* ctl) {
-  build_items_block<1024, false>(descs, n_scenes, gen_ix, rpi, item_pre, ctl);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1461,13 +1450,6 @@ hipError_t launch_trace(const SceneDesc* descs, int n_scenes, uint32_t gen, uint
   hipLaunchKernelGGL((trace_kernel<T, kTraceBlock>), dim3(grid), dim3(kTraceBlock), lds, stream, descs,
                      n_scenes, gen, chunk, launch_ix, item_pre, ctl, rpi, cap_recs, cap_objs, cap_verts,
                      item_pre_next);
-  return hipGetLastError();
-}
-
-hipError_t launch_build_trace_items(const SceneDesc* descs, int n_scenes, uint32_t gen, uint32_t rpi,
-                                    uint32_t* item_pre, BatchCtl* ctl, hipStream_t stream) {
-  hipLaunchKernelGGL(build_trace_items_kernel, dim3(1), dim3(1024), 0, stream, descs, n_scenes, gen, rpi,
-                     item_pre, ctl);
   return hipGetLastError();
 }
 
