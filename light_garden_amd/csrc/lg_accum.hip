@@ -815,43 +815,36 @@ __device__ __forceinline__ uint32_t packed_pairs(const uint32_t* row_start, uint
   return nt < kPackedPiece ? nt : kPackedPiece;
 }
 
-// Packed channel values travel as the bits of the float 2^23 + cq (exact: cq <= 2^22 < 2^23),
-// which are kMagicBits + cq: one FMA against 2^23 rounds a product to an integer and leaves
-// that integer in the low bits, so the deposits need no float-to-integer conversions.
+// One packed channel value of a sample: cq = round(max(v, 0) * 2^G), the low bits of one FMA against
+// 2^23 (round to nearest even; cq <= 2^22 leaves the exponent alone; a NaN deposits nothing).
 constexpr float kMagic = 8388608.0f;  // 2^23
-constexpr uint32_t kMagicBits = 0x4B000000u;
-constexpr uint64_t kNegMagic2 = 0ull - ((uint64_t)kMagicBits << 32 | kMagicBits);
+__device__ __forceinline__ uint32_t pack_q(float v, float scale) {
+  return __builtin_bit_cast(uint32_t, __builtin_fmaf(__builtin_fmaxf(v, 0.0f), scale, kMagic)) & 0x7FFFFFu;
+}
 
-// One packed channel value of a sample as kMagicBits + round(max(v, 0) * 2^G) (the FMA's
-// round-to-nearest-even; a NaN deposits nothing).
-__device__ __forceinline__ uint32_t pack_qm(float v, float scale) {
-  return __builtin_bit_cast(uint32_t, __builtin_fmaf(__builtin_fmaxf(v, 0.0f), scale, kMagic));
+// round(f * q) for 0 <= f < 1 and an integer q < 2^23, as one multiplication: the integer's bits
+// are the denormal float q * 2^-149, whose product with f rounds (to nearest even) to a multiple
+// of 2^-149, so its bits are the rounded integer. Never more than q.
+__device__ __forceinline__ uint32_t mul_frac(float f, uint32_t q) {
+  return __builtin_bit_cast(uint32_t, f * __builtin_bit_cast(float, q));
 }
 
 // The two-channel deposits of one sample at minor position m (fraction fr = m - floor(m))
-// into t (pixel jl of planes 0 and 1) and t + T (pixel jl + 1), channel values qm0..qm3 from
-// pack_qm. Pixel jl takes l = round((1 - fr) cq), as x = fma(1 - fr, 2^23 + cq, fr 2^23) =
-// 2^23 + (1 - fr) cq rounded to an integer: fr 2^23 is exact, and 1 - fr is exact or within
-// 2^-25 of it, which moves x by at most (2^23 + cq) 2^-25 < 1/2, so 0 <= l <= cq (x stays in
-// [2^23, 2^23 + cq]). Pixel jl + 1 takes cq - l = (2^23 + cq) - x in the integer bits; the two
-// deposits always add up to exactly cq.
+// into t (pixel jl of planes 0 and 1) and t + T (pixel jl + 1), channel values q0..q3 from
+// pack_q. Pixel jl + 1 takes r = round(fr q) and pixel jl the rest, q - r: the two deposits
+// always add up to exactly q, at one multiplication and one subtraction per channel (the form
+// before, an FMA against 2^23 and the subtractions of its exponent bits, took 14 instructions
+// for four channels and the weights where this takes 8; tile walk, us: 1M-ray frame 950 -> 915,
+// 1.6M segments at 4096x4096 4440 -> 4330; what binds it is the LDS, see the stream walk).
 template <int T, int STRIDE>
-__device__ __forceinline__ void deposit2(unsigned long long* t, float m, uint32_t qm0, uint32_t qm1, uint32_t qm2,
-                                         uint32_t qm3) {
+__device__ __forceinline__ void deposit2(unsigned long long* t, float m, uint32_t q0, uint32_t q1, uint32_t q2,
+                                         uint32_t q3) {
   const float fr = __builtin_amdgcn_fractf(m);
-  const float w = 1.0f - fr;
-  const float frm = fr * kMagic;
-  const uint32_t x0 = __builtin_bit_cast(uint32_t, __builtin_fmaf(w, __builtin_bit_cast(float, qm0), frm));
-  const uint32_t x1 = __builtin_bit_cast(uint32_t, __builtin_fmaf(w, __builtin_bit_cast(float, qm1), frm));
-  const uint32_t x2 = __builtin_bit_cast(uint32_t, __builtin_fmaf(w, __builtin_bit_cast(float, qm2), frm));
-  const uint32_t x3 = __builtin_bit_cast(uint32_t, __builtin_fmaf(w, __builtin_bit_cast(float, qm3), frm));
-  const uint64_t x01 = (uint64_t)x1 << 32 | x0, x23 = (uint64_t)x3 << 32 | x2;
-  // the fields of pixel jl + 1 as four 32-bit subtractions (no carry chain between them)
-  const uint64_t r01 = (uint64_t)(qm1 - x1) << 32 | (qm0 - x0), r23 = (uint64_t)(qm3 - x3) << 32 | (qm2 - x2);
-  atomicAdd(t, (unsigned long long)(x01 + kNegMagic2));
-  atomicAdd(t + STRIDE, (unsigned long long)(x23 + kNegMagic2));
-  atomicAdd(t + T, (unsigned long long)r01);
-  atomicAdd(t + T + STRIDE, (unsigned long long)r23);
+  const uint32_t r0 = mul_frac(fr, q0), r1 = mul_frac(fr, q1), r2 = mul_frac(fr, q2), r3 = mul_frac(fr, q3);
+  atomicAdd(t, (unsigned long long)(q1 - r1) << 32 | (q0 - r0));
+  atomicAdd(t + STRIDE, (unsigned long long)(q3 - r3) << 32 | (q2 - r2));
+  atomicAdd(t + T, (unsigned long long)r1 << 32 | r0);
+  atomicAdd(t + T + STRIDE, (unsigned long long)r3 << 32 | r2);
 }
 
 // The value one sample of colour channel c adds per unit weight: +-c * factor (BlendCode).
@@ -1128,10 +1121,10 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               s_first = (float)(u0 * g.inv_dM);
               ds = (float)g.inv_dM;
               if (two_ch) {
-                cq0 = (int)pack_qm(blend_value(bc0, ca.x, ca.w, bk0), cs0);
-                cq1 = (int)pack_qm(blend_value(bc1, ca.y, ca.w, bk1), cs1);
-                cq2 = (int)pack_qm(blend_value(bc2, ca.z, ca.w, bk2), cs2);
-                cq3 = (int)pack_qm(blend_value(bc3, ca.w, ca.w, bk3), cs3);
+                cq0 = (int)pack_q(blend_value(bc0, ca.x, ca.w, bk0), cs0);
+                cq1 = (int)pack_q(blend_value(bc1, ca.y, ca.w, bk1), cs1);
+                cq2 = (int)pack_q(blend_value(bc2, ca.z, ca.w, bk2), cs2);
+                cq3 = (int)pack_q(blend_value(bc3, ca.w, ca.w, bk3), cs3);
               } else {
                 cq0 = fx(blend_value(bc0, ca.x, ca.w, bk0), cs0);
                 cq1 = fx(blend_value(bc1, ca.y, ca.w, bk1), cs1);
@@ -1153,7 +1146,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
           // Sample stream: the c-th lane with samples owns positions pre_c .. pre_c + n_c - 1 of
           // the wave's stream (pre: exclusive prefix sum of n), and position k is column k +
           // q0_c - pre_c of the tile. Record c = {q0_c - pre_c, m_first, slope, 8 (q0_c - pre_c)},
-          // {qm0..qm3} (the column offset, and in bytes for the deposit address);
+          // {q0..q3} (the column offset, and in bytes for the deposit address);
           // record P (after the last pair) is empty (zero deposits in row 0), so the positions
           // past the end of the stream need no mask. Stream word i holds a bit per position
           // 64 i .. 64 i + 63 that starts a record; lane l of step s finds its record as the
@@ -1183,7 +1176,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             }
             if (lane == 0) {
               rec[2 * n_live] = make_uint4((uint32_t)(-total), 0u, 0u, (uint32_t)(-total * 8));
-              rec[2 * n_live + 1] = make_uint4(kMagicBits, kMagicBits, kMagicBits, kMagicBits);
+              rec[2 * n_live + 1] = make_uint4(0u, 0u, 0u, 0u);
               if (total & 63) atomicOr(&mask[total >> 6], 1ull << (total & 63));
             }
             // lane i keeps stream word i in registers; a step takes its word with a lane read
@@ -1304,10 +1297,10 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               const float d0 = bcast_f(dc.x, j), d1 = bcast_f(dc.y, j), d2 = bcast_f(dc.z, j), d3 = bcast_f(dc.w, j);
               const float sp = __builtin_fmaf(lane_f, jds, jsa);
               const float al = __builtin_fmaf(sp, d3, a3);
-              q0 = pack_qm(blend_value(bc0, __builtin_fmaf(sp, d0, a0), al, bk0), cs0);
-              q1 = pack_qm(blend_value(bc1, __builtin_fmaf(sp, d1, a1), al, bk1), cs1);
-              q2 = pack_qm(blend_value(bc2, __builtin_fmaf(sp, d2, a2), al, bk2), cs2);
-              q3 = pack_qm(blend_value(bc3, al, al, bk3), cs3);
+              q0 = pack_q(blend_value(bc0, __builtin_fmaf(sp, d0, a0), al, bk0), cs0);
+              q1 = pack_q(blend_value(bc1, __builtin_fmaf(sp, d1, a1), al, bk1), cs1);
+              q2 = pack_q(blend_value(bc2, __builtin_fmaf(sp, d2, a2), al, bk2), cs2);
+              q3 = pack_q(blend_value(bc3, al, al, bk3), cs3);
             }
             if (in) deposit2<T, kStride>(tile + e0, m, q0, q1, q2, q3);
             continue;
