@@ -751,7 +751,8 @@ __global__ __launch_bounds__(kScanThreads) void scan_add_kernel(uint32_t* out, u
 constexpr int kWBits = 20;
 constexpr int kWOne = 1 << kWBits;
 constexpr int kSlotU64 = kMergeSlotU64;
-static_assert(kSlotU64 == 4 * kTileMax * kTileMax, "a merge slot holds 4 planes of the largest tile");
+static_assert(kSlotU64 >= 4 * kTileMax * kTileMax && kSlotU64 >= 2 * kMaxHues * kTileMax * kTileMax,
+              "a merge slot holds 4 channel planes, or 2 planes per hue, of the largest tile");
 // A pair entry is the segment's index in its scene with the segment's major axis in bit 31
 // (1 = x); kNoPair marks lanes past the end of an item.
 constexpr uint32_t kPairIndex = 0x7FFFFFFFu;
@@ -799,14 +800,58 @@ __device__ __forceinline__ int scene_fixed_bits(const SceneDesc& D, int c) {
 // of the tile, kPackedPiece) (no item holds more), so the items' sums add up in the merge slot
 // and the launch tuning changes no bit.
 constexpr double kPackLevels = 4194304.0;  // 2^22
-__device__ __forceinline__ int packed_fixed_bits(const SceneDesc& D, int c, uint32_t n) {
-  const double bound = (double)D.color_max * (double)D.factor_max[c];
+__device__ __forceinline__ int packed_fixed_bits(double bound, uint32_t n) {
   if (!(bound > 0.0) || !(bound < 1e300)) return 0;
   const uint32_t q = 0xFFFFFFFFu / (n > 1u ? n : 1u);  // floor((2^32 - 1) / n)
   const double lim = (double)q < kPackLevels ? (double)q : kPackLevels;
   // the largest G with bound * 2^G <= lim - 1/2: v <= bound, rounded once in FP32, keeps
   // v * 2^G + 1/2 below lim + 1
   return clamp_fixed_bits(floor_log2_ratio(lim - 0.5, bound));
+}
+
+__device__ __forceinline__ int packed_fixed_bits(const SceneDesc& D, int c, uint32_t n) {
+  return packed_fixed_bits((double)D.color_max * (double)D.factor_max[c], n);
+}
+
+// Hue deposits (SCENE_HUES): a segment's colour is s times its light's hue, so its samples deposit
+// two numbers, s (the brightest channel's value) and the alpha deposit a * a, as the fields of ONE
+// word in the plane of its hue, where (R, G, B, A) take two words; the hue's RGB ratios come in
+// when a pixel's sums are converted. Half the LDS adds per sample, of which the walk is bound
+// (tile walk of the 1M-ray frame, us: 915 -> 776). The
+// fields' scales follow the packed rule with the hue's own bounds, so the brightest channel keeps
+// the levels it had and the others gain some.
+// What a tile's pairs and pixels need of each hue. It sits in LDS: the pairs of a batch mix hues
+// (a lane reads its own), and as registers of every wave it spilled the walk.
+struct HueScale {
+  double us, ua;     // 2^-G of the two fields
+  double ratio[3];   // the hue's RGB over its brightest channel
+  float ss, sa;      // 2^G
+  int32_t ch;        // the brightest channel
+  int32_t pad;
+};
+__device__ __forceinline__ HueScale hue_scale(const SceneDesc& D, int f, uint32_t n) {
+  HueScale h{};
+  if (f < D.n_hues) {
+    const int gs = packed_fixed_bits((double)D.hue_bound[f][0], n), ga = packed_fixed_bits((double)D.hue_bound[f][1], n);
+    h.us = __builtin_ldexp(1.0, -gs);
+    h.ua = __builtin_ldexp(1.0, -ga);
+    h.ss = __builtin_ldexpf(1.0f, gs);
+    h.sa = __builtin_ldexpf(1.0f, ga);
+    for (int k = 0; k < 3; k++) h.ratio[k] = D.hue_ratio[f][k];
+    h.ch = D.hue_ch[f];
+  }
+  return h;
+}
+
+// Adds hue h's exact sums s and a of a pixel to p: ratio s 2^-Gs and a 2^-Ga, in FP64 (rounded to
+// FP32 once, after the last hue). The one expression of the tile flush and of the merge of split
+// tiles.
+__device__ __forceinline__ void hue_add(double (&p)[4], const HueScale& h, unsigned long long s, unsigned long long a) {
+  const double v = (double)s * h.us;
+  p[0] = __builtin_fma(v, h.ratio[0], p[0]);
+  p[1] = __builtin_fma(v, h.ratio[1], p[1]);
+  p[2] = __builtin_fma(v, h.ratio[2], p[2]);
+  p[3] = __builtin_fma((double)a, h.ua, p[3]);
 }
 
 // The pair count that bounds a packed tile's fields (see packed_fixed_bits).
@@ -845,6 +890,16 @@ __device__ __forceinline__ void deposit2(unsigned long long* t, float m, uint32_
   atomicAdd(t + STRIDE, (unsigned long long)(q3 - r3) << 32 | (q2 - r2));
   atomicAdd(t + T, (unsigned long long)r1 << 32 | r0);
   atomicAdd(t + T + STRIDE, (unsigned long long)r3 << 32 | r2);
+}
+
+// The hue deposits of one sample: (s, a * a) as one word into t (pixel jl of the hue's plane) and
+// t + T.
+template <int T>
+__device__ __forceinline__ void deposit1(unsigned long long* t, float m, uint32_t qs, uint32_t qa) {
+  const float fr = __builtin_amdgcn_fractf(m);
+  const uint32_t r0 = mul_frac(fr, qs), r1 = mul_frac(fr, qa);
+  atomicAdd(t, (unsigned long long)(qa - r1) << 32 | (qs - r0));
+  atomicAdd(t + T, (unsigned long long)r1 << 32 | r0);
 }
 
 // The value one sample of colour channel c adds per unit weight: +-c * factor (BlendCode).
@@ -939,9 +994,11 @@ constexpr uint32_t kEarlyClaimPairs = 8192;
 // T is the tile edge of the frame (64 or 32; with 32 a pair has at most 32 samples in the
 // tile and lanes 32..63 only set up pairs). A scene with SCENE_PACKED (all its deposits
 // non-negative) keeps two channels per 64-bit word in the first two planes
-// (packed_fixed_bits); other scenes one channel per word in four. PACKED_ONLY: every scene of
-// the frame has SCENE_PACKED, so the LDS tile holds two planes only (half the LDS: two
-// workgroups share a compute unit at T = 64).
+// (packed_fixed_bits); one with SCENE_HUES a word per hue; other scenes one channel per word in
+// four. PACKED_ONLY: every scene of the frame has SCENE_PACKED, so the LDS tile holds two planes
+// only (half the LDS: two 512-thread workgroups share a compute unit at T = 64), or three in the
+// 1024-thread kernel, which serves up to three hues.
+enum WalkMode { WALK_COLOR, WALK_VERTEX_COLORS, WALK_HUES };
 template <int T, bool PACKED_ONLY, int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void tile_accum_kernel(const SceneDesc* __restrict__ descs,
                                                           const uint32_t* __restrict__ pairs,
@@ -950,7 +1007,10 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
   constexpr int kPlane = T * T;                         // pixels of a plane
   constexpr int kGuard = 2;                             // guard rows on each side of a plane
   constexpr int kStride = (T + 2 * kGuard) * T;         // elements from one plane to the next
-  constexpr int kPlanes = PACKED_ONLY ? 2 : 4;
+  constexpr bool kStreamKernel = PACKED_ONLY && T == 64 && BLOCK == 1024;
+  constexpr bool kHueKernel = T == 64 && BLOCK == 1024;  // the kernels frames with hues run
+  constexpr int kPlanes = kStreamKernel ? 3 : PACKED_ONLY ? 2 : 4;
+  static_assert(!kHueKernel || kPlanes >= kMaxHues, "a plane per hue");
   __shared__ unsigned long long s_tile[kPlanes * kStride];
   // the workgroup's next item and its index, double-buffered: thread 0 claims and loads item
   // i + 1 while item i runs and writes it into the other buffer
@@ -963,7 +1023,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
   // compute unit): each wave lays the samples of its 64 pairs end to end and walks that stream
   // 64 samples per step, every lane busy, instead of one pair per step. Per wave: a record per
   // pair with samples plus an empty one (two uint4 each) and a start bit per stream position.
-  constexpr bool kStreamKernel = PACKED_ONLY && T == 64 && BLOCK == 1024;
+  __shared__ HueScale s_hue[kHueKernel ? kMaxHues : 1];
   constexpr int kRecs = 66, kMaskWords = 64;
   __shared__ uint4 s_rec[kStreamKernel ? kWaves * kRecs * 2 : 1];
   __shared__ unsigned long long s_mask[kStreamKernel ? kWaves * kMaskWords : 1];
@@ -1019,11 +1079,17 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
     const float4* __restrict__ pos = gen(D.seg_pos);
     const float4* __restrict__ col0 = gen(D.seg_col);
     const float4* __restrict__ col1 = gen(D.seg_col1);
+    const uint64_t* __restrict__ keys = gen(D.seg_key);
     float4* accum = gen(D.accum);
     // two channels per word; uniform
     const bool two_ch = PACKED_ONLY || (D.flags & SCENE_PACKED) != 0;
-    int G[4];
-    if (two_ch) {
+    const bool hues = kHueKernel && (D.flags & SCENE_HUES) != 0;
+    const int n_hues = hues ? D.n_hues : 0;
+    if (kHueKernel && hues && threadIdx.x < kMaxHues) s_hue[threadIdx.x] = hue_scale(D, threadIdx.x, W.tile_pairs);
+    int G[4] = {0, 0, 0, 0};
+    if (hues) {
+      // (the channels' scales are not used)
+    } else if (two_ch) {
 #pragma unroll
       for (int c = 0; c < 4; c++) G[c] = packed_fixed_bits(D, c, W.tile_pairs);
     } else {
@@ -1056,7 +1122,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
       __syncthreads();
       continue;
     }
-    const int planes = two_ch ? 2 : 4;
+    const int planes = hues ? n_hues : two_ch ? 2 : 4;
     for (int k = threadIdx.x; k < planes * kPlane; k += BLOCK) tile[(k / kPlane) * kStride + k % kPlane] = 0ull;
     if (threadIdx.x == 0) s_batch[0] = s_batch[1] = 2u * kWaves;
     __syncthreads();
@@ -1084,17 +1150,23 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
           p = pos[s];
           ca = col0[s];
           if (col1) cb = col1[s];
+          if (n_hues > 1) {  // (such a scene has no col1: the key travels in its place)
+            const uint64_t k = keys[s];
+            cb.x = __uint_as_float((uint32_t)k);
+            cb.y = __uint_as_float((uint32_t)(k >> 32));
+          }
         }
       };
       uint32_t taken = 0;  // lane 0: the counter's previous value
       // One batch: set up the current batch's pairs from their loaded end points and colours,
       // issue the loads of the next batch and the pair entries of the one after, then walk.
-      // vc_tag: whether the scene's segments carry a colour per vertex (compiled twice, so that
+      // mode_tag: a colour per segment, a colour per vertex, or hues (compiled apart, so that
       // with one colour per segment a pair's channel values stay in scalar registers).
-      auto step = [&](auto vc_tag, const uint32_t e_cur, const float4& p_cur, const float4& a_cur,
+      auto step = [&](auto mode_tag, const uint32_t e_cur, const float4& p_cur, const float4& a_cur,
                       const float4& c_cur, const uint32_t e_nxt, float4& p_nxt, float4& a_nxt, float4& c_nxt,
                       uint32_t& b_aft, uint32_t& e_aft) {
-        constexpr bool kVC = decltype(vc_tag)::value;
+        constexpr bool kVC = decltype(mode_tag)::value == WALK_VERTEX_COLORS;
+        constexpr bool kHues = decltype(mode_tag)::value == WALK_HUES;
         // ---- per-lane setup of one pair of the current batch ----
         int packed = 0;  // n | q0 << 8 | xmajor << 16 | vertex colours << 17 | negative colour << 18
         float m_first = 0.f, slope = 0.f, s_first = 0.f, ds = 0.f;
@@ -1115,12 +1187,27 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               m_first = (float)(g.m0 + (((double)maj0 + 0.5) - g.M0) * g.slope - (double)min0 - 0.5);
               slope = (float)g.slope;
               ca = a_cur;
+              if constexpr (kHues) {
+                int f = 0;
+                if (n_hues > 1) {
+                  const uint64_t ray = ((uint64_t)__float_as_uint(c_cur.y) << 32 | __float_as_uint(c_cur.x)) >> kPathBits;
+                  f = (ray >= D.hue_ray[1] ? 1 : 0) + (n_hues > 2 && ray >= D.hue_ray[2] ? 1 : 0);
+                }
+                const HueScale& h = s_hue[f];
+                const int ch = h.ch;
+                const float v = ch == 0 ? ca.x : ch == 1 ? ca.y : ca.z;
+                cq0 = (int)pack_q(v, h.ss);
+                cq1 = (int)pack_q(ca.w * ca.w, h.sa);
+                cq2 = f * kStride;  // its plane
+              }
               const float4 cb = kVC ? c_cur : a_cur;
               dc = make_float4(cb.x - ca.x, cb.y - ca.y, cb.z - ca.z, cb.w - ca.w);
               const int vc = (dc.x != 0.f || dc.y != 0.f || dc.z != 0.f || dc.w != 0.f) ? 1 : 0;
               s_first = (float)(u0 * g.inv_dM);
               ds = (float)g.inv_dM;
-              if (two_ch) {
+              if constexpr (kHues) {
+                // (set above)
+              } else if (two_ch) {
                 cq0 = (int)pack_q(blend_value(bc0, ca.x, ca.w, bk0), cs0);
                 cq1 = (int)pack_q(blend_value(bc1, ca.y, ca.w, bk1), cs1);
                 cq2 = (int)pack_q(blend_value(bc2, ca.z, ca.w, bk2), cs2);
@@ -1170,8 +1257,11 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             if (n) {
               const int off = ((packed >> 8) & 0xff) - pre;
               rec[2 * c] = make_uint4((uint32_t)off, __float_as_uint(m_first), __float_as_uint(slope),
-                                      (uint32_t)(off * 8));
-              rec[2 * c + 1] = make_uint4((uint32_t)cq0, (uint32_t)cq1, (uint32_t)cq2, (uint32_t)cq3);
+                                      (uint32_t)((kHues ? off + cq2 : off) * 8));
+              if constexpr (kHues)
+                *reinterpret_cast<uint2*>(&rec[2 * c + 1]) = make_uint2((uint32_t)cq0, (uint32_t)cq1);
+              else
+                rec[2 * c + 1] = make_uint4((uint32_t)cq0, (uint32_t)cq1, (uint32_t)cq2, (uint32_t)cq3);
               atomicOr(&mask[pre >> 6], 1ull << (pre & 63));
             }
             if (lane == 0) {
@@ -1205,7 +1295,13 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               const char* const rbase = rec_m1 + (first + 1) * 32;
               const uint4* const r = reinterpret_cast<const uint4*>(rbase + k * 32u);
               r0 = r[0];
-              r1 = r[1];
+              if constexpr (kHues) {
+                const uint2 q = *reinterpret_cast<const uint2*>(&r[1]);
+                r1.x = q.x;
+                r1.y = q.y;
+              } else {
+                r1 = r[1];
+              }
             };
             // Step st at stream positions p = 64 st + lane: the sample's column is off + p, its
             // entry in plane 0 jl * T + column.
@@ -1219,25 +1315,30 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               // byte offset 8 (jl T + column) = (jl + st) 512 + 8 off + 8 lane
               const uint32_t eb = ((uint32_t)(jl + st) << 9) + r0.w + lane8;
               unsigned long long* const t = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(tile) + eb);
-              deposit2<T, kStride>(t, m, r1.x, r1.y, r1.z, r1.w);
+              if constexpr (kHues)
+                deposit1<T>(t, m, r1.x, r1.y);
+              else
+                deposit2<T, kStride>(t, m, r1.x, r1.y, r1.z, r1.w);
             };
             // One step ahead: the records of step s + 1 are read while step s deposits; two
             // steps per trip with the record registers swapped, so that nothing read ahead is
             // copied (a copy would wait for its read). Scheduling barriers keep the reads ahead
             // of the deposits they overlap.
-            uint4 ra, rb, rc, rd;
+            uint4 ra, rb{}, rc, rd{};
             read_recs(0, ra, rb);
-            // four zero adds into guard row -2: the loop is entered with the same LDS operations
-            // in flight as it loops back with (two reads, four adds), so that the compiler's
-            // wait counts inside the loop stay exact
+            // zero adds into guard row -2: the loop is entered with the same LDS operations
+            // in flight as it loops back with (two reads, four adds; two with hues), so that the
+            // compiler's wait counts inside the loop stay exact
             {
               unsigned long long zero = 0ull;
               asm volatile("" : "+v"(zero));  // an add the compiler cannot turn into a load
               unsigned long long* const g = tile + (-kGuard * T + lane);
               atomicAdd(g, zero);
-              atomicAdd(g + kStride, zero);
               atomicAdd(g + T, zero);
-              atomicAdd(g + T + kStride, zero);
+              if constexpr (!kHues) {
+                atomicAdd(g + kStride, zero);
+                atomicAdd(g + T + kStride, zero);
+              }
             }
             __builtin_amdgcn_sched_barrier(0);
             for (int st = 0;; st += 2) {
@@ -1253,7 +1354,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               if (st + 2 >= steps) break;
             }
             wave_samples += (unsigned long long)total;
-            wave_atomics += 4u * (unsigned)steps;
+            wave_atomics += (kHues ? 2u : 4u) * (unsigned)steps;
           }
           return;
         }
@@ -1269,7 +1370,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
           const int jn = jp & 0xff, jq0 = (jp >> 8) & 0xff, jvc = (jp >> 17) & 1;
           const int jneg = (jp >> 18) & 1;
           wave_samples += (unsigned long long)jn;
-          wave_atomics += two_ch ? 4u : 8u;
+          wave_atomics += kHues ? 2u : two_ch ? 4u : 8u;
           const float jm = bcast_f(m_first, j), jsl = bcast_f(slope, j);
           // lane's sample: minor pixel jl, weights wl (pixel jl) and wq (jl + 1), and the entry
           // t of (jl, jq0 + lane) in plane 0 (t2 in plane 2); the row below and the next plane
@@ -1284,6 +1385,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
           jl = jl < -kGuard ? -kGuard : (jl > T ? T : jl);
           const int e0 = jl * T + col;
           const bool in = lane < jn;
+          if constexpr (kHues) {
+            const uint32_t qs = (uint32_t)bcast_i(cq0, j), qa = (uint32_t)bcast_i(cq1, j);
+            const int plane = bcast_i(cq2, j);
+            if (in) deposit1<T>(tile + e0 + plane, m, qs, qa);
+            continue;
+          }
           if (two_ch) {
             uint32_t q0, q1, q2, q3;
             if (!kVC || !jvc) {
@@ -1371,24 +1478,33 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
       if (lane == 0) taken = atomicAdd(&s_batch[phase], 1u);
       // two batches per trip with the register sets swapped, so that every value loaded ahead is
       // written once per trip and none is copied (a copy would wait for its load)
-      auto run = [&](auto vc_tag) {
+      auto run = [&](auto mode_tag) {
         for (;;) {
           if (b0 >= n_batches) break;
           uint32_t b2, e2;
-          step(vc_tag, e0, p0, a0, c0v, e1, p1, a1, c1v, b2, e2);
+          step(mode_tag, e0, p0, a0, c0v, e1, p1, a1, c1v, b2, e2);
           if (b1 >= n_batches) break;
           uint32_t b3, e3;
-          step(vc_tag, e1, p1, a1, c1v, e2, p0, a0, c0v, b3, e3);
+          step(mode_tag, e1, p1, a1, c1v, e2, p0, a0, c0v, b3, e3);
           b0 = b2;
           e0 = e2;
           b1 = b3;
           e1 = e3;
         }
       };
-      if (col1)
-        run(std::true_type{});
-      else
-        run(std::false_type{});
+      bool walked = false;
+      if constexpr (kHueKernel) {
+        if (hues) {
+          run(std::integral_constant<int, WALK_HUES>{});
+          walked = true;
+        }
+      }
+      if (walked) {
+      } else if (col1) {
+        run(std::integral_constant<int, WALK_VERTEX_COLORS>{});
+      } else {
+        run(std::integral_constant<int, WALK_COLOR>{});
+      }
       __syncthreads();
       if (phase == 0) {
         transpose_tile<T, kStride, kWaves>(tile, planes, wave, lane);
@@ -1400,9 +1516,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
     if (split) {
       // exact partial sums into the tile's merge slot (integer atomics: order independent)
       unsigned long long* fx = split_fx + (size_t)W.slot * kSlotU64;
+      const int n_fields = hues ? 2 * n_hues : 4;
       for (int k = threadIdx.x; k < T * T; k += BLOCK) {
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
+        for (int c = 0; c < n_fields; c++) {
           const unsigned long long val =
               two_ch ? (tile[(c >> 1) * kStride + k] >> (32 * (c & 1))) & 0xffffffffull : tile[c * kStride + k];
           if (val) atomicAdd(&fx[c * T * T + k], val);
@@ -1424,7 +1540,17 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
         const int idx = k;  // row-major
         const size_t px = (size_t)gy * v.width + gx;
         float4 o = whole ? make_float4(0.f, 0.f, 0.f, 0.f) : accum[px];
-        if (two_ch) {
+        if (hues) {
+          double p[4] = {0.0, 0.0, 0.0, 0.0};
+          for (int f = 0; f < n_hues; f++) {
+            const unsigned long long w = tile[f * kStride + idx];
+            hue_add(p, s_hue[f], (uint32_t)w, w >> 32);
+          }
+          o.x += (float)p[0];
+          o.y += (float)p[1];
+          o.z += (float)p[2];
+          o.w += (float)p[3];
+        } else if (two_ch) {
           const unsigned long long w0 = tile[idx], w1 = tile[kStride + idx];
           o.x += field((uint32_t)w0, G[0]);
           o.y += field((uint32_t)(w0 >> 32), G[1]);
@@ -1460,6 +1586,7 @@ __global__ __launch_bounds__(256) void tile_merge_kernel(const SceneDesc* __rest
   if (ctl->flags & kCtlStop) return;
   uint32_t n_split = ctl->n_split;
   n_split = n_split < split_cap ? n_split : split_cap;
+  __shared__ HueScale s_hue[kMaxHues];
   for (uint32_t sl = blockIdx.x; sl < n_split; sl += gridDim.x) {
     const uint32_t g = split_tiles[sl];
     const SceneDesc& D = descs[tile_scene[g]];
@@ -1467,33 +1594,51 @@ __global__ __launch_bounds__(256) void tile_merge_kernel(const SceneDesc* __rest
     const uint32_t t = g - (uint32_t)D.tile_base;
     const int T = v.tile, TT = T * T;
     const int x0 = (int)(t % (uint32_t)v.tiles_x) * T, y0 = (int)(t / (uint32_t)v.tiles_x) * T;
-    double un[4];
-    if (D.flags & SCENE_PACKED) {
-      const uint32_t np = packed_pairs(row_start, g);
+    const bool hues = (D.flags & SCENE_HUES) != 0;
+    const uint32_t np = packed_pairs(row_start, g);
+    __syncthreads();  // (the slot before is done with the table)
+    if (hues && threadIdx.x < kMaxHues) s_hue[threadIdx.x] = hue_scale(D, threadIdx.x, np);
+    __syncthreads();
+    double un[4] = {0.0, 0.0, 0.0, 0.0};
+    if (!hues) {
 #pragma unroll
-      for (int c = 0; c < 4; c++) un[c] = __builtin_ldexp(1.0, -packed_fixed_bits(D, c, np));
-    } else {
-#pragma unroll
-      for (int c = 0; c < 4; c++) un[c] = __builtin_ldexp(1.0, -(scene_fixed_bits(D, c) + kWBits));
+      for (int c = 0; c < 4; c++)
+        un[c] = __builtin_ldexp(1.0, (D.flags & SCENE_PACKED) ? -packed_fixed_bits(D, c, np) : -(scene_fixed_bits(D, c) + kWBits));
     }
+    const int n_fields = hues ? 2 * D.n_hues : 4;
     const bool whole = (D.flags & SCENE_FRESH_IMAGE) != 0;  // the frame clears and resolves here
     unsigned long long* fx = split_fx + (size_t)sl * kSlotU64;
     for (int k = threadIdx.x; k < TT; k += blockDim.x) {
-      unsigned long long a[4];
+      unsigned long long a[2 * kMaxHues] = {}, any = 0ull;
 #pragma unroll
-      for (int c = 0; c < 4; c++) a[c] = fx[c * TT + k];
-      if ((a[0] | a[1] | a[2] | a[3]) == 0ull && !whole) continue;
+      for (int c = 0; c < 2 * kMaxHues; c++)
+        if (c < n_fields) {
+          a[c] = fx[c * TT + k];
+          any |= a[c];
+        }
+      if (any == 0ull && !whole) continue;
 #pragma unroll
-      for (int c = 0; c < 4; c++)
+      for (int c = 0; c < 2 * kMaxHues; c++)
         if (a[c]) fx[c * TT + k] = 0ull;
       const int gx = x0 + (k % T), gy = y0 + (k / T);
       if (gx >= v.width || gy >= v.height) continue;
       const size_t px = (size_t)gy * v.width + gx;
       float4 o = whole ? make_float4(0.f, 0.f, 0.f, 0.f) : gen(D.accum)[px];
-      o.x += (float)((double)(long long)a[0] * un[0]);
-      o.y += (float)((double)(long long)a[1] * un[1]);
-      o.z += (float)((double)(long long)a[2] * un[2]);
-      o.w += (float)((double)(long long)a[3] * un[3]);
+      if (hues) {
+        double p[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int f = 0; f < kMaxHues; f++)
+          if (2 * f < n_fields) hue_add(p, s_hue[f], a[2 * f], a[2 * f + 1]);
+        o.x += (float)p[0];
+        o.y += (float)p[1];
+        o.z += (float)p[2];
+        o.w += (float)p[3];
+      } else {
+        o.x += (float)((double)(long long)a[0] * un[0]);
+        o.y += (float)((double)(long long)a[1] * un[1]);
+        o.z += (float)((double)(long long)a[2] * un[2]);
+        o.w += (float)((double)(long long)a[3] * un[3]);
+      }
       gen(D.accum)[px] = o;
       if (whole) gen(D.out16)[px] = resolve_px(o);
     }

@@ -875,6 +875,7 @@ int lg_segments_upload(lg_segments* s, const float* pos, const float* color0, co
   if (rc) return rc;
   s->max_abs = 0.0f;
   s->nonneg = true;
+  s->hues = SceneHues{};
   // a color1 equal to color0 bit for bit is no per-vertex colour: the accumulation then takes
   // the one-colour walk, which deposits the same bits
   s->one_color = !color1 || !n || std::memcmp(color0, color1, n * 16) == 0;

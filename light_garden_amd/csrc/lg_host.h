@@ -182,6 +182,7 @@ struct lg_segments {
   // both vertices of every stored segment have colour col0 (traced segments, uploads without
   // or with an identical color1, StringMods without modulo colours): col1 is not read
   bool one_color = true;
+  lg::SceneHues hues;         // traced segments: the colours of their lights
   lg::DevBuf pos, col0, col1, key, pos64;
   bool has_pos64 = false;
 };
@@ -222,6 +223,10 @@ void begin_call(lg_ctx* ctx);
 void end_call(lg_ctx* ctx);
 // per channel, max |blend factor| of a BlendCode word over colours with |channel| <= m
 void blend_factor_bounds(uint32_t code, float m, const float k[4], float out[4]);
+// The hues of a scene's traced segments (n = 0 when its lights are more than kMaxHues), and their
+// form in a frame's descriptor.
+SceneHues scene_hues(const lg_scene* sc);
+void set_hues(SceneDesc& D, const SceneHues& h);
 // Whether every value colour * factor is >= 0 for colour channels in [0, m].
 bool blend_nonneg(uint32_t code, float m, const float k[4]);
 

@@ -197,7 +197,20 @@ enum SceneFlags : uint32_t {
   SCENE_FIXED_COUNT = 1u,     // accumulate `seg_fixed` uploaded segments (no trace)
   SCENE_FRESH_IMAGE = 2u,     // the frame clears, accumulates and resolves the image: the tile
                               // flushes write the accumulator and the RGBA16F target directly
-  SCENE_PACKED = 4u           // every deposit is non-negative: two channels per LDS word
+  SCENE_PACKED = 4u,          // every deposit is non-negative: two channels per LDS word
+  SCENE_HUES = 8u             // with SCENE_PACKED: the segments' colours are fractions of at most
+                              // kMaxHues light colours (SceneHues): one LDS word per deposit
+};
+
+// The colours of traced segments. A ray's RGB is its light's, scaled by one factor per surface it
+// met, and its alpha is its light's (tracer.rs:454-457): a segment's colour is one number times
+// its light's hue, and its light follows from the ray index in its key. Hue h covers the rays
+// from first_ray[h] (first_ray[0] = 0) up to the next hue's.
+constexpr int kMaxHues = 3;
+struct SceneHues {
+  int32_t n = 0;               // 0: the colours are not known to be of this form
+  uint64_t first_ray[kMaxHues] = {0, 0, 0};
+  float color[kMaxHues][4] = {};
 };
 
 // Device pointers kept in descriptors carry the global address space in their type: kernels
@@ -265,6 +278,13 @@ struct SceneDesc {
   uint32_t blend_code;
   float blend_k[4];
   float factor_max[4];
+  // SCENE_HUES: per hue the light's brightest RGB channel, the bounds of what a segment of it
+  // deposits there and in alpha (a * a), and the RGB channels over the brightest
+  int32_t n_hues;
+  int32_t hue_ch[kMaxHues];
+  uint64_t hue_ray[kMaxHues];
+  float hue_bound[kMaxHues][2];
+  double hue_ratio[kMaxHues][3];
 };
 
 // Source factors of the supported blends, per channel c of the interpolated colour (a = its
@@ -319,8 +339,8 @@ struct alignas(16) WorkItem {
 };
 constexpr uint32_t kSplitBit = 0x80000000u;
 // One merge slot of a tile split over several work items: 4 channel planes of the largest
-// tile (64 x 64), 64-bit fixed point.
-constexpr int kMergeSlotU64 = 4 * 64 * 64;
+// tile (64 x 64), or two per hue, 64-bit fixed point.
+constexpr int kMergeSlotU64 = 2 * kMaxHues * 64 * 64;
 // Pairs per tile work item at most: the fixed point of a tile that accumulates two channels
 // per LDS word follows min(pairs of the tile, kPackedPiece), whatever the launch tuning, so
 // results do not depend on it.

@@ -132,6 +132,8 @@ int lg_accumulate_noalloc(lg_ctx* ctx, const lg_segments* segs, lg_image* img) {
   const bool packed = ctx->packed_accum && segs->nonneg && std::isfinite(segs->max_abs) &&
                       blend_nonneg(D.blend_code, segs->max_abs, D.blend_k);
   if (packed) D.flags |= SCENE_PACKED;
+  const bool hues = packed && segs->hues.n && D.blend_code == kBlendDefault && tile == 64;
+  if (hues) set_hues(D, segs->hues);
   const uint32_t min_piece = std::max(kNaMinPiece, std::min(ctx->tune.min_piece, kPackedPiece));
   const uint32_t max_piece = std::max(min_piece, std::min(ctx->tune.max_piece, kPackedPiece));
 
@@ -166,7 +168,7 @@ int lg_accumulate_noalloc(lg_ctx* ctx, const lg_segments* segs, lg_image* img) {
                              split_tiles, kNaSplit, kNaPairs, min_piece, max_piece, (uint32_t)ctx->n_cu, false, st));
     LG_HIP(launch_bin(1, d_desc, 1, chunk_pre, cbase, d_ctl, counts, row_start, pairs, kNaPairs, n_tiles, bin_grid, st));
     LG_HIP(launch_tile_accum(d_desc, pairs, items, split_fx, d_ctl,
-                             tile, packed, (int)ctx->tune.tile_block, ctx->n_cu, st));
+                             tile, packed, hues ? 1024 : (int)ctx->tune.tile_block, ctx->n_cu, st));
     LG_HIP(launch_tile_merge(d_desc, tile_scene, row_start, split_tiles, d_ctl, split_fx, kNaSplit, ctx->n_cu, st));
     LG_HIP(hipMemcpyAsync(&hc, d_ctl, sizeof(BatchCtl), hipMemcpyDeviceToHost, st));
     LG_HIP(hipStreamSynchronize(st));

@@ -126,11 +126,39 @@ struct Layout {
   int n_tiles = 0, max_tiles = 0;
   int tile = 64;                     // screen tile edge of the frame
   bool packed_only = false;          // every accumulated scene keeps two channels per LDS word
+  bool hues = false;                 // some scene's deposits are one LDS word (SCENE_HUES)
   uint64_t n_counts = 0, n_px = 0;  // n_counts: capacity of the per-frame [chunk][tile][axis] matrix
   uint32_t bin_target = 0;           // bin chunks per frame
   std::vector<int> tile_base;
   std::vector<uint64_t> px_base;
 };
+
+SceneHues scene_hues(const lg_scene* sc) {
+  SceneHues h;
+  if (sc->lights.empty() || sc->lights.size() > (size_t)kMaxHues) return h;
+  uint64_t ray = 0;
+  for (const lg_light& l : sc->lights) {
+    h.first_ray[h.n] = ray;
+    for (int c = 0; c < 4; c++) h.color[h.n][c] = l.color[c];
+    h.n++;
+    ray += l.num_rays;
+  }
+  return h;
+}
+
+void set_hues(SceneDesc& D, const SceneHues& h) {
+  D.flags |= SCENE_HUES;
+  D.n_hues = h.n;
+  for (int f = 0; f < h.n; f++) {
+    const float* c = h.color[f];
+    const int p = c[1] > c[0] ? (c[2] > c[1] ? 2 : 1) : (c[2] > c[0] ? 2 : 0);
+    D.hue_ch[f] = p;
+    D.hue_ray[f] = h.first_ray[f];
+    D.hue_bound[f][0] = c[p];
+    D.hue_bound[f][1] = c[3] * c[3];
+    for (int k = 0; k < 3; k++) D.hue_ratio[f][k] = c[p] > 0.0f ? (double)c[k] / (double)c[p] : 0.0;
+  }
+}
 
 // Stage events only where the caller asked for them (the synchronous entry points on the
 // context's own stream).
@@ -198,7 +226,7 @@ static int enqueue(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, const
       Scope s(ctx, profile, "tile_accum", 0);
       LG_HIP(launch_tile_accum(d_descs, P.pairs.as<uint32_t>(), P.items.as<WorkItem>(),
                                P.split_fx.as<unsigned long long>(), d_ctl, L.tile, L.packed_only,
-                               (int)ctx->tune.tile_block, ctx->n_cu, st));
+                               L.hues ? 1024 : (int)ctx->tune.tile_block, ctx->n_cu, st));
     }
     {
       Scope s(ctx, profile, "tile_merge", 0);
@@ -376,6 +404,7 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
   if ((rc = P.stage_out.ensure(F.out_bytes()))) return rc;
   // ---- descriptors ----
   L.packed_only = accum;
+  L.hues = false;
   char* in = P.stage_in.as<char>();
   SceneDesc* hd = reinterpret_cast<SceneDesc*>(in);
   uint32_t* h_tile_scene = reinterpret_cast<uint32_t*>(in + F.tile_scene);
@@ -391,6 +420,7 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
     D.gen_count = gbl(reinterpret_cast<uint32_t*>(P.counters.as<char>() + i * kCounterStride + kGenCountOffset));
     float max_abs = 0.0f;
     bool nonneg = true;
+    SceneHues hues;
     if (trace) {
       lg_scene* sc = e.scene;
       D.recs = gbl(L.fp64 ? sc->recs64.p : sc->recs32.p);
@@ -423,6 +453,7 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
       D.q_cap = sc->q_cap;
       max_abs = sc->light_max;
       nonneg = sc->light_nonneg;
+      hues = scene_hues(sc);
     }
     if (e.segs) {
       D.seg_pos = gbl(e.segs->pos.as<float4>());
@@ -437,6 +468,7 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
         D.seg_fixed = e.segs->count;
         max_abs = e.segs->max_abs;
         nonneg = e.segs->nonneg;
+        hues = e.segs->hues;
       }
     }
     if (e.img) {
@@ -454,10 +486,17 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
     for (int c = 0; c < 4; c++) D.blend_k[c] = e.img ? e.img->blend.constant[c] : 0.0f;
     blend_factor_bounds(D.blend_code, max_abs, D.blend_k, D.factor_max);
     // two channels per LDS word when every deposit of the scene is non-negative
-    if (ctx->packed_accum && nonneg && std::isfinite(max_abs) && blend_nonneg(D.blend_code, max_abs, D.blend_k))
+    if (ctx->packed_accum && nonneg && std::isfinite(max_abs) && blend_nonneg(D.blend_code, max_abs, D.blend_k)) {
       D.flags |= SCENE_PACKED;
-    else if (accum)
+      // one LDS word per deposit where the blend keeps the hue: RGB One, alpha SrcAlpha (the
+      // default); not with 32-pixel tiles, whose kernels do not have that walk
+      if (hues.n && D.blend_code == kBlendDefault && L.tile == 64) {
+        set_hues(D, hues);
+        L.hues = true;
+      }
+    } else if (accum) {
       L.packed_only = false;
+    }
     D.tile_base = L.tile_base[i];
     if (accum) {
       int t = D.view.tiles_x * D.view.tiles_y;
@@ -471,7 +510,8 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
                                  (uint64_t)L.max_tiles, L.n_counts, L.n_px, L.bin_target, P.pairs_cap, P.items_cap,
                                  P.split_cap, ctx->tune.rays_per_item, ctx->tune.min_piece, ctx->tune.max_piece,
                                  ctx->tune.trace_waves, ctx->tune.bvh_min_objects,
-                                 (uint64_t)L.tile, (uint64_t)L.packed_only, L.chunk, ctx->tune.tile_block};
+                                 (uint64_t)L.tile, (uint64_t)L.packed_only, (uint64_t)L.hues, L.chunk,
+                                 ctx->tune.tile_block};
   for (DevBuf* b : {&P.frame_in, &P.item_pre, &P.chunk_pre, &P.cbase, &P.places, &P.scan_scratch, &P.row_start,
                     &P.pairs, &P.items, &P.split_tiles, &P.split_fx})
     shape.push_back((uint64_t)b->p);
@@ -576,6 +616,7 @@ static int batch_finish(lg_ctx* ctx, Pipeline& P, bool profile, Batch& B, bool* 
       e.segs->max_abs = e.scene->light_max;
       e.segs->nonneg = e.scene->light_nonneg;
       e.segs->one_color = true;
+      e.segs->hues = scene_hues(e.scene);
       e.scene->seg_hint = std::max(e.scene->seg_hint, segs);
     }
   }

@@ -78,6 +78,7 @@ int copy_segments(lg_segments* dst, const lg_segments* src) {
   dst->has_pos64 = false;
   dst->max_abs = src->max_abs;
   dst->nonneg = src->nonneg;
+  dst->hues = src->hues;
   return LG_OK;
 }
 
