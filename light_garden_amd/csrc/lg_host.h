@@ -107,7 +107,7 @@ hipError_t launch_tile_accum(const SceneDesc* descs, const uint32_t* pairs, cons
                              int n_cu, hipStream_t st);
 hipError_t launch_tile_merge(const SceneDesc* descs, const uint32_t* tile_scene, const uint32_t* row_start,
                              const uint32_t* split_tiles, const BatchCtl* ctl, unsigned long long* split_fx,
-                             uint32_t split_cap, int grid, hipStream_t st);
+                             uint32_t split_cap, int tile, int n_cu, hipStream_t st);
 uint64_t merge_slot_u64();
 // The 64-bit LDS atomic issue-rate probe (lg_calibrate_lds_atomics): `sink` holds 2 * n_cu
 // words; *wave_instructions = the atomic wave instructions the launch issues.

@@ -169,7 +169,8 @@ int lg_accumulate_noalloc(lg_ctx* ctx, const lg_segments* segs, lg_image* img) {
     LG_HIP(launch_bin(1, d_desc, 1, chunk_pre, cbase, d_ctl, counts, row_start, pairs, kNaPairs, n_tiles, bin_grid, st));
     LG_HIP(launch_tile_accum(d_desc, pairs, items, split_fx, d_ctl,
                              tile, packed, hues ? 1024 : (int)ctx->tune.tile_block, ctx->n_cu, st));
-    LG_HIP(launch_tile_merge(d_desc, tile_scene, row_start, split_tiles, d_ctl, split_fx, kNaSplit, ctx->n_cu, st));
+    LG_HIP(launch_tile_merge(d_desc, tile_scene, row_start, split_tiles, d_ctl, split_fx, kNaSplit, tile, ctx->n_cu,
+                             st));
     LG_HIP(hipMemcpyAsync(&hc, d_ctl, sizeof(BatchCtl), hipMemcpyDeviceToHost, st));
     LG_HIP(hipStreamSynchronize(st));
   }

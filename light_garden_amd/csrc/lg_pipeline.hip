@@ -232,7 +232,7 @@ static int enqueue(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, const
       Scope s(ctx, profile, "tile_merge", 0);
       LG_HIP(launch_tile_merge(d_descs, P.tile_scene.as<uint32_t>(), P.row_start.as<uint32_t>(),
                                P.split_tiles.as<uint32_t>(), d_ctl, P.split_fx.as<unsigned long long>(), P.split_cap,
-                               ctx->n_cu, st));
+                               L.tile, ctx->n_cu, st));
     }
   }
   if ((stages & ST_RESOLVE) && !whole) {
