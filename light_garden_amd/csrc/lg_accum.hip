@@ -283,7 +283,7 @@ __global__ __launch_bounds__(256) void bin_kernel(const SceneDesc* __restrict__ 
   const uint32_t chunk = ctl->chunk;
   bool first = true;
   for (;;) {
-    if (threadIdx.x == 0) s_chunk = next_work_item(&ctl->chunk_cursor[PASS], n_chunks, first);
+    if (threadIdx.x == 0) s_chunk = next_work_item(PASS == 0 ? &ctl->chunk_cursor0 : &ctl->chunk_cursor1, n_chunks, first);
     first = false;
     __syncthreads();
     const uint32_t ci = __builtin_amdgcn_readfirstlane(s_chunk);
@@ -979,7 +979,8 @@ template <int T, bool PACKED_ONLY, int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void tile_accum_kernel(const SceneDesc* __restrict__ descs,
                                                           const uint32_t* __restrict__ pairs,
                                                           const WorkItem* __restrict__ items,
-                                                          unsigned long long* split_fx, BatchCtl* ctl) {
+                                                          unsigned long long* split_fx, BatchCtl* ctl,
+                                                          uint32_t count_work) {
   constexpr int kPlane = T * T;                         // pixels of a plane
   constexpr int kGuard = 2;                             // guard rows on each side of a plane
   constexpr int kStride = (T + 2 * kGuard) * T;         // elements from one plane to the next
@@ -1030,11 +1031,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
     // starts from LDS. A small item claims at its start (the claim returns while it runs); a
     // large one at its flush, since a workgroup holding a claimed item while its current one
     // runs for long leaves others idle at the end of the launch. After the last item every
-    // workgroup claims one more, past the end.
+    // workgroup claims one more, past the end; a frame with an item per workgroup or fewer claims
+    // none.
     const bool claim_early = W.end - W.begin <= kEarlyClaimPairs;
     uint32_t it_next = 0;
     auto claim = [&]() {
-      if (threadIdx.x == 0) it_next = atomicAdd(&ctl->work_cursor, 1u) + gridDim.x;
+      if (threadIdx.x == 0) it_next = n_items > gridDim.x ? atomicAdd(&ctl->work_cursor, 1u) + gridDim.x : n_items;
     };
     if (claim_early) claim();
     // publishes the next item for the loop's next trip (before the workgroup's last barrier)
@@ -1583,9 +1585,22 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
     publish_next(wn);
     __syncthreads();
   }
-  if (lane == 0 && wave_samples) {
-    atomicAdd(&ctl->samples, wave_samples);
-    atomicAdd(&ctl->lds_atomics, wave_atomics);
+  // Profiled frames: the walk's work, one global add per workgroup. (An add per wave to either
+  // word in every frame held up the claims of the work items, 8192 adds of 12 ns to one line: the
+  // tile walk of a 20k-ray frame took 90 us where it takes 62.)
+  if (count_work) {
+    __shared__ unsigned long long s_work[2];
+    if (threadIdx.x < 2) s_work[threadIdx.x] = 0ull;
+    __syncthreads();
+    if (lane == 0 && wave_samples) {
+      atomicAdd(&s_work[0], wave_samples);
+      atomicAdd(&s_work[1], wave_atomics);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && s_work[0]) {
+      atomicAdd(&ctl->samples, s_work[0]);
+      atomicAdd(&ctl->lds_atomics, s_work[1]);
+    }
   }
 }
 
@@ -1808,10 +1823,10 @@ hipError_t launch_work_items(const SceneDesc* descs, const uint32_t* tile_scene,
 // persistent grid fills every compute unit.
 hipError_t launch_tile_accum(const SceneDesc* descs, const uint32_t* pairs, const WorkItem* items,
                              unsigned long long* split_fx, BatchCtl* ctl, int tile, bool packed_only, int block,
-                             int n_cu, hipStream_t st) {
+                             bool count_work, int n_cu, hipStream_t st) {
 #define LG_TILE_LAUNCH(T, P, B, PER_CU)                                                                     \
   hipLaunchKernelGGL((tile_accum_kernel<T, P, B>), dim3(n_cu * (PER_CU)), dim3(B), 0, st, descs, pairs, items, \
-                     split_fx, ctl)
+                     split_fx, ctl, count_work ? 1u : 0u)
   if (tile == 64) {
     if (packed_only && block == 512)
       LG_TILE_LAUNCH(64, true, 512, 2);

@@ -104,7 +104,7 @@ hipError_t launch_work_items(const SceneDesc* descs, const uint32_t* tile_scene,
                              bool whole_images, hipStream_t st);
 hipError_t launch_tile_accum(const SceneDesc* descs, const uint32_t* pairs, const WorkItem* items,
                              unsigned long long* split_fx, BatchCtl* ctl, int tile, bool packed_only, int block,
-                             int n_cu, hipStream_t st);
+                             bool count_work, int n_cu, hipStream_t st);
 hipError_t launch_tile_merge(const SceneDesc* descs, const uint32_t* tile_scene, const uint32_t* row_start,
                              const uint32_t* split_tiles, const BatchCtl* ctl, unsigned long long* split_fx,
                              uint32_t split_cap, int tile, int n_cu, hipStream_t st);

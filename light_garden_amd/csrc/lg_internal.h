@@ -298,29 +298,37 @@ constexpr uint32_t kBlendDefault = BC_ONE | (BC_ONE << 4) | (BC_ONE << 8) | (BC_
 
 constexpr int kMaxGen = kPathBits;
 
-// Device-side control block of one batched frame.
+// Device-side control block of one batched frame. Atomic adds to one line of memory are served one
+// after another, 12 ns each over the whole chip, so the words that persistent workgroups count on
+// have lines of their own: a workgroup waits for its claim, and behind other words' adds it waits
+// for those too.
 struct BatchCtl {
   uint32_t n_items_gen[kMaxGen];   // trace items per generation
-  uint32_t item_cursor[kMaxGen];
   uint32_t gen_done[kMaxGen];      // trace workgroups finished per generation
   uint32_t n_chunks;
   uint32_t chunk;                  // segments per bin chunk (at least; see scene_chunk)
   uint32_t bin_groups;             // bin workgroups of the frame
   uint32_t spread;                 // segments per bin workgroup of the frame (see scene_chunk)
-  uint32_t chunk_cursor[2];        // bin_count, bin_fill
-  uint32_t piece;                  // pairs per work item
   unsigned long long total_pairs;
   uint32_t n_work;
-  uint32_t work_cursor;
   uint32_t flags;                  // CTL_* overflow bits
-  uint32_t n_split;                // tiles split over several work items (merge slots used)
-  unsigned long long samples;      // anti-aliased samples walked by tile_accum (2 pixels x 4 channels each)
-  unsigned long long lds_atomics;  // 64-bit LDS atomic wave instructions tile_accum's walk issued
+  uint32_t n_split;                // tiles split over several work items
+  uint32_t pad0;
+  // profiled frames only: anti-aliased samples walked by tile_accum (2 pixels x 4 channels each),
+  // and the 64-bit LDS atomic wave instructions its walk issued
+  unsigned long long samples;
+  unsigned long long lds_atomics;
   // tile work items ordered by size class (floor(log2(pairs))), largest class first: items per
-  // class, and the slots each class has handed out
+  // class, and the slots each class has handed out (frames above kPlanTiles tiles)
   uint32_t class_count[32];
   uint32_t class_cursor[32];
+  alignas(128) uint32_t item_cursor[kMaxGen];
+  alignas(128) uint32_t chunk_cursor0;  // bin_count
+  alignas(128) uint32_t chunk_cursor1;  // bin_fill
+  alignas(128) uint32_t work_cursor;    // tile_accum
+  uint32_t pad[31];
 };
+static_assert(sizeof(BatchCtl) % 128 == 0, "the cursors' lines end with the block");
 
 enum CtlFlags : uint32_t { CTL_PAIRS_OVERFLOW = 1u, CTL_ITEMS_OVERFLOW = 2u, CTL_SPLIT_OVERFLOW = 4u };
 // Any of these makes the frame's tile stage a no-op; the host grows the buffer and reruns.

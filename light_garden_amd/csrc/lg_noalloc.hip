@@ -168,7 +168,7 @@ int lg_accumulate_noalloc(lg_ctx* ctx, const lg_segments* segs, lg_image* img) {
                              split_tiles, kNaSplit, kNaPairs, min_piece, max_piece, (uint32_t)ctx->n_cu, false, st));
     LG_HIP(launch_bin(1, d_desc, 1, chunk_pre, cbase, d_ctl, counts, row_start, pairs, kNaPairs, n_tiles, bin_grid, st));
     LG_HIP(launch_tile_accum(d_desc, pairs, items, split_fx, d_ctl,
-                             tile, packed, hues ? 1024 : (int)ctx->tune.tile_block, ctx->n_cu, st));
+                             tile, packed, hues ? 1024 : (int)ctx->tune.tile_block, false, ctx->n_cu, st));
     LG_HIP(launch_tile_merge(d_desc, tile_scene, row_start, split_tiles, d_ctl, split_fx, kNaSplit, tile, ctx->n_cu,
                              st));
     LG_HIP(hipMemcpyAsync(&hc, d_ctl, sizeof(BatchCtl), hipMemcpyDeviceToHost, st));

@@ -40,11 +40,11 @@ struct DevView {
   }
 };
 
-// Byte offsets of a frame's parts in frame_in and stage_in, each a multiple of 16.
+// Byte offsets of a frame's parts in frame_in and stage_in, each a multiple of 128.
 struct FrameLayout {
   size_t tile_scene, px_pre, item_pre0, counters, ctl, row_count, total;
   FrameLayout(int n, int n_tiles) {
-    auto up = [](size_t b) { return (b + 15) & ~size_t(15); };
+    auto up = [](size_t b) { return (b + 127) & ~size_t(127); };  // (the control block's lines)
     tile_scene = up((size_t)n * sizeof(SceneDesc));
     px_pre = tile_scene + up((size_t)n_tiles * 4);
     item_pre0 = px_pre + up((size_t)n * 8);
@@ -226,7 +226,7 @@ static int enqueue(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, const
       Scope s(ctx, profile, "tile_accum", 0);
       LG_HIP(launch_tile_accum(d_descs, P.pairs.as<uint32_t>(), P.items.as<WorkItem>(),
                                P.split_fx.as<unsigned long long>(), d_ctl, L.tile, L.packed_only,
-                               L.hues ? 1024 : (int)ctx->tune.tile_block, ctx->n_cu, st));
+                               L.hues ? 1024 : (int)ctx->tune.tile_block, profile, ctx->n_cu, st));
     }
     {
       Scope s(ctx, profile, "tile_merge", 0);
