@@ -306,7 +306,7 @@ int lg_accumulate(lg_ctx* ctx, const lg_segments* segs, lg_image* img);
 /* lg_accumulate without device allocation. No counterpart in the reference: it is for callers
  * that cannot allocate device memory (serving loops with a fixed footprint, harnesses that
  * forbid hipMalloc). The same kernels and the same result bits as lg_accumulate, with their
- * scratch in one static device array of about 59 MB (56.4 MiB) per device (kept until the
+ * scratch in one static device array of about 63 MB (60.3 MiB) per device (kept until the
  * process ends): an image of at most 4096 x 4096 pixels (2048 x 2048 with 32-pixel tiles), at
  * most 8,388,608 segment-tile pairs and at most 128 tiles split over several work items per
  * call. Beyond a limit it returns LG_E_CAPACITY and deposits nothing. Calls on one device share
@@ -375,8 +375,8 @@ int lg_batch_render(lg_ctx* ctx, uint32_t n, lg_scene* const* scenes, const lg_p
  * `tile` none of them changes results: images are the same bits for every setting. */
 typedef struct lg_tuning {
   uint32_t rays_per_item;  /* rays per trace work item, [64, 2^20]; default 256 */
-  uint32_t min_piece;      /* smallest tile work item in segment-tile pairs, >= 64; default 4096 */
-  uint32_t max_piece;      /* largest tile work item, >= min_piece; default 8192; work items
+  uint32_t min_piece;      /* smallest tile work item in segment-tile pairs, >= 64; default 2048 */
+  uint32_t max_piece;      /* largest tile work item, >= min_piece; default 32768; work items
                               hold at most 32768 pairs whatever the setting (the fixed point
                               of two channels per LDS word is sized for that) */
   uint32_t trace_waves;    /* trace workgroups per compute unit, [1, 16]; default 4 */
@@ -396,7 +396,9 @@ typedef struct lg_tuning {
                               scene leaves no LDS room for it */
   uint32_t tile_block;     /* threads per tile workgroup, 1024 (one per compute unit) or 512
                               (two per compute unit), for frames at 64-pixel tiles whose every
-                              scene keeps two colour channels per LDS word; default 1024 */
+                              scene keeps two colour channels per LDS word; default 1024.
+                              Frames with traced scenes of one to three lights under the
+                              default blend always take 1024 */
 } lg_tuning;
 int lg_ctx_get_tuning(const lg_ctx* ctx, lg_tuning* out);
 int lg_ctx_set_tuning(lg_ctx* ctx, const lg_tuning* tuning);

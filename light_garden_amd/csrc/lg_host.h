@@ -131,7 +131,13 @@ struct lg_ctx {
   bool profiling = false;
   bool use_graphs = true;
   bool packed_accum = true;   // two channels per LDS word for scenes whose deposits are all >= 0
-  lg_tuning tune{256u, 4096u, 8192u, 4u, 16u, 64u, 2u, 1024u};
+  // Pieces: half a tile workgroup's even share, within [2048, 32768]. Below 2048 pairs the merge
+  // costs what the balance gains, above, the piece at a light's centre is the frame's tail (tile
+  // walk + merge, us, at 1024 / 2048 / 4096: 20k-ray frame 64 / 61 / 70, 75k-ray frame 93 / 91 /
+  // 101, 60k lines with vertex colours 319 / 316 / 362); a cap of 8192 splits tiles for nothing
+  // where the share is larger (8192 / 32768: 1M-ray frame 720 / 622, 1.6M segments at 4096x4096
+  // 4350 / 3730, 20 uneven scenes 736 / 678).
+  lg_tuning tune{256u, 2048u, 32768u, 4u, 16u, 64u, 2u, 1024u};
   std::vector<lg::StageRec> pending;  // events of the current call
   std::vector<hipEvent_t> event_pool;
   std::vector<lg_stage_time> last_times;
