@@ -232,6 +232,13 @@ int lg_segments_download(lg_segments* segs, float* pos, float* color0, float* co
  * reference's P2 = Point2<f64> vertices, tracer.rs:451-452). */
 int lg_segments_download_pos64(lg_segments* segs, double* pos64, uint64_t cap, uint64_t* count);
 
+/* The buffer's vertex pairs in ascending key order, which for traced segments is trace_all's
+ * order: xy gets 2 doubles and rgba 4 floats per vertex, 2 vertices per segment (FP64 end points
+ * of an LG_TRACE_FP64 trace, else the stored FP32 ones). LG_E_CAPACITY with *n_vertices set to the
+ * needed count when cap_vertices is too small. */
+int lg_segments_download_vertices(lg_segments* segs, double* xy, float* rgba, uint64_t cap_vertices,
+                                  uint64_t* n_vertices);
+
 /* ---- trace: Tracer::trace_all / Tracer::trace (tracer.rs:276-358, 360-493) ------------ */
 /* Traces every light of the scene into `out` (device). Segment order in the buffer is
  * unspecified; the key gives each segment's identity and the reference's emission order. */

@@ -187,6 +187,7 @@ FUNCTIONS = {
     "lg_segments_upload": (C.c_int, [_P, _P, _P, _P, C.c_uint64]),
     "lg_segments_download": (C.c_int, [_P, _P, _P, _P, _P, C.c_uint64, C.POINTER(C.c_uint64)]),
     "lg_segments_download_pos64": (C.c_int, [_P, _P, C.c_uint64, C.POINTER(C.c_uint64)]),
+    "lg_segments_download_vertices": (C.c_int, [_P, _P, _P, C.c_uint64, C.POINTER(C.c_uint64)]),
     "lg_trace": (C.c_int, [_P, C.POINTER(LgParams), _P]),
     "lg_trace_all": (C.c_int, [_P, C.POINTER(LgParams), _P, _P, C.c_uint64,
                                C.POINTER(C.c_uint64)]),

@@ -10,7 +10,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "build")
 LIB = os.path.join(BUILD, "liblg.so")
 SOURCES = ["lg_api.hip", "lg_pipeline.hip", "lg_server.hip", "lg_ron.hip", "lg_stringmod.hip", "lg_encode.hip",
-           "lg_trace.hip", "lg_accum.hip", "lg_noalloc.hip"]
+           "lg_trace.hip", "lg_accum.hip", "lg_noalloc.hip", "lg_order.hip"]
 
 # -packed-fp32-ops: no v_pk_{add,mul,fma}_f32 (packed FP32 has given wrong results on this
 # hardware pool); the host pass warns that it does not know the feature.

@@ -1738,7 +1738,7 @@ __global__ void fill_u32_kernel(uint32_t* p, uint64_t n, uint32_t v) {
 bool tile_size_supported(int tile) { return tile == 32 || tile == 64; }
 uint64_t merge_slot_u64() { return kSlotU64; }
 
-static uint64_t scan_scratch_elems(uint64_t n) {
+uint64_t scan_scratch_elems(uint64_t n) {
   uint64_t total = 0;
   while (n > 1) {
     uint64_t nb = (n + kScanBlock - 1) / kScanBlock;
@@ -1748,9 +1748,8 @@ static uint64_t scan_scratch_elems(uint64_t n) {
   return total + 1;
 }
 
-// Exclusive scan of n u32 (out may not alias in). scratch holds scan_scratch_elems(n) u32.
-static hipError_t launch_scan_exclusive(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* scratch,
-                                        hipStream_t st, unsigned long long* total) {
+hipError_t launch_scan_exclusive(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* scratch,
+                                 hipStream_t st, unsigned long long* total) {
   if (n == 0) return hipSuccess;
   uint64_t nb = (n + kScanBlock - 1) / kScanBlock;
   uint32_t* sums = scratch;

@@ -876,6 +876,7 @@ int lg_segments_upload(lg_segments* s, const float* pos, const float* color0, co
   s->max_abs = 0.0f;
   s->nonneg = true;
   s->hues = SceneHues{};
+  s->n_rays = 0;
   // a color1 equal to color0 bit for bit is no per-vertex colour: the accumulation then takes
   // the one-colour walk, which deposits the same bits
   s->one_color = !color1 || !n || std::memcmp(color0, color1, n * 16) == 0;
@@ -964,34 +965,9 @@ int lg_trace_all(lg_scene* scene, const lg_params* params, double* xy, float* rg
     lg_segments_destroy(segs);
     return rc;
   }
-  uint64_t n = segs->count;
-  *n_vertices = 2 * n;
-  if (cap_vertices < 2 * n || (n && (!xy || !rgba))) {
-    lg_segments_destroy(segs);
-    return fail(LG_E_CAPACITY, "trace_all: output too small");
-  }
-  std::vector<float> pos(4 * n), col(4 * n);
-  std::vector<double> pos64;
-  std::vector<uint64_t> key(n);
-  rc = lg_segments_download(segs, pos.data(), col.data(), nullptr, key.data(), n, nullptr);
-  if (!rc && segs->has_pos64) {
-    pos64.resize(4 * n);
-    rc = lg_segments_download_pos64(segs, pos64.data(), n, nullptr);
-  }
+  rc = lg_segments_download_vertices(segs, xy, rgba, cap_vertices, n_vertices);
   lg_segments_destroy(segs);
-  if (rc) return rc;
-  std::vector<uint64_t> order(n);
-  std::iota(order.begin(), order.end(), 0ull);
-  std::sort(order.begin(), order.end(), [&](uint64_t a, uint64_t b) { return key[a] < key[b]; });
-  for (uint64_t i = 0; i < n; i++) {
-    uint64_t s = order[i];
-    for (int v = 0; v < 2; v++) {
-      xy[4 * i + 2 * v] = pos64.empty() ? (double)pos[4 * s + 2 * v] : pos64[4 * s + 2 * v];
-      xy[4 * i + 2 * v + 1] = pos64.empty() ? (double)pos[4 * s + 2 * v + 1] : pos64[4 * s + 2 * v + 1];
-      std::memcpy(rgba + 8 * i + 4 * v, &col[4 * s], 16);
-    }
-  }
-  return LG_OK;
+  return rc;
 }
 
 // ---- image ---------------------------------------------------------------------------------

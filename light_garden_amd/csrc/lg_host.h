@@ -68,6 +68,11 @@ struct SmScratchDeleter {
   void operator()(SmScratch* p) const;
 };
 
+struct OrderScratch;  // ordered downloads (lg_order.hip)
+struct OrderScratchDeleter {
+  void operator()(OrderScratch* s) const;
+};
+
 int fail(int code, const std::string& msg);
 
 // ---- kernel launchers (lg_trace.hip, lg_accum.hip) ---------------------------------------------
@@ -83,6 +88,12 @@ hipError_t launch_trace(const SceneDesc* descs, int n_scenes, uint32_t gen, uint
                         int cap_verts, uint32_t* item_pre_next, int grid, hipStream_t stream);
 int trace_block();
 bool tile_size_supported(int tile);
+// Exclusive scan of n u32 (out may not alias in). scratch holds scan_scratch_elems(n) u32. With
+// total (zeroed by an earlier kernel): *total += the 64-bit sum of the elements, or bit 63 set when
+// 2048 consecutive elements sum to 2^32 or more (the 32-bit offsets wrapped).
+uint64_t scan_scratch_elems(uint64_t n);
+hipError_t launch_scan_exclusive(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* scratch, hipStream_t st,
+                                 unsigned long long* total);
 hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t st);
 hipError_t launch_build_chunks(const SceneDesc* descs, int n_scenes, uint32_t chunk_min, uint32_t target,
                                uint32_t groups, uint32_t* chunk_pre, uint32_t* cbase, BatchCtl* ctl, hipStream_t st);
@@ -143,6 +154,7 @@ struct lg_ctx {
   std::vector<lg_stage_time> last_times;
   std::unique_ptr<lg::Pipeline, lg::PipelineDeleter> pipe;
   std::unique_ptr<lg::SmScratch, lg::SmScratchDeleter> sm;
+  std::unique_ptr<lg::OrderScratch, lg::OrderScratchDeleter> order;
   lg::DevBuf encode_table;  // 65536 u8: the 8-bit encode of every half (built on first use)
   bool encode_table_ready = false;
 
@@ -189,6 +201,7 @@ struct lg_segments {
   // or with an identical color1, StringMods without modulo colours): col1 is not read
   bool one_color = true;
   lg::SceneHues hues;         // traced segments: the colours of their lights
+  uint64_t n_rays = 0;        // traced segments: the scene's rays (keys hold their index); else 0
   lg::DevBuf pos, col0, col1, key, pos64;
   bool has_pos64 = false;
 };

@@ -617,6 +617,7 @@ static int batch_finish(lg_ctx* ctx, Pipeline& P, bool profile, Batch& B, bool* 
       e.segs->nonneg = e.scene->light_nonneg;
       e.segs->one_color = true;
       e.segs->hues = scene_hues(e.scene);
+      e.segs->n_rays = e.scene->n_primary;
       e.scene->seg_hint = std::max(e.scene->seg_hint, segs);
     }
   }

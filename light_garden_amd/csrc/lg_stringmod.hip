@@ -554,6 +554,7 @@ int lg_string_mod_draw(lg_ctx* ctx, uint32_t n, const lg_string_mod* mods, lg_se
   out->max_abs = max_abs;
   out->nonneg = nonneg;
   out->hues = lg::SceneHues{};
+  out->n_rays = 0;
   // without modulo colours both ends of every segment take their StringMod's colour
   // (get_color, string_mod.rs:124-150): col1 is then neither written nor read
   out->one_color = mrc.empty();

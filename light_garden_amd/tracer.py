@@ -324,6 +324,16 @@ class Segments:
                  c1.ctypes.data, key.ctypes.data, n, C.byref(cnt))
         return pos, c0, c1, key
 
+    def vertices(self):
+        """The vertex pairs in key order (lg_segments_download_vertices): xy float64 (2S, 2), rgba
+        float32 (2S, 4)."""
+        n = self.count()
+        xy = np.empty((2 * n, 2), np.float64)
+        rgba = np.empty((2 * n, 4), np.float32)
+        cnt = C.c_uint64()
+        abi.call("lg_segments_download_vertices", self._h, xy.ctypes.data, rgba.ctypes.data, 2 * n, C.byref(cnt))
+        return xy, rgba
+
     def download_pos64(self):
         n = self.count()
         pos = np.empty((n, 4), np.float64)
@@ -453,6 +463,7 @@ class Tracer:
         self.chunk_size = 100               # tracer.rs:39 (rayon chunking; no GPU meaning)
         self.canvas_bounds = tuple(canvas_bounds)  # left, right, bottom, top
         self.fp64 = False
+        self._trace_segs = None
         self._h = C.c_void_p()
         abi.call("lg_scene_create", self.ctx.handle, C.byref(self._h))
         self.ctx._adopt(self)
@@ -543,17 +554,11 @@ class Tracer:
 
     def trace_all(self):
         """Tracer::trace_all (tracer.rs:276): vertex pairs in the reference's order, as
-        (xy float64 (2S, 2), rgba float32 (2S, 4)). One trace; the segment keys give the
-        order (light, ray, depth, parent, reflected before refracted)."""
-        segs = self.trace()
-        pos, col, _, key = segs.download()
-        if self.fp64:
-            pos = segs.download_pos64()
-        segs.close()
-        order = np.argsort(key, kind="stable")
-        xy = np.asarray(pos, np.float64)[order].reshape(-1, 2)
-        rgba = np.repeat(col[order], 2, axis=0)
-        return xy, rgba
+        (xy float64 (2S, 2), rgba float32 (2S, 4)). One trace into a buffer that the tracer
+        keeps; the library orders it (light, ray, depth, parent, reflected before refracted)."""
+        if self._trace_segs is None or not self._trace_segs.handle:
+            self._trace_segs = Segments(self.ctx)
+        return self.trace(self._trace_segs).vertices()
 
     def render(self, segs: Segments, img: Image):
         """One frame: clear, trace, accumulate, resolve (LightGarden::draw + Renderer::render)."""
@@ -562,6 +567,8 @@ class Tracer:
         abi.call("lg_render", self._h, C.byref(p), segs.handle, img.handle)
 
     def close(self):
+        if getattr(self, "_trace_segs", None) is not None:
+            self._trace_segs.close()
         if self._h:
             abi.load().lg_scene_destroy(self._h)
             self._h = C.c_void_p()
