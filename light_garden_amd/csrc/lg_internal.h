@@ -304,7 +304,6 @@ constexpr int kMaxGen = kPathBits;
 // for those too.
 struct BatchCtl {
   uint32_t n_items_gen[kMaxGen];   // trace items per generation
-  uint32_t gen_done[kMaxGen];      // trace workgroups finished per generation
   uint32_t n_chunks;
   uint32_t chunk;                  // segments per bin chunk (at least; see scene_chunk)
   uint32_t bin_groups;             // bin workgroups of the frame
@@ -323,6 +322,7 @@ struct BatchCtl {
   uint32_t class_count[32];
   uint32_t class_cursor[32];
   alignas(128) uint32_t item_cursor[kMaxGen];
+  alignas(128) uint32_t gen_done[kMaxGen];  // trace workgroups finished per generation
   alignas(128) uint32_t chunk_cursor0;  // bin_count
   alignas(128) uint32_t chunk_cursor1;  // bin_fill
   alignas(128) uint32_t work_cursor;    // tile_accum

@@ -1147,6 +1147,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const uint32_t n_items = ctl->n_items_gen[gen_ix];
+  // Workgroup b's first item is b: the others have none. They leave before any atomic or fence
+  // (with both, the 900 idle workgroups of a late generation held up the working ones by 13 us).
+  if (blockIdx.x >= n_items) return;
   int loaded = -1;
   if (threadIdx.x < kMaxChunk) s_lcnt[threadIdx.x] = 0;
 
@@ -1411,20 +1414,19 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
       }
     }
   }
-  // The last workgroup to finish builds the next launch's work list (its child counts are
-  // final once every workgroup of this launch is done).
+  // The last of the workgroups that had items builds the next launch's work list. Its child counts
+  // are final then: every add to them has returned its value before its workgroup counts itself
+  // done, and both are performed where all XCDs see them, so no fence is needed (a device-scope
+  // release writes back an XCD's whole L2). The rays themselves are read by the next launch only.
   if (item_pre_next) {
     __shared__ bool s_last;
     __syncthreads();
     if (threadIdx.x == 0) {
-      __threadfence();
-      s_last = atomicAdd(&ctl->gen_done[gen_ix], 1u) == gridDim.x - 1;
+      const uint32_t working = n_items < gridDim.x ? n_items : gridDim.x;
+      s_last = __hip_atomic_fetch_add(&ctl->gen_done[gen_ix], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == working - 1;
     }
     __syncthreads();
-    if (s_last) {
-      __threadfence();
-      build_items_block<BLOCK>(descs, n_scenes, gen_ix + chunk, rpi, item_pre_next, ctl);
-    }
+    if (s_last) build_items_block<BLOCK>(descs, n_scenes, gen_ix + chunk, rpi, item_pre_next, ctl);
   }
 }
 
