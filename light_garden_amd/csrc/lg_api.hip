@@ -526,6 +526,12 @@ int compile_scene(lg_scene* sc, hipStream_t st) {
     box32[o] = make_float4(round_down(boxes[o].lo[0]), round_down(boxes[o].lo[1]), round_up(boxes[o].hi[0]),
                            round_up(boxes[o].hi[1]));
   if ((rc = upload(sc->obj_box, box32.data(), box32.size(), st))) return rc;
+  std::vector<float4> medium(box32);
+  const float4 none = make_float4(INFINITY, INFINITY, -INFINITY, -INFINITY);
+  for (size_t o = 0; o < medium.size(); o++)
+    if ((flags[o] & (OBJ_MATERIAL | OBJ_CLOSED)) != (OBJ_MATERIAL | OBJ_CLOSED)) medium[o] = none;
+  while (medium.size() % kMediumBlock) medium.push_back(none);
+  if ((rc = upload(sc->medium_box, medium.data(), medium.size(), st))) return rc;
   std::vector<Box2> walk_boxes;  // the BVH holds the objects of the walk
   std::vector<int32_t> walk_rec;
   for (size_t o = 0; o < obj_rec.size(); o++)

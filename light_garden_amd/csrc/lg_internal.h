@@ -150,6 +150,10 @@ struct alignas(16) BvhNode {
 };
 static_assert(sizeof(BvhNode) == 48, "BvhNode is three float4");
 
+// Boxes of SceneDesc::medium_box are read in groups of this many (the list is padded with empty
+// ones).
+constexpr int kMediumBlock = 4;
+
 constexpr int kMaxRecords = 1024;      // records resident in LDS per trace workgroup
 constexpr int kMaxObjects = 1024;
 constexpr int kMaxPolyVertices = 1024; // vertices of all polygons in a scene
@@ -236,6 +240,8 @@ struct SceneDesc {
   const LG_G uint32_t* obj_flags;
   const LG_G int32_t* obj_rec;
   const LG_G float4* obj_box;      // per object: padded world box {lo.x, lo.y, hi.x, hi.y}
+  const LG_G float4* medium_box;   // the same for objects with a material and an inside, an empty
+                                   // box for others; kMediumBlock of them at a time
   const LG_G void* verts;          // polygon vertices in the culling precision
   const LG_G double* verts64;
   const LG_G DevLight* lights;

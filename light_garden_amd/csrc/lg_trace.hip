@@ -1272,24 +1272,44 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
         }
       }
       // The medium a ray exits into: the first other material object, in scene order, that
-      // contains the exit point (tracer.rs:431-440), else air. The loop over objects is
-      // uniform across the wave (its flags and padded boxes are scalar loads); a lane runs the
-      // exact FP64 inside test only for objects whose box holds its point, and stops at the
-      // first that contains it.
-      {
-        // the object's flags and padded box: wave-uniform, read with scalar loads
-        const LG_K uint32_t* kflags = (const LG_K uint32_t*)D.obj_flags;
-        const LG_K float* kbox = (const LG_K float*)D.obj_box;
-        uint64_t seeking = __ballot(seek);
-        for (int o = 0; seeking && o < n_objs; o++) {
-          if (!(kflags[o] & OBJ_MATERIAL)) continue;
-          const float bx0 = kbox[4 * o], bx1 = kbox[4 * o + 1], bx2 = kbox[4 * o + 2], bx3 = kbox[4 * o + 3];
-          if (seek && o != obj && px >= (double)bx0 && px <= (double)bx2 && py >= (double)bx1 &&
-              py <= (double)bx3 && contains_object<double>(recs64, verts64, s_obj_rec[o], px, py)) {
-            n2 = gen(D.obj_n64)[o];
-            seek = false;
+      // contains the exit point (tracer.rs:431-440), else air. The boxes of 64 objects at a time
+      // are tested for every lane, without a branch between them (they are the same for the wave:
+      // scalar loads, four boxes each), and leave a bit per object whose padded box holds the
+      // lane's point; a lane then runs the exact FP64 inside test on its own few candidates, in
+      // order, up to the first that contains it. FP32 points will do for the boxes, which are
+      // padded by 1e-5 (1 + |coordinates|). (With a branch and two dependent scalar loads per
+      // object the search took 4 to 8 us of a 33 us step with 64 objects; frames, us: 75k rays, 23
+      // objects 419 -> 398, 20 scenes of 1 to 160 objects 2174 -> 2000.)
+      if (__ballot(seek)) {
+        const LG_K float* const boxes = (const LG_K float*)D.medium_box;
+        const float fx = (float)px, fy = (float)py;
+        for (int base = 0; base < n_objs; base += 64) {
+          const int n = n_objs - base < 64 ? n_objs - base : 64;
+          uint32_t half[2] = {0u, 0u};
+#pragma unroll
+          for (int h = 0; h < 2; h++)
+            for (int o = 32 * h; o < n && o < 32 * (h + 1); o += kMediumBlock) {
+              const LG_K float* const b = boxes + 4 * (base + o);
+#pragma unroll
+              for (int k = 0; k < kMediumBlock; k++)
+                if ((fx >= b[4 * k]) & (fy >= b[4 * k + 1]) & (fx <= b[4 * k + 2]) & (fy <= b[4 * k + 3]))
+                  half[h] |= 1u << ((o + k) & 31);
+            }
+          uint64_t cand = (uint64_t)half[1] << 32 | half[0];
+          if ((unsigned)(obj - base) < 64u) cand &= ~(1ull << (obj - base));
+          if (!seek) cand = 0ull;
+          while (__ballot(cand != 0ull)) {
+            if (cand) {
+              const int o = base + __builtin_ctzll(cand);
+              cand &= cand - 1ull;
+              if (contains_object<double>(recs64, verts64, s_obj_rec[o], px, py)) {
+                n2 = gen(D.obj_n64)[o];
+                seek = false;
+                cand = 0ull;
+              }
+            }
           }
-          seeking = __ballot(seek);
+          if (!__ballot(seek)) break;
         }
       }
       if (hit) {
