@@ -3,7 +3,7 @@
 The GPU path has eight launch knobs (lg_tuning in include/lg.h): rays per trace work item,
 trace workgroups per compute unit, bounce generations per trace launch (bounce-chunking: the
 children of the launch's earlier generations stay on chip), the smallest / largest tile work
-item in segment-tile pairs, the object count from which a scene's culling pass walks its BVH,
+item in segment-tile pairs, the object count from which a scene's culling pass goes by boxes,
 the screen tile edge of the accumulation (32 or 64 pixels) and the threads of a tile
 workgroup (one of 1024 or two of 512 per compute unit). All but the tile edge change
 no result (images are the same bits for every setting); the tile edge moves images within the

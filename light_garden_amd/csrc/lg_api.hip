@@ -381,34 +381,6 @@ static uint32_t spread_bits(uint32_t v) {  // 16 bits -> even bit positions
   return v;
 }
 
-// Preorder node of objects order[lo, hi) (median split); returns its index.
-static int bvh_build(std::vector<BvhNode>& nodes, const std::vector<int>& order, const std::vector<Box2>& boxes,
-                     const std::vector<int32_t>& obj_rec, int lo, int hi) {
-  const int idx = (int)nodes.size();
-  nodes.push_back(BvhNode{});
-  Box2 b = empty_box();
-  if (hi - lo <= kBvhLeaf) {
-    BvhNode& N = nodes[idx];
-    N.count = hi - lo;
-    for (int k = 0; k < kBvhLeaf; k++) N.top[k] = k < hi - lo ? obj_rec[order[lo + k]] : -1;
-    for (int k = lo; k < hi; k++) b.add(boxes[order[k]]);
-  } else {
-    const int mid = (lo + hi) / 2;
-    bvh_build(nodes, order, boxes, obj_rec, lo, mid);
-    bvh_build(nodes, order, boxes, obj_rec, mid, hi);
-    for (int k = lo; k < hi; k++) b.add(boxes[order[k]]);
-    nodes[idx].count = 0;
-    for (int k = 0; k < kBvhLeaf; k++) nodes[idx].top[k] = -1;
-  }
-  BvhNode& N = nodes[idx];
-  N.lo[0] = round_down(b.lo[0]);
-  N.lo[1] = round_down(b.lo[1]);
-  N.hi[0] = round_up(b.hi[0]);
-  N.hi[1] = round_up(b.hi[1]);
-  N.skip = (int)nodes.size();
-  return idx;
-}
-
 // Object boxes padded by 1e-5 (1 + |coordinates|), far more than the FP32 culling pass's
 // error and than the rounding of an FP64 inside test: a point outside an object's padded box
 // is neither hit by a culled ray nor contained.
@@ -437,10 +409,9 @@ static std::vector<Box2> object_boxes(const std::vector<Rec<double>>& recs, cons
   return boxes;
 }
 
-// The scene's BVH over the padded object boxes: leaves of kBvhLeaf objects in Morton order of
-// their box centres.
-static std::vector<BvhNode> build_bvh(const std::vector<Box2>& boxes, const std::vector<int32_t>& obj_rec) {
-  const int n = (int)obj_rec.size();
+// Objects in Morton order of their box centres.
+static std::vector<int> morton_order(const std::vector<Box2>& boxes) {
+  const int n = (int)boxes.size();
   Box2 all = empty_box();
   for (int o = 0; o < n; o++) all.add(boxes[o]);
   std::vector<uint32_t> code(n);
@@ -455,9 +426,52 @@ static std::vector<BvhNode> build_bvh(const std::vector<Box2>& boxes, const std:
   std::vector<int> order(n);
   for (int o = 0; o < n; o++) order[o] = o;
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return code[a] < code[b]; });
-  std::vector<BvhNode> nodes;
-  if (n > 0) bvh_build(nodes, order, boxes, obj_rec, 0, n);
-  return nodes;
+  return order;
+}
+
+static float4 box_f32(const Box2& b) {
+  return make_float4(round_down(b.lo[0]), round_down(b.lo[1]), round_up(b.hi[0]), round_up(b.hi[1]));
+}
+
+// The culling blocks of objects with the given boxes and first records (CullBlock).
+struct CullLists {
+  std::vector<CullBlock> blocks;
+  std::vector<float4> box;
+  std::vector<int32_t> rec;
+};
+static CullLists build_blocks(const std::vector<Box2>& boxes, const std::vector<int32_t>& top,
+                              const std::vector<Rec<double>>& recs) {
+  CullLists C;
+  const std::vector<int> order = morton_order(boxes);
+  for (size_t b = 0; b < order.size(); b += kCullBlock) {
+    const size_t n = std::min<size_t>(kCullBlock, order.size() - b);
+    CullBlock B;
+    std::memset(&B, 0, sizeof(B));
+    B.first = (int32_t)C.box.size();
+    B.n = (int32_t)n;
+    Box2 all = empty_box();
+    uint64_t mask[8] = {};
+    for (size_t k = 0; k < n; k++) {
+      const int o = order[b + k];
+      all.add(boxes[o]);
+      mask[recs[top[o]].kind & 7] |= 1ull << k;
+      C.box.push_back(box_f32(boxes[o]));
+      C.rec.push_back(top[o]);
+    }
+    const float4 u = box_f32(all);
+    B.box[0] = u.x;
+    B.box[1] = u.y;
+    B.box[2] = u.z;
+    B.box[3] = u.w;
+    for (uint64_t m : mask)
+      if (m) B.kind[B.n_kinds++] = m;
+    while (C.box.size() % kBoxGroup) {  // (no kind has a bit for these)
+      C.box.push_back(u);
+      C.rec.push_back(-1);
+    }
+    C.blocks.push_back(B);
+  }
+  return C;
 }
 
 // Uploads on `st`, the stream of the frame that will read the scene.
@@ -522,26 +536,26 @@ int compile_scene(lg_scene* sc, hipStream_t st) {
   if ((rc = upload(sc->verts64, verts.data(), verts.size(), st))) return rc;
   const std::vector<Box2> boxes = object_boxes(recs, verts, obj_rec);
   std::vector<float4> box32(boxes.size());
-  for (size_t o = 0; o < boxes.size(); o++)
-    box32[o] = make_float4(round_down(boxes[o].lo[0]), round_down(boxes[o].lo[1]), round_up(boxes[o].hi[0]),
-                           round_up(boxes[o].hi[1]));
+  for (size_t o = 0; o < boxes.size(); o++) box32[o] = box_f32(boxes[o]);
   if ((rc = upload(sc->obj_box, box32.data(), box32.size(), st))) return rc;
   std::vector<float4> medium(box32);
   const float4 none = make_float4(INFINITY, INFINITY, -INFINITY, -INFINITY);
   for (size_t o = 0; o < medium.size(); o++)
     if ((flags[o] & (OBJ_MATERIAL | OBJ_CLOSED)) != (OBJ_MATERIAL | OBJ_CLOSED)) medium[o] = none;
-  while (medium.size() % kMediumBlock) medium.push_back(none);
+  while (medium.size() % kBoxGroup) medium.push_back(none);
   if ((rc = upload(sc->medium_box, medium.data(), medium.size(), st))) return rc;
-  std::vector<Box2> walk_boxes;  // the BVH holds the objects of the walk
+  std::vector<Box2> walk_boxes;  // the blocks hold the objects of the walk
   std::vector<int32_t> walk_rec;
   for (size_t o = 0; o < obj_rec.size(); o++)
     if (recs[obj_rec[o]].kind != REC_TREE) {
       walk_boxes.push_back(boxes[o]);
       walk_rec.push_back(obj_rec[o]);
     }
-  const std::vector<BvhNode> bvh = build_bvh(walk_boxes, walk_rec);
-  if ((rc = upload(sc->bvh_dev, bvh.data(), bvh.size(), st))) return rc;
-  sc->n_bvh = (int)bvh.size();
+  const CullLists cull = build_blocks(walk_boxes, walk_rec, recs);
+  if ((rc = upload(sc->blocks, cull.blocks.data(), cull.blocks.size(), st))) return rc;
+  if ((rc = upload(sc->block_box, cull.box.data(), cull.box.size(), st))) return rc;
+  if ((rc = upload(sc->block_rec, cull.rec.data(), cull.rec.size(), st))) return rc;
+  sc->n_blocks = (int)cull.blocks.size();
   // lights
   if (sc->lights.size() > (size_t)kMaxLights) return fail(LG_E_UNSUPPORTED, "scene: too many lights");
   std::vector<DevLight> dl;

@@ -148,7 +148,7 @@ struct lg_ctx {
   // 101, 60k lines with vertex colours 319 / 316 / 362); a cap of 8192 splits tiles for nothing
   // where the share is larger (8192 / 32768: 1M-ray frame 720 / 622, 1.6M segments at 4096x4096
   // 4350 / 3730, 20 uneven scenes 736 / 678).
-  lg_tuning tune{256u, 2048u, 32768u, 4u, 16u, 64u, 2u, 1024u};
+  lg_tuning tune{256u, 2048u, 32768u, 4u, 8u, 64u, 2u, 1024u};
   std::vector<lg::StageRec> pending;  // events of the current call
   std::vector<hipEvent_t> event_pool;
   std::vector<lg_stage_time> last_times;
@@ -179,9 +179,10 @@ struct lg_scene {
   std::vector<int32_t> h_obj_rec;
   std::vector<double> h_verts64;
   int n_recs = 0, n_objs = 0, n_verts = 0;
-  lg::DevBuf recs32, recs64, obj_n64, obj_flags, obj_rec, obj_box, medium_box, verts32, verts64, lights_dev, bvh_dev;
+  lg::DevBuf recs32, recs64, obj_n64, obj_flags, obj_rec, obj_box, medium_box, verts32, verts64, lights_dev;
+  lg::DevBuf blocks, block_box, block_rec;  // culling blocks (CullBlock)
   lg::DevBuf tree_rec;        // first records of the Logic trees of more than two primitives
-  int n_bvh = 0;              // BVH nodes built for the scene (0: none)
+  int n_blocks = 0;
   int n_trees = 0;
   lg::DevBuf q0, q1;          // ray queues (QRay<double>)
   uint64_t q_cap = 0;         // rays per queue

@@ -137,22 +137,22 @@ __host__ __device__ inline bool contains_object(const Rec<T>* recs, const T* ver
 // Per-object flags.
 enum ObjFlags : uint32_t { OBJ_MATERIAL = 1u, OBJ_CLOSED = 2u };
 
-// Bounding-volume hierarchy over a scene's objects, nodes in preorder: an internal node's
-// first child follows it, `skip` is the node after its subtree. A leaf (count > 0) names up
-// to kBvhLeaf objects by their first record. Boxes are FP32, padded so that every hit the
-// FP32 culling pass can report lies inside its object's box.
-constexpr int kBvhLeaf = 4;
-struct alignas(16) BvhNode {
-  float lo[2], hi[2];
-  int32_t skip;
-  int32_t count;
-  int32_t top[kBvhLeaf];
+// Bounding volumes over a scene's objects (Logic trees of more than two primitives aside): the
+// objects in Morton order of their box centres, cut into blocks of up to kCullBlock. A block has
+// the union of its objects' boxes and, per shape kind, the objects of that kind as bits. The
+// boxes, kBoxGroup to a read (a block's are padded to that), are FP32 and padded so that every hit
+// the FP32 culling pass can report lies inside its object's box.
+constexpr int kCullBlock = 64;
+constexpr int kBoxGroup = 4;
+struct alignas(16) CullBlock {
+  float box[4];         // lo.x lo.y hi.x hi.y
+  uint64_t kind[8];     // n_kinds masks, disjoint, together the block's objects
+  int32_t first;        // of its boxes and first records
+  int32_t n;
+  int32_t n_kinds;
+  int32_t pad;
 };
-static_assert(sizeof(BvhNode) == 48, "BvhNode is three float4");
-
-// Boxes of SceneDesc::medium_box are read in groups of this many (the list is padded with empty
-// ones).
-constexpr int kMediumBlock = 4;
+static_assert(sizeof(CullBlock) == 96, "six float4");
 
 constexpr int kMaxRecords = 1024;      // records resident in LDS per trace workgroup
 constexpr int kMaxObjects = 1024;
@@ -241,14 +241,16 @@ struct SceneDesc {
   const LG_G int32_t* obj_rec;
   const LG_G float4* obj_box;      // per object: padded world box {lo.x, lo.y, hi.x, hi.y}
   const LG_G float4* medium_box;   // the same for objects with a material and an inside, an empty
-                                   // box for others; kMediumBlock of them at a time
+                                   // box for others, padded to kBoxGroup
   const LG_G void* verts;          // polygon vertices in the culling precision
   const LG_G double* verts64;
   const LG_G DevLight* lights;
-  const LG_G BvhNode* bvh;         // NULL: the culling pass walks every record
+  const LG_G CullBlock* blocks;    // culling by boxes; n_blocks = 0: the pass walks every record
+  const LG_G float4* block_box;    // the blocks' objects: padded boxes,
+  const LG_G int32_t* block_rec;   // and first records
   const LG_G int32_t* tree_rec;    // first record of each object that is a Logic tree of more
                                    // than two primitives (the object walk skips these)
-  int32_t n_bvh;                   // nodes
+  int32_t n_blocks;
   int32_t n_trees;
   int32_t n_recs, n_objs, n_verts, n_lights;
   uint64_t n_primary;

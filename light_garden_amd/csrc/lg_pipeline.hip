@@ -112,9 +112,9 @@ void PipelineDeleter::operator()(Pipeline* p) const { delete p; }
 
 void pipeline_destroy(lg_ctx* ctx) { ctx->pipe.reset(); }
 
-// Whether a scene's culling pass walks its BVH (FP32 traces of scenes with enough objects).
-static bool scene_uses_bvh(const lg_ctx* ctx, const lg_scene* sc, bool fp64) {
-  return !fp64 && sc->n_bvh > 0 && (uint32_t)sc->n_objs >= ctx->tune.bvh_min_objects;
+// Whether a scene's culling pass goes by its objects' boxes.
+static bool scene_uses_boxes(const lg_ctx* ctx, const lg_scene* sc) {
+  return sc->n_blocks > 0 && (uint32_t)sc->n_objs >= ctx->tune.bvh_min_objects;
 }
 
 struct Layout {
@@ -433,9 +433,10 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
       D.verts = gbl(L.fp64 ? sc->verts64.p : sc->verts32.p);
       D.verts64 = gbl(sc->verts64.as<const double>());
       D.lights = gbl(sc->lights_dev.as<const DevLight>());
-      const bool bvh = scene_uses_bvh(ctx, sc, L.fp64);
-      D.bvh = gbl(bvh ? sc->bvh_dev.as<const BvhNode>() : nullptr);
-      D.n_bvh = bvh ? sc->n_bvh : 0;
+      D.blocks = gbl(sc->blocks.as<const CullBlock>());
+      D.block_box = gbl(sc->block_box.as<const float4>());
+      D.block_rec = gbl(sc->block_rec.as<const int32_t>());
+      D.n_blocks = scene_uses_boxes(ctx, sc) ? sc->n_blocks : 0;
       D.tree_rec = gbl(sc->tree_rec.as<const int32_t>());
       D.n_trees = sc->n_trees;
       D.n_recs = sc->n_recs;

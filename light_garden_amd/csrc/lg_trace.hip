@@ -71,15 +71,18 @@ __device__ __forceinline__ void normalize_v(T& x, T& y) {
   }
 }
 
-// The FP32 culling pass reads its records and BVH nodes with wave-uniform indices (the object
+// The FP32 culling pass over every object reads its records with wave-uniform indices (the object
 // loop is the same for every lane). Read through the constant address space from the scene's
 // device buffers, those loads become scalar loads: a record's fields arrive in SGPRs and feed
 // the vector ALU directly, instead of taking VGPRs after an LDS read, and the scalar data
-// cache holds a scene's records (64 B each) for every wave of the compute unit.
+// cache holds a scene's records (64 B each) for every wave of the compute unit. The pass by boxes
+// reads the boxes so, and the records of its candidates, each lane its own, as four 16-byte vector
+// loads (they hit the L1).
 #define LG_K __attribute__((address_space(4)))
 typedef int lg_v4i __attribute__((ext_vector_type(4)));
-struct RecK {
-  const LG_K lg_v4i* p;  // four per record
+template <typename P>
+struct RecAt {
+  P p;  // four lg_v4i per record
   __device__ __forceinline__ Rec<float> operator[](int i) const {
     struct V {
       lg_v4i a, b, c, d;
@@ -88,30 +91,17 @@ struct RecK {
     return __builtin_bit_cast(Rec<float>, v);
   }
 };
-struct NodeK {
-  const LG_K lg_v4i* p;  // three per node
-  __device__ __forceinline__ BvhNode operator[](int i) const {
-    struct V {
-      lg_v4i a, b, c;
-    };
-    const V v{p[3 * i], p[3 * i + 1], p[3 * i + 2]};
-    return __builtin_bit_cast(BvhNode, v);
-  }
-};
+using RecK = RecAt<const LG_K lg_v4i*>;  // the same record for every lane
+using RecV = RecAt<const lg_v4i*>;       // a record per lane
 
-// One field of a record or node at an index known only at run time (still wave-uniform): read
-// from the source itself, since indexing into a copy of the whole record would put the copy on
-// the stack.
+// One field of a record at an index known only at run time: read from the source itself, since
+// indexing into a copy of the whole record would put the copy on the stack.
 template <typename T>
 __device__ __forceinline__ T rec_param(const Rec<T>* recs, int i, int m) {
   return recs[i].p[m];
 }
 __device__ __forceinline__ float rec_param(const RecK& recs, int i, int m) {
   return reinterpret_cast<const LG_K float*>(recs.p + 4 * i)[offsetof(Rec<float>, p) / 4 + m];
-}
-__device__ __forceinline__ int node_top(const BvhNode* nodes, int i, int k) { return nodes[i].top[k]; }
-__device__ __forceinline__ int node_top(const NodeK& nodes, int i, int k) {
-  return reinterpret_cast<const LG_K int*>(nodes.p + 3 * i)[offsetof(BvhNode, top) / 4 + k];
 }
 
 // FP32 -> FP64 step threshold: a branch quantity q is recomputed in FP64 when
@@ -720,54 +710,84 @@ __device__ __forceinline__ int eval_object(const RayT<T>& r, RS recs, const Rec<
   return i + 1;
 }
 
-// The culling pass for one ray: every object in scene order, or (n_nodes > 0) the objects
-// of the BVH leaves the wave enters. The node index is wave-uniform; a node is entered when
-// some lane's ray meets its box at a t in [tmin, t_best + 4e-5 (1 + t_best)], and an
-// entered leaf's objects are evaluated for every lane, as the full walk evaluates every
-// object. Each object that can hit within that window lies in an entered leaf (boxes are
-// padded beyond the FP32 error), so the winner, and any runner-up that the FP64 refinement
-// looks at (within 1e-5 (1 + t)), are those of the full walk. One loop serves both walks so
-// that eval_object is inlined once. Inlined, so that the compiler sees which records are in
-// LDS and which in global memory. Logic trees of more than two primitives are skipped here.
-template <typename T, typename RS, typename NS>
-__device__ __forceinline__ Nearest<T> walk_objects(const RayT<T>& r, RS recs, const Rec<double>* recs64,
-                                                   const T* verts, int n_recs, NS nodes, int n_nodes) {
-  Nearest<T> nb;
-  nearest_init(nb);
+// The culling pass for one ray over every object in scene order. Logic trees of more than two
+// primitives are not among them. Inlined, so that the compiler sees which records are in LDS and
+// which in global memory.
+template <typename T, typename RS>
+__device__ __forceinline__ void walk_objects(const RayT<T>& r, RS recs, const Rec<double>* recs64, const T* verts,
+                                             int n_recs, Nearest<T>& nb) {
+  for (int rec = 0; rec < n_recs;) rec = eval_object<T, false>(r, recs, recs64, verts, rec, nb);
+}
+
+// The scene's culling blocks; tops: the blocks' first records in LDS.
+struct CullView {
+  const LG_K CullBlock* blocks;
+  const LG_K float* box;
+  const int32_t* tops;
+  int n;
+};
+
+// The culling pass by boxes: every lane tests its ray against the boxes of a block's objects
+// (uniform, branch-free, four boxes to a scalar load, 13 vector instructions each) for a t in
+// [tmin, t_best + 4e-5 (1 + t_best)], which leaves a bit per candidate; then, kind by kind, each
+// lane evaluates its own candidates, as many rounds as the lane with the most has of that kind. A
+// walk that evaluates an object for the whole wave when one lane needs it (a hierarchy does that
+// too) runs nearly all of them once rays have split up, since a wave's rays are in no order then.
+// Bound: instruction issue and the serial loads of the rounds. A million rays, 64 objects, 10
+// bounces: trace launches 894 us over every object, 716 us through a hierarchy of boxes, 600 us
+// so; 75011 rays, 23 objects, 8 bounces: 263, 256 and 206 us; FP64, 40009 rays, 12 objects, 6
+// bounces: 110 and 97 us (records in LDS). With 4 objects (20000 rays): 93 us over every object,
+// 99 us so: by boxes from lg_tuning.bvh_min_objects (8) objects.
+//
+// Every object that can hit within the window is a candidate (boxes are padded beyond the FP32
+// error of the test), so the winner, and any runner-up that the FP64 refinement looks at (within
+// 1e-5 (1 + t)), are those of the full walk: `consider` does not depend on the order.
+template <typename T, typename RS>
+__device__ __forceinline__ void walk_boxes(const RayT<T>& r, RS recs, const Rec<double>* recs64, const T* verts,
+                                           const CullView& C, Nearest<T>& nb) {
+  // (1e-18: the products stay finite for coordinates below 1e20)
   const float ox = (float)r.ox, oy = (float)r.oy, dx = (float)r.dx, dy = (float)r.dy;
-  const float ix = 1.0f / (fabsf(dx) > 1e-30f ? dx : __builtin_copysignf(1e-30f, dx));
-  const float iy = 1.0f / (fabsf(dy) > 1e-30f ? dy : __builtin_copysignf(1e-30f, dy));
-  int rec = 0, node = 0, leaf = 0, k = 0, cnt = 0;
-  for (;;) {
-    int top;
-    if (n_nodes == 0) {
-      if (rec >= n_recs) return nb;
-      top = rec;
-    } else {
-      while (k >= cnt) {
-        if (node >= n_nodes) return nb;
-        const BvhNode N = nodes[node];
-        const float tx0 = (N.lo[0] - ox) * ix, tx1 = (N.hi[0] - ox) * ix;
-        const float ty0 = (N.lo[1] - oy) * iy, ty1 = (N.hi[1] - oy) * iy;
-        const float tn = fmaxf(fminf(tx0, tx1), fminf(ty0, ty1));
-        const float tf = fminf(fmaxf(tx0, tx1), fmaxf(ty0, ty1));
-        const float bt = (float)nb.t;
-        const float lim = bt + 4e-5f * (1.0f + bt);
-        const bool need = tn <= tf && tf >= 1e-5f && tn <= lim;
-        int next = N.skip, c = 0;
-        if (__ballot(need)) {
-          c = N.count;
-          if (!c) next = node + 1;
-        }
-        leaf = __builtin_amdgcn_readfirstlane(node);
-        cnt = __builtin_amdgcn_readfirstlane(c);
-        k = 0;
-        node = __builtin_amdgcn_readfirstlane(next);
+  const float ix = 1.0f / (fabsf(dx) > 1e-18f ? dx : __builtin_copysignf(1e-18f, dx));
+  const float iy = 1.0f / (fabsf(dy) > 1e-18f ? dy : __builtin_copysignf(1e-18f, dy));
+  const float ax = -ox * ix, ay = -oy * iy;
+  // an FP64 ray's rounding to FP32 moves it by up to 2^-24 of its origin's coordinates; the boxes'
+  // padding covers the same of theirs
+  const float slack = sizeof(T) == 8 ? 6e-7f * (fabsf(ax) + fabsf(ay)) : 0.0f;
+  // whether the ray meets the box within [1e-5, lim]
+  auto meets = [&](const LG_K float* b, float lim) {
+    const float x0 = __builtin_fmaf(b[0], ix, ax), x1 = __builtin_fmaf(b[2], ix, ax);
+    const float y0 = __builtin_fmaf(b[1], iy, ay), y1 = __builtin_fmaf(b[3], iy, ay);
+    const float tn = fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)), 1e-5f);
+    const float tf = fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), lim);
+    if constexpr (sizeof(T) == 8) return !(tn > tf + slack);  // (NaN: a candidate)
+    return tn <= tf;
+  };
+  for (int b = 0; b < C.n; b++) {
+    const LG_K CullBlock* const B = C.blocks + b;
+    const float bt = (float)nb.t;
+    const float lim = bt + 4e-5f * (1.0f + bt);
+    if (C.n > 1 && !__ballot(meets(B->box, lim))) continue;
+    const int n = B->n, first = B->first;
+    uint32_t half[2] = {0u, 0u};
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+      for (int o = 32 * h; o < n && o < 32 * (h + 1); o += kBoxGroup) {
+        const LG_K float* const x = C.box + 4 * (first + o);
+#pragma unroll
+        for (int k = 0; k < kBoxGroup; k++)
+          if (meets(x + 4 * k, lim)) half[h] |= 1u << ((o + k) & 31);
       }
-      top = __builtin_amdgcn_readfirstlane(node_top(nodes, leaf, k));
-      k++;
+    const uint64_t cand = (uint64_t)half[1] << 32 | half[0];
+    for (int k = 0; k < B->n_kinds; k++) {
+      uint64_t m = cand & B->kind[k];
+      while (__ballot(m != 0ull)) {
+        if (m) {
+          const int top = C.tops[first + __builtin_ctzll(m)];
+          m &= m - 1ull;
+          eval_object<T, false>(r, recs, recs64, verts, top, nb);
+        }
+      }
     }
-    rec = eval_object<T, false>(r, recs, recs64, verts, top, nb);
   }
 }
 
@@ -779,19 +799,24 @@ struct TreeList {
   int n;
 };
 
-// Nearest hit over every object: the object walk over the records before the first Logic tree
-// of more than two primitives, then those trees in a wave-uniform loop of their own, where the
+// Records of the object walk: those before the first such tree.
+__device__ __forceinline__ int walk_records(const TreeList& trees, int n_recs) {
+  return trees.n ? __builtin_amdgcn_readfirstlane(trees.top[0]) : n_recs;
+}
+
+// Nearest hit over every object: walk(nb) offers those before the first Logic tree of more than
+// two primitives, then come those trees in a wave-uniform loop of their own, where the
 // walk's state is no longer live (such trees are rare; a test for them inside the walk raises
 // its register pressure). `consider` keeps the lexicographic minimum of (t, scene order) and
 // the nearest t of another object, so the order in which objects are offered does not change
-// the result. A tree whose box the ray does not enter within the window of the BVH walk is
+// the result. A tree whose box the ray does not enter within the window of the walk by boxes is
 // skipped, for the same reason.
-template <typename T, typename RS, typename NS = const BvhNode*>
+template <typename T, typename RS, typename Walk>
 __device__ __forceinline__ Nearest<T> nearest_hit(const RayT<T>& r, RS recs, const Rec<double>* recs64,
-                                                  const T* verts, int n_recs, const TreeList& trees,
-                                                  NS nodes = nullptr, int n_nodes = 0) {
-  const int n_walk = trees.n ? __builtin_amdgcn_readfirstlane(trees.top[0]) : n_recs;
-  Nearest<T> nb = walk_objects(r, recs, recs64, verts, n_walk, nodes, n_nodes);
+                                                  const T* verts, const TreeList& trees, Walk&& walk) {
+  Nearest<T> nb;
+  nearest_init(nb);
+  walk(nb);
   if (trees.n == 0) return nb;
   const T ix = (T)1 / (fabs(r.dx) > (T)1e-30 ? r.dx : (T)__builtin_copysign(1e-30, (double)r.dx));
   const T iy = (T)1 / (fabs(r.dy) > (T)1e-30 ? r.dy : (T)__builtin_copysign(1e-30, (double)r.dy));
@@ -1003,7 +1028,9 @@ __device__ __forceinline__ double tie_tol(double t) { return 1e-5 * (1.0 + t); }
 // the main path's registers and code small.
 __device__ __forceinline__ Nearest<double> rescan_fp64(const RayT<double>& rd, const Rec<double>* recs64,
                                                     const double* verts64, int n_recs, const TreeList& trees) {
-  return nearest_hit<double>(rd, recs64, recs64, verts64, n_recs, trees);
+  return nearest_hit<double>(rd, recs64, recs64, verts64, trees, [&](Nearest<double>& nb) {
+    walk_objects<double>(rd, recs64, recs64, verts64, walk_records(trees, n_recs), nb);
+  });
 }
 
 // FP64 answer for a ray whose FP32 culling pass found `nb`.
@@ -1102,18 +1129,19 @@ __device__ __forceinline__ void build_items_block(const SceneDesc* __restrict__ 
 // index in the frame) picks the ping-pong queues.
 constexpr uint32_t kMaxChunk = 3;
 
-// LDS of one trace workgroup: object flags and first records, polygon vertices, the FP64
-// trace's records (the FP32 culling pass reads its records and BVH nodes with scalar loads),
-// then the level buffers of a chunked launch.
+// LDS of one trace workgroup: the objects' first records and flags in scene order, first records
+// in the culling blocks' order (without padding, which only the last block has), polygon
+// vertices, the FP64 trace's records (the FP32 culling pass reads its records from global
+// memory), then the level buffers of a chunked launch.
 struct TraceLds {
-  size_t flags, obj_rec, verts, recs, levels, total;
+  size_t obj, tops, verts, recs, levels, total;
 };
 template <typename T>
 __host__ __device__ inline TraceLds trace_lds(int n_recs, int n_objs, int n_verts, uint32_t chunk, int block) {
   TraceLds L;
-  L.flags = 0;
-  L.obj_rec = L.flags + (size_t)n_objs * 4;
-  L.verts = (L.obj_rec + (size_t)n_objs * 4 + 15) & ~size_t(15);
+  L.obj = 0;
+  L.tops = (size_t)n_objs * 4;
+  L.verts = (L.tops + (size_t)n_objs * 4 + 15) & ~size_t(15);
   L.recs = (L.verts + (size_t)n_verts * 2 * sizeof(T) + 15) & ~size_t(15);
   const bool fp64 = sizeof(T) == 8;
   L.levels = (L.recs + (fp64 ? (size_t)n_recs * sizeof(Rec<T>) : 0) + 15) & ~size_t(15);
@@ -1138,8 +1166,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
   __shared__ uint32_t s_lcnt[kMaxChunk];  // rays in the LDS buffer of each level (1 .. chunk - 1)
 
   const TraceLds lay = trace_lds<T>(cap_recs, cap_objs, cap_verts, chunk, BLOCK);
-  uint32_t* s_obj_flags = reinterpret_cast<uint32_t*>(smem + lay.flags);
-  int32_t* s_obj_rec = reinterpret_cast<int32_t*>(smem + lay.obj_rec);
+  uint32_t* s_obj = reinterpret_cast<uint32_t*>(smem + lay.obj);  // first record << 2 | ObjFlags
+  int32_t* s_tops = reinterpret_cast<int32_t*>(smem + lay.tops);
   T* s_verts = reinterpret_cast<T*>(smem + lay.verts);
   Rec<T>* s_rec = reinterpret_cast<Rec<T>*>(smem + lay.recs);
   QRay<double>* s_lvl = reinterpret_cast<QRay<double>*>(smem + lay.levels);  // level j at (j - 1) * 2 * BLOCK
@@ -1167,6 +1195,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
     const double* verts64 = gen(D.verts64);
     const int n_recs = D.n_recs, n_objs = D.n_objs;
     const TreeList trees{gen(D.tree_rec), gen(D.obj_box), D.n_trees};
+    const CullView cull{(const LG_K CullBlock*)D.blocks, (const LG_K float*)D.block_box, s_tops, D.n_blocks};
     if (sid != loaded) {
       if (sizeof(T) == 8) {  // the FP32 pass reads its records with scalar loads instead
         const int4* src = reinterpret_cast<const int4*>(gen(D.recs));
@@ -1174,9 +1203,10 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
         const int n16 = n_recs * (int)(sizeof(Rec<T>) / 16);
         for (int k = threadIdx.x; k < n16; k += BLOCK) dst[k] = src[k];
       }
+      const int n_walk = n_objs - D.n_trees;  // the objects that the blocks hold
       for (int k = threadIdx.x; k < n_objs; k += BLOCK) {
-        s_obj_flags[k] = gen(D.obj_flags)[k];
-        s_obj_rec[k] = gen(D.obj_rec)[k];
+        s_obj[k] = (uint32_t)gen(D.obj_rec)[k] << 2 | gen(D.obj_flags)[k];
+        if (D.n_blocks && k < n_walk) s_tops[k] = gen(D.block_rec)[k];
       }
       const T* vsrc = reinterpret_cast<const T*>(gen(D.verts));
       for (int k = threadIdx.x; k < 2 * D.n_verts; k += BLOCK) s_verts[k] = vsrc[k];
@@ -1239,12 +1269,22 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
         const RayT<double> rd{ox, oy, dx, dy};
         Nearest<double> h;
         if constexpr (sizeof(T) == 8) {
-          h = nearest_hit<double>(rd, s_rec, recs64, s_verts, n_recs, trees);
+          h = nearest_hit<double>(rd, s_rec, recs64, s_verts, trees, [&](Nearest<double>& nb) {
+            if (cull.n)
+              walk_boxes<double>(rd, s_rec, recs64, s_verts, cull, nb);
+            else
+              walk_objects<double>(rd, s_rec, recs64, s_verts, walk_records(trees, n_recs), nb);
+          });
         } else {
           const RayT<float> rf{(float)ox, (float)oy, (float)dx, (float)dy};
           const RecK krec{(const LG_K lg_v4i*)D.recs};
-          const NodeK knode{(const LG_K lg_v4i*)D.bvh};
-          Nearest<float> nb = nearest_hit<float>(rf, krec, recs64, s_verts, n_recs, trees, knode, D.n_bvh);
+          const RecV vrec{(const lg_v4i*)gen(D.recs)};
+          Nearest<float> nb = nearest_hit<float>(rf, krec, recs64, s_verts, trees, [&](Nearest<float>& nf) {
+            if (cull.n)
+              walk_boxes<float>(rf, vrec, recs64, s_verts, cull, nf);
+            else
+              walk_objects<float>(rf, krec, recs64, s_verts, walk_records(trees, n_recs), nf);
+          });
           nearest_init(h);
           if (nb.top >= 0) refine_fp64(rd, nb, recs64, verts64, n_recs, trees, h);
         }
@@ -1260,7 +1300,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
           }
           hit_normal<double>(R, verts64, h.code, h.s, px, py, nx, ny);
           obj = R.obj;
-          fl = s_obj_flags[obj];
+          fl = s_obj[obj] & 3u;
           hit = true;
           emit = true;
           if (fl & OBJ_MATERIAL) {
@@ -1288,10 +1328,10 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
           uint32_t half[2] = {0u, 0u};
 #pragma unroll
           for (int h = 0; h < 2; h++)
-            for (int o = 32 * h; o < n && o < 32 * (h + 1); o += kMediumBlock) {
+            for (int o = 32 * h; o < n && o < 32 * (h + 1); o += kBoxGroup) {
               const LG_K float* const b = boxes + 4 * (base + o);
 #pragma unroll
-              for (int k = 0; k < kMediumBlock; k++)
+              for (int k = 0; k < kBoxGroup; k++)
                 if ((fx >= b[4 * k]) & (fy >= b[4 * k + 1]) & (fx <= b[4 * k + 2]) & (fy <= b[4 * k + 3]))
                   half[h] |= 1u << ((o + k) & 31);
             }
@@ -1302,7 +1342,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             if (cand) {
               const int o = base + __builtin_ctzll(cand);
               cand &= cand - 1ull;
-              if (contains_object<double>(recs64, verts64, s_obj_rec[o], px, py)) {
+              if (contains_object<double>(recs64, verts64, (int)(s_obj[o] >> 2), px, py)) {
                 n2 = gen(D.obj_n64)[o];
                 seek = false;
                 cand = 0ull;
