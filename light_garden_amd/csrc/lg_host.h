@@ -179,9 +179,18 @@ struct lg_scene {
   std::vector<int32_t> h_obj_rec;
   std::vector<double> h_verts64;
   int n_recs = 0, n_objs = 0, n_verts = 0;
-  lg::DevBuf recs32, recs64, obj_n64, obj_flags, obj_rec, obj_box, medium_box, verts32, verts64, lights_dev;
-  lg::DevBuf blocks, block_box, block_rec;  // culling blocks (CullBlock)
-  lg::DevBuf tree_rec;        // first records of the Logic trees of more than two primitives
+  // The compiled scene on the device: one allocation, written with one copy; byte offsets of its
+  // tables.
+  lg::DevBuf tables;
+  struct {
+    size_t recs32, recs64, obj_n64, obj_flags, obj_rec, obj_box, medium_box, verts32, verts64, lights;
+    size_t blocks, block_box, block_rec;  // culling blocks (CullBlock)
+    size_t tree_rec;                      // first records of the Logic trees of more than two primitives
+  } at{};
+  template <typename U>
+  const U* table(size_t off) const {
+    return reinterpret_cast<const U*>(tables.as<char>() + off);
+  }
   int n_blocks = 0;
   int n_trees = 0;
   lg::DevBuf q0, q1;          // ray queues (QRay<double>)

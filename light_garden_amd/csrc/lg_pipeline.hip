@@ -423,21 +423,21 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
     SceneHues hues;
     if (trace) {
       lg_scene* sc = e.scene;
-      D.recs = gbl(L.fp64 ? sc->recs64.p : sc->recs32.p);
-      D.recs64 = gbl(sc->recs64.as<const Rec<double>>());
-      D.obj_n64 = gbl(sc->obj_n64.as<const double>());
-      D.obj_flags = gbl(sc->obj_flags.as<const uint32_t>());
-      D.obj_rec = gbl(sc->obj_rec.as<const int32_t>());
-      D.obj_box = gbl(sc->obj_box.as<const float4>());
-      D.medium_box = gbl(sc->medium_box.as<const float4>());
-      D.verts = gbl(L.fp64 ? sc->verts64.p : sc->verts32.p);
-      D.verts64 = gbl(sc->verts64.as<const double>());
-      D.lights = gbl(sc->lights_dev.as<const DevLight>());
-      D.blocks = gbl(sc->blocks.as<const CullBlock>());
-      D.block_box = gbl(sc->block_box.as<const float4>());
-      D.block_rec = gbl(sc->block_rec.as<const int32_t>());
+      D.recs = gbl(sc->table<void>(L.fp64 ? sc->at.recs64 : sc->at.recs32));
+      D.recs64 = gbl(sc->table<Rec<double>>(sc->at.recs64));
+      D.obj_n64 = gbl(sc->table<double>(sc->at.obj_n64));
+      D.obj_flags = gbl(sc->table<uint32_t>(sc->at.obj_flags));
+      D.obj_rec = gbl(sc->table<int32_t>(sc->at.obj_rec));
+      D.obj_box = gbl(sc->table<float4>(sc->at.obj_box));
+      D.medium_box = gbl(sc->table<float4>(sc->at.medium_box));
+      D.verts = gbl(sc->table<void>(L.fp64 ? sc->at.verts64 : sc->at.verts32));
+      D.verts64 = gbl(sc->table<double>(sc->at.verts64));
+      D.lights = gbl(sc->table<DevLight>(sc->at.lights));
+      D.blocks = gbl(sc->table<CullBlock>(sc->at.blocks));
+      D.block_box = gbl(sc->table<float4>(sc->at.block_box));
+      D.block_rec = gbl(sc->table<int32_t>(sc->at.block_rec));
       D.n_blocks = scene_uses_boxes(ctx, sc) ? sc->n_blocks : 0;
-      D.tree_rec = gbl(sc->tree_rec.as<const int32_t>());
+      D.tree_rec = gbl(sc->table<int32_t>(sc->at.tree_rec));
       D.n_trees = sc->n_trees;
       D.n_recs = sc->n_recs;
       D.n_objs = sc->n_objs;
