@@ -952,7 +952,7 @@ constexpr uint32_t kEarlyClaimPairs = 8192;
 // lane l loads pair l's segment and computes its sample range inside the tile plus the
 // tile-relative FP32 parameters of its samples. Two-channel frames at T = 64 with 1024-thread
 // workgroups then walk the batch as one stream of samples, 64 per step (see the stream
-// comment in the walk); other shapes walk the pairs one after another with one sample per
+// comment in the walk; not under blends with factors when colours vary along a segment); other shapes walk the pairs one after another with one sample per
 // lane, reading the pair's setup from scalar registers.
 //
 // An item is walked twice: first its y-major pairs with the tile held transposed (pixel
@@ -974,7 +974,7 @@ constexpr uint32_t kEarlyClaimPairs = 8192;
 // four. PACKED_ONLY: every scene of the frame has SCENE_PACKED, so the LDS tile holds two planes
 // only (half the LDS: two 512-thread workgroups share a compute unit at T = 64), or three in the
 // 1024-thread kernel, which serves up to three hues.
-enum WalkMode { WALK_COLOR, WALK_VERTEX_COLORS, WALK_HUES };
+enum WalkMode { WALK_COLOR, WALK_VERTEX_COLORS, WALK_VERTEX_STREAM, WALK_HUES };
 template <int T, bool PACKED_ONLY, int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void tile_accum_kernel(const SceneDesc* __restrict__ descs,
                                                           const uint32_t* __restrict__ pairs,
@@ -996,8 +996,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
   __shared__ uint32_t s_batch[2];  // next batch of 64 pairs, per phase
   unsigned long long* const tile = s_tile + kGuard * T;  // row 0 of plane 0
   constexpr int kWaves = BLOCK / 64;
-  // Sample-stream walk (two-channel frames, one colour per segment, T = 64, one workgroup per
-  // compute unit): each wave lays the samples of its 64 pairs end to end and walks that stream
+  // Sample-stream walk (two-channel frames, T = 64, one workgroup per compute unit; with a colour
+  // per vertex under the default blend, whose channel values need no factors): each wave lays the samples of its 64 pairs end to end and walks that stream
   // 64 samples per step, every lane busy, instead of one pair per step. Per wave: a record per
   // pair with samples plus an empty one (two uint4 each) and a start bit per stream position.
   __shared__ HueScale s_hue[kHueKernel ? kMaxHues : 1];
@@ -1147,7 +1147,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
       auto step = [&](auto mode_tag, const uint32_t e_cur, const float4& p_cur, const float4& a_cur,
                       const float4& c_cur, const uint32_t e_nxt, float4& p_nxt, float4& a_nxt, float4& c_nxt,
                       uint32_t& b_aft, uint32_t& e_aft) {
-        constexpr bool kVC = decltype(mode_tag)::value == WALK_VERTEX_COLORS;
+        constexpr bool kVS = decltype(mode_tag)::value == WALK_VERTEX_STREAM;
+        constexpr bool kVC = kVS || decltype(mode_tag)::value == WALK_VERTEX_COLORS;
         constexpr bool kHues = decltype(mode_tag)::value == WALK_HUES;
         // ---- per-lane setup of one pair of the current batch ----
         int packed = 0;  // n | q0 << 8 | vertex colours << 17 | negative colour << 18
@@ -1245,11 +1246,14 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
         e_aft = entry(b_aft);
         if (lane == 0) taken = atomicAdd(&s_batch[phase], 1u);
         // ---- walk the pairs that have samples ----
-        if constexpr (kStreamKernel && !kVC) {
+        if constexpr (kStreamKernel && (kVS || !kVC)) {
           // Sample stream: the c-th lane with samples owns positions pre_c .. pre_c + n_c - 1 of
           // the wave's stream (pre: exclusive prefix sum of n), and position k is column k +
           // q0_c - pre_c of the tile. Record c = {q0_c - pre_c, m_first, slope, 8 (q0_c - pre_c)},
-          // {q0..q3} (the column offset, and in bytes for the deposit address);
+          // {q0..q3} (the column offset, and in bytes for the deposit address); with a colour per
+          // vertex {q0_c, s_first, ds} in the second part and the first colour and the difference in
+          // two more (60033 string-mod lines of two colours at 2048x1536: 144 us, pair by pair 292,
+          // where a pair of 40 samples pays the step of 64 and the reads of 14 lanes' registers);
           // record P (after the last pair) is empty (zero deposits in row 0), so the positions
           // past the end of the stream need no mask. Stream word i holds a bit per position
           // 64 i .. 64 i + 63 that starts a record; lane l of step s finds its record as the
@@ -1266,6 +1270,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
                                                          __builtin_amdgcn_mbcnt_lo((uint32_t)live, 0u));
             const int wv = __builtin_amdgcn_readfirstlane(wave);
             uint4* const rec = s_rec + wv * (kRecs * 2);
+            // the vertex colours' part of the records: in the third plane, which such frames do not use
+            uint4* const vrec = reinterpret_cast<uint4*>(s_tile + 2 * kStride) + wv * (kRecs * 2);
+            static_assert(!kVS || (kPlanes > 2 && kWaves * kRecs * 32 <= kStride * 8), "the third plane holds them");
             unsigned long long* const mask = s_mask + wv * kMaskWords;
             // (one wave's LDS operations execute in order: the words are cleared before the
             // starts are set, and the previous batch's reads are done before these writes)
@@ -1274,15 +1281,22 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               const int off = ((packed >> 8) & 0xff) - pre;
               rec[2 * c] = make_uint4((uint32_t)off, __float_as_uint(m_first), __float_as_uint(slope),
                                       (uint32_t)((kHues ? off + cq2 : off) * 8));
-              if constexpr (kHues)
+              if constexpr (kHues) {
                 *reinterpret_cast<uint2*>(&rec[2 * c + 1]) = make_uint2((uint32_t)cq0, (uint32_t)cq1);
-              else
+              } else if constexpr (kVS) {
+                rec[2 * c + 1] = make_uint4(__float_as_uint((float)((packed >> 8) & 0xff)), __float_as_uint(s_first),
+                                            __float_as_uint(ds), 0u);
+                vrec[2 * c] = __builtin_bit_cast(uint4, ca);
+                vrec[2 * c + 1] = __builtin_bit_cast(uint4, dc);
+              } else {
                 rec[2 * c + 1] = make_uint4((uint32_t)cq0, (uint32_t)cq1, (uint32_t)cq2, (uint32_t)cq3);
+              }
               atomicOr(&mask[pre >> 6], 1ull << (pre & 63));
             }
             if (lane == 0) {
               rec[2 * n_live] = make_uint4((uint32_t)(-total), 0u, 0u, (uint32_t)(-total * 8));
               rec[2 * n_live + 1] = make_uint4(0u, 0u, 0u, 0u);
+              if constexpr (kVS) vrec[2 * n_live] = vrec[2 * n_live + 1] = make_uint4(0u, 0u, 0u, 0u);
               if (total & 63) atomicOr(&mask[total >> 6], 1ull << (total & 63));
             }
             // lane i keeps stream word i in registers; a step takes its word with a lane read
@@ -1295,7 +1309,10 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             // lane then names record seen <= 65.
             uint32_t seen = 0;
             const char* const rec_m1 = reinterpret_cast<const char*>(rec) - 32;  // record -1
-            auto read_recs = [&](int s, uint4& r0, uint4& r1) {
+            struct StepRec {
+              uint4 r0, r1, a, d;
+            };
+            auto read_recs = [&](int s, StepRec& R) {
               const int sl = s < 63 ? s : 63;
               uint32_t lo = __builtin_amdgcn_readlane(mw_lo, sl);
               uint32_t hi = __builtin_amdgcn_readlane(mw_hi, sl);
@@ -1310,19 +1327,25 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               // the wave-uniform part of the address apart: one lane operation adds k
               const char* const rbase = rec_m1 + (first + 1) * 32;
               const uint4* const r = reinterpret_cast<const uint4*>(rbase + k * 32u);
-              r0 = r[0];
+              R.r0 = r[0];
               if constexpr (kHues) {
                 const uint2 q = *reinterpret_cast<const uint2*>(&r[1]);
-                r1.x = q.x;
-                r1.y = q.y;
+                R.r1.x = q.x;
+                R.r1.y = q.y;
               } else {
-                r1 = r[1];
+                R.r1 = r[1];
+              }
+              if constexpr (kVS) {
+                const uint4* const rv = r + (vrec - rec);
+                R.a = rv[0];
+                R.d = rv[1];
               }
             };
             // Step st at stream positions p = 64 st + lane: the sample's column is off + p, its
             // entry in plane 0 jl * T + column.
             const uint32_t lane8 = (uint32_t)lane * 8u;
-            auto deposit_step = [&](int st, const uint4& r0, const uint4& r1) {
+            auto deposit_step = [&](int st, const StepRec& R) {
+              const uint4 r0 = R.r0, r1 = R.r1;
               const int col = (int)r0.x + lane + (st << 6);
               const float m = __builtin_fmaf((float)col, __uint_as_float(r0.z), __uint_as_float(r0.y));
               int jl;
@@ -1331,17 +1354,27 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               // byte offset 8 (jl T + column) = (jl + st) 512 + 8 off + 8 lane
               const uint32_t eb = ((uint32_t)(jl + st) << 9) + r0.w + lane8;
               unsigned long long* const t = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(tile) + eb);
-              if constexpr (kHues)
+              if constexpr (kHues) {
                 deposit1<T>(t, m, r1.x, r1.y);
-              else
+              } else if constexpr (kVS) {
+                // the per-pair walk's expressions: the same bits
+                const float4 a = __builtin_bit_cast(float4, R.a), d = __builtin_bit_cast(float4, R.d);
+                const float sp = __builtin_fmaf((float)col - __uint_as_float(r1.x), __uint_as_float(r1.z),
+                                                __uint_as_float(r1.y));
+                const float al = __builtin_fmaf(sp, d.w, a.w);
+                deposit2<T, kStride>(t, m, pack_q(__builtin_fmaf(sp, d.x, a.x), cs0),
+                                     pack_q(__builtin_fmaf(sp, d.y, a.y), cs1),
+                                     pack_q(__builtin_fmaf(sp, d.z, a.z), cs2), pack_q(al * al, cs3));
+              } else {
                 deposit2<T, kStride>(t, m, r1.x, r1.y, r1.z, r1.w);
+              }
             };
             // One step ahead: the records of step s + 1 are read while step s deposits; two
             // steps per trip with the record registers swapped, so that nothing read ahead is
             // copied (a copy would wait for its read). Scheduling barriers keep the reads ahead
             // of the deposits they overlap.
-            uint4 ra, rb{}, rc, rd{};
-            read_recs(0, ra, rb);
+            StepRec ra{}, rb{};
+            read_recs(0, ra);
             // zero adds into guard row -2: the loop is entered with the same LDS operations
             // in flight as it loops back with (two reads, four adds; two with hues), so that the
             // compiler's wait counts inside the loop stay exact
@@ -1358,14 +1391,14 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             }
             __builtin_amdgcn_sched_barrier(0);
             for (int st = 0;; st += 2) {
-              read_recs(st + 1, rc, rd);
+              read_recs(st + 1, rb);
               __builtin_amdgcn_sched_barrier(0);
-              deposit_step(st, ra, rb);
+              deposit_step(st, ra);
               __builtin_amdgcn_sched_barrier(0);
               if (st + 1 >= steps) break;
-              read_recs(st + 2, ra, rb);
+              read_recs(st + 2, ra);
               __builtin_amdgcn_sched_barrier(0);
-              deposit_step(st + 1, rc, rd);
+              deposit_step(st + 1, rb);
               __builtin_amdgcn_sched_barrier(0);
               if (st + 2 >= steps) break;
             }
@@ -1516,6 +1549,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
         }
       }
       if (walked) {
+      } else if (kStreamKernel && col1 && bc == kBlendDefault) {
+        run(std::integral_constant<int, kStreamKernel ? WALK_VERTEX_STREAM : WALK_VERTEX_COLORS>{});
       } else if (col1) {
         run(std::integral_constant<int, WALK_VERTEX_COLORS>{});
       } else {
