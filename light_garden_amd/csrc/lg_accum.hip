@@ -95,6 +95,20 @@ __device__ __forceinline__ double rcp_newton(double x) {
   return __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
 }
 
+// LDS by byte address: a uniform part of an address that comes from a lane read stays an integer.
+#define LG_L __attribute__((address_space(3)))
+typedef uint32_t lg_v4u __attribute__((ext_vector_type(4)));
+typedef uint32_t lg_v2u __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+  return (uint32_t)(uintptr_t)(const LG_L char*)p;
+}
+__device__ __forceinline__ uint4 lds_read16(uint32_t a) {
+  return __builtin_bit_cast(uint4, *(const LG_L lg_v4u*)(uintptr_t)a);
+}
+__device__ __forceinline__ uint2 lds_read8(uint32_t a) {
+  return __builtin_bit_cast(uint2, *(const LG_L lg_v2u*)(uintptr_t)a);
+}
+
 // Inclusive sum over the lanes of a wave with DPP lane moves (no LDS round trips): shifts by
 // 1, 2, 4, 8 within each row of 16 lanes, then the totals of rows 0 and 2 broadcast into rows
 // 1 and 3, and the total of rows 0-1 into rows 2-3. Lanes a move has no source for add 0.
@@ -294,13 +308,14 @@ __global__ __launch_bounds__(256) void bin_kernel(const SceneDesc* __restrict__ 
     const int n_tiles = v.tiles_x * v.tiles_y;
     const uint32_t local = ci - chunk_pre[sid];
     uint2* const mat = reinterpret_cast<uint2*>(places + cbase[sid]) + (uint64_t)local * n_tiles;
-    uint2* const tile_rows = reinterpret_cast<uint2*>(rows) + D.tile_base;
+    uint2* const tile_rows = reinterpret_cast<uint2*>(rows) + D.row_base;
+    const uint32_t row_stride = D.row_stride;
     uint2* const hist2 = reinterpret_cast<uint2*>(s_hist);
     for (int t = threadIdx.x; t < n_tiles; t += blockDim.x) {
       if (PASS == 0) {
         hist2[t] = make_uint2(0u, 0u);
       } else {
-        const uint2 a = tile_rows[t], b = mat[t];
+        const uint2 a = tile_rows[t * row_stride], b = mat[t];
         hist2[t] = make_uint2(a.x + b.x, a.y + b.y);
       }
     }
@@ -402,7 +417,7 @@ __global__ __launch_bounds__(256) void bin_kernel(const SceneDesc* __restrict__ 
       for (int t = threadIdx.x; t < n_tiles; t += blockDim.x) {
         const uint2 h = hist2[t];
         if (h.x | h.y) {  // (a tile the chunk does not touch has no pairs to place)
-          const unsigned long long before = atomicAdd(reinterpret_cast<unsigned long long*>(tile_rows + t),
+          const unsigned long long before = atomicAdd(reinterpret_cast<unsigned long long*>(tile_rows + t * row_stride),
                                                       (unsigned long long)h.y << 32 | h.x);
           mat[t] = make_uint2((uint32_t)before, (uint32_t)(before >> 32));
         }
@@ -414,7 +429,7 @@ __global__ __launch_bounds__(256) void bin_kernel(const SceneDesc* __restrict__ 
 
 // ---- tile work items ------------------------------------------------------------------------
 // Tile g's list is pairs [rows[2 g], rows[2 g + 2]) of the scanned row totals, its x-major part
-// from rows[2 g + 1] on. A tile is cut into full pieces and at most one remainder; the items are
+// from rows[2 g + 1] on (with layers 2 * layers rows per tile, y-major and x-major of each). A tile is cut into full pieces and at most one remainder; the items are
 // ordered by size class (floor(log2(pairs))), largest class first. With `whole` (the frame clears,
 // accumulates and resolves every image) a tile without pairs gets one empty item (size class 0),
 // which writes its cleared pixels.
@@ -424,6 +439,7 @@ struct PlanLimits {
   uint32_t min_piece, max_piece;
   uint32_t grid;   // tile workgroups
   uint32_t whole;
+  uint32_t layers; // pairs of rows per tile
 };
 
 __device__ __forceinline__ uint32_t piece_size(unsigned long long total, const PlanLimits& L) {
@@ -490,10 +506,19 @@ __global__ __launch_bounds__(1024) void plan_items_kernel(const SceneDesc* __res
   const int t1 = t0 + per < n_tiles ? t0 + per : n_tiles;
   const uint2* counts = reinterpret_cast<const uint2*>(row_count);
   uint2* starts = reinterpret_cast<uint2*>(row_start);
+  const uint32_t nl = L.layers;
+  auto tile_count = [&](int t) {
+    uint32_t n = 0;
+    for (uint32_t l = 0; l < nl; l++) {
+      const uint2 c = counts[t * nl + l];
+      n += c.x + c.y;
+    }
+    return n;
+  };
   if (threadIdx.x < 32) s_cls[threadIdx.x] = 0u;
   if (threadIdx.x == 0) s_nsplit = 0u;
   unsigned long long own = 0;
-  for (int t = t0; t < t1; t++) {
+  for (uint32_t t = t0 * nl; t < t1 * nl; t++) {
     const uint2 c = counts[t];
     own += (unsigned long long)c.x + c.y;
   }
@@ -515,12 +540,15 @@ __global__ __launch_bounds__(1024) void plan_items_kernel(const SceneDesc* __res
   const int cls_full = 31 - __clz(piece);
   uint32_t b = first;
   for (int t = t0; t < t1; t++) {
-    const uint2 c = counts[t];
-    starts[t] = make_uint2(b, b + c.x);
-    const TileCut k = cut_tile(c.x + c.y, piece, L.whole);
+    const uint32_t b0 = b;
+    for (uint32_t l = 0; l < nl; l++) {
+      const uint2 c = counts[t * nl + l];
+      starts[t * nl + l] = make_uint2(b, b + c.x);
+      b += c.x + c.y;
+    }
+    const TileCut k = cut_tile(b - b0, piece, L.whole);
     if (k.full) atomicAdd(&s_cls[cls_full], k.full);
     if (k.items > k.full) atomicAdd(&s_cls[k.cls_rem], 1u);
-    b += c.x + c.y;
   }
   __syncthreads();
   if (threadIdx.x < 32) {  // first slot of each size class, largest class first
@@ -529,7 +557,7 @@ __global__ __launch_bounds__(1024) void plan_items_kernel(const SceneDesc* __res
     s_cur[threadIdx.x] = base;
     if (threadIdx.x == 0) {
       const uint32_t n_items = base + s_cls[0];
-      row_start[2 * n_tiles] = (uint32_t)total;
+      row_start[2 * n_tiles * nl] = (uint32_t)total;
       ctl->total_pairs = total;
       ctl->n_work = n_items < L.items_cap ? n_items : L.items_cap;
       uint32_t f = 0;
@@ -541,8 +569,7 @@ __global__ __launch_bounds__(1024) void plan_items_kernel(const SceneDesc* __res
   __syncthreads();
   b = first;
   for (int t = t0; t < t1; t++) {
-    const uint2 c = counts[t];
-    const uint32_t cnt = c.x + c.y;
+    const uint32_t cnt = tile_count(t);
     const TileCut k = cut_tile(cnt, piece, L.whole);
     if (k.items) {
       uint32_t split_slot = 0, full_slot = 0, rem_slot = 0;
@@ -553,7 +580,7 @@ __global__ __launch_bounds__(1024) void plan_items_kernel(const SceneDesc* __res
       if (k.full) full_slot = atomicAdd(&s_cur[cls_full], k.full);
       if (k.items > k.full) rem_slot = atomicAdd(&s_cur[k.cls_rem], 1u);
       const uint32_t sid = tile_scene[t];
-      put_items(items, L.items_cap, sid, (uint32_t)(t - descs[sid].tile_base), b, b + cnt, b + c.x, piece, k,
+      put_items(items, L.items_cap, sid, (uint32_t)(t - descs[sid].tile_base), b, b + cnt, b + counts[t * nl].x, piece, k,
                 split_slot, full_slot, rem_slot);
     }
     b += cnt;
@@ -578,7 +605,7 @@ __global__ __launch_bounds__(256) void tile_classes_kernel(int n_tiles, const ui
   const unsigned long long total = ctl->total_pairs;
   const uint32_t piece = piece_size(total, L);
   if (g < n_tiles) {
-    const TileCut k = cut_tile(row_start[2 * g + 2] - row_start[2 * g], piece, L.whole);
+    const TileCut k = cut_tile(row_start[2 * (g + 1) * L.layers] - row_start[2 * g * L.layers], piece, L.whole);
     if (k.full) atomicAdd(&s_cls[31 - __clz(piece)], k.full);
     if (k.items > k.full) atomicAdd(&s_cls[k.cls_rem], 1u);
   }
@@ -617,9 +644,9 @@ __global__ __launch_bounds__(256) void write_items_kernel(const SceneDesc* __res
   uint32_t b = 0, e = 0, mid = 0;
   TileCut k{0u, 0u, 0};
   if (g < n_tiles) {
-    b = row_start[2 * g];
-    mid = row_start[2 * g + 1];
-    e = row_start[2 * g + 2];
+    b = row_start[2 * g * L.layers];
+    mid = row_start[2 * g * L.layers + 1];
+    e = row_start[2 * (g + 1) * L.layers];
     k = cut_tile(e - b, piece, L.whole);
   }
   const int cls_full = 31 - __clz(piece);
@@ -830,10 +857,32 @@ __device__ __forceinline__ void hue_add(double (&p)[4], const HueScale& h, unsig
   p[3] = __builtin_fma((double)a, h.ua, p[3]);
 }
 
-// The pair count that bounds a packed tile's fields (see packed_fixed_bits).
-__device__ __forceinline__ uint32_t packed_pairs(const uint32_t* row_start, uint32_t g) {
-  const uint32_t nt = row_start[2 * g + 2] - row_start[2 * g];
-  return nt < kPackedPiece ? nt : kPackedPiece;
+// Run weights (SCENE_RUNS). A run's segments have one colour, so a tile sums one number per pixel
+// and run: the weights of the deposits, each sample's 2^G cut into round(fr 2^G) at pixel jl + 1
+// and the rest at jl, as 32-bit words (a pair deposits at most once into a pixel, so n pairs keep a
+// word below n 2^G <= 2^32 - 1). The colours come in when a layer's sums are converted: channel c of
+// run f adds weight times C = round(value 2^K_c), exact 64-bit products, so neither the split of a
+// tile's list into items nor the order of anything changes a bit. C <= 2^30, less where the
+// tile's pairs would pass 2^62 in total. A deposit costs two 32-bit adds where two-channel words
+// take four of 64 bits, no colour is loaded, and instruction issue instead of the LDS is what bounds the
+// walk (1.6M segments in 16 runs at 4096x4096, 78M pairs: 3727 us by colours, 2255 us so).
+// Finer than the colours' fixed point: a weight has the levels the brightest channel had, and
+// no colour is rounded to them.
+constexpr int kFxBits = 22;  // of a sample's place below the pixel; |slope| 2^22 is a 24-bit number
+__device__ __forceinline__ int weight_bits(uint32_t n) {
+  const int G = 31 - __clz((int)(0xFFFFFFFFu / (n > 1u ? n : 1u)));
+  return G < kFxBits ? G : kFxBits;
+}
+// K of channel c in a tile of n pairs.
+__device__ __forceinline__ int run_color_bits(const SceneDesc& D, int c, uint32_t n) {
+  const double bound = (double)D.color_max * (double)D.factor_max[c];
+  if (!(bound > 0.0) || !(bound < 1e300)) return 0;
+  const uint32_t over = n / kPackedPiece;  // n 2^G <= 2^32 (over + 1)
+  return 30 - (over ? 32 - __clz((int)over) : 0) - 1 - floor_log2_ratio(bound, 1.0);
+}
+__device__ __forceinline__ uint32_t run_color(float v, int K) {
+  const double x = __builtin_ldexp((double)v, K);
+  return x > 0.0 && x < 4294967295.0 ? (uint32_t)__builtin_rint(x) : 0u;
 }
 
 // One packed channel value of a sample: cq = round(max(v, 0) * 2^G), the low bits of one FMA against
@@ -927,18 +976,18 @@ __device__ __forceinline__ ushort4 resolve_px(const float4 a) {
 // 0 .. T/2-1 alone; lanes from T on idle). Every element off the main diagonal is swapped
 // exactly once, and the lanes' addresses step by T + 1 elements, which keeps the swaps free of
 // bank conflicts.
-template <int T, int STRIDE, int WAVES>
-__device__ __forceinline__ void transpose_tile(unsigned long long* t, int planes, int wave, int lane) {
+template <int T, int STRIDE, int WAVES, typename W>
+__device__ __forceinline__ void transpose_tile(W* t, int planes, int wave, int lane) {
   constexpr int H = T / 2;
   for (int j = wave; j < planes * H; j += WAVES) {
     const int d = (j % H) + 1;
-    unsigned long long* pl = t + (j / H) * STRIDE;
+    W* pl = t + (j / H) * STRIDE;
     const bool first_diag = lane < T - d;
     const int r = first_diag ? lane : lane - (T - d);
     const int c = first_diag ? lane + d : r + (T - d);
     if (lane < T && (d < H || lane < H)) {
       const int a = r * T + c, b = c * T + r;
-      const unsigned long long va = pl[a], vb = pl[b];
+      const W va = pl[a], vb = pl[b];
       pl[a] = vb;
       pl[b] = va;
     }
@@ -971,21 +1020,25 @@ constexpr uint32_t kEarlyClaimPairs = 8192;
 // tile and lanes 32..63 only set up pairs). A scene with SCENE_PACKED (all its deposits
 // non-negative) keeps two channels per 64-bit word in the first two planes
 // (packed_fixed_bits); one with SCENE_HUES a word per hue; other scenes one channel per word in
-// four. PACKED_ONLY: every scene of the frame has SCENE_PACKED, so the LDS tile holds two planes
+// four. RUNS: the kernel of a SCENE_RUNS frame, whose tiles go through the layers' lists one after
+// another with a 32-bit weight plane per run, and keep the pixels' channel sums in registers from
+// layer to layer. PACKED_ONLY: every scene of the frame has SCENE_PACKED, so the LDS tile holds two planes
 // only (half the LDS: two 512-thread workgroups share a compute unit at T = 64), or three in the
 // 1024-thread kernel, which serves up to three hues.
-enum WalkMode { WALK_COLOR, WALK_VERTEX_COLORS, WALK_VERTEX_STREAM, WALK_HUES };
-template <int T, bool PACKED_ONLY, int BLOCK>
+enum WalkMode { WALK_COLOR, WALK_VERTEX_COLORS, WALK_VERTEX_STREAM, WALK_HUES, WALK_RUNS };
+template <int T, bool PACKED_ONLY, int BLOCK, bool RUNS>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void tile_accum_kernel(const SceneDesc* __restrict__ descs,
                                                           const uint32_t* __restrict__ pairs,
                                                           const WorkItem* __restrict__ items,
+                                                          const uint32_t* __restrict__ row_start,
                                                           unsigned long long* split_fx, BatchCtl* ctl,
                                                           uint32_t count_work) {
   constexpr int kPlane = T * T;                         // pixels of a plane
   constexpr int kGuard = 2;                             // guard rows on each side of a plane
   constexpr int kStride = (T + 2 * kGuard) * T;         // elements from one plane to the next
   constexpr bool kStreamKernel = PACKED_ONLY && T == 64 && BLOCK == 1024;
-  constexpr bool kHueKernel = T == 64 && BLOCK == 1024;  // the kernels frames with hues run
+  static_assert(!RUNS || kStreamKernel, "runs are walked as streams");
+  constexpr bool kHueKernel = T == 64 && BLOCK == 1024 && !RUNS;  // the kernels frames with hues run
   constexpr int kPlanes = kStreamKernel ? 3 : PACKED_ONLY ? 2 : 4;
   static_assert(!kHueKernel || kPlanes >= kMaxHues, "a plane per hue");
   __shared__ unsigned long long s_tile[kPlanes * kStride];
@@ -995,6 +1048,10 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
   __shared__ uint32_t s_item[2];
   __shared__ uint32_t s_batch[2];  // next batch of 64 pairs, per phase
   unsigned long long* const tile = s_tile + kGuard * T;  // row 0 of plane 0
+  // RUNS: planes of 32-bit words in the same memory, a weight plane per run of the layer
+  static_assert(2 * kPlanes >= kRunPlanes || !RUNS, "a plane per run");
+  uint32_t* const tile32 = reinterpret_cast<uint32_t*>(s_tile) + kGuard * T;
+  __shared__ uint32_t s_run[RUNS ? kRunPlanes : 1][4];  // the runs' colours (run_color)
   constexpr int kWaves = BLOCK / 64;
   // Sample-stream walk (two-channel frames, T = 64, one workgroup per compute unit; with a colour
   // per vertex under the default blend, whose channel values need no factors): each wave lays the samples of its 64 pairs end to end and walks that stream
@@ -1065,7 +1122,18 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
     const int n_hues = hues ? D.n_hues : 0;
     if (kHueKernel && hues && threadIdx.x < kMaxHues) s_hue[threadIdx.x] = hue_scale(D, threadIdx.x, W.tile_pairs);
     int G[4] = {0, 0, 0, 0};
-    if (hues) {
+    const uint32_t n_layers = RUNS ? D.row_stride : 1u;
+    const uint32_t* const tile_rows = row_start + 2u * n_layers * W.tile;
+    int K[4] = {0, 0, 0, 0};
+    const int wG = RUNS ? weight_bits(W.tile_pairs) : 0;
+    const uint32_t wq = 1u << wG;  // a sample's weight
+    unsigned long long acc[RUNS ? T * T / BLOCK : 1][4] = {};
+    if constexpr (RUNS) {
+      const uint32_t nt = tile_rows[2u * n_layers] - tile_rows[0];
+#pragma unroll
+      for (int c = 0; c < 4; c++) K[c] = run_color_bits(D, c, nt);
+    }
+    if (RUNS || hues) {
       // (the channels' scales are not used)
     } else if (two_ch) {
 #pragma unroll
@@ -1100,15 +1168,44 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
       __syncthreads();
       continue;
     }
-    const int planes = hues ? n_hues : two_ch ? 2 : 4;
-    for (int k = threadIdx.x; k < planes * kPlane; k += BLOCK) tile[(k / kPlane) * kStride + k % kPlane] = 0ull;
+    for (uint32_t layer = 0; layer < n_layers; layer++) {
+    uint32_t r_beg = W.begin, r_end = W.end;  // the item's part of the layer's list
+    // the list holds its y-major pairs before `mid`, its x-major pairs from there
+    uint32_t mid = W.mid;
+    int planes = hues ? n_hues : two_ch ? 2 : 4;
+    uint32_t run1 = 0, run2 = 0, run3 = 0, run4 = 0, run5 = 0;  // RUNS: the layer's first segments
+    if constexpr (RUNS) {
+      const uint32_t lb = tile_rows[2u * layer], le = tile_rows[2u * layer + 2u];
+      mid = tile_rows[2u * layer + 1u];
+      r_beg = r_beg > lb ? r_beg : lb;
+      r_end = r_end < le ? r_end : le;
+      if (r_beg >= r_end) continue;
+      const SceneDesc& DL = descs[layer];
+      pos = gen(DL.seg_pos);
+      planes = DL.n_runs;
+      static_assert(kRunPlanes == 6, "run1 .. run5");
+      run1 = DL.run_first[1];
+      run2 = DL.run_first[2];
+      run3 = DL.run_first[3];
+      run4 = DL.run_first[4];
+      run5 = DL.run_first[5];
+      if (threadIdx.x < kRunPlanes * 4) {
+        const int f = threadIdx.x >> 2, c = threadIdx.x & 3;
+        const uint32_t code = (bc >> (4 * c)) & 15u;
+        const float v = blend_value(code, DL.run_color[f][c], DL.run_color[f][3], DL.blend_k[c]);
+        s_run[f][c] = run_color(v, c == 0 ? K[0] : c == 1 ? K[1] : c == 2 ? K[2] : K[3]);
+      }
+      // (a thread zeroes and converts the same pixels, so the layer before needs no barrier here;
+      // s_run's readers have all passed the barriers of this layer's walk only after this write)
+      for (int k = threadIdx.x; k < planes * kPlane; k += BLOCK) tile32[(k / kPlane) * kStride + k % kPlane] = 0u;
+    } else {
+      for (int k = threadIdx.x; k < planes * kPlane; k += BLOCK) tile[(k / kPlane) * kStride + k % kPlane] = 0ull;
+    }
     if (threadIdx.x == 0) s_batch[0] = s_batch[1] = 2u * kWaves;
     __syncthreads();
-    // the tile's list holds its y-major pairs before `mid`, its x-major pairs from there
-    const uint32_t mid = W.mid;
     for (int phase = 0; phase < 2; phase++) {  // 0: y-major pairs, 1: x-major pairs
-      const uint32_t pb = phase ? (W.begin > mid ? W.begin : mid) : W.begin;
-      const uint32_t pe = phase ? W.end : (W.end < mid ? W.end : mid);
+      const uint32_t pb = phase ? (r_beg > mid ? r_beg : mid) : r_beg;
+      const uint32_t pe = phase ? r_end : (r_end < mid ? r_end : mid);
       const uint32_t n_batches = pe > pb ? (pe - pb + 63u) >> 6 : 0u;
       // an empty phase deposits nothing: without y-major pairs the tile stays zero, so it
       // needs no transpose either
@@ -1130,6 +1227,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
         if (e != kNoPair) {
           const uint32_t s = e & kPairIndex;
           p = pos[s];
+          if constexpr (RUNS) return;  // (a run's colour comes in with its sums)
           ca = col0[s];
           if (col1) cb = col1[s];
           if (n_hues > 1) {  // (such a scene has no col1: the key travels in its place)
@@ -1150,6 +1248,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
         constexpr bool kVS = decltype(mode_tag)::value == WALK_VERTEX_STREAM;
         constexpr bool kVC = kVS || decltype(mode_tag)::value == WALK_VERTEX_COLORS;
         constexpr bool kHues = decltype(mode_tag)::value == WALK_HUES;
+        constexpr bool kRuns = decltype(mode_tag)::value == WALK_RUNS;
+        int fx_m = 0, fx_s = 0;  // kRuns: m at the tile's middle column and the slope, times 2^kFxBits
         // ---- per-lane setup of one pair of the current batch ----
         int packed = 0;  // n | q0 << 8 | vertex colours << 17 | negative colour << 18
         float m_first = 0.f, slope = 0.f, s_first = 0.f, ds = 0.f;
@@ -1198,8 +1298,15 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             b = b < wb ? b : wb;
           }
           if (a <= b) {
-            ca = a_cur;
-            if constexpr (kHues) {
+            if constexpr (!kRuns) ca = a_cur;
+            if constexpr (kRuns) {
+              const double mc = m0 + ((maj0 + (T / 2 + 0.5)) - M0) * sl - min0 - 0.5;
+              // (a weight rounds to nearest, with the carry into jl, by half a unit added here)
+              fx_m = (int)__builtin_rint(mc * (double)(1 << kFxBits)) + ((1 << (kFxBits - wG)) >> 1);
+              fx_s = (int)__builtin_rint(sl * (double)(1 << kFxBits));
+              const uint32_t s = e_cur & kPairIndex;
+              cq2 = ((s >= run1) + (s >= run2) + (s >= run3) + (s >= run4) + (s >= run5)) * kStride;  // its plane
+            } else if constexpr (kHues) {
               int f = 0;
               if (n_hues > 1) {
                 const uint64_t ray = ((uint64_t)__float_as_uint(c_cur.y) << 32 | __float_as_uint(c_cur.x)) >> kPathBits;
@@ -1258,7 +1365,15 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
           // past the end of the stream need no mask. Stream word i holds a bit per position
           // 64 i .. 64 i + 63 that starts a record; lane l of step s finds its record as the
           // number of starts at positions <= 64 s + l, minus one.
-          const int n = packed & 0xff;
+          //
+          // With runs a lane takes two samples of a pair, columns c and c + ceil(n / 2), at one
+          // position: the record search and its read, a third of a step's instructions, serve both
+          // (the second is left out at the last position of an odd n). The line is in fixed point there, 22
+          // bits below the pixel: m = M + S position, both modulo 2^32 and exact, its pixel M >> 22
+          // and the weight the G bits below. Record c: {M at position 0, S, 4 (q0_c - pre_c) and
+          // the plane, last position with a second sample}, {S ceil(n / 2), 4 ceil(n / 2)}.
+          const int n_all = packed & 0xff;
+          const int n = kRuns ? (n_all + 1) >> 1 : n_all;  // positions
           const uint64_t live = __ballot(n != 0);
           if (live) {
             const int incl = wave_sum_incl(n);
@@ -1279,9 +1394,16 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             if (lane < steps) mask[lane] = 0ull;
             if (n) {
               const int off = ((packed >> 8) & 0xff) - pre;
-              rec[2 * c] = make_uint4((uint32_t)off, __float_as_uint(m_first), __float_as_uint(slope),
-                                      (uint32_t)((kHues ? off + cq2 : off) * 8));
-              if constexpr (kHues) {
+              if constexpr (kRuns) {
+                rec[2 * c] = make_uint4((uint32_t)(fx_m + __mul24(off - T / 2, fx_s)), (uint32_t)fx_s,
+                                        (uint32_t)((off + cq2) * 4), (uint32_t)(pre + n_all - n - 1));
+                *reinterpret_cast<uint2*>(&rec[2 * c + 1]) = make_uint2((uint32_t)__mul24(n, fx_s), (uint32_t)(4 * n));
+              } else {
+                rec[2 * c] = make_uint4((uint32_t)off, __float_as_uint(m_first), __float_as_uint(slope),
+                                        (uint32_t)((kHues ? off + cq2 : off) * 8));
+              }
+              if constexpr (kRuns) {
+              } else if constexpr (kHues) {
                 *reinterpret_cast<uint2*>(&rec[2 * c + 1]) = make_uint2((uint32_t)cq0, (uint32_t)cq1);
               } else if constexpr (kVS) {
                 rec[2 * c + 1] = make_uint4(__float_as_uint((float)((packed >> 8) & 0xff)), __float_as_uint(s_first),
@@ -1294,57 +1416,74 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               atomicOr(&mask[pre >> 6], 1ull << (pre & 63));
             }
             if (lane == 0) {
-              rec[2 * n_live] = make_uint4((uint32_t)(-total), 0u, 0u, (uint32_t)(-total * 8));
-              rec[2 * n_live + 1] = make_uint4(0u, 0u, 0u, 0u);
+              if constexpr (kRuns) {
+                // (no colour to be zero: the empty record's line lies above the tile, in guard row -2)
+                rec[2 * n_live] = make_uint4((uint32_t)(-4 << kFxBits), 0u, (uint32_t)(-total * 4), 0xffffffffu);
+                rec[2 * n_live + 1] = make_uint4(0u, 0u, 0u, 0u);
+              } else {
+                rec[2 * n_live] = make_uint4((uint32_t)(-total), 0u, 0u, (uint32_t)(-total * 8));
+                rec[2 * n_live + 1] = make_uint4(0u, 0u, 0u, 0u);
+              }
               if constexpr (kVS) vrec[2 * n_live] = vrec[2 * n_live + 1] = make_uint4(0u, 0u, 0u, 0u);
               if (total & 63) atomicOr(&mask[total >> 6], 1ull << (total & 63));
             }
-            // lane i keeps stream word i in registers; a step takes its word with a lane read
+            // Lane i keeps, for step i, the stream word's starts at positions 64 i + 1 .. 64 i + 63 and
+            // the address of the record before the first of those: a step takes them with three lane
+            // reads, and its lane l reads the record that many starts further on. (With the record
+            // count kept by scalar instructions, 17 of them a step, the scalar unit took as long as
+            // the vector ALU: 1M-ray frame 590 -> 549 us, 1.6M segments in runs 2920 -> 2700.) Past the last step (the read one step ahead, never used) the words
+            // are empty and every lane names the last record.
             const unsigned long long my_word = lane < steps ? mask[lane] : 0ull;
-            const uint32_t mw_lo = (uint32_t)my_word, mw_hi = (uint32_t)(my_word >> 32);
-            // Records of this lane's position in step s, read into (r0, r1); `seen` counts the
-            // starts of the words before s (wave-uniform). The record index is seen + [position
-            // 64 s starts a record] - 1 + the starts at positions 64 s + 1 .. 64 s + lane. Past
-            // the last step (the read one step ahead, never used) the word is taken as 1: every
-            // lane then names record seen <= 65.
-            uint32_t seen = 0;
-            const char* const rec_m1 = reinterpret_cast<const char*>(rec) - 32;  // record -1
+            const uint32_t my_lo = (uint32_t)(my_word >> 1), my_hi = (uint32_t)(my_word >> 33);
+            const int my_n = __builtin_popcountll(my_word);
+            const int my_first = wave_sum_incl(my_n) - my_n + (int)(my_word & 1ull) - 1;
+            const uint32_t my_rec = lds_address(rec) + (uint32_t)(my_first * 32);
             struct StepRec {
               uint4 r0, r1, a, d;
             };
             auto read_recs = [&](int s, StepRec& R) {
               const int sl = s < 63 ? s : 63;
-              uint32_t lo = __builtin_amdgcn_readlane(mw_lo, sl);
-              uint32_t hi = __builtin_amdgcn_readlane(mw_hi, sl);
-              if (s >= steps) {
-                lo = 1u;
-                hi = 0u;
-              }
-              const uint64_t X = ((uint64_t)hi << 32 | lo) >> 1;
-              const uint32_t k = __builtin_amdgcn_mbcnt_hi((uint32_t)(X >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)X, 0u));
-              const int first = (int)seen + (int)(lo & 1u) - 1;
-              seen += (uint32_t)__builtin_popcountll((uint64_t)hi << 32 | lo);
-              // the wave-uniform part of the address apart: one lane operation adds k
-              const char* const rbase = rec_m1 + (first + 1) * 32;
-              const uint4* const r = reinterpret_cast<const uint4*>(rbase + k * 32u);
-              R.r0 = r[0];
-              if constexpr (kHues) {
-                const uint2 q = *reinterpret_cast<const uint2*>(&r[1]);
+              const uint32_t lo = __builtin_amdgcn_readlane(my_lo, sl), hi = __builtin_amdgcn_readlane(my_hi, sl);
+              const uint32_t k = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+              const uint32_t ra = __builtin_amdgcn_readlane(my_rec, sl) + k * 32u;
+              R.r0 = lds_read16(ra);
+              if constexpr (kHues || kRuns) {
+                const uint2 q = lds_read8(ra + 16u);
                 R.r1.x = q.x;
                 R.r1.y = q.y;
               } else {
-                R.r1 = r[1];
+                R.r1 = lds_read16(ra + 16u);
               }
               if constexpr (kVS) {
-                const uint4* const rv = r + (vrec - rec);
-                R.a = rv[0];
-                R.d = rv[1];
+                const uint32_t rv = ra + (lds_address(vrec) - lds_address(rec));
+                R.a = lds_read16(rv);
+                R.d = lds_read16(rv + 16u);
               }
             };
             // Step st at stream positions p = 64 st + lane: the sample's column is off + p, its
             // entry in plane 0 jl * T + column.
             const uint32_t lane8 = (uint32_t)lane * 8u;
+            uint32_t w_bits = (uint32_t)wG;  // in a lane register: the field extract takes one scalar only
+            if constexpr (kRuns) asm volatile("" : "+v"(w_bits));
             auto deposit_step = [&](int st, const StepRec& R) {
+              if constexpr (kRuns) {
+                const int p = lane + (st << 6);
+                auto put = [&](int M, uint32_t b) {
+                  int jl = M >> kFxBits;
+                  jl = jl < -kGuard ? -kGuard : (jl > T ? T : jl);
+                  uint32_t* const t = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(tile32) + (((uint32_t)jl << 8) + b));
+                  const uint32_t r = __builtin_amdgcn_ubfe((uint32_t)M, (uint32_t)(kFxBits - wG), w_bits);
+                  atomicAdd(t, wq - r);
+                  atomicAdd(t + T, r);
+                };
+                int M;
+                asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(M) : "v"(p), "v"((int)R.r0.y), "v"((int)R.r0.x));
+                const uint32_t base = ((uint32_t)p << 2) + R.r0.z;
+                put(M, base);
+                // (no second sample: above the tile, into the guard rows)
+                put(p <= (int)R.r0.w ? M + (int)R.r1.x : -4 << kFxBits, base + R.r1.y);
+                return;
+              }
               const uint4 r0 = R.r0, r1 = R.r1;
               const int col = (int)r0.x + lane + (st << 6);
               const float m = __builtin_fmaf((float)col, __uint_as_float(r0.z), __uint_as_float(r0.y));
@@ -1378,7 +1517,15 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             // zero adds into guard row -2: the loop is entered with the same LDS operations
             // in flight as it loops back with (two reads, four adds; two with hues), so that the
             // compiler's wait counts inside the loop stay exact
-            {
+            if constexpr (kRuns) {
+              uint32_t zero = 0u;
+              asm volatile("" : "+v"(zero));
+              uint32_t* const g = tile32 + (-kGuard * T + lane);
+              for (int k = 0; k < 2; k++) {
+                atomicAdd(g, zero);
+                atomicAdd(g + T, zero);
+              }
+            } else {
               unsigned long long zero = 0ull;
               asm volatile("" : "+v"(zero));  // an add the compiler cannot turn into a load
               unsigned long long* const g = tile + (-kGuard * T + lane);
@@ -1402,7 +1549,10 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               __builtin_amdgcn_sched_barrier(0);
               if (st + 2 >= steps) break;
             }
-            wave_samples += (unsigned long long)total;
+            if (!kRuns)
+              wave_samples += (unsigned long long)total;
+            else if (count_work)
+              wave_samples += (unsigned long long)__builtin_amdgcn_readlane(wave_sum_incl(n_all), 63);
             wave_atomics += (kHues ? 2u : 4u) * (unsigned)steps;
           }
           return;
@@ -1541,14 +1691,16 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
           e1 = e3;
         }
       };
-      bool walked = false;
+      bool walked = RUNS;
+      if constexpr (RUNS) run(std::integral_constant<int, WALK_RUNS>{});
       if constexpr (kHueKernel) {
         if (hues) {
           run(std::integral_constant<int, WALK_HUES>{});
           walked = true;
         }
       }
-      if (walked) {
+      if constexpr (RUNS) {
+      } else if (walked) {
       } else if (kStreamKernel && col1 && bc == kBlendDefault) {
         run(std::integral_constant<int, kStreamKernel ? WALK_VERTEX_STREAM : WALK_VERTEX_COLORS>{});
       } else if (col1) {
@@ -1558,13 +1710,55 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
       }
       __syncthreads();
       if (phase == 0) {
-        transpose_tile<T, kStride, kWaves>(tile, planes, wave, lane);
+        if constexpr (RUNS)
+          transpose_tile<T, kStride, kWaves>(tile32, planes, wave, lane);
+        else
+          transpose_tile<T, kStride, kWaves>(tile, planes, wave, lane);
         __syncthreads();
       }
     }
+    if constexpr (RUNS) {
+      for (int f = 0; f < planes; f++) {
+        const uint32_t q0 = s_run[f][0], q1 = s_run[f][1], q2 = s_run[f][2], q3 = s_run[f][3];
+#pragma unroll
+        for (int i = 0; i < T * T / BLOCK; i++) {
+          const uint32_t w = tile32[f * kStride + i * BLOCK + (int)threadIdx.x];
+          acc[i][0] += (unsigned long long)w * q0;
+          acc[i][1] += (unsigned long long)w * q1;
+          acc[i][2] += (unsigned long long)w * q2;
+          acc[i][3] += (unsigned long long)w * q3;
+        }
+      }
+      __syncthreads();  // the next layer writes s_run
+    }
+    }
     if (!claim_early) claim();
     const WorkItem wn = load_next();  // in flight during the flush
-    if (split) {
+    if constexpr (RUNS) {
+      unsigned long long* fx = split_fx + (size_t)W.slot * kSlotU64;
+      double un[4];
+#pragma unroll
+      for (int c = 0; c < 4; c++) un[c] = __builtin_ldexp(1.0, -(wG + K[c]));
+#pragma unroll
+      for (int i = 0; i < T * T / BLOCK; i++) {
+        const int k = i * BLOCK + (int)threadIdx.x;
+        if (split) {  // (the merge converts the tile's sums)
+#pragma unroll
+          for (int c = 0; c < 4; c++)
+            if (acc[i][c]) atomicAdd(&fx[c * T * T + k], acc[i][c]);
+          continue;
+        }
+        const int gx = x0 + k % T, gy = y0 + k / T;
+        if (gx >= v.width || gy >= v.height) continue;
+        const size_t px = (size_t)gy * v.width + gx;
+        float4 o = accum[px];
+        o.x += (float)((double)(long long)acc[i][0] * un[0]);
+        o.y += (float)((double)(long long)acc[i][1] * un[1]);
+        o.z += (float)((double)(long long)acc[i][2] * un[2]);
+        o.w += (float)((double)(long long)acc[i][3] * un[3]);
+        accum[px] = o;
+      }
+    } else if (split) {
       // exact partial sums into the tile's merge slot (integer atomics: order independent)
       unsigned long long* fx = split_fx + (size_t)W.slot * kSlotU64;
       const int n_fields = hues ? 2 * n_hues : 4;
@@ -1666,7 +1860,10 @@ __global__ __launch_bounds__(kMergeBlock) void tile_merge_kernel(const SceneDesc
     const int T = v.tile, TT = tile_px;
     const int x0 = (int)(t % (uint32_t)v.tiles_x) * T, y0 = (int)(t / (uint32_t)v.tiles_x) * T;
     const bool hues = (D.flags & SCENE_HUES) != 0;
-    const uint32_t np = packed_pairs(row_start, g);
+    const bool runs = (D.flags & SCENE_RUNS) != 0;
+    const uint32_t nl = runs ? D.row_stride : 1u;
+    const uint32_t nt = row_start[2u * nl * (g + 1u)] - row_start[2u * nl * g];
+    const uint32_t np = nt < kPackedPiece ? nt : kPackedPiece;
     __syncthreads();  // (the slot before is done with the table)
     if (hues && threadIdx.x < kMaxHues) s_hue[threadIdx.x] = hue_scale(D, threadIdx.x, np);
     __syncthreads();
@@ -1674,7 +1871,9 @@ __global__ __launch_bounds__(kMergeBlock) void tile_merge_kernel(const SceneDesc
     if (!hues) {
 #pragma unroll
       for (int c = 0; c < 4; c++)
-        un[c] = __builtin_ldexp(1.0, (D.flags & SCENE_PACKED) ? -packed_fixed_bits(D, c, np) : -(scene_fixed_bits(D, c) + kWBits));
+        un[c] = __builtin_ldexp(1.0, runs ? -(weight_bits(np) + run_color_bits(D, c, nt))
+                                     : (D.flags & SCENE_PACKED) ? -packed_fixed_bits(D, c, np)
+                                                                : -(scene_fixed_bits(D, c) + kWBits));
     }
     const int n_fields = hues ? 2 * D.n_hues : 4;
     const bool whole = (D.flags & SCENE_FRESH_IMAGE) != 0;  // the frame clears and resolves here
@@ -1829,19 +2028,20 @@ uint64_t work_items_scratch_elems(int n_tiles_total) {
   return n_tiles_total <= kPlanTiles ? 1 : scan_scratch_elems(2 * (uint64_t)n_tiles_total + 1);
 }
 
-hipError_t launch_work_items(const SceneDesc* descs, const uint32_t* tile_scene, int n_tiles_total,
+hipError_t launch_work_items(const SceneDesc* descs, const uint32_t* tile_scene, int n_tiles_total, int layers,
                              const uint32_t* row_count, uint32_t* row_start, uint32_t* scan_scratch, BatchCtl* ctl,
                              WorkItem* items, uint32_t items_cap, uint32_t* split_tiles, uint32_t split_cap,
                              uint64_t pairs_cap, uint32_t min_piece, uint32_t max_piece, uint32_t grid,
                              bool whole_images, hipStream_t st) {
-  const PlanLimits L{pairs_cap, items_cap, split_cap, min_piece, max_piece, grid, whole_images ? 1u : 0u};
+  const PlanLimits L{pairs_cap, items_cap, split_cap, min_piece, max_piece, grid, whole_images ? 1u : 0u,
+                     (uint32_t)layers};
   const int n = n_tiles_total;
   if (n <= kPlanTiles) {
     hipLaunchKernelGGL(plan_items_kernel, dim3(1), dim3(1024), 0, st, descs, tile_scene, n, row_count, ctl, row_start,
                        items, split_tiles, L);
     return hipGetLastError();
   }
-  hipError_t e = launch_scan_exclusive(row_count, row_start, 2 * (uint64_t)n + 1, scan_scratch, st, &ctl->total_pairs);
+  hipError_t e = launch_scan_exclusive(row_count, row_start, 2 * (uint64_t)n * layers + 1, scan_scratch, st, &ctl->total_pairs);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(tile_classes_kernel, dim3((n + 255) / 256), dim3(256), 0, st, n, row_start, ctl, L);
   if ((e = hipGetLastError()) != hipSuccess) return e;
@@ -1856,12 +2056,14 @@ hipError_t launch_work_items(const SceneDesc* descs, const uint32_t* tile_scene,
 // block = 512, two of 512), 32 with four 36.9 KB and with two 18.4 KB (four of 256); the
 // persistent grid fills every compute unit.
 hipError_t launch_tile_accum(const SceneDesc* descs, const uint32_t* pairs, const WorkItem* items,
-                             unsigned long long* split_fx, BatchCtl* ctl, int tile, bool packed_only, int block,
-                             bool count_work, int n_cu, hipStream_t st) {
-#define LG_TILE_LAUNCH(T, P, B, PER_CU)                                                                     \
-  hipLaunchKernelGGL((tile_accum_kernel<T, P, B>), dim3(n_cu * (PER_CU)), dim3(B), 0, st, descs, pairs, items, \
-                     split_fx, ctl, count_work ? 1u : 0u)
-  if (tile == 64) {
+                             const uint32_t* row_start, unsigned long long* split_fx, BatchCtl* ctl, int tile,
+                             bool packed_only, int block, bool runs, bool count_work, int n_cu, hipStream_t st) {
+#define LG_TILE_LAUNCH(T, P, B, PER_CU, ...)                                                                     \
+  hipLaunchKernelGGL((tile_accum_kernel<T, P, B, bool(__VA_ARGS__ + 0)>), dim3(n_cu * (PER_CU)), dim3(B), 0, st, \
+                     descs, pairs, items, row_start, split_fx, ctl, count_work ? 1u : 0u)
+  if (runs) {
+    LG_TILE_LAUNCH(64, true, 1024, 1, 1);
+  } else if (tile == 64) {
     if (packed_only && block == 512)
       LG_TILE_LAUNCH(64, true, 512, 2);
     else if (packed_only)

@@ -908,6 +908,7 @@ int lg_segments_upload(lg_segments* s, const float* pos, const float* color0, co
   s->max_abs = 0.0f;
   s->nonneg = true;
   s->hues = SceneHues{};
+  s->runs = SegRuns{};
   s->n_rays = 0;
   // a color1 equal to color0 bit for bit is no per-vertex colour: the accumulation then takes
   // the one-colour walk, which deposits the same bits
@@ -931,6 +932,9 @@ int lg_segments_upload(lg_segments* s, const float* pos, const float* color0, co
       }
     s->max_abs = mx;
     s->nonneg = nonneg;
+    if (s->one_color)
+      for (uint64_t i = 0; i < n && s->runs.add(i, color0 + 4 * i); i++) {
+      }
     LG_HIP(hipMemcpyAsync(s->key.p, keys.data(), n * 8, hipMemcpyHostToDevice, st));
     LG_HIP(hipStreamSynchronize(st));
   }

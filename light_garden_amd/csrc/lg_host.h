@@ -108,14 +108,15 @@ hipError_t launch_bin(int pass, const SceneDesc* descs, int n_scenes, const uint
 // its y-major and x-major pairs, and where they start; scan_scratch holds
 // work_items_scratch_elems(n_tiles_total) u32.
 uint64_t work_items_scratch_elems(int n_tiles_total);
-hipError_t launch_work_items(const SceneDesc* descs, const uint32_t* tile_scene, int n_tiles_total,
+// layers: pairs of rows per tile (1, or a SCENE_RUNS frame's layers)
+hipError_t launch_work_items(const SceneDesc* descs, const uint32_t* tile_scene, int n_tiles_total, int layers,
                              const uint32_t* row_count, uint32_t* row_start, uint32_t* scan_scratch, BatchCtl* ctl,
                              WorkItem* items, uint32_t items_cap, uint32_t* split_tiles, uint32_t split_cap,
                              uint64_t pairs_cap, uint32_t min_piece, uint32_t max_piece, uint32_t grid,
                              bool whole_images, hipStream_t st);
 hipError_t launch_tile_accum(const SceneDesc* descs, const uint32_t* pairs, const WorkItem* items,
-                             unsigned long long* split_fx, BatchCtl* ctl, int tile, bool packed_only, int block,
-                             bool count_work, int n_cu, hipStream_t st);
+                             const uint32_t* row_start, unsigned long long* split_fx, BatchCtl* ctl, int tile,
+                             bool packed_only, int block, bool runs, bool count_work, int n_cu, hipStream_t st);
 hipError_t launch_tile_merge(const SceneDesc* descs, const uint32_t* tile_scene, const uint32_t* row_start,
                              const uint32_t* split_tiles, const BatchCtl* ctl, unsigned long long* split_fx,
                              uint32_t split_cap, int tile, int n_cu, hipStream_t st);
@@ -211,6 +212,7 @@ struct lg_segments {
   // or with an identical color1, StringMods without modulo colours): col1 is not read
   bool one_color = true;
   lg::SceneHues hues;         // traced segments: the colours of their lights
+  lg::SegRuns runs;           // segments of one colour each: their runs of equal colours, if few
   uint64_t n_rays = 0;        // traced segments: the scene's rays (keys hold their index); else 0
   lg::DevBuf pos, col0, col1, key, pos64;
   bool has_pos64 = false;
@@ -256,6 +258,11 @@ void blend_factor_bounds(uint32_t code, float m, const float k[4], float out[4])
 // form in a frame's descriptor.
 SceneHues scene_hues(const lg_scene* sc);
 void set_hues(SceneDesc& D, const SceneHues& h);
+// Whether an accumulation goes by runs; the layers of such a frame, and the descriptor of one of them from the whole
+// scene's. All layers of a frame have the same tiles.
+bool use_runs(const lg_segments& s);
+int run_layers(const SegRuns& r);
+SceneDesc run_layer(const SceneDesc& D, const SegRuns& r, int layer, int n_layers);
 // Whether every value colour * factor is >= 0 for colour channels in [0, m].
 bool blend_nonneg(uint32_t code, float m, const float k[4]);
 

@@ -1,6 +1,7 @@
 // lg_internal.h — layouts shared by the host side (lg_api.hip) and the kernels
 // (lg_trace.hip, lg_accum.hip). gfx950 only.
 #pragma once
+#include <cstring>
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -202,8 +203,33 @@ enum SceneFlags : uint32_t {
   SCENE_FRESH_IMAGE = 2u,     // the frame clears, accumulates and resolves the image: the tile
                               // flushes write the accumulator and the RGBA16F target directly
   SCENE_PACKED = 4u,          // every deposit is non-negative: two channels per LDS word
-  SCENE_HUES = 8u             // with SCENE_PACKED: the segments' colours are fractions of at most
+  SCENE_HUES = 8u,            // with SCENE_PACKED: the segments' colours are fractions of at most
                               // kMaxHues light colours (SceneHues): one LDS word per deposit
+  SCENE_RUNS = 16u            // with SCENE_PACKED: runs of segments of one colour (SegRuns): the
+                              // tiles sum one weight per run. The frame's only scene, cut into
+                              // layers of up to kRunPlanes runs with a descriptor each
+};
+
+// Segments in runs of one colour (StringMods without modulo colours, or uploads): run r holds the segments from
+// first[r] (first[0] = 0) up to the next run's, all of colour color[r].
+constexpr int kRunPlanes = 6;   // runs whose weight planes fit a tile kernel's LDS
+constexpr int kMaxLayers = 4;
+constexpr int kMaxRuns = kRunPlanes * kMaxLayers;
+struct SegRuns {
+  int32_t n = 0;                // 0: the segments are not known to be of this form
+  uint32_t first[kMaxRuns] = {};
+  float color[kMaxRuns][4] = {};
+  // A segment of the given colour at index i follows; false: too many runs (n = 0 from then on).
+  bool add(uint64_t i, const float* c) {
+    if (n && std::memcmp(color[n - 1], c, sizeof(color[0])) == 0) return true;
+    if (n == kMaxRuns || i > 0xffffffffull) {
+      n = 0;
+      return false;
+    }
+    first[n] = (uint32_t)i;
+    std::memcpy(color[n++], c, sizeof(color[0]));
+    return true;
+  }
 };
 
 // The colours of traced segments. A ray's RGB is its light's, scaled by one factor per surface it
@@ -293,6 +319,13 @@ struct SceneDesc {
   uint64_t hue_ray[kMaxHues];
   float hue_bound[kMaxHues][2];
   double hue_ratio[kMaxHues][3];
+  // Tile t's pair rows (y-major, x-major) are rows 2 (row_base + row_stride t) and the next.
+  // row_stride is 1 but for the layers of a SCENE_RUNS frame, whose rows of a tile follow each other.
+  uint32_t row_base, row_stride;
+  // SCENE_RUNS: this layer's runs, by first segment in the layer, and their colours
+  int32_t n_runs;
+  uint32_t run_first[kRunPlanes];
+  float run_color[kRunPlanes][4];
 };
 
 // Source factors of the supported blends, per channel c of the interpolated colour (a = its

@@ -31,18 +31,18 @@ constexpr uint32_t kNaSplit = 128;          // tiles split over several work ite
 constexpr uint32_t kNaBinTarget = 128;      // bin chunks of one call
 constexpr uint32_t kNaChunkMin = 256;       // segments per bin chunk, at least
 constexpr uint32_t kNaMinPiece = 4096;      // smallest tile work item (bounds the item count)
-constexpr uint64_t kNaCounts = 2 * (uint64_t)kNaMaxTiles * (kNaBinTarget + 1);  // [chunk][tile][axis]
-constexpr uint64_t kNaRows = 2 * (uint64_t)kNaMaxTiles + 1;
+constexpr uint64_t kNaCounts = 2 * (uint64_t)kNaMaxTiles * (kNaBinTarget + kMaxLayers);  // [chunk][tile][axis]
+constexpr uint64_t kNaRows = 2 * (uint64_t)kNaMaxTiles * kMaxLayers + 1;
 constexpr uint64_t kNaScan = 64;  // >= work_items_scratch_elems(kNaMaxTiles)
 constexpr uint64_t kNaItems = kNaMaxTiles + kNaPairs / kNaMinPiece + 1024;
 
 constexpr uint64_t na_align(uint64_t x) { return (x + 255) & ~uint64_t(255); }
 // byte offsets of the partition
 constexpr uint64_t kOffDesc = 0;
-constexpr uint64_t kOffCtl = na_align(kOffDesc + sizeof(SceneDesc));
+constexpr uint64_t kOffCtl = na_align(kOffDesc + kMaxLayers * sizeof(SceneDesc));
 constexpr uint64_t kOffChunkPre = na_align(kOffCtl + sizeof(BatchCtl));
-constexpr uint64_t kOffCbase = na_align(kOffChunkPre + 2 * 4);
-constexpr uint64_t kOffCounts = na_align(kOffCbase + 2 * 4);
+constexpr uint64_t kOffCbase = na_align(kOffChunkPre + (kMaxLayers + 1) * 4);
+constexpr uint64_t kOffCounts = na_align(kOffCbase + (kMaxLayers + 1) * 4);
 constexpr uint64_t kOffRowCount = na_align(kOffCounts + kNaCounts * 4);
 constexpr uint64_t kOffRowStart = na_align(kOffRowCount + kNaRows * 4);
 constexpr uint64_t kOffScan = na_align(kOffRowStart + kNaRows * 4);
@@ -134,6 +134,9 @@ int lg_accumulate_noalloc(lg_ctx* ctx, const lg_segments* segs, lg_image* img) {
   if (packed) D.flags |= SCENE_PACKED;
   const bool hues = packed && segs->hues.n && D.blend_code == kBlendDefault && tile == 64;
   if (hues) set_hues(D, segs->hues);
+  D.row_stride = 1u;
+  const bool runs = packed && use_runs(*segs) && tile == 64;
+  const int layers = runs ? run_layers(segs->runs) : 1;
   const uint32_t min_piece = std::max(kNaMinPiece, std::min(ctx->tune.min_piece, kPackedPiece));
   const uint32_t max_piece = std::max(min_piece, std::min(ctx->tune.max_piece, kPackedPiece));
 
@@ -156,19 +159,22 @@ int lg_accumulate_noalloc(lg_ctx* ctx, const lg_segments* segs, lg_image* img) {
   BatchCtl hc;
   {
     std::lock_guard<std::mutex> lk(g_call_mu[ctx->device]);
-    hipLaunchKernelGGL(na_put_desc_kernel, dim3(1), dim3(64), 0, st, D, d_desc);
-    LG_HIP(hipGetLastError());
+    for (int l = 0; l < layers; l++) {
+      hipLaunchKernelGGL(na_put_desc_kernel, dim3(1), dim3(64), 0, st, runs ? run_layer(D, segs->runs, l, layers) : D,
+                         d_desc + l);
+      LG_HIP(hipGetLastError());
+    }
     LG_HIP(launch_fill_u32(reinterpret_cast<uint32_t*>(d_ctl), sizeof(BatchCtl) / 4, 0u, st));
     LG_HIP(launch_fill_u32(tile_scene, (uint64_t)n_tiles, 0u, st));
-    LG_HIP(launch_fill_u32(row_count, 2 * (uint64_t)n_tiles + 1, 0u, st));
+    LG_HIP(launch_fill_u32(row_count, 2 * (uint64_t)n_tiles * layers + 1, 0u, st));
     const int bin_grid = ctx->n_cu * (int)kBinWaves;
-    LG_HIP(launch_build_chunks(d_desc, 1, kNaChunkMin, kNaBinTarget, (uint32_t)bin_grid, chunk_pre, cbase, d_ctl, st));
-    LG_HIP(launch_bin(0, d_desc, 1, chunk_pre, cbase, d_ctl, counts, row_count, nullptr, 0, n_tiles, bin_grid, st));
-    LG_HIP(launch_work_items(d_desc, tile_scene, n_tiles, row_count, row_start, scan, d_ctl, items, (uint32_t)kNaItems,
+    LG_HIP(launch_build_chunks(d_desc, layers, kNaChunkMin, kNaBinTarget, (uint32_t)bin_grid, chunk_pre, cbase, d_ctl, st));
+    LG_HIP(launch_bin(0, d_desc, layers, chunk_pre, cbase, d_ctl, counts, row_count, nullptr, 0, n_tiles, bin_grid, st));
+    LG_HIP(launch_work_items(d_desc, tile_scene, n_tiles, layers, row_count, row_start, scan, d_ctl, items, (uint32_t)kNaItems,
                              split_tiles, kNaSplit, kNaPairs, min_piece, max_piece, (uint32_t)ctx->n_cu, false, st));
-    LG_HIP(launch_bin(1, d_desc, 1, chunk_pre, cbase, d_ctl, counts, row_start, pairs, kNaPairs, n_tiles, bin_grid, st));
-    LG_HIP(launch_tile_accum(d_desc, pairs, items, split_fx, d_ctl,
-                             tile, packed, hues ? 1024 : (int)ctx->tune.tile_block, false, ctx->n_cu, st));
+    LG_HIP(launch_bin(1, d_desc, layers, chunk_pre, cbase, d_ctl, counts, row_start, pairs, kNaPairs, n_tiles, bin_grid, st));
+    LG_HIP(launch_tile_accum(d_desc, pairs, items, row_start, split_fx, d_ctl, tile, packed,
+                             hues ? 1024 : (int)ctx->tune.tile_block, runs, false, ctx->n_cu, st));
     LG_HIP(launch_tile_merge(d_desc, tile_scene, row_start, split_tiles, d_ctl, split_fx, kNaSplit, tile, ctx->n_cu,
                              st));
     LG_HIP(hipMemcpyAsync(&hc, d_ctl, sizeof(BatchCtl), hipMemcpyDeviceToHost, st));

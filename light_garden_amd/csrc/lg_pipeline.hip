@@ -43,7 +43,7 @@ struct DevView {
 // Byte offsets of a frame's parts in frame_in and stage_in, each a multiple of 128.
 struct FrameLayout {
   size_t tile_scene, px_pre, item_pre0, counters, ctl, row_count, total;
-  FrameLayout(int n, int n_tiles) {
+  FrameLayout(int n, int n_tiles, int layers) {
     auto up = [](size_t b) { return (b + 127) & ~size_t(127); };  // (the control block's lines)
     tile_scene = up((size_t)n * sizeof(SceneDesc));
     px_pre = tile_scene + up((size_t)n_tiles * 4);
@@ -51,7 +51,7 @@ struct FrameLayout {
     counters = item_pre0 + up((size_t)(n + 1) * 4);
     ctl = counters + (size_t)n * kCounterStride;
     row_count = ctl + up(sizeof(BatchCtl));
-    total = row_count + up((size_t)(2 * n_tiles + 1) * 4);
+    total = row_count + up((size_t)(2 * n_tiles * layers + 1) * 4);
   }
   size_t out_bytes() const { return row_count - counters; }
 };
@@ -118,7 +118,8 @@ static bool scene_uses_boxes(const lg_ctx* ctx, const lg_scene* sc) {
 }
 
 struct Layout {
-  int n = 0;
+  int n = 0;                         // descriptors: one per entry, or one per layer
+  int layers = 1;                    // of a frame over segments in runs (SCENE_RUNS)
   bool fp64 = false;
   uint32_t max_bounce = 0;
   int cap_recs = 0, cap_objs = 0, cap_verts = 0;
@@ -127,6 +128,7 @@ struct Layout {
   int tile = 64;                     // screen tile edge of the frame
   bool packed_only = false;          // every accumulated scene keeps two channels per LDS word
   bool hues = false;                 // some scene's deposits are one LDS word (SCENE_HUES)
+  bool runs = false;                 // the frame's tiles sum weights of runs (SCENE_RUNS)
   uint64_t n_counts = 0, n_px = 0;  // n_counts: capacity of the per-frame [chunk][tile][axis] matrix
   uint32_t bin_target = 0;           // bin chunks per frame
   std::vector<int> tile_base;
@@ -160,6 +162,36 @@ void set_hues(SceneDesc& D, const SceneHues& h) {
   }
 }
 
+// Runs of a few segments are not worth a plane each: they average a batch of 64 pairs at least.
+bool use_runs(const lg_segments& s) { return s.runs.n > 0 && s.count >= 64ull * (uint64_t)s.runs.n; }
+
+int run_layers(const SegRuns& r) { return (r.n + kRunPlanes - 1) / kRunPlanes; }
+
+SceneDesc run_layer(const SceneDesc& D, const SegRuns& r, int layer, int n_layers) {
+  SceneDesc d = D;
+  const int per = (r.n + n_layers - 1) / n_layers;
+  const int a = std::min(layer * per, r.n), b = std::min(a + per, r.n);
+  const uint64_t first = a < r.n ? r.first[a] : D.seg_fixed;
+  const uint64_t end = b < r.n ? r.first[b] : D.seg_fixed;
+  d.flags |= SCENE_RUNS;
+  d.seg_pos = D.seg_pos + first;
+  d.seg_fixed = end - first;
+  d.row_base = (uint32_t)layer;
+  d.row_stride = (uint32_t)n_layers;
+  d.n_runs = b - a;
+  for (int f = 0; f < kRunPlanes; f++) {
+    d.run_first[f] = f < d.n_runs ? (uint32_t)(r.first[a + f] - first) : 0xffffffffu;
+    for (int c = 0; c < 4; c++) d.run_color[f][c] = f < d.n_runs ? r.color[a + f][c] : 0.0f;
+  }
+  return d;
+}
+
+// Whether every deposit of the segments into the image is non-negative (SCENE_PACKED).
+static bool scene_packed(const lg_ctx* ctx, const lg_segments& segs, const lg_image& img) {
+  return ctx->packed_accum && segs.nonneg && std::isfinite(segs.max_abs) &&
+         blend_nonneg(img.blend_code, segs.max_abs, img.blend.constant);
+}
+
 // Stage events only where the caller asked for them (the synchronous entry points on the
 // context's own stream).
 struct Scope {
@@ -175,7 +207,7 @@ static int enqueue(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, const
   const bool whole = whole_images(stages);
   SceneDesc* d_descs = P.descs.as<SceneDesc>();
   BatchCtl* d_ctl = P.ctl.as<BatchCtl>();
-  const FrameLayout F(n, L.n_tiles);
+  const FrameLayout F(n, L.n_tiles, L.layers);
   LG_HIP(hipMemcpyAsync(P.frame_in.p, P.stage_in.p, F.total, hipMemcpyHostToDevice, st));
   if ((stages & ST_CLEAR) && !whole) {
     Scope s(ctx, profile, "clear", L.n_px);
@@ -210,7 +242,7 @@ static int enqueue(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, const
     }
     {
       Scope s(ctx, profile, "bin_scan", 2 * (uint64_t)L.n_tiles);
-      LG_HIP(launch_work_items(d_descs, P.tile_scene.as<uint32_t>(), L.n_tiles, P.row_count.as<uint32_t>(),
+      LG_HIP(launch_work_items(d_descs, P.tile_scene.as<uint32_t>(), L.n_tiles, L.layers, P.row_count.as<uint32_t>(),
                                P.row_start.as<uint32_t>(), P.scan_scratch.as<uint32_t>(), d_ctl,
                                P.items.as<WorkItem>(), P.items_cap, P.split_tiles.as<uint32_t>(), P.split_cap,
                                P.pairs_cap, std::min(ctx->tune.min_piece, kPackedPiece),
@@ -224,9 +256,9 @@ static int enqueue(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, const
     }
     {
       Scope s(ctx, profile, "tile_accum", 0);
-      LG_HIP(launch_tile_accum(d_descs, P.pairs.as<uint32_t>(), P.items.as<WorkItem>(),
+      LG_HIP(launch_tile_accum(d_descs, P.pairs.as<uint32_t>(), P.items.as<WorkItem>(), P.row_start.as<uint32_t>(),
                                P.split_fx.as<unsigned long long>(), d_ctl, L.tile, L.packed_only,
-                               L.hues ? 1024 : (int)ctx->tune.tile_block, profile, ctx->n_cu, st));
+                               L.hues ? 1024 : (int)ctx->tune.tile_block, L.runs, profile, ctx->n_cu, st));
     }
     {
       Scope s(ctx, profile, "tile_merge", 0);
@@ -289,10 +321,16 @@ static int batch_validate(lg_ctx* ctx, hipStream_t st, Batch& B) {
 static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, bool allow_graph, Batch& B) {
   const std::vector<Entry>& E = B.E;
   const uint32_t stages = B.stages;
-  const int n = (int)E.size();
   const bool trace = stages & ST_TRACE, accum = stages & ST_ACCUM;
   int rc;
   Layout& L = B.L;
+  // Segments in runs of one colour, every deposit non-negative: the tiles sum weights (not with
+  // 32-pixel tiles, whose kernels do not have that walk)
+  L.runs = accum && !trace && E.size() == 1 && use_runs(*E[0].segs) && ctx->tune.tile == 64 &&
+           scene_packed(ctx, *E[0].segs, *E[0].img);
+  L.layers = L.runs ? run_layers(E[0].segs->runs) : 1;
+  const int entries = (int)E.size();
+  const int n = L.n = L.runs ? L.layers : entries;
   // ---- capacities ----
   L.max_bounce = 0;
   L.cap_recs = L.cap_objs = L.cap_verts = 1;
@@ -333,7 +371,7 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
   L.n_counts = 0;
   L.n_px = 0;
   L.tile = (int)ctx->tune.tile;
-  for (int i = 0; i < n; i++) {
+  for (int i = 0; i < entries; i++) {
     const Entry& e = E[i];
     if (e.img) {
       L.px_base[i] = L.n_px;
@@ -367,7 +405,7 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
   const uint32_t items_need =
       (uint32_t)std::min<uint64_t>(0xffffffffull, (uint64_t)L.n_tiles + P.pairs_cap / ctx->tune.min_piece + 1024);
   P.items_cap = std::max(P.items_cap, items_need);
-  const FrameLayout F(n, L.n_tiles);
+  const FrameLayout F(n, L.n_tiles, L.layers);
   {
     if ((rc = P.frame_in.ensure(F.total))) return rc;
     char* fi = P.frame_in.as<char>();
@@ -383,8 +421,8 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
   if ((rc = P.chunk_pre.ensure((size_t)(n + 1) * 4))) return rc;
   if ((rc = P.cbase.ensure((size_t)(n + 1) * 4))) return rc;
   if ((rc = P.places.ensure(std::max<uint64_t>(L.n_counts, 1) * 4))) return rc;
-  if ((rc = P.scan_scratch.ensure(work_items_scratch_elems(L.n_tiles) * 4))) return rc;
-  if ((rc = P.row_start.ensure((size_t)(2 * L.n_tiles + 1) * 4))) return rc;
+  if ((rc = P.scan_scratch.ensure(work_items_scratch_elems(L.n_tiles * L.layers) * 4))) return rc;
+  if ((rc = P.row_start.ensure((size_t)(2 * L.n_tiles * L.layers + 1) * 4))) return rc;
   if ((rc = P.pairs.ensure(P.pairs_cap * 4))) return rc;
   if ((rc = P.items.ensure((size_t)P.items_cap * sizeof(WorkItem)))) return rc;
   {
@@ -412,7 +450,7 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
   uint32_t* h_pre = reinterpret_cast<uint32_t*>(in + F.item_pre0);
   std::memset(in + F.counters, 0, F.total - F.counters);
   h_pre[0] = 0;
-  for (int i = 0; i < n; i++) {
+  for (int i = 0; i < entries; i++) {
     const Entry& e = E[i];
     SceneDesc& D = hd[i];
     std::memset(&D, 0, sizeof(D));
@@ -500,9 +538,18 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
       L.packed_only = false;
     }
     D.tile_base = L.tile_base[i];
+    D.row_base = (uint32_t)L.tile_base[i];
+    D.row_stride = 1u;
     if (accum) {
       int t = D.view.tiles_x * D.view.tiles_y;
       for (int k = 0; k < t; k++) h_tile_scene[L.tile_base[i] + k] = (uint32_t)i;
+    }
+  }
+  if (L.runs) {
+    const SceneDesc whole = hd[0];
+    for (int l = 0; l < n; l++) {
+      hd[l] = run_layer(whole, E[0].segs->runs, l, n);
+      h_px[l] = l ? L.n_px : 0;  // (the image's pixels are the first layer's)
     }
   }
   if (trace) reinterpret_cast<BatchCtl*>(in + F.ctl)->n_items_gen[0] = h_pre[n];
@@ -512,7 +559,7 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
                                  (uint64_t)L.max_tiles, L.n_counts, L.n_px, L.bin_target, P.pairs_cap, P.items_cap,
                                  P.split_cap, ctx->tune.rays_per_item, ctx->tune.min_piece, ctx->tune.max_piece,
                                  ctx->tune.trace_waves, ctx->tune.bvh_min_objects,
-                                 (uint64_t)L.tile, (uint64_t)L.packed_only, (uint64_t)L.hues, L.chunk,
+                                 (uint64_t)L.tile, (uint64_t)L.packed_only, (uint64_t)L.hues, (uint64_t)L.runs, L.chunk,
                                  ctx->tune.tile_block};
   for (DevBuf* b : {&P.frame_in, &P.item_pre, &P.chunk_pre, &P.cbase, &P.places, &P.scan_scratch, &P.row_start,
                     &P.pairs, &P.items, &P.split_tiles, &P.split_fx})
@@ -557,9 +604,9 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
 static int batch_finish(lg_ctx* ctx, Pipeline& P, bool profile, Batch& B, bool* rerun) {
   const std::vector<Entry>& E = B.E;
   const uint32_t stages = B.stages;
-  const int n = (int)E.size();
-  const bool trace = stages & ST_TRACE, accum = stages & ST_ACCUM;
   const Layout& L = B.L;
+  const int n = L.n;
+  const bool trace = stages & ST_TRACE, accum = stages & ST_ACCUM;
   // ---- overflow check ----
   const char* out = P.stage_out.as<const char>();
   const BatchCtl* hc = reinterpret_cast<const BatchCtl*>(out + n * kCounterStride);
@@ -619,6 +666,7 @@ static int batch_finish(lg_ctx* ctx, Pipeline& P, bool profile, Batch& B, bool* 
       e.segs->nonneg = e.scene->light_nonneg;
       e.segs->one_color = true;
       e.segs->hues = scene_hues(e.scene);
+      e.segs->runs = SegRuns{};
       e.segs->n_rays = e.scene->n_primary;
       e.scene->seg_hint = std::max(e.scene->seg_hint, segs);
     }

@@ -79,6 +79,7 @@ int copy_segments(lg_segments* dst, const lg_segments* src) {
   dst->max_abs = src->max_abs;
   dst->nonneg = src->nonneg;
   dst->hues = src->hues;
+  dst->runs = src->runs;
   dst->n_rays = src->n_rays;
   return LG_OK;
 }

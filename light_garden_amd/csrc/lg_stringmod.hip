@@ -494,6 +494,8 @@ int lg_string_mod_draw(lg_ctx* ctx, uint32_t n, const lg_string_mod* mods, lg_se
   std::vector<lg_mod_rem_color> mrc;
   uint64_t total = 0;
   bool nonneg = true;  // a segment's colour is the StringMod's or a mean of its modulo colours
+  lg::SegRuns runs;    // consecutive StringMods of one colour
+  bool in_runs = true;
   for (uint32_t i = 0; i < n; i++) {
     const lg_string_mod& outer = mods[i];
     const lg_string_mod& m = outer.nested ? *outer.nested : outer;
@@ -515,6 +517,7 @@ int lg_string_mod_draw(lg_ctx* ctx, uint32_t n, const lg_string_mod* mods, lg_se
     const uint64_t segs = d.n_points ? m.modulo : 0;
     if (!segs) continue;
     d.seg_base = total;
+    in_runs = in_runs && !m.n_modulo_colors && runs.add(total, m.color);
     total += segs;
     descs.push_back(d);
   }
@@ -554,6 +557,7 @@ int lg_string_mod_draw(lg_ctx* ctx, uint32_t n, const lg_string_mod* mods, lg_se
   out->max_abs = max_abs;
   out->nonneg = nonneg;
   out->hues = lg::SceneHues{};
+  out->runs = in_runs ? runs : lg::SegRuns{};
   out->n_rays = 0;
   // without modulo colours both ends of every segment take their StringMod's colour
   // (get_color, string_mod.rs:124-150): col1 is then neither written nor read
