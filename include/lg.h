@@ -381,7 +381,7 @@ int lg_batch_render(lg_ctx* ctx, uint32_t n, lg_scene* const* scenes, const lg_p
  * these are the knobs of the persistent GPU work lists, read by the autotuner. Apart from
  * `tile` none of them changes results: images are the same bits for every setting. */
 typedef struct lg_tuning {
-  uint32_t rays_per_item;  /* rays per trace work item, [64, 2^20]; default 256 */
+  uint32_t rays_per_item;  /* rays per trace work item, at most, [64, 2^20]; default 256 */
   uint32_t min_piece;      /* smallest tile work item in segment-tile pairs, >= 64; default 2048 */
   uint32_t max_piece;      /* largest tile work item, >= min_piece; default 32768; work items
                               hold at most 32768 pairs whatever the setting (the fixed point

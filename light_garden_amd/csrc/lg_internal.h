@@ -343,8 +343,22 @@ constexpr int kMaxGen = kPathBits;
 // after another, 12 ns each over the whole chip, so the words that persistent workgroups count on
 // have lines of their own: a workgroup waits for its claim, and behind other words' adds it waits
 // for those too.
+// Rays of a trace item when a launch has `total`: at most the tuning's (`rpi`), fewer, down to 64,
+// when there would be fewer items than the grid has workgroups. A workgroup waits for its
+// slowest wave at every append, and a launch for its slowest workgroup, so few rays are done sooner by
+// workgroups of one wave. (us of trace launches, items of 256 rays and so: 20000 rays, 4
+// objects 94 and 86; 12000 rays, 3 objects 97 and 79; 75011 rays, 23 objects 213 and 214. Sharing
+// the rays of an item out over its four waves gave no more: every further wave fetches the
+// kernel's code through its own compute unit's cache.)
+__host__ __device__ inline uint32_t trace_item_rays(uint64_t total, uint32_t rpi, uint32_t groups) {
+  const uint64_t waves = (total + 64ull * groups - 1) / (64ull * groups);  // per item
+  const uint64_t m = waves > 1 ? 64 * waves : 64;
+  return m < rpi ? (uint32_t)m : rpi;
+}
+
 struct BatchCtl {
   uint32_t n_items_gen[kMaxGen];   // trace items per generation
+  uint32_t item_rays[kMaxGen];     // rays of an item, per generation
   uint32_t n_chunks;
   uint32_t chunk;                  // segments per bin chunk (at least; see scene_chunk)
   uint32_t bin_groups;             // bin workgroups of the frame

@@ -450,6 +450,10 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
   uint32_t* h_pre = reinterpret_cast<uint32_t*>(in + F.item_pre0);
   std::memset(in + F.counters, 0, F.total - F.counters);
   h_pre[0] = 0;
+  uint64_t rays = 0;
+  for (const Entry& e : E)
+    if (trace && e.params.max_bounce) rays += e.scene->n_primary;
+  const uint32_t rpi = trace_item_rays(rays, ctx->tune.rays_per_item, (uint32_t)ctx->n_cu * ctx->tune.trace_waves);
   for (int i = 0; i < entries; i++) {
     const Entry& e = E[i];
     SceneDesc& D = hd[i];
@@ -483,7 +487,6 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
       D.n_lights = (int32_t)sc->lights.size();
       D.n_primary = sc->n_primary;
       // trace items of the first launch
-      const uint64_t rpi = ctx->tune.rays_per_item;
       h_pre[i + 1] = h_pre[i] + (e.params.max_bounce ? (uint32_t)((sc->n_primary + rpi - 1) / rpi) : 0u);
       D.max_bounce = e.params.max_bounce;
       for (int c = 0; c < 4; c++) D.cutoff[c] = e.params.cutoff_color[c];
@@ -552,7 +555,11 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
       h_px[l] = l ? L.n_px : 0;  // (the image's pixels are the first layer's)
     }
   }
-  if (trace) reinterpret_cast<BatchCtl*>(in + F.ctl)->n_items_gen[0] = h_pre[n];
+  if (trace) {
+    BatchCtl* c = reinterpret_cast<BatchCtl*>(in + F.ctl);
+    c->n_items_gen[0] = h_pre[n];
+    c->item_rays[0] = rpi;
+  }
   // ---- launch (graph replay when the shape is unchanged) ----
   std::vector<uint64_t> shape = {(uint64_t)n, stages, L.fp64, L.max_bounce, (uint64_t)L.cap_recs,
                                  (uint64_t)L.cap_objs, (uint64_t)L.cap_verts, (uint64_t)L.n_tiles,

@@ -1075,25 +1075,33 @@ __device__ __forceinline__ int find_scene(const uint32_t* pre, int n, uint32_t x
 // kernel, so they are read with device-scope atomic loads (not through this CU's cache).
 template <int BLOCK>
 __device__ __forceinline__ void build_items_block(const SceneDesc* __restrict__ descs, int n_scenes,
-                                                  uint32_t gen_ix, uint32_t rpi, uint32_t* item_pre,
+                                                  uint32_t gen_ix, uint32_t max_rpi, uint32_t* item_pre,
                                                   BatchCtl* ctl) {
   constexpr int kW = BLOCK / 64;
   __shared__ uint32_t s_w[kW];
   __shared__ uint32_t s_carry;
-  if (threadIdx.x == 0) s_carry = 0;
+  __shared__ unsigned long long s_rays;
+  auto scene_rays = [&](int sid) -> uint64_t {
+    if (sid >= n_scenes) return 0;
+    const SceneDesc& D = descs[sid];
+    if (gen_ix >= D.max_bounce) return 0;
+    const uint32_t g = __hip_atomic_load(gen(D.gen_count) + gen_ix - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return g < D.q_cap ? g : D.q_cap;
+  };
+  if (threadIdx.x == 0) {
+    s_carry = 0;
+    s_rays = 0;
+  }
   __syncthreads();
+  for (int sid = threadIdx.x; sid < n_scenes; sid += BLOCK) {
+    const uint64_t c = scene_rays(sid);
+    if (c) atomicAdd(&s_rays, (unsigned long long)c);
+  }
+  __syncthreads();
+  const uint32_t rpi = trace_item_rays(s_rays, max_rpi, gridDim.x);
   for (int base = 0; base < n_scenes; base += BLOCK) {
     const int sid = base + threadIdx.x;
-    uint32_t n_it = 0;
-    if (sid < n_scenes) {
-      const SceneDesc& D = descs[sid];
-      if (gen_ix < D.max_bounce) {
-        const uint32_t g = __hip_atomic_load(gen(D.gen_count) + gen_ix - 1, __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_AGENT);
-        const uint64_t c = g < D.q_cap ? g : D.q_cap;
-        n_it = (uint32_t)((c + rpi - 1) / rpi);
-      }
-    }
+    const uint32_t n_it = (uint32_t)((scene_rays(sid) + rpi - 1) / rpi);
     // block exclusive scan
     uint32_t x = n_it;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1115,6 +1123,7 @@ __device__ __forceinline__ void build_items_block(const SceneDesc* __restrict__ 
   if (threadIdx.x == 0) {
     item_pre[n_scenes] = s_carry;
     ctl->n_items_gen[gen_ix] = s_carry;
+    ctl->item_rays[gen_ix] = rpi;
     ctl->item_cursor[gen_ix] = 0;
   }
 }
@@ -1153,7 +1162,7 @@ template <typename T, int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void trace_kernel(const SceneDesc* __restrict__ descs, int n_scenes,
                                                       uint32_t gen_ix, uint32_t chunk, uint32_t launch_ix,
                                                       const uint32_t* __restrict__ item_pre,
-                                                      BatchCtl* ctl, uint32_t rpi, int cap_recs,
+                                                      BatchCtl* ctl, uint32_t max_rpi, int cap_recs,
                                                       int cap_objs, int cap_verts,
                                                       uint32_t* __restrict__ item_pre_next) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -1175,6 +1184,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const uint32_t n_items = ctl->n_items_gen[gen_ix];
+  const uint32_t rpi = ctl->item_rays[gen_ix];
   // Workgroup b's first item is b: the others have none. They leave before any atomic or fence
   // (with both, the 900 idle workgroups of a late generation held up the working ones by 13 us).
   if (blockIdx.x >= n_items) return;
@@ -1486,7 +1496,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
       s_last = __hip_atomic_fetch_add(&ctl->gen_done[gen_ix], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == working - 1;
     }
     __syncthreads();
-    if (s_last) build_items_block<BLOCK>(descs, n_scenes, gen_ix + chunk, rpi, item_pre_next, ctl);
+    if (s_last) build_items_block<BLOCK>(descs, n_scenes, gen_ix + chunk, max_rpi, item_pre_next, ctl);
   }
 }
 
