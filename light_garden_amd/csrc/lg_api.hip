@@ -439,6 +439,43 @@ static float4 box_f32(const Box2& b) {
   return make_float4(round_down(b.lo[0]), round_down(b.lo[1]), round_up(b.hi[0]), round_up(b.hi[1]));
 }
 
+// MediumMasks of objects with the given boxes, and the map of their buckets.
+static std::vector<MediumMasks> medium_masks(const std::vector<float4>& box, const std::vector<uint32_t>& flags,
+                                             float map[4]) {
+  std::vector<MediumMasks> M((box.size() + 63) / 64);
+  if (!M.empty()) std::memset(M.data(), 0, M.size() * sizeof(M[0]));
+  auto has = [&](size_t o) {
+    return (flags[o] & (OBJ_MATERIAL | OBJ_CLOSED)) == (OBJ_MATERIAL | OBJ_CLOSED);
+  };
+  float4 all = make_float4(INFINITY, INFINITY, -INFINITY, -INFINITY);
+  for (size_t o = 0; o < box.size(); o++)
+    if (has(o))
+      all = make_float4(std::min(all.x, box[o].x), std::min(all.y, box[o].y), std::max(all.z, box[o].z),
+                        std::max(all.w, box[o].w));
+  auto axis = [](float lo, float hi, float* m) {
+    m[0] = kMediumBuckets / (hi - lo);
+    m[1] = -lo * m[0];
+    if (!std::isfinite(m[0]) || !std::isfinite(m[1])) m[0] = m[1] = 0.0f;  // one bucket for all
+  };
+  axis(all.x, all.z, map);
+  axis(all.y, all.w, map + 2);
+  for (size_t o = 0; o < box.size(); o++) {
+    if (!has(o)) continue;
+    MediumMasks& m = M[o / 64];
+    const uint64_t bit = 1ull << (o % 64);
+    for (int k = medium_bucket(box[o].x, map[0], map[1]); k <= medium_bucket(box[o].z, map[0], map[1]); k++) m.x[k] |= bit;
+    for (int k = medium_bucket(box[o].y, map[2], map[3]); k <= medium_bucket(box[o].w, map[2], map[3]); k++) m.y[k] |= bit;
+  }
+  return M;
+}
+
+// Centre and half sizes of a box, in FP32 and not smaller.
+static float4 centre_f32(const Box2& b) {
+  const float cx = (float)(0.5 * (b.lo[0] + b.hi[0])), cy = (float)(0.5 * (b.lo[1] + b.hi[1]));
+  return make_float4(cx, cy, round_up(std::max(b.hi[0] - cx, cx - b.lo[0])),
+                     round_up(std::max(b.hi[1] - cy, cy - b.lo[1])));
+}
+
 // The culling blocks of objects with the given boxes and first records (CullBlock).
 struct CullLists {
   std::vector<CullBlock> blocks;
@@ -461,10 +498,10 @@ static CullLists build_blocks(const std::vector<Box2>& boxes, const std::vector<
       const int o = order[b + k];
       all.add(boxes[o]);
       mask[recs[top[o]].kind & 7] |= 1ull << k;
-      C.box.push_back(box_f32(boxes[o]));
+      C.box.push_back(centre_f32(boxes[o]));
       C.rec.push_back(top[o]);
     }
-    const float4 u = box_f32(all);
+    const float4 u = centre_f32(all);
     B.box[0] = u.x;
     B.box[1] = u.y;
     B.box[2] = u.z;
@@ -544,12 +581,8 @@ int compile_scene(lg_scene* sc, hipStream_t st) {
   std::vector<float4> box32(boxes.size());
   for (size_t o = 0; o < boxes.size(); o++) box32[o] = box_f32(boxes[o]);
   at.obj_box = pack.add(box32);
-  std::vector<float4> medium(box32);
-  const float4 none = make_float4(INFINITY, INFINITY, -INFINITY, -INFINITY);
-  for (size_t o = 0; o < medium.size(); o++)
-    if ((flags[o] & (OBJ_MATERIAL | OBJ_CLOSED)) != (OBJ_MATERIAL | OBJ_CLOSED)) medium[o] = none;
-  while (medium.size() % kBoxGroup) medium.push_back(none);
-  at.medium_box = pack.add(medium);
+  float medium_map[4];
+  at.medium = pack.add(medium_masks(box32, flags, medium_map));
   std::vector<Box2> walk_boxes;  // the blocks hold the objects of the walk
   std::vector<int32_t> walk_rec;
   for (size_t o = 0; o < obj_rec.size(); o++)
@@ -612,6 +645,7 @@ int compile_scene(lg_scene* sc, hipStream_t st) {
   sc->at = at;
   sc->n_trees = (int)tree_rec.size();
   sc->n_blocks = (int)cull.blocks.size();
+  std::memcpy(sc->medium_map, medium_map, sizeof(medium_map));
   sc->n_primary = base;
   float lmax = 0.0f;
   bool nonneg = true;

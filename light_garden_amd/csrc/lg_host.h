@@ -184,7 +184,7 @@ struct lg_scene {
   // tables.
   lg::DevBuf tables;
   struct {
-    size_t recs32, recs64, obj_n64, obj_flags, obj_rec, obj_box, medium_box, verts32, verts64, lights;
+    size_t recs32, recs64, obj_n64, obj_flags, obj_rec, obj_box, medium, verts32, verts64, lights;
     size_t blocks, block_box, block_rec;  // culling blocks (CullBlock)
     size_t tree_rec;                      // first records of the Logic trees of more than two primitives
   } at{};
@@ -193,6 +193,7 @@ struct lg_scene {
     return reinterpret_cast<const U*>(tables.as<char>() + off);
   }
   int n_blocks = 0;
+  float medium_map[4] = {};
   int n_trees = 0;
   lg::DevBuf q0, q1;          // ray queues (QRay<double>)
   uint64_t q_cap = 0;         // rays per queue

@@ -146,7 +146,7 @@ enum ObjFlags : uint32_t { OBJ_MATERIAL = 1u, OBJ_CLOSED = 2u };
 constexpr int kCullBlock = 64;
 constexpr int kBoxGroup = 4;
 struct alignas(16) CullBlock {
-  float box[4];         // lo.x lo.y hi.x hi.y
+  float box[4];         // centre x, y, half sizes x, y
   uint64_t kind[8];     // n_kinds masks, disjoint, together the block's objects
   int32_t first;        // of its boxes and first records
   int32_t n;
@@ -258,6 +258,19 @@ __host__ __device__ __forceinline__ T* gen(LG_G T* p) {
   return (T*)p;
 }
 
+// Which of 64 objects (with a material and an inside; others have no bit) have a padded box over a
+// bucket of x, and of y: a point lies in none but those of both its buckets.
+constexpr int kMediumBuckets = 64;
+struct MediumMasks {
+  uint64_t x[kMediumBuckets], y[kMediumBuckets];
+};
+// Monotone in v, so a point between a box's ends has a bucket between theirs.
+__host__ __device__ inline int medium_bucket(float v, float scale, float offset) {
+  const float b = __builtin_fmaf(v, scale, offset);
+  const float c = __builtin_fminf(__builtin_fmaxf(b, 0.0f), (float)(kMediumBuckets - 1));
+  return (int)c;
+}
+
 struct SceneDesc {
   // geometry (device buffers of the lg_scene)
   const LG_G void* recs;           // culling records, Rec<float> or Rec<double>
@@ -266,13 +279,13 @@ struct SceneDesc {
   const LG_G uint32_t* obj_flags;
   const LG_G int32_t* obj_rec;
   const LG_G float4* obj_box;      // per object: padded world box {lo.x, lo.y, hi.x, hi.y}
-  const LG_G float4* medium_box;   // the same for objects with a material and an inside, an empty
-                                   // box for others, padded to kBoxGroup
+  const LG_G MediumMasks* medium;  // per 64 objects
+  float medium_map[4];             // bucket of x: x * [0] + [1]; of y: y * [2] + [3] (medium_bucket)
   const LG_G void* verts;          // polygon vertices in the culling precision
   const LG_G double* verts64;
   const LG_G DevLight* lights;
   const LG_G CullBlock* blocks;    // culling by boxes; n_blocks = 0: the pass walks every record
-  const LG_G float4* block_box;    // the blocks' objects: padded boxes,
+  const LG_G float4* block_box;    // the blocks' objects: padded boxes (centre and half sizes),
   const LG_G int32_t* block_rec;   // and first records
   const LG_G int32_t* tree_rec;    // first record of each object that is a Logic tree of more
                                    // than two primitives (the object walk skips these)

@@ -471,7 +471,8 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
       D.obj_flags = gbl(sc->table<uint32_t>(sc->at.obj_flags));
       D.obj_rec = gbl(sc->table<int32_t>(sc->at.obj_rec));
       D.obj_box = gbl(sc->table<float4>(sc->at.obj_box));
-      D.medium_box = gbl(sc->table<float4>(sc->at.medium_box));
+      D.medium = gbl(sc->table<MediumMasks>(sc->at.medium));
+      std::memcpy(D.medium_map, sc->medium_map, sizeof(D.medium_map));
       D.verts = gbl(sc->table<void>(L.fp64 ? sc->at.verts64 : sc->at.verts32));
       D.verts64 = gbl(sc->table<double>(sc->at.verts64));
       D.lights = gbl(sc->table<DevLight>(sc->at.lights));

@@ -719,6 +719,14 @@ __device__ __forceinline__ void walk_objects(const RayT<T>& r, RS recs, const Re
   for (int rec = 0; rec < n_recs;) rec = eval_object<T, false>(r, recs, recs64, verts, rec, nb);
 }
 
+// a + b + the lane's bit of `carry`.
+__device__ __forceinline__ uint32_t add_carry(uint32_t a, uint32_t b, uint64_t carry) {
+  uint32_t r;
+  uint64_t out;
+  asm("v_addc_co_u32 %0, %1, %2, %3, %4" : "=v"(r), "=s"(out) : "v"(a), "v"(b), "s"(carry));
+  return r;
+}
+
 // The scene's culling blocks; tops: the blocks' first records in LDS.
 struct CullView {
   const LG_K CullBlock* blocks;
@@ -728,14 +736,14 @@ struct CullView {
 };
 
 // The culling pass by boxes: every lane tests its ray against the boxes of a block's objects
-// (uniform, branch-free, four boxes to a scalar load, 13 vector instructions each) for a t in
+// (uniform, branch-free, four boxes to a scalar load, ten vector instructions each) for a t in
 // [tmin, t_best + 4e-5 (1 + t_best)], which leaves a bit per candidate; then, kind by kind, each
 // lane evaluates its own candidates, as many rounds as the lane with the most has of that kind. A
 // walk that evaluates an object for the whole wave when one lane needs it (a hierarchy does that
 // too) runs nearly all of them once rays have split up, since a wave's rays are in no order then.
 // Bound: instruction issue and the serial loads of the rounds. A million rays, 64 objects, 10
-// bounces: trace launches 894 us over every object, 716 us through a hierarchy of boxes, 600 us
-// so; 75011 rays, 23 objects, 8 bounces: 263, 256 and 206 us; FP64, 40009 rays, 12 objects, 6
+// bounces: trace launches 894 us over every object, 716 us through a hierarchy of boxes, 582 us
+// so; 75011 rays, 23 objects, 8 bounces: 263, 256 and 204 us; FP64, 40009 rays, 12 objects, 6
 // bounces: 110 and 97 us (records in LDS). With 4 objects (20000 rays): 93 us over every object,
 // 99 us so: by boxes from lg_tuning.bvh_min_objects (8) objects.
 //
@@ -753,12 +761,12 @@ __device__ __forceinline__ void walk_boxes(const RayT<T>& r, RS recs, const Rec<
   // an FP64 ray's rounding to FP32 moves it by up to 2^-24 of its origin's coordinates; the boxes'
   // padding covers the same of theirs
   const float slack = sizeof(T) == 8 ? 6e-7f * (fabsf(ax) + fabsf(ay)) : 0.0f;
-  // whether the ray meets the box within [1e-5, lim]
+  const float wx = fabsf(ix), wy = fabsf(iy);
+  // whether the ray meets the box (centre and half sizes) within [1e-5, lim]
   auto meets = [&](const LG_K float* b, float lim) {
-    const float x0 = __builtin_fmaf(b[0], ix, ax), x1 = __builtin_fmaf(b[2], ix, ax);
-    const float y0 = __builtin_fmaf(b[1], iy, ay), y1 = __builtin_fmaf(b[3], iy, ay);
-    const float tn = fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)), 1e-5f);
-    const float tf = fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), lim);
+    const float cx = __builtin_fmaf(b[0], ix, ax), cy = __builtin_fmaf(b[1], iy, ay);
+    const float tn = fmaxf(fmaxf(__builtin_fmaf(-b[2], wx, cx), __builtin_fmaf(-b[3], wy, cy)), 1e-5f);
+    const float tf = fminf(fminf(__builtin_fmaf(b[2], wx, cx), __builtin_fmaf(b[3], wy, cy)), lim);
     if constexpr (sizeof(T) == 8) return !(tn > tf + slack);  // (NaN: a candidate)
     return tn <= tf;
   };
@@ -768,14 +776,16 @@ __device__ __forceinline__ void walk_boxes(const RayT<T>& r, RS recs, const Rec<
     const float lim = bt + 4e-5f * (1.0f + bt);
     if (C.n > 1 && !__ballot(meets(B->box, lim))) continue;
     const int n = B->n, first = B->first;
+    // from the last box down: each moves the bits up by one and adds its own, one instruction (an
+    // add with the comparison as carry)
     uint32_t half[2] = {0u, 0u};
 #pragma unroll
-    for (int h = 0; h < 2; h++)
-      for (int o = 32 * h; o < n && o < 32 * (h + 1); o += kBoxGroup) {
+    for (int h = 1; h >= 0; h--)
+      for (int o = (n < 32 * (h + 1) ? n + kBoxGroup - 1 : 32 * (h + 1)) / kBoxGroup * kBoxGroup - kBoxGroup; o >= 32 * h;
+           o -= kBoxGroup) {
         const LG_K float* const x = C.box + 4 * (first + o);
 #pragma unroll
-        for (int k = 0; k < kBoxGroup; k++)
-          if (meets(x + 4 * k, lim)) half[h] |= 1u << ((o + k) & 31);
+        for (int k = kBoxGroup - 1; k >= 0; k--) half[h] = add_carry(half[h], half[h], __ballot(meets(x + 4 * k, lim)));
       }
     const uint64_t cand = (uint64_t)half[1] << 32 | half[0];
     for (int k = 0; k < B->n_kinds; k++) {
@@ -1322,37 +1332,28 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
         }
       }
       // The medium a ray exits into: the first other material object, in scene order, that
-      // contains the exit point (tracer.rs:431-440), else air. The boxes of 64 objects at a time
-      // are tested for every lane, without a branch between them (they are the same for the wave:
-      // scalar loads, four boxes each), and leave a bit per object whose padded box holds the
-      // lane's point; a lane then runs the exact FP64 inside test on its own few candidates, in
-      // order, up to the first that contains it. FP32 points will do for the boxes, which are
-      // padded by 1e-5 (1 + |coordinates|). (With a branch and two dependent scalar loads per
-      // object the search took 4 to 8 us of a 33 us step with 64 objects; frames, us: 75k rays, 23
-      // objects 419 -> 398, 20 scenes of 1 to 160 objects 2174 -> 2000.)
+      // contains the exit point (tracer.rs:431-440), else air. The masks of the point's bucket in x
+      // and in y give the few of 64 objects at a time that can; a lane looks at its own, in
+      // order, up to the first whose padded box holds the point (in FP32: the padding of 1e-5 (1 +
+      // |coordinates|) covers that) and that contains it by the exact FP64 test. (A test of every
+      // box by every lane, without branches, was a quarter of the vector instructions of a step with
+      // 64 objects. With ten instead of thirteen instructions per box in the culling pass,
+      // trace launches: a million rays, 64 objects 618 -> 582 us; 75011 rays, 23 objects 215 -> 204.)
       if (__ballot(seek)) {
-        const LG_K float* const boxes = (const LG_K float*)D.medium_box;
-        const float fx = (float)px, fy = (float)py;
+        const int kx = medium_bucket((float)px, D.medium_map[0], D.medium_map[1]);
+        const int ky = medium_bucket((float)py, D.medium_map[2], D.medium_map[3]);
         for (int base = 0; base < n_objs; base += 64) {
-          const int n = n_objs - base < 64 ? n_objs - base : 64;
-          uint32_t half[2] = {0u, 0u};
-#pragma unroll
-          for (int h = 0; h < 2; h++)
-            for (int o = 32 * h; o < n && o < 32 * (h + 1); o += kBoxGroup) {
-              const LG_K float* const b = boxes + 4 * (base + o);
-#pragma unroll
-              for (int k = 0; k < kBoxGroup; k++)
-                if ((fx >= b[4 * k]) & (fy >= b[4 * k + 1]) & (fx <= b[4 * k + 2]) & (fy <= b[4 * k + 3]))
-                  half[h] |= 1u << ((o + k) & 31);
-            }
-          uint64_t cand = (uint64_t)half[1] << 32 | half[0];
+          const MediumMasks* const m = gen(D.medium) + base / 64;
+          uint64_t cand = seek ? m->x[kx] & m->y[ky] : 0ull;
           if ((unsigned)(obj - base) < 64u) cand &= ~(1ull << (obj - base));
-          if (!seek) cand = 0ull;
           while (__ballot(cand != 0ull)) {
             if (cand) {
               const int o = base + __builtin_ctzll(cand);
               cand &= cand - 1ull;
-              if (contains_object<double>(recs64, verts64, (int)(s_obj[o] >> 2), px, py)) {
+              const float4 b = gen(D.obj_box)[o];
+              const float fx = (float)px, fy = (float)py;
+              if ((fx >= b.x) & (fy >= b.y) & (fx <= b.z) & (fy <= b.w) &&
+                  contains_object<double>(recs64, verts64, (int)(s_obj[o] >> 2), px, py)) {
                 n2 = gen(D.obj_n64)[o];
                 seek = false;
                 cand = 0ull;
