@@ -865,7 +865,7 @@ __device__ __forceinline__ void hue_add(double (&p)[4], const HueScale& h, unsig
 // tile's list into items nor the order of anything changes a bit. C <= 2^30, less where the
 // tile's pairs would pass 2^62 in total. A deposit costs two 32-bit adds where two-channel words
 // take four of 64 bits, no colour is loaded, and instruction issue instead of the LDS is what bounds the
-// walk (1.6M segments in 16 runs at 4096x4096, 78M pairs: 3727 us by colours, 2255 us so).
+// walk (1.6M segments in 16 runs at 4096x4096, 78M pairs: 3727 us by colours, 2210 us so).
 // Finer than the colours' fixed point: a weight has the levels the brightest channel had, and
 // no colour is rounded to them.
 constexpr int kFxBits = 22;  // of a sample's place below the pixel; |slope| 2^22 is a 24-bit number
@@ -1366,14 +1366,17 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
           // 64 i .. 64 i + 63 that starts a record; lane l of step s finds its record as the
           // number of starts at positions <= 64 s + l, minus one.
           //
-          // With runs a lane takes two samples of a pair, columns c and c + ceil(n / 2), at one
-          // position: the record search and its read, a third of a step's instructions, serve both
-          // (the second is left out at the last position of an odd n). The line is in fixed point there, 22
-          // bits below the pixel: m = M + S position, both modulo 2^32 and exact, its pixel M >> 22
+          // With hues and with runs a lane takes two samples of a pair, columns c and c + ceil(n / 2),
+          // at one position: the record search and its reads, a third of a step's instructions,
+          // serve both (at the last position of an odd n the second goes to the guard rows). Instruction
+          // issue bounds these walks, the LDS the others. Record c with hues: {q0_c - pre_c, m_first,
+          // slope, 8 (q0_c - pre_c) and the plane}, {s, a a, last position with a second sample,
+          // its distance in columns} (1M-ray frame 541 -> 506 us, 20 uneven scenes 604 -> 563). With runs the line is in fixed point, 22 bits below the pixel: m = M + S position, both modulo 2^32 and exact, its pixel M >> 22
           // and the weight the G bits below. Record c: {M at position 0, S, 4 (q0_c - pre_c) and
-          // the plane, last position with a second sample}, {S ceil(n / 2), 4 ceil(n / 2)}.
+          // the plane, last position with a second sample}, {S distance, 4 distance}.
           const int n_all = packed & 0xff;
-          const int n = kRuns ? (n_all + 1) >> 1 : n_all;  // positions
+          constexpr bool kTwo = kRuns || kHues;
+          const int n = kTwo ? (n_all + 1) >> 1 : n_all;  // positions
           const uint64_t live = __ballot(n != 0);
           if (live) {
             const int incl = wave_sum_incl(n);
@@ -1393,18 +1396,23 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             // starts are set, and the previous batch's reads are done before these writes)
             if (lane < steps) mask[lane] = 0ull;
             if (n) {
-              const int off = ((packed >> 8) & 0xff) - pre;
+              // the two samples of an even record are columns c and c + n, of an odd one c + m and c (m =
+              // n_all - n): neighbouring pairs, often of the same columns, then mostly meet other banks
+              // (without that the 1M-ray frame's walk took 550 us, 506 so)
+              const int m2 = n_all - n;
+              const int off = ((packed >> 8) & 0xff) - pre + (kTwo && (c & 1) ? m2 : 0);
+              const int delta = (c & 1) ? -m2 : n;  // kTwo: from the first sample's column to the second's
               if constexpr (kRuns) {
                 rec[2 * c] = make_uint4((uint32_t)(fx_m + __mul24(off - T / 2, fx_s)), (uint32_t)fx_s,
-                                        (uint32_t)((off + cq2) * 4), (uint32_t)(pre + n_all - n - 1));
-                *reinterpret_cast<uint2*>(&rec[2 * c + 1]) = make_uint2((uint32_t)__mul24(n, fx_s), (uint32_t)(4 * n));
+                                        (uint32_t)((off + cq2) * 4), (uint32_t)(pre + m2 - 1));
+                *reinterpret_cast<uint2*>(&rec[2 * c + 1]) = make_uint2((uint32_t)__mul24(delta, fx_s), (uint32_t)(4 * delta));
               } else {
                 rec[2 * c] = make_uint4((uint32_t)off, __float_as_uint(m_first), __float_as_uint(slope),
                                         (uint32_t)((kHues ? off + cq2 : off) * 8));
               }
               if constexpr (kRuns) {
               } else if constexpr (kHues) {
-                *reinterpret_cast<uint2*>(&rec[2 * c + 1]) = make_uint2((uint32_t)cq0, (uint32_t)cq1);
+                rec[2 * c + 1] = make_uint4((uint32_t)cq0, (uint32_t)cq1, (uint32_t)(pre + m2 - 1), (uint32_t)delta);
               } else if constexpr (kVS) {
                 rec[2 * c + 1] = make_uint4(__float_as_uint((float)((packed >> 8) & 0xff)), __float_as_uint(s_first),
                                             __float_as_uint(ds), 0u);
@@ -1422,7 +1430,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
                 rec[2 * n_live + 1] = make_uint4(0u, 0u, 0u, 0u);
               } else {
                 rec[2 * n_live] = make_uint4((uint32_t)(-total), 0u, 0u, (uint32_t)(-total * 8));
-                rec[2 * n_live + 1] = make_uint4(0u, 0u, 0u, 0u);
+                rec[2 * n_live + 1] = make_uint4(0u, 0u, kHues ? 0xffffffffu : 0u, 0u);
               }
               if constexpr (kVS) vrec[2 * n_live] = vrec[2 * n_live + 1] = make_uint4(0u, 0u, 0u, 0u);
               if (total & 63) atomicOr(&mask[total >> 6], 1ull << (total & 63));
@@ -1447,7 +1455,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               const uint32_t k = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
               const uint32_t ra = __builtin_amdgcn_readlane(my_rec, sl) + k * 32u;
               R.r0 = lds_read16(ra);
-              if constexpr (kHues || kRuns) {
+              if constexpr (kRuns) {
                 const uint2 q = lds_read8(ra + 16u);
                 R.r1.x = q.x;
                 R.r1.y = q.y;
@@ -1485,6 +1493,22 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
                 return;
               }
               const uint4 r0 = R.r0, r1 = R.r1;
+              if constexpr (kHues) {
+                const int p = lane + (st << 6), col = (int)r0.x + p;
+                auto put = [&](float m, uint32_t b) {
+                  int jl;
+                  asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(jl) : "v"(m));
+                  jl = jl < -kGuard ? -kGuard : (jl > T ? T : jl);
+                  char* const t = reinterpret_cast<char*>(tile) + (((uint32_t)jl << 9) + b);
+                  deposit1<T>(reinterpret_cast<unsigned long long*>(t), m, r1.x, r1.y);
+                };
+                const float m = __builtin_fmaf((float)col, __uint_as_float(r0.z), __uint_as_float(r0.y));
+                const float m2 = __builtin_fmaf((float)(col + (int)r1.w), __uint_as_float(r0.z), __uint_as_float(r0.y));
+                const uint32_t base = ((uint32_t)p << 3) + r0.w;
+                put(m, base);
+                put(p <= (int)r1.z ? m2 : -4.0f, base + (r1.w << 3));
+                return;
+              }
               const int col = (int)r0.x + lane + (st << 6);
               const float m = __builtin_fmaf((float)col, __uint_as_float(r0.z), __uint_as_float(r0.y));
               int jl;
@@ -1493,9 +1517,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               // byte offset 8 (jl T + column) = (jl + st) 512 + 8 off + 8 lane
               const uint32_t eb = ((uint32_t)(jl + st) << 9) + r0.w + lane8;
               unsigned long long* const t = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(tile) + eb);
-              if constexpr (kHues) {
-                deposit1<T>(t, m, r1.x, r1.y);
-              } else if constexpr (kVS) {
+              if constexpr (kVS) {
                 // the per-pair walk's expressions: the same bits
                 const float4 a = __builtin_bit_cast(float4, R.a), d = __builtin_bit_cast(float4, R.d);
                 const float sp = __builtin_fmaf((float)col - __uint_as_float(r1.x), __uint_as_float(r1.z),
@@ -1515,7 +1537,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             StepRec ra{}, rb{};
             read_recs(0, ra);
             // zero adds into guard row -2: the loop is entered with the same LDS operations
-            // in flight as it loops back with (two reads, four adds; two with hues), so that the
+            // in flight as it loops back with (two reads, four adds), so that the
             // compiler's wait counts inside the loop stay exact
             if constexpr (kRuns) {
               uint32_t zero = 0u;
@@ -1531,10 +1553,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               unsigned long long* const g = tile + (-kGuard * T + lane);
               atomicAdd(g, zero);
               atomicAdd(g + T, zero);
-              if constexpr (!kHues) {
-                atomicAdd(g + kStride, zero);
-                atomicAdd(g + T + kStride, zero);
-              }
+              atomicAdd(g + kStride, zero);
+              atomicAdd(g + T + kStride, zero);
             }
             __builtin_amdgcn_sched_barrier(0);
             for (int st = 0;; st += 2) {
@@ -1549,11 +1569,11 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               __builtin_amdgcn_sched_barrier(0);
               if (st + 2 >= steps) break;
             }
-            if (!kRuns)
+            if (!kTwo)
               wave_samples += (unsigned long long)total;
             else if (count_work)
               wave_samples += (unsigned long long)__builtin_amdgcn_readlane(wave_sum_incl(n_all), 63);
-            wave_atomics += (kHues ? 2u : 4u) * (unsigned)steps;
+            wave_atomics += 4u * (unsigned)steps;
           }
           return;
         }
