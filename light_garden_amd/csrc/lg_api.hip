@@ -1073,16 +1073,24 @@ int lg_image_destroy(lg_image* img) {
   return LG_OK;
 }
 
+// Clears (mode 0) or resolves (1) an image.
+static int image_pass(lg_ctx* ctx, lg_image* img, int mode) {
+  begin_call(ctx);
+  const uint64_t n = (uint64_t)img->view.width * img->view.height;
+  {
+    StageScope s(ctx, mode ? "resolve" : "clear", n);
+    LG_HIP(launch_pixels(mode, img->accum.as<float4>(), img->out16.as<ushort4>(), n, ctx->stream));
+  }
+  LG_HIP(hipStreamSynchronize(ctx->stream));
+  end_call(ctx);
+  return LG_OK;
+}
+
 int lg_image_clear(lg_image* img) {
   if (!img) return fail(LG_E_INVALID, "image is NULL");
   lg_ctx* ctx = img->ctx;
   LG_HIP(hipSetDevice(ctx->device));
-  begin_call(ctx);
-  Entry e;
-  e.img = img;
-  int rc = pipeline_run(ctx, {e}, ST_CLEAR);
-  end_call(ctx);
-  return rc;
+  return image_pass(ctx, img, 0);
 }
 
 int lg_image_device_ptrs(lg_image* img, void** accum, void** rgba16f) {
@@ -1129,12 +1137,8 @@ int lg_accumulate(lg_ctx* ctx, const lg_segments* segs, lg_image* img) {
 int lg_resolve(lg_ctx* ctx, lg_image* img) {
   if (!ctx || !img) return fail(LG_E_INVALID, "ctx or image is NULL");
   LG_HIP(hipSetDevice(ctx->device));
-  begin_call(ctx);
-  Entry e;
-  e.img = img;
-  int rc = pipeline_run(ctx, {e}, ST_RESOLVE);
-  end_call(ctx);
-  return rc;
+  if (img->ctx != ctx) return fail(LG_E_INVALID, "resolve: image of another context");
+  return image_pass(ctx, img, 1);
 }
 
 int lg_render(lg_scene* scene, const lg_params* params, lg_segments* segs, lg_image* img) {
@@ -1158,7 +1162,7 @@ int lg_batch_render(lg_ctx* ctx, uint32_t n, lg_scene* const* scenes, const lg_p
     E[i].segs = segs[i];
     E[i].img = images[i];
   }
-  int rc = pipeline_run(ctx, E, ST_CLEAR | ST_TRACE | ST_ACCUM | ST_RESOLVE);
+  int rc = pipeline_run(ctx, E, ST_TRACE | ST_ACCUM | ST_FRESH);
   if (rc) return rc;
   end_call(ctx);
   return LG_OK;

@@ -129,8 +129,8 @@ hipError_t launch_lds_atomic_rate(int n_cu, uint32_t iters, unsigned long long* 
 // once per device (the device must be current); its size in bytes.
 int noalloc_init(int device, hipStream_t st);
 uint64_t noalloc_scratch_bytes();
-hipError_t launch_pixels(int mode, const SceneDesc* descs, const uint64_t* px_pre, int n_scenes, uint64_t n_px,
-                         hipStream_t st);
+// Clears (mode 0) or resolves (1) the n pixels of an image.
+hipError_t launch_pixels(int mode, float4* accum, ushort4* out16, uint64_t n, hipStream_t st);
 
 }  // namespace lg
 
@@ -230,12 +230,9 @@ struct lg_image {
 
 namespace lg {
 
-enum Stage : uint32_t { ST_CLEAR = 1u, ST_TRACE = 2u, ST_ACCUM = 4u, ST_RESOLVE = 8u };
-// The frame clears, accumulates into and resolves every image (lg_render, lg_batch_render,
-// the server): clear and resolve fold into the tile flushes.
-inline bool whole_images(uint32_t stages) {
-  return (stages & (ST_CLEAR | ST_ACCUM | ST_RESOLVE)) == (ST_CLEAR | ST_ACCUM | ST_RESOLVE);
-}
+// ST_FRESH with ST_ACCUM: the frame clears, accumulates into and resolves every image (lg_render,
+// lg_batch_render, the server), clear and resolve as part of the tile flushes.
+enum Stage : uint32_t { ST_TRACE = 1u, ST_ACCUM = 2u, ST_FRESH = 4u };
 
 struct Entry {
   lg_scene* scene = nullptr;

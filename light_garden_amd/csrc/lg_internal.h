@@ -318,7 +318,6 @@ struct SceneDesc {
   LG_G ushort4* out16;
   int32_t tile_base;          // first global tile of this scene
   float color_max;            // bound on |colour channel| of the scene's segments
-  uint64_t px_base;           // first pixel of this scene in the batch's pixel range
   // blend of the image (lg_image_set_blend): per channel (r, g, b, a) 4 bits at 4 * channel,
   // a BlendCode factor in the low 3 bits and bit 3 set for ReverseSubtract; the constant;
   // per channel, the largest |factor| over |colour| <= color_max

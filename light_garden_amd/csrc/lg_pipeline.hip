@@ -42,12 +42,11 @@ struct DevView {
 
 // Byte offsets of a frame's parts in frame_in and stage_in, each a multiple of 128.
 struct FrameLayout {
-  size_t tile_scene, px_pre, item_pre0, counters, ctl, row_count, total;
+  size_t tile_scene, item_pre0, counters, ctl, row_count, total;
   FrameLayout(int n, int n_tiles, int layers) {
     auto up = [](size_t b) { return (b + 127) & ~size_t(127); };  // (the control block's lines)
     tile_scene = up((size_t)n * sizeof(SceneDesc));
-    px_pre = tile_scene + up((size_t)n_tiles * 4);
-    item_pre0 = px_pre + up((size_t)n * 8);
+    item_pre0 = tile_scene + up((size_t)n_tiles * 4);
     counters = item_pre0 + up((size_t)(n + 1) * 4);
     ctl = counters + (size_t)n * kCounterStride;
     row_count = ctl + up(sizeof(BatchCtl));
@@ -57,11 +56,11 @@ struct FrameLayout {
 };
 
 struct Pipeline {
-  // One allocation that a frame uploads with one copy: descs | tile_scene | px_pre | item_pre0 |
+  // One allocation that a frame uploads with one copy: descs | tile_scene | item_pre0 |
   // counters | ctl | row_count (FrameLayout; the layout of stage_in, whose counters, control block
   // and row totals are the frame's zeros). One copy reads counters | ctl back.
   DevBuf frame_in;
-  DevView descs, tile_scene, px_pre, item_pre0, counters, ctl, row_count;
+  DevView descs, tile_scene, item_pre0, counters, ctl, row_count;
   DevBuf item_pre, chunk_pre, cbase, places, row_start, scan_scratch;
   DevBuf pairs, items;
   DevBuf split_tiles, split_fx;  // merge slots of tiles split over several items
@@ -129,10 +128,9 @@ struct Layout {
   bool packed_only = false;          // every accumulated scene keeps two channels per LDS word
   bool hues = false;                 // some scene's deposits are one LDS word (SCENE_HUES)
   bool runs = false;                 // the frame's tiles sum weights of runs (SCENE_RUNS)
-  uint64_t n_counts = 0, n_px = 0;  // n_counts: capacity of the per-frame [chunk][tile][axis] matrix
+  uint64_t n_counts = 0;             // capacity of the per-frame [chunk][tile][axis] matrix
   uint32_t bin_target = 0;           // bin chunks per frame
   std::vector<int> tile_base;
-  std::vector<uint64_t> px_base;
 };
 
 SceneHues scene_hues(const lg_scene* sc) {
@@ -204,15 +202,11 @@ struct Scope {
 
 static int enqueue(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, const Layout& L, uint32_t stages) {
   const int n = L.n;
-  const bool whole = whole_images(stages);
+  const bool whole = stages & ST_FRESH;
   SceneDesc* d_descs = P.descs.as<SceneDesc>();
   BatchCtl* d_ctl = P.ctl.as<BatchCtl>();
   const FrameLayout F(n, L.n_tiles, L.layers);
   LG_HIP(hipMemcpyAsync(P.frame_in.p, P.stage_in.p, F.total, hipMemcpyHostToDevice, st));
-  if ((stages & ST_CLEAR) && !whole) {
-    Scope s(ctx, profile, "clear", L.n_px);
-    LG_HIP(launch_pixels(0, d_descs, P.px_pre.as<uint64_t>(), n, L.n_px, st));
-  }
   if (stages & ST_TRACE) {
     Scope s(ctx, profile, L.fp64 ? "trace_fp64" : "trace", L.max_bounce);
     const int grid = ctx->n_cu * (int)ctx->tune.trace_waves;
@@ -267,10 +261,6 @@ static int enqueue(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, const
                                L.tile, ctx->n_cu, st));
     }
   }
-  if ((stages & ST_RESOLVE) && !whole) {
-    Scope s(ctx, profile, "resolve", L.n_px);
-    LG_HIP(launch_pixels(1, d_descs, P.px_pre.as<uint64_t>(), n, L.n_px, st));
-  }
   LG_HIP(hipMemcpyAsync(P.stage_out.p, P.counters.p, F.out_bytes(), hipMemcpyDeviceToHost, st));
   return LG_OK;
 }
@@ -288,7 +278,6 @@ static int batch_validate(lg_ctx* ctx, hipStream_t st, Batch& B) {
   const uint32_t stages = B.stages;
   const int n = (int)E.size();
   const bool trace = stages & ST_TRACE, accum = stages & ST_ACCUM;
-  const bool pixels = stages & (ST_CLEAR | ST_RESOLVE | ST_ACCUM);
   int rc;
   Layout& L = B.L;
   L.n = n;
@@ -305,7 +294,7 @@ static int batch_validate(lg_ctx* ctx, hipStream_t st, Batch& B) {
       if ((rc = compile_scene(e.scene, st))) return rc;
     }
     if (accum && !e.segs) return fail(LG_E_INVALID, "batch: accumulation needs a segment buffer");
-    if (pixels && !e.img) return fail(LG_E_INVALID, "batch: an image is needed");
+    if (accum && !e.img) return fail(LG_E_INVALID, "batch: an image is needed");
     if (e.img && e.img->ctx != ctx) return fail(LG_E_INVALID, "batch: image of another context");
     for (int j = 0; j < i; j++) {
       if ((e.scene && e.scene == E[j].scene) || (e.segs && e.segs == E[j].segs) || (e.img && e.img == E[j].img))
@@ -365,18 +354,12 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
   }
   // ---- layout ----
   L.tile_base.assign(n, 0);
-  L.px_base.assign(n, 0);
   L.n_tiles = 0;
   L.max_tiles = 1;
   L.n_counts = 0;
-  L.n_px = 0;
   L.tile = (int)ctx->tune.tile;
   for (int i = 0; i < entries; i++) {
     const Entry& e = E[i];
-    if (e.img) {
-      L.px_base[i] = L.n_px;
-      L.n_px += (uint64_t)e.img->view.width * e.img->view.height;
-    }
     if (accum) {
       AccumView v = make_view(e.img->view, L.tile);
       int t = v.tiles_x * v.tiles_y;
@@ -411,7 +394,6 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
     char* fi = P.frame_in.as<char>();
     P.descs.p = fi;
     P.tile_scene.p = fi + F.tile_scene;
-    P.px_pre.p = fi + F.px_pre;
     P.item_pre0.p = fi + F.item_pre0;
     P.counters.p = fi + F.counters;
     P.ctl.p = fi + F.ctl;
@@ -446,7 +428,6 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
   char* in = P.stage_in.as<char>();
   SceneDesc* hd = reinterpret_cast<SceneDesc*>(in);
   uint32_t* h_tile_scene = reinterpret_cast<uint32_t*>(in + F.tile_scene);
-  uint64_t* h_px = reinterpret_cast<uint64_t*>(in + F.px_pre);
   uint32_t* h_pre = reinterpret_cast<uint32_t*>(in + F.item_pre0);
   std::memset(in + F.counters, 0, F.total - F.counters);
   h_pre[0] = 0;
@@ -516,14 +497,10 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
       }
     }
     if (e.img) {
-      if (whole_images(stages)) D.flags |= SCENE_FRESH_IMAGE;
+      if (stages & ST_FRESH) D.flags |= SCENE_FRESH_IMAGE;
       D.view = make_view(e.img->view, L.tile);
       D.accum = gbl(e.img->accum.as<float4>());
       D.out16 = gbl(e.img->out16.as<ushort4>());
-      D.px_base = L.px_base[i];
-      h_px[i] = L.px_base[i];
-    } else {
-      h_px[i] = L.n_px;
     }
     D.color_max = max_abs;
     D.blend_code = e.img ? e.img->blend_code : kBlendDefault;
@@ -551,10 +528,7 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
   }
   if (L.runs) {
     const SceneDesc whole = hd[0];
-    for (int l = 0; l < n; l++) {
-      hd[l] = run_layer(whole, E[0].segs->runs, l, n);
-      h_px[l] = l ? L.n_px : 0;  // (the image's pixels are the first layer's)
-    }
+    for (int l = 0; l < n; l++) hd[l] = run_layer(whole, E[0].segs->runs, l, n);
   }
   if (trace) {
     BatchCtl* c = reinterpret_cast<BatchCtl*>(in + F.ctl);
@@ -564,7 +538,7 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
   // ---- launch (graph replay when the shape is unchanged) ----
   std::vector<uint64_t> shape = {(uint64_t)n, stages, L.fp64, L.max_bounce, (uint64_t)L.cap_recs,
                                  (uint64_t)L.cap_objs, (uint64_t)L.cap_verts, (uint64_t)L.n_tiles,
-                                 (uint64_t)L.max_tiles, L.n_counts, L.n_px, L.bin_target, P.pairs_cap, P.items_cap,
+                                 (uint64_t)L.max_tiles, L.n_counts, L.bin_target, P.pairs_cap, P.items_cap,
                                  P.split_cap, ctx->tune.rays_per_item, ctx->tune.min_piece, ctx->tune.max_piece,
                                  ctx->tune.trace_waves, ctx->tune.bvh_min_objects,
                                  (uint64_t)L.tile, (uint64_t)L.packed_only, (uint64_t)L.hues, (uint64_t)L.runs, L.chunk,

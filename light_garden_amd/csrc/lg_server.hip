@@ -260,7 +260,7 @@ struct lg_server {
     s.start_us = now_us();
     s.busy = true;
     stats.frames++;
-    if (status == LG_OK) status = frame_job_start(s.job, std::move(E), ST_CLEAR | ST_TRACE | ST_ACCUM | ST_RESOLVE);
+    if (status == LG_OK) status = frame_job_start(s.job, std::move(E), ST_TRACE | ST_ACCUM | ST_FRESH);
     if (status != LG_OK) complete(s, status);
     size_t rb = resident_bytes();
     stats.resident_bytes = rb;
