@@ -156,20 +156,19 @@ __device__ __forceinline__ uint64_t scene_segments(const SceneDesc& D) {
   return c < D.seg_cap ? c : D.seg_cap;
 }
 
-// Segments per bin chunk of a scene: the frame's chunk size, and at least kBinSegsPerCounter
-// per counter of the scene's [tile][axis] histogram, which every chunk initialises, adds to the
-// row totals and writes back (short chunks of a large image would spend their time there) --
-// unless that would leave the frame fewer chunks than it has bin workgroups (`spread` segments
-// each). A scene with more chunks than workgroups gets a whole multiple of their number
-// (a count just above it leaves most workgroups idle while the rest take one more chunk).
-// Never more chunks than the frame's chunk size gives, so the count matrix keeps its capacity.
-constexpr uint32_t kBinSegsPerCounter = 2;
+// Segments per bin chunk of a scene: the frame's chunk size, or a bin workgroup's share of the frame's
+// segments (`spread`) where that is more. Every chunk initialises the scene's [tile][axis]
+// histogram and writes it back, which short chunks of a large image would spend their time on, and
+// adds it to the row totals, which many chunks of a small image queue up for (its totals are a few
+// lines, and a line takes some 15 ns per chunk: a scene of a million segments on 64 tiles, cut
+// into 4600 chunks beside 19 others, held the frame's count pass up: 152 us, 60 so; the fill pass 210 and 88). A scene with more
+// chunks than workgroups gets a whole multiple of their number (a count just above it leaves
+// most workgroups idle while the rest take one more chunk). Never more chunks than the frame's
+// chunk size gives, so the count matrix keeps its capacity.
 __device__ __forceinline__ uint32_t scene_chunk(uint32_t chunk, uint32_t groups, uint32_t spread, const SceneDesc& D) {
   const uint64_t n = scene_segments(D);
   const uint64_t g = groups ? groups : 1u;
-  uint64_t m = (uint64_t)kBinSegsPerCounter * 2u * (uint64_t)(D.view.tiles_x * D.view.tiles_y);
-  m = m < spread ? m : spread;
-  uint64_t sc = m > chunk ? m : chunk;
+  uint64_t sc = spread > chunk ? spread : chunk;
   const uint64_t nch = (n + sc - 1) / sc;
   if (nch > g) {
     const uint64_t whole = nch / g * g;
