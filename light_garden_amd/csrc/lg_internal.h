@@ -284,12 +284,13 @@ struct SceneDesc {
   const LG_G void* verts;          // polygon vertices in the culling precision
   const LG_G double* verts64;
   const LG_G DevLight* lights;
-  const LG_G CullBlock* blocks;    // culling by boxes; n_blocks = 0: the pass walks every record
+  const LG_G CullBlock* blocks;    // culling by boxes (every object's; see by_boxes)
   const LG_G float4* block_box;    // the blocks' objects: padded boxes (centre and half sizes),
   const LG_G int32_t* block_rec;   // and first records
   const LG_G int32_t* tree_rec;    // first record of each object that is a Logic tree of more
                                    // than two primitives (the object walk skips these)
   int32_t n_blocks;
+  int32_t by_boxes;                // 0: the culling pass walks every record
   int32_t n_trees;
   int32_t n_recs, n_objs, n_verts, n_lights;
   uint64_t n_primary;

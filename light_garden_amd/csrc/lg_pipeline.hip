@@ -460,7 +460,8 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
       D.blocks = gbl(sc->table<CullBlock>(sc->at.blocks));
       D.block_box = gbl(sc->table<float4>(sc->at.block_box));
       D.block_rec = gbl(sc->table<int32_t>(sc->at.block_rec));
-      D.n_blocks = scene_uses_boxes(ctx, sc) ? sc->n_blocks : 0;
+      D.n_blocks = sc->n_blocks;
+      D.by_boxes = scene_uses_boxes(ctx, sc) ? 1 : 0;
       D.tree_rec = gbl(sc->table<int32_t>(sc->at.tree_rec));
       D.n_trees = sc->n_trees;
       D.n_recs = sc->n_recs;

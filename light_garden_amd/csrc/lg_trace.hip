@@ -1034,19 +1034,21 @@ __device__ __forceinline__ bool canvas_exit(const RayT<T>& r, const double* cv, 
 // ---------------------------------------------------------------------------------------
 __device__ __forceinline__ double tie_tol(double t) { return 1e-5 * (1.0 + t); }
 
-// Full FP64 scan for the rare ray whose FP32 winner was not confirmed; out of line to keep
-// the main path's registers and code small.
+// Full FP64 scan for the rare ray whose FP32 winner was not confirmed, by boxes whatever the scene's
+// size: a wave waits for its slowest lane. (Over every object, with a record's loads waited for one
+// after another, one such ray of a scene of 64 objects took 225 us, most of a launch of a million.)
 __device__ __forceinline__ Nearest<double> rescan_fp64(const RayT<double>& rd, const Rec<double>* recs64,
-                                                    const double* verts64, int n_recs, const TreeList& trees) {
+                                                    const double* verts64, const CullView& blocks,
+                                                    const TreeList& trees) {
   return nearest_hit<double>(rd, recs64, recs64, verts64, trees, [&](Nearest<double>& nb) {
-    walk_objects<double>(rd, recs64, recs64, verts64, walk_records(trees, n_recs), nb);
+    walk_boxes<double>(rd, recs64, recs64, verts64, blocks, nb);
   });
 }
 
 // FP64 answer for a ray whose FP32 culling pass found `nb`.
 __device__ __forceinline__ void refine_fp64(const RayT<double>& rd, const Nearest<float>& nb,
                                             const Rec<double>* recs64, const double* verts64,
-                                            int n_recs, const TreeList& trees, Nearest<double>& h) {
+                                            const CullView& blocks, const TreeList& trees, Nearest<double>& h) {
   const bool tie = nb.top2 >= 0 && (double)nb.t2 <= (double)nb.t + tie_tol(nb.t);
   if (tie) {
     int a = nb.top < nb.top2 ? nb.top : nb.top2;
@@ -1057,7 +1059,7 @@ __device__ __forceinline__ void refine_fp64(const RayT<double>& rd, const Neares
     eval_object<double>(rd, recs64, recs64, verts64, nb.top, h);
   }
   const bool unsure = h.top < 0 || (!tie && nb.top2 >= 0 && h.t > (double)nb.t2 - tie_tol(nb.t2));
-  if (unsure) h = rescan_fp64(rd, recs64, verts64, n_recs, trees);
+  if (unsure) h = rescan_fp64(rd, recs64, verts64, blocks, trees);
 }
 
 __device__ __forceinline__ uint64_t gen_input_count(const SceneDesc& D, uint32_t gen_ix) {
@@ -1215,7 +1217,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
     const double* verts64 = gen(D.verts64);
     const int n_recs = D.n_recs, n_objs = D.n_objs;
     const TreeList trees{gen(D.tree_rec), gen(D.obj_box), D.n_trees};
-    const CullView cull{(const LG_K CullBlock*)D.blocks, (const LG_K float*)D.block_box, s_tops, D.n_blocks};
+    const CullView blocks{(const LG_K CullBlock*)D.blocks, (const LG_K float*)D.block_box, s_tops, D.n_blocks};
+    CullView cull = blocks;
+    if (!D.by_boxes) cull.n = 0;
     if (sid != loaded) {
       if (sizeof(T) == 8) {  // the FP32 pass reads its records with scalar loads instead
         const int4* src = reinterpret_cast<const int4*>(gen(D.recs));
@@ -1226,7 +1230,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
       const int n_walk = n_objs - D.n_trees;  // the objects that the blocks hold
       for (int k = threadIdx.x; k < n_objs; k += BLOCK) {
         s_obj[k] = (uint32_t)gen(D.obj_rec)[k] << 2 | gen(D.obj_flags)[k];
-        if (D.n_blocks && k < n_walk) s_tops[k] = gen(D.block_rec)[k];
+        if (k < n_walk) s_tops[k] = gen(D.block_rec)[k];
       }
       const T* vsrc = reinterpret_cast<const T*>(gen(D.verts));
       for (int k = threadIdx.x; k < 2 * D.n_verts; k += BLOCK) s_verts[k] = vsrc[k];
@@ -1306,7 +1310,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               walk_objects<float>(rf, krec, recs64, s_verts, walk_records(trees, n_recs), nf);
           });
           nearest_init(h);
-          if (nb.top >= 0) refine_fp64(rd, nb, recs64, verts64, n_recs, trees, h);
+          if (nb.top >= 0) refine_fp64(rd, nb, recs64, verts64, blocks, trees, h);
         }
         if (h.rec >= 0) {
           const Rec<double>& R = recs64[h.rec];
