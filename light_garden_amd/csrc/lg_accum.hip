@@ -180,9 +180,22 @@ __device__ __forceinline__ uint32_t scene_chunk(uint32_t chunk, uint32_t groups,
 // Bin layout of one frame, from the segment counts the trace just produced: the chunk size
 // gives about `target` chunks over the whole batch (at least `chunk_min` segments each);
 // chunk_pre[s] = first chunk of scene s, cbase[s] = first entry of scene s's [chunk][tile][axis]
-// matrix (2 x tiles x its chunk count). One block of 1024.
-__global__ __launch_bounds__(1024) void build_chunks_kernel(const SceneDesc* __restrict__ descs, int n_scenes,
-                                                           uint32_t chunk_min, uint32_t target, uint32_t groups,
+// matrix (2 x tiles x its chunk count). Frames of up to kBinScenes scenes have a wave of every
+// workgroup of the count pass make it (bin_kernel): a launch less, which at 5 us was a twentieth
+// of the smallest frames (20000 rays 185 -> 182 us a frame). For more scenes, one block of 1024:
+constexpr int kBinScenes = 64;
+struct BinPlan {
+  uint32_t chunk_min, target, groups;
+};
+// Segments per chunk and per workgroup of a frame of `total` segments.
+__device__ __forceinline__ uint2 frame_chunk(unsigned long long total, const BinPlan& P) {
+  const unsigned long long ch = (total + P.target - 1) / P.target;
+  const unsigned long long sp = P.groups ? (total + P.groups - 1) / P.groups : total;
+  return make_uint2((uint32_t)(ch > P.chunk_min ? (ch < 0x80000000ull ? ch : 0x80000000ull) : P.chunk_min),
+                    (uint32_t)(sp < 0x80000000ull ? sp : 0x80000000ull));
+}
+
+__global__ __launch_bounds__(1024) void build_chunks_kernel(const SceneDesc* __restrict__ descs, int n_scenes, BinPlan P,
                                                            uint32_t* chunk_pre, uint32_t* cbase, BatchCtl* ctl) {
   __shared__ unsigned long long s_tot[16];
   __shared__ uint32_t s_wa[16], s_wb[16];
@@ -197,10 +210,8 @@ __global__ __launch_bounds__(1024) void build_chunks_kernel(const SceneDesc* __r
   __syncthreads();
   unsigned long long total = 0;
   for (int w = 0; w < 16; w++) total += s_tot[w];
-  unsigned long long ch = (total + target - 1) / target;
-  const uint32_t chunk = (uint32_t)(ch > chunk_min ? (ch < 0x80000000ull ? ch : 0x80000000ull) : chunk_min);
-  const unsigned long long sp = groups ? (total + groups - 1) / groups : total;
-  const uint32_t spread = (uint32_t)(sp < 0x80000000ull ? sp : 0x80000000ull);
+  const uint2 fc = frame_chunk(total, P);
+  const uint32_t chunk = fc.x, spread = fc.y, groups = P.groups;
   for (int base = 0; base < n_scenes; base += 1024) {
     const int sid = base + threadIdx.x;
     uint32_t nch = 0, ncnt = 0;
@@ -266,8 +277,7 @@ __global__ __launch_bounds__(1024) void build_chunks_kernel(const SceneDesc* __r
 // scene's; 1.6M segments at 4096x4096 754 -> 630; 20k-ray frame at 1024x1024 45 -> 25).
 template <int PASS>
 __global__ __launch_bounds__(256) void bin_kernel(const SceneDesc* __restrict__ descs, int n_scenes,
-                                                  const uint32_t* __restrict__ chunk_pre,
-                                                  const uint32_t* __restrict__ cbase, BatchCtl* ctl,
+                                                  BinPlan P, uint32_t* chunk_pre, uint32_t* cbase, BatchCtl* ctl,
                                                   uint32_t* places, uint32_t* rows, uint32_t* pairs,
                                                   uint64_t pairs_cap) {
   // rows: PASS 0 the row totals (zeroed before the frame), PASS 1 the rows' starts; both
@@ -280,8 +290,50 @@ __global__ __launch_bounds__(256) void bin_kernel(const SceneDesc* __restrict__ 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   ColumnRec* const rec = s_rec[wave];
   unsigned long long* const mask = s_mask[wave];
-  const uint32_t n_chunks = ctl->n_chunks;
-  const uint32_t chunk = ctl->chunk;
+  // PASS 0 of a frame of few scenes makes the layout; its first workgroup writes it for PASS 1
+  const bool own_layout = PASS == 0 && n_scenes <= kBinScenes;
+  __shared__ uint32_t s_pre[PASS == 0 ? kBinScenes + 1 : 1], s_cbase[PASS == 0 ? kBinScenes : 1], s_chunk_spread[2];
+  if (own_layout) {
+    if (wave == 0) {
+      const SceneDesc& D = descs[lane < n_scenes ? lane : 0];
+      const unsigned long long n_own = lane < n_scenes ? scene_segments(D) : 0ull;
+      unsigned long long total = n_own;
+#pragma unroll
+      for (int d = 32; d > 0; d >>= 1) total += __shfl_xor(total, d, 64);
+      const uint2 fc = frame_chunk(total, P);
+      const uint32_t sc = scene_chunk(fc.x, P.groups, fc.y, D);
+      const uint32_t nch = (uint32_t)((n_own + sc - 1) / sc);
+      const uint32_t ncnt = 2u * nch * (uint32_t)(D.view.tiles_x * D.view.tiles_y);
+      const uint32_t pre = (uint32_t)wave_sum_incl((int)nch) - nch, cb = (uint32_t)wave_sum_incl((int)ncnt) - ncnt;
+      if (lane < n_scenes) {
+        s_pre[lane] = pre;
+        s_cbase[lane] = cb;
+        if (lane == n_scenes - 1) s_pre[n_scenes] = pre + nch;
+        if (blockIdx.x == 0) {
+          chunk_pre[lane] = pre;
+          cbase[lane] = cb;
+          if (lane == n_scenes - 1) {
+            chunk_pre[n_scenes] = pre + nch;
+            ctl->n_chunks = pre + nch;
+          }
+        }
+      }
+      if (lane == 0) {
+        s_chunk_spread[0] = fc.x;
+        s_chunk_spread[1] = fc.y;
+        if (blockIdx.x == 0) {
+          ctl->chunk = fc.x;
+          ctl->spread = fc.y;
+          ctl->bin_groups = P.groups;
+        }
+      }
+    }
+    __syncthreads();
+  }
+  const uint32_t n_chunks = own_layout ? s_pre[n_scenes] : ctl->n_chunks;
+  const uint32_t chunk = own_layout ? s_chunk_spread[0] : ctl->chunk;
+  const uint32_t spread = own_layout ? s_chunk_spread[1] : ctl->spread;
+  const uint32_t groups = own_layout ? P.groups : ctl->bin_groups;
   bool first = true;
   for (;;) {
     if (threadIdx.x == 0) s_chunk = next_work_item(PASS == 0 ? &ctl->chunk_cursor0 : &ctl->chunk_cursor1, n_chunks, first);
@@ -289,12 +341,13 @@ __global__ __launch_bounds__(256) void bin_kernel(const SceneDesc* __restrict__ 
     __syncthreads();
     const uint32_t ci = __builtin_amdgcn_readfirstlane(s_chunk);
     if (ci >= n_chunks) break;
-    const int sid = __builtin_amdgcn_readfirstlane(find_u32(chunk_pre, n_scenes, ci));
+    const int sid = __builtin_amdgcn_readfirstlane(own_layout ? find_u32(s_pre, n_scenes, ci) : find_u32(chunk_pre, n_scenes, ci));
     const SceneDesc& D = descs[sid];
     const AccumView v = D.view;
     const int n_tiles = v.tiles_x * v.tiles_y;
-    const uint32_t local = ci - chunk_pre[sid];
-    uint2* const mat = reinterpret_cast<uint2*>(places + cbase[sid]) + (uint64_t)local * n_tiles;
+    const uint32_t local = ci - (own_layout ? s_pre[sid] : chunk_pre[sid]);
+    uint2* const mat =
+        reinterpret_cast<uint2*>(places + (own_layout ? s_cbase[sid] : cbase[sid])) + (uint64_t)local * n_tiles;
     uint2* const tile_rows = reinterpret_cast<uint2*>(rows) + D.row_base;
     const uint32_t row_stride = D.row_stride;
     uint2* const hist2 = reinterpret_cast<uint2*>(s_hist);
@@ -308,7 +361,7 @@ __global__ __launch_bounds__(256) void bin_kernel(const SceneDesc* __restrict__ 
     }
     __syncthreads();
     const uint64_t n = scene_segments(D);
-    const uint32_t sc = scene_chunk(chunk, ctl->bin_groups, ctl->spread, D);
+    const uint32_t sc = scene_chunk(chunk, groups, spread, D);
     const uint64_t s0 = (uint64_t)local * sc;
     const uint64_t s1 = s0 + sc < n ? s0 + sc : n;
     const int sh = v.tile_shift;
@@ -2008,23 +2061,25 @@ hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t st) 
   return hipGetLastError();
 }
 
-hipError_t launch_build_chunks(const SceneDesc* descs, int n_scenes, uint32_t chunk_min, uint32_t target,
-                               uint32_t groups, uint32_t* chunk_pre, uint32_t* cbase, BatchCtl* ctl, hipStream_t st) {
-  hipLaunchKernelGGL(build_chunks_kernel, dim3(1), dim3(1024), 0, st, descs, n_scenes, chunk_min, target, groups,
-                     chunk_pre, cbase, ctl);
+hipError_t launch_bin_count(const SceneDesc* descs, int n_scenes, uint32_t chunk_min, uint32_t target,
+                            uint32_t* chunk_pre, uint32_t* cbase, BatchCtl* ctl, uint32_t* places, uint32_t* row_count,
+                            int max_tiles, int grid, hipStream_t st) {
+  const BinPlan P{chunk_min, target, (uint32_t)grid};
+  if (n_scenes > kBinScenes) {
+    hipLaunchKernelGGL(build_chunks_kernel, dim3(1), dim3(1024), 0, st, descs, n_scenes, P, chunk_pre, cbase, ctl);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(bin_kernel<0>, dim3(grid), dim3(256), (size_t)max_tiles * 2 * sizeof(uint32_t), st, descs, n_scenes,
+                     P, chunk_pre, cbase, ctl, places, row_count, nullptr, 0);
   return hipGetLastError();
 }
 
-hipError_t launch_bin(int pass, const SceneDesc* descs, int n_scenes, const uint32_t* chunk_pre,
-                      const uint32_t* cbase, BatchCtl* ctl, uint32_t* places, uint32_t* rows, uint32_t* pairs,
-                      uint64_t pairs_cap, int max_tiles, int grid, hipStream_t st) {
-  size_t lds = (size_t)max_tiles * 2 * sizeof(uint32_t);
-  if (pass == 0)
-    hipLaunchKernelGGL(bin_kernel<0>, dim3(grid), dim3(256), lds, st, descs, n_scenes, chunk_pre, cbase, ctl, places,
-                       rows, pairs, pairs_cap);
-  else
-    hipLaunchKernelGGL(bin_kernel<1>, dim3(grid), dim3(256), lds, st, descs, n_scenes, chunk_pre, cbase, ctl, places,
-                       rows, pairs, pairs_cap);
+hipError_t launch_bin_fill(const SceneDesc* descs, int n_scenes, uint32_t* chunk_pre, uint32_t* cbase, BatchCtl* ctl,
+                           uint32_t* places, uint32_t* row_start, uint32_t* pairs, uint64_t pairs_cap, int max_tiles,
+                           int grid, hipStream_t st) {
+  hipLaunchKernelGGL(bin_kernel<1>, dim3(grid), dim3(256), (size_t)max_tiles * 2 * sizeof(uint32_t), st, descs, n_scenes,
+                     BinPlan{}, chunk_pre, cbase, ctl, places, row_start, pairs, pairs_cap);
   return hipGetLastError();
 }
 

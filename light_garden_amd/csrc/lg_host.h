@@ -95,15 +95,17 @@ uint64_t scan_scratch_elems(uint64_t n);
 hipError_t launch_scan_exclusive(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* scratch, hipStream_t st,
                                  unsigned long long* total);
 hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t st);
-hipError_t launch_build_chunks(const SceneDesc* descs, int n_scenes, uint32_t chunk_min, uint32_t target,
-                               uint32_t groups, uint32_t* chunk_pre, uint32_t* cbase, BatchCtl* ctl, hipStream_t st);
 // bin workgroups per compute unit (as many as the LDS allows run at once)
 constexpr uint32_t kBinWaves = 6;
-// rows: pass 0 the row totals (2 per tile, zeroed by the caller), pass 1 the rows' starts; places:
-// the [scene][chunk][tile][axis] matrix
-hipError_t launch_bin(int pass, const SceneDesc* descs, int n_scenes, const uint32_t* chunk_pre,
-                      const uint32_t* cbase, BatchCtl* ctl, uint32_t* places, uint32_t* rows, uint32_t* pairs,
-                      uint64_t pairs_cap, int max_tiles, int grid, hipStream_t st);
+// The bin layout (chunk_pre, cbase: see the kernels) and the count pass: row_count are the row totals
+// (2 per tile, zeroed by the caller), places the [scene][chunk][tile][axis] matrix.
+hipError_t launch_bin_count(const SceneDesc* descs, int n_scenes, uint32_t chunk_min, uint32_t target,
+                            uint32_t* chunk_pre, uint32_t* cbase, BatchCtl* ctl, uint32_t* places, uint32_t* row_count,
+                            int max_tiles, int grid, hipStream_t st);
+// The fill pass, of the same grid: row_start are the rows' starts.
+hipError_t launch_bin_fill(const SceneDesc* descs, int n_scenes, uint32_t* chunk_pre, uint32_t* cbase, BatchCtl* ctl,
+                           uint32_t* places, uint32_t* row_start, uint32_t* pairs, uint64_t pairs_cap, int max_tiles,
+                           int grid, hipStream_t st);
 // row_count and row_start hold 2 * n_tiles_total + 1 entries (row_count's last is zero): per tile
 // its y-major and x-major pairs, and where they start; scan_scratch holds
 // work_items_scratch_elems(n_tiles_total) u32.

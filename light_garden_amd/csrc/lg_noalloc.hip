@@ -168,11 +168,12 @@ int lg_accumulate_noalloc(lg_ctx* ctx, const lg_segments* segs, lg_image* img) {
     LG_HIP(launch_fill_u32(tile_scene, (uint64_t)n_tiles, 0u, st));
     LG_HIP(launch_fill_u32(row_count, 2 * (uint64_t)n_tiles * layers + 1, 0u, st));
     const int bin_grid = ctx->n_cu * (int)kBinWaves;
-    LG_HIP(launch_build_chunks(d_desc, layers, kNaChunkMin, kNaBinTarget, (uint32_t)bin_grid, chunk_pre, cbase, d_ctl, st));
-    LG_HIP(launch_bin(0, d_desc, layers, chunk_pre, cbase, d_ctl, counts, row_count, nullptr, 0, n_tiles, bin_grid, st));
+    LG_HIP(launch_bin_count(d_desc, layers, kNaChunkMin, kNaBinTarget, chunk_pre, cbase, d_ctl, counts, row_count,
+                            n_tiles, bin_grid, st));
     LG_HIP(launch_work_items(d_desc, tile_scene, n_tiles, layers, row_count, row_start, scan, d_ctl, items, (uint32_t)kNaItems,
                              split_tiles, kNaSplit, kNaPairs, min_piece, max_piece, (uint32_t)ctx->n_cu, false, st));
-    LG_HIP(launch_bin(1, d_desc, layers, chunk_pre, cbase, d_ctl, counts, row_start, pairs, kNaPairs, n_tiles, bin_grid, st));
+    LG_HIP(launch_bin_fill(d_desc, layers, chunk_pre, cbase, d_ctl, counts, row_start, pairs, kNaPairs, n_tiles,
+                           bin_grid, st));
     LG_HIP(launch_tile_accum(d_desc, pairs, items, row_start, split_fx, d_ctl, tile, packed,
                              hues ? 1024 : (int)ctx->tune.tile_block, runs, false, ctx->n_cu, st));
     LG_HIP(launch_tile_merge(d_desc, tile_scene, row_start, split_tiles, d_ctl, split_fx, kNaSplit, tile, ctx->n_cu,

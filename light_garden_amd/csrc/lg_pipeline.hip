@@ -229,10 +229,8 @@ static int enqueue(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, const
     const int grid = ctx->n_cu * (int)kBinWaves;
     {
       Scope s(ctx, profile, "bin_count", 0);
-      LG_HIP(launch_build_chunks(d_descs, n, kChunkMin, L.bin_target, (uint32_t)grid, P.chunk_pre.as<uint32_t>(),
-                                 P.cbase.as<uint32_t>(), d_ctl, st));
-      LG_HIP(launch_bin(0, d_descs, n, P.chunk_pre.as<uint32_t>(), P.cbase.as<uint32_t>(), d_ctl,
-                        P.places.as<uint32_t>(), P.row_count.as<uint32_t>(), nullptr, 0, L.max_tiles, grid, st));
+      LG_HIP(launch_bin_count(d_descs, n, kChunkMin, L.bin_target, P.chunk_pre.as<uint32_t>(), P.cbase.as<uint32_t>(),
+                              d_ctl, P.places.as<uint32_t>(), P.row_count.as<uint32_t>(), L.max_tiles, grid, st));
     }
     {
       Scope s(ctx, profile, "bin_scan", 2 * (uint64_t)L.n_tiles);
@@ -244,9 +242,9 @@ static int enqueue(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, const
     }
     {
       Scope s(ctx, profile, "bin_fill", 0);
-      LG_HIP(launch_bin(1, d_descs, n, P.chunk_pre.as<uint32_t>(), P.cbase.as<uint32_t>(), d_ctl,
-                        P.places.as<uint32_t>(), P.row_start.as<uint32_t>(), P.pairs.as<uint32_t>(), P.pairs_cap,
-                        L.max_tiles, grid, st));
+      LG_HIP(launch_bin_fill(d_descs, n, P.chunk_pre.as<uint32_t>(), P.cbase.as<uint32_t>(), d_ctl,
+                             P.places.as<uint32_t>(), P.row_start.as<uint32_t>(), P.pairs.as<uint32_t>(), P.pairs_cap,
+                             L.max_tiles, grid, st));
     }
     {
       Scope s(ctx, profile, "tile_accum", 0);
