@@ -2020,6 +2020,11 @@ hipError_t launch_lds_atomic_rate(int n_cu, uint32_t iters, unsigned long long* 
   return hipGetLastError();
 }
 
+__global__ __launch_bounds__(256) void iota_u64_kernel(uint64_t* p, uint64_t n) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = i;
+}
+
 __global__ void fill_u32_kernel(uint32_t* p, uint64_t n, uint32_t v) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
     p[i] = v;
@@ -2050,6 +2055,11 @@ hipError_t launch_scan_exclusive(const uint32_t* in, uint32_t* out, uint64_t n, 
   e = launch_scan_exclusive(sums, sums, nb, scratch + nb, st, total);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(scan_add_kernel, dim3((unsigned)nb), dim3(kScanThreads), 0, st, out, n, sums);
+  return hipGetLastError();
+}
+
+hipError_t launch_iota_u64(uint64_t* p, uint64_t n, hipStream_t st) {
+  hipLaunchKernelGGL(iota_u64_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p, n);
   return hipGetLastError();
 }
 

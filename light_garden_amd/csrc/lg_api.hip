@@ -9,7 +9,6 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
-#include <numeric>
 #include <string>
 #include <vector>
 
@@ -931,6 +930,37 @@ int lg_segments_count(const lg_segments* s, uint64_t* count) {
   return LG_OK;
 }
 
+// The largest |value| and whether every value is >= 0, over the bits, in 32-bit integer
+// operations that the compiler vectorises (with float comparisons, whose order NaN fixes, one value
+// after another: 100003 segments took 150 us of an upload's 266). NaN, rare, goes value by value.
+struct ColorBounds {
+  uint32_t top = 0, sign = 0;  // the largest magnitude's bits; some value is below zero, or NaN
+  float rest = 0.0f;
+  void add(const float* v, uint64_t n) {
+    uint32_t t = 0, neg = 0;
+    for (uint64_t i = 0; i < n; i++) {
+      uint32_t b;
+      std::memcpy(&b, v + i, sizeof(b));
+      const uint32_t m = b & 0x7fffffffu;
+      t = t > m ? t : m;
+      neg |= b > 0x80000000u ? 1u : 0u;  // (-0 is not below zero)
+    }
+    sign |= neg;
+    if (t <= 0x7f800000u) {
+      top = std::max(top, t);
+      return;
+    }
+    sign = 1u;
+    for (uint64_t i = 0; i < n; i++) rest = std::max(rest, std::fabs(v[i]));
+  }
+  float max_abs() const {
+    float m;
+    std::memcpy(&m, &top, sizeof(m));
+    return std::max(m, rest);
+  }
+  bool nonneg() const { return sign == 0u; }
+};
+
 int lg_segments_upload(lg_segments* s, const float* pos, const float* color0, const float* color1,
                        uint64_t n) {
   if (!s || (n && (!pos || !color0))) return fail(LG_E_INVALID, "segments, pos or color0 is NULL");
@@ -951,25 +981,15 @@ int lg_segments_upload(lg_segments* s, const float* pos, const float* color0, co
     LG_HIP(hipMemcpyAsync(s->pos.p, pos, n * 16, hipMemcpyHostToDevice, st));
     LG_HIP(hipMemcpyAsync(s->col0.p, color0, n * 16, hipMemcpyHostToDevice, st));
     if (!s->one_color) LG_HIP(hipMemcpyAsync(s->col1.p, color1, n * 16, hipMemcpyHostToDevice, st));
-    std::vector<uint64_t> keys(n);
-    std::iota(keys.begin(), keys.end(), 0ull);
-    float mx = 0.0f;
-    bool nonneg = true;
-    for (uint64_t i = 0; i < 4 * n; i++) {
-      mx = std::max(mx, std::fabs(color0[i]));
-      nonneg = nonneg && color0[i] >= 0.0f;
-    }
-    if (color1)
-      for (uint64_t i = 0; i < 4 * n; i++) {
-        mx = std::max(mx, std::fabs(color1[i]));
-        nonneg = nonneg && color1[i] >= 0.0f;
-      }
-    s->max_abs = mx;
-    s->nonneg = nonneg;
+    LG_HIP(launch_iota_u64(s->key.as<uint64_t>(), n, st));
+    ColorBounds b;
+    b.add(color0, 4 * n);
+    if (color1) b.add(color1, 4 * n);
+    s->max_abs = b.max_abs();
+    s->nonneg = b.nonneg();
     if (s->one_color)
       for (uint64_t i = 0; i < n && s->runs.add(i, color0 + 4 * i); i++) {
       }
-    LG_HIP(hipMemcpyAsync(s->key.p, keys.data(), n * 8, hipMemcpyHostToDevice, st));
     LG_HIP(hipStreamSynchronize(st));
   }
   s->count = n;

@@ -95,6 +95,7 @@ uint64_t scan_scratch_elems(uint64_t n);
 hipError_t launch_scan_exclusive(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* scratch, hipStream_t st,
                                  unsigned long long* total);
 hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t st);
+hipError_t launch_iota_u64(uint64_t* p, uint64_t n, hipStream_t st);  // p[i] = i
 // bin workgroups per compute unit (as many as the LDS allows run at once)
 constexpr uint32_t kBinWaves = 6;
 // The bin layout (chunk_pre, cbase: see the kernels) and the count pass: row_count are the row totals
