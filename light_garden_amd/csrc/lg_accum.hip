@@ -1395,28 +1395,27 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
         // ---- walk the pairs that have samples ----
         if constexpr (kStreamKernel && (kVS || !kVC)) {
           // Sample stream: the c-th lane with samples owns positions pre_c .. pre_c + n_c - 1 of
-          // the wave's stream (pre: exclusive prefix sum of n), and position k is column k +
-          // q0_c - pre_c of the tile. Record c = {q0_c - pre_c, m_first, slope, 8 (q0_c - pre_c)},
-          // {q0..q3} (the column offset, and in bytes for the deposit address); with a colour per
-          // vertex {q0_c, s_first, ds} in the second part and the first colour and the difference in
-          // two more (60033 string-mod lines of two colours at 2048x1536: 144 us, pair by pair 292,
-          // where a pair of 40 samples pays the step of 64 and the reads of 14 lanes' registers);
-          // record P (after the last pair) is empty (zero deposits in row 0), so the positions
-          // past the end of the stream need no mask. Stream word i holds a bit per position
+          // the wave's stream (pre: exclusive prefix sum of n), n_c half its samples, rounded up: at
+          // position k a lane takes two, columns k + off_c and k + off_c + delta_c of the tile, so
+          // that the search for the record and its reads serve both (at the last position of an odd
+          // number the second goes to the guard rows). Record c = {off_c, delta_c and the first
+          // position without a second sample, m_first, slope, 8 off_c}, {q0..q3}; with a colour
+          // per vertex {q0_c, s_first, ds} in the second part and the first colour and the difference in
+          // two more; with hues {off_c, m_first, slope, 8 off_c and the plane}, {s, a a, last position
+          // with a second sample, delta_c}. With runs the line is in fixed point, 22 bits below the
+          // pixel: m = M + S position, both modulo 2^32 and exact, its pixel M >> 22 and the weight
+          // the G bits below; {M at position 0, S, 4 off_c and the plane, last position with a
+          // second sample}, {S delta_c, 4 delta_c}. Record P (after the last pair) is empty, so the
+          // positions past the end of the stream need no mask. Stream word i holds a bit per position
           // 64 i .. 64 i + 63 that starts a record; lane l of step s finds its record as the
           // number of starts at positions <= 64 s + l, minus one.
           //
-          // With hues and with runs a lane takes two samples of a pair, columns c and c + ceil(n / 2),
-          // at one position: the record search and its reads, a third of a step's instructions,
-          // serve both (at the last position of an odd n the second goes to the guard rows). Instruction
-          // issue bounds these walks, the LDS the others. Record c with hues: {q0_c - pre_c, m_first,
-          // slope, 8 (q0_c - pre_c) and the plane}, {s, a a, last position with a second sample,
-          // its distance in columns} (1M-ray frame 541 -> 506 us, 20 uneven scenes 604 -> 563). With runs the line is in fixed point, 22 bits below the pixel: m = M + S position, both modulo 2^32 and exact, its pixel M >> 22
-          // and the weight the G bits below. Record c: {M at position 0, S, 4 (q0_c - pre_c) and
-          // the plane, last position with a second sample}, {S distance, 4 distance}.
+          // Hues and runs are bound by instruction issue, channels by the LDS. Tile walk, us, a
+          // sample to a lane and two: 1M-ray frame 541 and 506, 20 uneven scenes 604 and 563, 60033
+          // string-mod lines of two colours at 2048x1536 142 and 134 (pair by pair 292), 100003 lines of a colour
+          // each at 1920x1080 52 and 50.
           const int n_all = packed & 0xff;
-          constexpr bool kTwo = kRuns || kHues;
-          const int n = kTwo ? (n_all + 1) >> 1 : n_all;  // positions
+          const int n = (n_all + 1) >> 1;  // positions
           const uint64_t live = __ballot(n != 0);
           if (live) {
             const int incl = wave_sum_incl(n);
@@ -1440,14 +1439,16 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               // n_all - n): neighbouring pairs, often of the same columns, then mostly meet other banks
               // (without that the 1M-ray frame's walk took 550 us, 506 so)
               const int m2 = n_all - n;
-              const int off = ((packed >> 8) & 0xff) - pre + (kTwo && (c & 1) ? m2 : 0);
-              const int delta = (c & 1) ? -m2 : n;  // kTwo: from the first sample's column to the second's
+              const int off = ((packed >> 8) & 0xff) - pre + ((c & 1) ? m2 : 0);
+              const int delta = (c & 1) ? -m2 : n;  // from the first sample's column to the second's
               if constexpr (kRuns) {
                 rec[2 * c] = make_uint4((uint32_t)(fx_m + __mul24(off - T / 2, fx_s)), (uint32_t)fx_s,
                                         (uint32_t)((off + cq2) * 4), (uint32_t)(pre + m2 - 1));
                 *reinterpret_cast<uint2*>(&rec[2 * c + 1]) = make_uint2((uint32_t)__mul24(delta, fx_s), (uint32_t)(4 * delta));
               } else {
-                rec[2 * c] = make_uint4((uint32_t)off, __float_as_uint(m_first), __float_as_uint(slope),
+                const uint32_t place = kHues ? (uint32_t)off
+                                             : (uint32_t)off << 19 | ((uint32_t)delta & 127u) << 12 | (uint32_t)(pre + m2);
+                rec[2 * c] = make_uint4(place, __float_as_uint(m_first), __float_as_uint(slope),
                                         (uint32_t)((kHues ? off + cq2 : off) * 8));
               }
               if constexpr (kRuns) {
@@ -1469,7 +1470,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
                 rec[2 * n_live] = make_uint4((uint32_t)(-4 << kFxBits), 0u, (uint32_t)(-total * 4), 0xffffffffu);
                 rec[2 * n_live + 1] = make_uint4(0u, 0u, 0u, 0u);
               } else {
-                rec[2 * n_live] = make_uint4((uint32_t)(-total), 0u, 0u, (uint32_t)(-total * 8));
+                rec[2 * n_live] = make_uint4(kHues ? (uint32_t)(-total) : (uint32_t)(-total) << 19, 0u, 0u,
+                                             (uint32_t)(-total * 8));
                 rec[2 * n_live + 1] = make_uint4(0u, 0u, kHues ? 0xffffffffu : 0u, 0u);
               }
               if constexpr (kVS) vrec[2 * n_live] = vrec[2 * n_live + 1] = make_uint4(0u, 0u, 0u, 0u);
@@ -1479,8 +1481,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             // the address of the record before the first of those: a step takes them with three lane
             // reads, and its lane l reads the record that many starts further on. (With the record
             // count kept by scalar instructions, 17 of them a step, the scalar unit took as long as
-            // the vector ALU: 1M-ray frame 590 -> 549 us, 1.6M segments in runs 2920 -> 2700.) Past the last step (the read one step ahead, never used) the words
-            // are empty and every lane names the last record.
+            // the vector ALU: 1M-ray frame 590 -> 549 us, 1.6M segments in runs 2920 -> 2700.) Past the
+            // last step (the read one step ahead, never used) the words are empty and every lane names
+            // the last record.
             const unsigned long long my_word = lane < steps ? mask[lane] : 0ull;
             const uint32_t my_lo = (uint32_t)(my_word >> 1), my_hi = (uint32_t)(my_word >> 33);
             const int my_n = __builtin_popcountll(my_word);
@@ -1510,7 +1513,6 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             };
             // Step st at stream positions p = 64 st + lane: the sample's column is off + p, its
             // entry in plane 0 jl * T + column.
-            const uint32_t lane8 = (uint32_t)lane * 8u;
             uint32_t w_bits = (uint32_t)wG;  // in a lane register: the field extract takes one scalar only
             if constexpr (kRuns) asm volatile("" : "+v"(w_bits));
             auto deposit_step = [&](int st, const StepRec& R) {
@@ -1549,26 +1551,32 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
                 put(p <= (int)r1.z ? m2 : -4.0f, base + (r1.w << 3));
                 return;
               }
-              const int col = (int)r0.x + lane + (st << 6);
+              const int p = lane + (st << 6), col = ((int)r0.x >> 19) + p;
+              const int delta = __builtin_amdgcn_sbfe((int)r0.x, 12, 7);
+              auto put = [&](int column, float m, uint32_t b) {
+                int jl;
+                asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(jl) : "v"(m));
+                jl = jl < -kGuard ? -kGuard : (jl > T ? T : jl);
+                unsigned long long* const t =
+                    reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(tile) + (((uint32_t)jl << 9) + b));
+                if constexpr (kVS) {
+                  // the per-pair walk's expressions: the same bits
+                  const float4 a = __builtin_bit_cast(float4, R.a), d = __builtin_bit_cast(float4, R.d);
+                  const float sp = __builtin_fmaf((float)column - __uint_as_float(r1.x), __uint_as_float(r1.z),
+                                                  __uint_as_float(r1.y));
+                  const float al = __builtin_fmaf(sp, d.w, a.w);
+                  deposit2<T, kStride>(t, m, pack_q(__builtin_fmaf(sp, d.x, a.x), cs0),
+                                       pack_q(__builtin_fmaf(sp, d.y, a.y), cs1),
+                                       pack_q(__builtin_fmaf(sp, d.z, a.z), cs2), pack_q(al * al, cs3));
+                } else {
+                  deposit2<T, kStride>(t, m, r1.x, r1.y, r1.z, r1.w);
+                }
+              };
               const float m = __builtin_fmaf((float)col, __uint_as_float(r0.z), __uint_as_float(r0.y));
-              int jl;
-              asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(jl) : "v"(m));
-              jl = jl < -kGuard ? -kGuard : (jl > T ? T : jl);
-              // byte offset 8 (jl T + column) = (jl + st) 512 + 8 off + 8 lane
-              const uint32_t eb = ((uint32_t)(jl + st) << 9) + r0.w + lane8;
-              unsigned long long* const t = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(tile) + eb);
-              if constexpr (kVS) {
-                // the per-pair walk's expressions: the same bits
-                const float4 a = __builtin_bit_cast(float4, R.a), d = __builtin_bit_cast(float4, R.d);
-                const float sp = __builtin_fmaf((float)col - __uint_as_float(r1.x), __uint_as_float(r1.z),
-                                                __uint_as_float(r1.y));
-                const float al = __builtin_fmaf(sp, d.w, a.w);
-                deposit2<T, kStride>(t, m, pack_q(__builtin_fmaf(sp, d.x, a.x), cs0),
-                                     pack_q(__builtin_fmaf(sp, d.y, a.y), cs1),
-                                     pack_q(__builtin_fmaf(sp, d.z, a.z), cs2), pack_q(al * al, cs3));
-              } else {
-                deposit2<T, kStride>(t, m, r1.x, r1.y, r1.z, r1.w);
-              }
+              const float m2 = __builtin_fmaf((float)(col + delta), __uint_as_float(r0.z), __uint_as_float(r0.y));
+              const uint32_t base = ((uint32_t)p << 3) + r0.w;
+              put(col, m, base);
+              put(col + delta, p < (int)(r0.x & 0xfffu) ? m2 : -4.0f, base + ((uint32_t)delta << 3));
             };
             // One step ahead: the records of step s + 1 are read while step s deposits; two
             // steps per trip with the record registers swapped, so that nothing read ahead is
@@ -1577,7 +1585,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             StepRec ra{}, rb{};
             read_recs(0, ra);
             // zero adds into guard row -2: the loop is entered with the same LDS operations
-            // in flight as it loops back with (two reads, four adds), so that the
+            // in flight as it loops back with (two reads and four adds; more with
+            // channels), so that the
             // compiler's wait counts inside the loop stay exact
             if constexpr (kRuns) {
               uint32_t zero = 0u;
@@ -1591,10 +1600,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               unsigned long long zero = 0ull;
               asm volatile("" : "+v"(zero));  // an add the compiler cannot turn into a load
               unsigned long long* const g = tile + (-kGuard * T + lane);
-              atomicAdd(g, zero);
-              atomicAdd(g + T, zero);
-              atomicAdd(g + kStride, zero);
-              atomicAdd(g + T + kStride, zero);
+              for (int k = 0; k < (kHues ? 1 : 2); k++) {
+                atomicAdd(g, zero);
+                atomicAdd(g + T, zero);
+                atomicAdd(g + kStride, zero);
+                atomicAdd(g + T + kStride, zero);
+              }
             }
             __builtin_amdgcn_sched_barrier(0);
             for (int st = 0;; st += 2) {
@@ -1609,11 +1620,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               __builtin_amdgcn_sched_barrier(0);
               if (st + 2 >= steps) break;
             }
-            if (!kTwo)
-              wave_samples += (unsigned long long)total;
-            else if (count_work)
+            if (count_work)
               wave_samples += (unsigned long long)__builtin_amdgcn_readlane(wave_sum_incl(n_all), 63);
-            wave_atomics += 4u * (unsigned)steps;
+            wave_atomics += (kHues || kRuns ? 4u : 8u) * (unsigned)steps;
           }
           return;
         }
