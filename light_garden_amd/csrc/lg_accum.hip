@@ -897,6 +897,12 @@ __device__ __forceinline__ void hue_add(double (&p)[4], const HueScale& h, unsig
   p[3] = __builtin_fma((double)a, h.ua, p[3]);
 }
 
+// Whether the items of a split tile of two fields to a word add the words as they are to the merge
+// slot: with the whole tile's pairs in the fields' bound no sum carries. (n: its pairs, at most
+// kPackedPiece.) Half the adds and loads: every item of a tile of nearly full pixels took 17 us for
+// them where 256 do so at a time (60033 string-mod lines of two colours, us of walk and merge: 135 + 25 and 117 + 23).
+__device__ __forceinline__ bool slot_words(uint32_t n) { return n < kPackedPiece; }
+
 // Run weights (SCENE_RUNS). A run's segments have one colour, so a tile sums one number per pixel
 // and run: the weights of the deposits, each sample's 2^G cut into round(fr 2^G) at pixel jl + 1
 // and the rest at jl, as 32-bit words (a pair deposits at most once into a pixel, so n pairs keep a
@@ -1831,11 +1837,19 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
       // exact partial sums into the tile's merge slot (integer atomics: order independent)
       unsigned long long* fx = split_fx + (size_t)W.slot * kSlotU64;
       const int n_fields = hues ? 2 * n_hues : 4;
-      for (int k = threadIdx.x; k < T * T; k += BLOCK) {
-        for (int c = 0; c < n_fields; c++) {
-          const unsigned long long val =
-              two_ch ? (tile[(c >> 1) * kStride + k] >> (32 * (c & 1))) & 0xffffffffull : tile[c * kStride + k];
-          if (val) atomicAdd(&fx[c * T * T + k], val);
+      if (two_ch && slot_words(W.tile_pairs)) {
+        for (int k = threadIdx.x; k < T * T; k += BLOCK)
+          for (int f = 0; f < n_fields / 2; f++) {
+            const unsigned long long val = tile[f * kStride + k];
+            if (val) atomicAdd(&fx[f * T * T + k], val);
+          }
+      } else {
+        for (int k = threadIdx.x; k < T * T; k += BLOCK) {
+          for (int c = 0; c < n_fields; c++) {
+            const unsigned long long val =
+                two_ch ? (tile[(c >> 1) * kStride + k] >> (32 * (c & 1))) & 0xffffffffull : tile[c * kStride + k];
+            if (val) atomicAdd(&fx[c * T * T + k], val);
+          }
         }
       }
     } else {
@@ -1948,9 +1962,11 @@ __global__ __launch_bounds__(kMergeBlock) void tile_merge_kernel(const SceneDesc
     const bool whole = (D.flags & SCENE_FRESH_IMAGE) != 0;  // the frame clears and resolves here
     unsigned long long* fx = split_fx + (size_t)sl * kSlotU64;
     unsigned long long a[2 * kMaxHues] = {}, any = 0ull;
+    const bool words = (D.flags & SCENE_PACKED) && !runs && slot_words(np);
+    const int n_slot = words ? n_fields / 2 : n_fields;
 #pragma unroll
     for (int c = 0; c < 2 * kMaxHues; c++)
-      if (c < n_fields) {
+      if (c < n_slot) {
         a[c] = fx[c * TT + k];
         any |= a[c];
       }
@@ -1958,6 +1974,14 @@ __global__ __launch_bounds__(kMergeBlock) void tile_merge_kernel(const SceneDesc
 #pragma unroll
     for (int c = 0; c < 2 * kMaxHues; c++)
       if (a[c]) fx[c * TT + k] = 0ull;
+    if (words) {
+#pragma unroll
+      for (int f = kMaxHues - 1; f >= 0; f--) {
+        const unsigned long long w = a[f];
+        a[2 * f] = w & 0xffffffffull;
+        a[2 * f + 1] = w >> 32;
+      }
+    }
     const int gx = x0 + (k % T), gy = y0 + (k / T);
     if (gx >= v.width || gy >= v.height) continue;
     const size_t px = (size_t)gy * v.width + gx;
