@@ -1473,7 +1473,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             if (lane == 0) {
               if constexpr (kRuns) {
                 // (no colour to be zero: the empty record's line lies above the tile, in guard row -2)
-                rec[2 * n_live] = make_uint4((uint32_t)(-4 << kFxBits), 0u, (uint32_t)(-total * 4), 0xffffffffu);
+                rec[2 * n_live] = make_uint4((uint32_t)(-(4 << kFxBits)), 0u, (uint32_t)(-total * 4), 0xffffffffu);
                 rec[2 * n_live + 1] = make_uint4(0u, 0u, 0u, 0u);
               } else {
                 rec[2 * n_live] = make_uint4(kHues ? (uint32_t)(-total) : (uint32_t)(-total) << 19, 0u, 0u,
@@ -1537,7 +1537,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
                 const uint32_t base = ((uint32_t)p << 2) + R.r0.z;
                 put(M, base);
                 // (no second sample: above the tile, into the guard rows)
-                put(p <= (int)R.r0.w ? M + (int)R.r1.x : -4 << kFxBits, base + R.r1.y);
+                put(p <= (int)R.r0.w ? M + (int)R.r1.x : -(4 << kFxBits), base + R.r1.y);
                 return;
               }
               const uint4 r0 = R.r0, r1 = R.r1;

@@ -505,8 +505,11 @@ static CullLists build_blocks(const std::vector<Box2>& boxes, const std::vector<
     B.box[1] = u.y;
     B.box[2] = u.z;
     B.box[3] = u.w;
-    for (uint64_t m : mask)
-      if (m) B.kind[B.n_kinds++] = m;
+    for (int k = 0; k < 8; k++)
+      if (mask[k]) {
+        B.kinds |= (uint32_t)k << (4 * B.n_kinds);
+        B.kind[B.n_kinds++] = mask[k];
+      }
     while (C.box.size() % kBoxGroup) {  // (no kind has a bit for these)
       C.box.push_back(u);
       C.rec.push_back(-1);

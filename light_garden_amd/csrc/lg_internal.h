@@ -151,7 +151,7 @@ struct alignas(16) CullBlock {
   int32_t first;        // of its boxes and first records
   int32_t n;
   int32_t n_kinds;
-  int32_t pad;
+  uint32_t kinds;       // their RecKinds, 4 bits each
 };
 static_assert(sizeof(CullBlock) == 96, "six float4");
 

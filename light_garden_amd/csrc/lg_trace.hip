@@ -437,11 +437,11 @@ __device__ __forceinline__ bool bezier_nearest(const RayT<T>& r, const T* a, T& 
 // aux_in / aux_out: face or edge index of the chord ends (rect/polygon).
 // ---------------------------------------------------------------------------------------
 template <typename T>
-__device__ __forceinline__ bool chord_any(const RayT<T>& r, const Rec<T>& R,
+__device__ __forceinline__ bool chord_any(const RayT<T>& r, int kind, const Rec<T>& R,
                                           const Rec<double>* R64, const T* verts, T& tin,
                                           T& tout, int& ain, int& aout) {
   ain = aout = 0;
-  switch (R.kind) {
+  switch (kind) {
     case REC_CIRCLE: return chord_circle(r, R.p, R64, tin, tout);
     case REC_RECT: return chord_rect(r, R.p, tin, tout, ain, aout);
     case REC_ELLIPSE: return chord_ellipse(r, R.p, R64, tin, tout);
@@ -591,7 +591,7 @@ __device__ __forceinline__ TreeHit<T> logic_tree(const RayT<T>& r, RS recs, cons
     const int leaf = i + (int)rec_param(recs, i, m);
     T tin, tout;
     int ain, aout;
-    if (!chord_any(r, recs[leaf], recs64 + leaf, verts, tin, tout, ain, aout)) continue;
+    if (!chord_any(r, recs[leaf].kind, recs[leaf], recs64 + leaf, verts, tin, tout, ain, aout)) continue;
     for (int side = 0; side < 2; side++) {
       const T t = side ? tout : tin;
       if (!(t > tmin_v<T>()) || (best_k >= 0 && !(t < best))) continue;
@@ -601,7 +601,7 @@ __device__ __forceinline__ TreeHit<T> logic_tree(const RayT<T>& r, RS recs, cons
         const int kq = i + (int)rec_param(recs, i, q);
         T qin, qout;
         int qa, qb;
-        if (chord_any(r, recs[kq], recs64 + kq, verts, qin, qout, qa, qb) && t > qin && t < qout)
+        if (chord_any(r, recs[kq].kind, recs[kq], recs64 + kq, verts, qin, qout, qa, qb) && t > qin && t < qout)
           leaf_in |= 1u << q;
       }
       // insideness of every subtree at t (bit k - i for the subtree whose root record is k)
@@ -657,9 +657,8 @@ __device__ __forceinline__ TreeHit<T> logic_tree(const RayT<T>& r, RS recs, cons
 // records follow the walk's.
 template <typename T, bool kTrees = true, typename RS>
 __device__ __forceinline__ int eval_object(const RayT<T>& r, RS recs, const Rec<double>* recs64, const T* verts,
-                                           int i, Nearest<T>& nb) {
+                                           int i, int kind, Nearest<T>& nb) {
   const Rec<T>& R = recs[i];
-  const int kind = R.kind;
   if (kind == REC_SEG) {
     T t;
     if (hit_segment(r, R.p, t)) consider(nb, t, i, 0, (T)0, i);
@@ -693,15 +692,15 @@ __device__ __forceinline__ int eval_object(const RayT<T>& r, RS recs, const Rec<
   if (kind == REC_LOGIC) {
     T inA = 0, outA = 0, inB = 0, outB = 0;
     int ainA, aoutA, ainB, aoutB;
-    bool hA = chord_any(r, recs[i + 1], recs64 + i + 1, verts, inA, outA, ainA, aoutA);
-    bool hB = chord_any(r, recs[i + 2], recs64 + i + 2, verts, inB, outB, ainB, aoutB);
+    bool hA = chord_any(r, recs[i + 1].kind, recs[i + 1], recs64 + i + 1, verts, inA, outA, ainA, aoutA);
+    bool hB = chord_any(r, recs[i + 2].kind, recs[i + 2], recs64 + i + 2, verts, inB, outB, ainB, aoutB);
     logic_candidates(nb, R.op, hA, inA, outA, ainA, aoutA, i + 1, hB, inB, outB, ainB, aoutB,
                      i + 2, i);
     return i + 3;
   }
   T tin, tout;
   int ain, aout;
-  if (chord_any(r, R, recs64 + i, verts, tin, tout, ain, aout)) {
+  if (chord_any(r, kind, R, recs64 + i, verts, tin, tout, ain, aout)) {
     if (tin > tmin_v<T>())
       consider(nb, tin, i, ain << 8, (T)0, i);
     else
@@ -716,7 +715,7 @@ __device__ __forceinline__ int eval_object(const RayT<T>& r, RS recs, const Rec<
 template <typename T, typename RS>
 __device__ __forceinline__ void walk_objects(const RayT<T>& r, RS recs, const Rec<double>* recs64, const T* verts,
                                              int n_recs, Nearest<T>& nb) {
-  for (int rec = 0; rec < n_recs;) rec = eval_object<T, false>(r, recs, recs64, verts, rec, nb);
+  for (int rec = 0; rec < n_recs;) rec = eval_object<T, false>(r, recs, recs64, verts, rec, recs[rec].kind, nb);
 }
 
 // a + b + the lane's bit of `carry`.
@@ -742,8 +741,9 @@ struct CullView {
 // walk that evaluates an object for the whole wave when one lane needs it (a hierarchy does that
 // too) runs nearly all of them once rays have split up, since a wave's rays are in no order then.
 // Bound: instruction issue and the serial loads of the rounds. A million rays, 64 objects, 10
-// bounces: trace launches 894 us over every object, 716 us through a hierarchy of boxes, 582 us
-// so; 75011 rays, 23 objects, 8 bounces: 263, 256 and 204 us; FP64, 40009 rays, 12 objects, 6
+// bounces: trace launches 894 us over every object, 716 us through a hierarchy of boxes, 553 us
+// so (573 with the kind read from each lane's record: branches over execution masks); 75011 rays,
+// 23 objects, 8 bounces: 263, 256 and 200 us; FP64, 40009 rays, 12 objects, 6
 // bounces: 110 and 97 us (records in LDS). With 4 objects (20000 rays): 93 us over every object,
 // 99 us so: by boxes from lg_tuning.bvh_min_objects (8) objects.
 //
@@ -790,11 +790,12 @@ __device__ __forceinline__ void walk_boxes(const RayT<T>& r, RS recs, const Rec<
     const uint64_t cand = (uint64_t)half[1] << 32 | half[0];
     for (int k = 0; k < B->n_kinds; k++) {
       uint64_t m = cand & B->kind[k];
+      const int kind = (int)(B->kinds >> (4 * k) & 15u);  // the same for every lane: scalar branches
       while (__ballot(m != 0ull)) {
         if (m) {
           const int top = C.tops[first + __builtin_ctzll(m)];
           m &= m - 1ull;
-          eval_object<T, false>(r, recs, recs64, verts, top, nb);
+          eval_object<T, false>(r, recs, recs64, verts, top, kind, nb);
         }
       }
     }
@@ -1053,10 +1054,10 @@ __device__ __forceinline__ void refine_fp64(const RayT<double>& rd, const Neares
   if (tie) {
     int a = nb.top < nb.top2 ? nb.top : nb.top2;
     int b = nb.top < nb.top2 ? nb.top2 : nb.top;
-    eval_object<double>(rd, recs64, recs64, verts64, a, h);
-    eval_object<double>(rd, recs64, recs64, verts64, b, h);
+    eval_object<double>(rd, recs64, recs64, verts64, a, recs64[a].kind, h);
+    eval_object<double>(rd, recs64, recs64, verts64, b, recs64[b].kind, h);
   } else {
-    eval_object<double>(rd, recs64, recs64, verts64, nb.top, h);
+    eval_object<double>(rd, recs64, recs64, verts64, nb.top, recs64[nb.top].kind, h);
   }
   const bool unsure = h.top < 0 || (!tie && nb.top2 >= 0 && h.t > (double)nb.t2 - tie_tol(nb.t2));
   if (unsure) h = rescan_fp64(rd, recs64, verts64, blocks, trees);
