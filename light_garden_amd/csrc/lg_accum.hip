@@ -186,7 +186,9 @@ __device__ __forceinline__ uint32_t scene_chunk(uint32_t chunk, uint32_t groups,
 constexpr int kBinScenes = 64;
 struct BinPlan {
   uint32_t chunk_min, target, groups;
+  uint32_t lds_counters;  // LDS words of the histogram; the layout's follow
 };
+constexpr uint32_t bin_layout_words(int n_scenes) { return 2u * (uint32_t)n_scenes + 3u; }
 // Segments per chunk and per workgroup of a frame of `total` segments.
 __device__ __forceinline__ uint2 frame_chunk(unsigned long long total, const BinPlan& P) {
   const unsigned long long ch = (total + P.target - 1) / P.target;
@@ -292,7 +294,11 @@ __global__ __launch_bounds__(256) void bin_kernel(const SceneDesc* __restrict__ 
   unsigned long long* const mask = s_mask[wave];
   // PASS 0 of a frame of few scenes makes the layout; its first workgroup writes it for PASS 1
   const bool own_layout = PASS == 0 && n_scenes <= kBinScenes;
-  __shared__ uint32_t s_pre[PASS == 0 ? kBinScenes + 1 : 1], s_cbase[PASS == 0 ? kBinScenes : 1], s_chunk_spread[2];
+  // (after the histogram, sized for the frame's scenes: with room for kBinScenes apart, a 4096x4096
+  // image's workgroups were two to a compute unit instead of three, count pass 225 -> 282 us)
+  uint32_t* const s_pre = s_hist + P.lds_counters;
+  uint32_t* const s_cbase = s_pre + n_scenes + 1;
+  uint32_t* const s_chunk_spread = s_cbase + n_scenes;
   if (own_layout) {
     if (wave == 0) {
       const SceneDesc& D = descs[lane < n_scenes ? lane : 0];
@@ -2107,14 +2113,15 @@ hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t st) 
 hipError_t launch_bin_count(const SceneDesc* descs, int n_scenes, uint32_t chunk_min, uint32_t target,
                             uint32_t* chunk_pre, uint32_t* cbase, BatchCtl* ctl, uint32_t* places, uint32_t* row_count,
                             int max_tiles, int grid, hipStream_t st) {
-  const BinPlan P{chunk_min, target, (uint32_t)grid};
+  const BinPlan P{chunk_min, target, (uint32_t)grid, 2u * (uint32_t)max_tiles};
   if (n_scenes > kBinScenes) {
     hipLaunchKernelGGL(build_chunks_kernel, dim3(1), dim3(1024), 0, st, descs, n_scenes, P, chunk_pre, cbase, ctl);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(bin_kernel<0>, dim3(grid), dim3(256), (size_t)max_tiles * 2 * sizeof(uint32_t), st, descs, n_scenes,
-                     P, chunk_pre, cbase, ctl, places, row_count, nullptr, 0);
+  const size_t words = P.lds_counters + (n_scenes > kBinScenes ? 0u : bin_layout_words(n_scenes));
+  hipLaunchKernelGGL(bin_kernel<0>, dim3(grid), dim3(256), words * sizeof(uint32_t), st, descs, n_scenes, P, chunk_pre,
+                     cbase, ctl, places, row_count, nullptr, 0);
   return hipGetLastError();
 }
 
