@@ -1348,11 +1348,17 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             const int wa = (int)__builtin_ceilf(cl), wb = (int)__builtin_floorf(ch);
             a = a > wa ? a : wa;
             b = b < wb ? b : wb;
+          } else if (!(m_first >= -1.02f && m_first <= (float)T + 0.02f)) {
+            b = -1;  // (the binning lists a row or two more than the deposits touch)
           }
           if (a <= b) {
             if constexpr (!kRuns) ca = a_cur;
             if constexpr (kRuns) {
-              const double mc = m0 + ((maj0 + (T / 2 + 0.5)) - M0) * sl - min0 - 0.5;
+              const double ml = (double)m_first + (double)(T / 2) * (double)slope;
+              double mc = m0 + ((maj0 + (T / 2 + 0.5)) - M0) * sl - min0 - 0.5;
+              // (far outside end points leave FP64 pixels too coarse for two evaluations to agree; the
+              // sample range, and so the rows that the walk may touch, follows m_first)
+              mc = __builtin_fabs(mc - ml) < 0.25 ? mc : ml;
               // (a weight rounds to nearest, with the carry into jl, by half a unit added here)
               fx_m = (int)__builtin_rint(mc * (double)(1 << kFxBits)) + ((1 << (kFxBits - wG)) >> 1);
               fx_s = (int)__builtin_rint(sl * (double)(1 << kFxBits));
@@ -1422,6 +1428,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
           // 64 i .. 64 i + 63 that starts a record; lane l of step s finds its record as the
           // number of starts at positions <= 64 s + l, minus one.
           //
+          // A sample's pixel needs no clamp here: the setup keeps samples at m in [-1.02, T + 0.02] only,
+          // off by some 1e-5, so jl and jl + 1 lie in the tile's rows and the two guard rows on either side.
+          //
           // Hues and runs are bound by instruction issue, channels by the LDS. Tile walk, us, a
           // sample to a lane and two: 1M-ray frame 541 and 506, 20 uneven scenes 604 and 563, 60033
           // string-mod lines of two colours at 2048x1536 142 and 134 (pair by pair 292), 100003 lines of a colour
@@ -1479,7 +1488,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
             if (lane == 0) {
               if constexpr (kRuns) {
                 // (no colour to be zero: the empty record's line lies above the tile, in guard row -2)
-                rec[2 * n_live] = make_uint4((uint32_t)(-(4 << kFxBits)), 0u, (uint32_t)(-total * 4), 0xffffffffu);
+                rec[2 * n_live] = make_uint4((uint32_t)(-(kGuard << kFxBits)), 0u, (uint32_t)(-total * 4), 0xffffffffu);
                 rec[2 * n_live + 1] = make_uint4(0u, 0u, 0u, 0u);
               } else {
                 rec[2 * n_live] = make_uint4(kHues ? (uint32_t)(-total) : (uint32_t)(-total) << 19, 0u, 0u,
@@ -1531,8 +1540,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               if constexpr (kRuns) {
                 const int p = lane + (st << 6);
                 auto put = [&](int M, uint32_t b) {
-                  int jl = M >> kFxBits;
-                  jl = jl < -kGuard ? -kGuard : (jl > T ? T : jl);
+                  const int jl = M >> kFxBits;
                   uint32_t* const t = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(tile32) + (((uint32_t)jl << 8) + b));
                   const uint32_t r = __builtin_amdgcn_ubfe((uint32_t)M, (uint32_t)(kFxBits - wG), w_bits);
                   atomicAdd(t, wq - r);
@@ -1543,7 +1551,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
                 const uint32_t base = ((uint32_t)p << 2) + R.r0.z;
                 put(M, base);
                 // (no second sample: above the tile, into the guard rows)
-                put(p <= (int)R.r0.w ? M + (int)R.r1.x : -(4 << kFxBits), base + R.r1.y);
+                put(p <= (int)R.r0.w ? M + (int)R.r1.x : -(kGuard << kFxBits), base + R.r1.y);
                 return;
               }
               const uint4 r0 = R.r0, r1 = R.r1;
@@ -1552,7 +1560,6 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
                 auto put = [&](float m, uint32_t b) {
                   int jl;
                   asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(jl) : "v"(m));
-                  jl = jl < -kGuard ? -kGuard : (jl > T ? T : jl);
                   char* const t = reinterpret_cast<char*>(tile) + (((uint32_t)jl << 9) + b);
                   deposit1<T>(reinterpret_cast<unsigned long long*>(t), m, r1.x, r1.y);
                 };
@@ -1560,7 +1567,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
                 const float m2 = __builtin_fmaf((float)(col + (int)r1.w), __uint_as_float(r0.z), __uint_as_float(r0.y));
                 const uint32_t base = ((uint32_t)p << 3) + r0.w;
                 put(m, base);
-                put(p <= (int)r1.z ? m2 : -4.0f, base + (r1.w << 3));
+                put(p <= (int)r1.z ? m2 : (float)-kGuard, base + (r1.w << 3));
                 return;
               }
               const int p = lane + (st << 6), col = ((int)r0.x >> 19) + p;
@@ -1568,7 +1575,6 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               auto put = [&](int column, float m, uint32_t b) {
                 int jl;
                 asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(jl) : "v"(m));
-                jl = jl < -kGuard ? -kGuard : (jl > T ? T : jl);
                 unsigned long long* const t =
                     reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(tile) + (((uint32_t)jl << 9) + b));
                 if constexpr (kVS) {
@@ -1588,7 +1594,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
               const float m2 = __builtin_fmaf((float)(col + delta), __uint_as_float(r0.z), __uint_as_float(r0.y));
               const uint32_t base = ((uint32_t)p << 3) + r0.w;
               put(col, m, base);
-              put(col + delta, p < (int)(r0.x & 0xfffu) ? m2 : -4.0f, base + ((uint32_t)delta << 3));
+              put(col + delta, p < (int)(r0.x & 0xfffu) ? m2 : (float)-kGuard, base + ((uint32_t)delta << 3));
             };
             // One step ahead: the records of step s + 1 are read while step s deposits; two
             // steps per trip with the record registers swapped, so that nothing read ahead is

@@ -72,3 +72,24 @@ def test_runs_other_blend_and_large_image(ctx, orc):
     np.testing.assert_array_equal(got, accumulated(ctx, segs, w, h, min_piece=64, max_piece=64))
     ref = orc.accumulate_f64(pos.astype(np.float64), c0, None, abi.LgView(*BOUNDS, w, h), threads=8)
     assert orc.rel_l1(got, ref) < 1e-5
+
+
+@pytest.mark.parametrize("far", [1e6, 1e15, 1e18], ids=lambda f: "%.0e" % f)
+def test_runs_of_far_end_points(ctx, far):
+    """Lines across the image from far outside (FP32 end points, so they come from anywhere in it): the
+    tiles of the walk by weights and of the walk by colours hold the same amount."""
+    rng = np.random.default_rng(int(np.log10(far)))
+    n = 4000
+    a = rng.uniform(0.0, 2 * np.pi, n)
+    c = rng.uniform(-1.0, 1.0, (n, 2))
+    d = np.stack([np.cos(a), np.sin(a)], 1) * far
+    pos = np.concatenate([c - d, c + d], 1).astype(np.float32)
+    col = np.full((n, 4), 0.002, np.float32)
+    runs, colours = lg.Segments(ctx), lg.Segments(ctx)
+    runs.upload(pos, col)
+    col2 = col.copy()
+    col2[::2] *= np.float32(1.0 + 2.0 ** -20)  # (a run each: the walk by colours)
+    colours.upload(pos, col2)
+    x, y = accumulated(ctx, runs, 512, 512), accumulated(ctx, colours, 512, 512)
+    assert np.isfinite(x).all()
+    np.testing.assert_allclose(x.sum(), y.sum(), rtol=1e-3)
