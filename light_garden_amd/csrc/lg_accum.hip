@@ -11,10 +11,11 @@
 //      row totals are scanned, and a second pass writes segment indices into per-tile lists,
 //      y-major pairs first.
 //   2. tiles: a persistent workgroup takes a (tile, pair range) work item, walks each of
-//      its segments' column (x-major) or row (y-major) samples that fall in the tile, one
-//      sample per lane (the samples of 64 pairs laid end to end, 64 per step, in two-channel
-//      frames), and adds the two anti-aliased deposits per sample into a 64-bit
-//      fixed-point LDS tile (4 colour planes, or 2 when two channels share a word).
+//      its segments' column (x-major) or row (y-major) samples that fall in the tile (in
+//      two-channel frames the samples of 64 pairs laid end to end, two to a lane, 128 per
+//      step; else one per lane), and adds the two anti-aliased deposits per sample into a
+//      64-bit fixed-point LDS tile: 4 colour planes, or 2 when two channels share a word, or
+//      up to 3 hues' or 6 one-colour runs' weight planes, whose colours come in afterwards.
 //      Integer sums make the image independent of the order of the deposits. When one item
 //      owns the tile it converts the sums to FP32 and adds them to the accumulator with
 //      coalesced read-add-write; the items of a heavy tile split over several items add
@@ -161,10 +162,10 @@ __device__ __forceinline__ uint64_t scene_segments(const SceneDesc& D) {
 // histogram and writes it back, which short chunks of a large image would spend their time on, and
 // adds it to the row totals, which many chunks of a small image queue up for (its totals are a few
 // lines, and a line takes some 15 ns per chunk: a scene of a million segments on 64 tiles, cut
-// into 4600 chunks beside 19 others, held the frame's count pass up: 152 us, 60 so; the fill pass 210 and 88). A scene with more
-// chunks than workgroups gets a whole multiple of their number (a count just above it leaves
-// most workgroups idle while the rest take one more chunk). Never more chunks than the frame's
-// chunk size gives, so the count matrix keeps its capacity.
+// into 4600 chunks beside 19 others, held the frame's count pass up: 152 us, 60 so; the fill pass
+// 210 and 88). A scene with more chunks than workgroups gets a whole multiple of their number (a
+// count just above it leaves most workgroups idle while the rest take one more chunk). Never more
+// chunks than the frame's chunk size gives, so the count matrix keeps its capacity.
 __device__ __forceinline__ uint32_t scene_chunk(uint32_t chunk, uint32_t groups, uint32_t spread, const SceneDesc& D) {
   const uint64_t n = scene_segments(D);
   const uint64_t g = groups ? groups : 1u;
@@ -475,10 +476,11 @@ __global__ __launch_bounds__(256) void bin_kernel(const SceneDesc* __restrict__ 
 
 // ---- tile work items ------------------------------------------------------------------------
 // Tile g's list is pairs [rows[2 g], rows[2 g + 2]) of the scanned row totals, its x-major part
-// from rows[2 g + 1] on (with layers 2 * layers rows per tile, y-major and x-major of each). A tile is cut into full pieces and at most one remainder; the items are
-// ordered by size class (floor(log2(pairs))), largest class first. With `whole` (the frame clears,
-// accumulates and resolves every image) a tile without pairs gets one empty item (size class 0),
-// which writes its cleared pixels.
+// from rows[2 g + 1] on (with layers 2 * layers rows per tile, y-major and x-major of each). A tile
+// is cut into full pieces and at most one remainder; the items are ordered by size class
+// (floor(log2(pairs))), largest class first. With `whole` (the frame clears, accumulates and
+// resolves every image) a tile without pairs gets one empty item (size class 0), which writes its
+// cleared pixels.
 struct PlanLimits {
   uint64_t pairs_cap;
   uint32_t items_cap, split_cap;
@@ -906,7 +908,8 @@ __device__ __forceinline__ void hue_add(double (&p)[4], const HueScale& h, unsig
 // Whether the items of a split tile of two fields to a word add the words as they are to the merge
 // slot: with the whole tile's pairs in the fields' bound no sum carries. (n: its pairs, at most
 // kPackedPiece.) Half the adds and loads: every item of a tile of nearly full pixels took 17 us for
-// them where 256 do so at a time (60033 string-mod lines of two colours, us of walk and merge: 135 + 25 and 117 + 23).
+// them where 256 do so at a time (60033 string-mod lines of two colours, us of walk and merge:
+// 135 + 25 and 117 + 23).
 __device__ __forceinline__ bool slot_words(uint32_t n) { return n < kPackedPiece; }
 
 // Run weights (SCENE_RUNS). A run's segments have one colour, so a tile sums one number per pixel
@@ -917,7 +920,7 @@ __device__ __forceinline__ bool slot_words(uint32_t n) { return n < kPackedPiece
 // tile's list into items nor the order of anything changes a bit. C <= 2^30, less where the
 // tile's pairs would pass 2^62 in total. A deposit costs two 32-bit adds where two-channel words
 // take four of 64 bits, no colour is loaded, and instruction issue instead of the LDS is what bounds the
-// walk (1.6M segments in 16 runs at 4096x4096, 78M pairs: 3727 us by colours, 2210 us so).
+// walk (1.6M segments in 16 runs at 4096x4096, 78M pairs: 3727 us by colours, 2110 us so).
 // Finer than the colours' fixed point: a weight has the levels the brightest channel had, and
 // no colour is rounded to them.
 constexpr int kFxBits = 22;  // of a sample's place below the pixel; |slope| 2^22 is a 24-bit number
@@ -1052,9 +1055,10 @@ constexpr uint32_t kEarlyClaimPairs = 8192;
 // One persistent workgroup per (tile, pair range) item. Each wave takes 64 pairs at a time:
 // lane l loads pair l's segment and computes its sample range inside the tile plus the
 // tile-relative FP32 parameters of its samples. Two-channel frames at T = 64 with 1024-thread
-// workgroups then walk the batch as one stream of samples, 64 per step (see the stream
-// comment in the walk; not under blends with factors when colours vary along a segment); other shapes walk the pairs one after another with one sample per
-// lane, reading the pair's setup from scalar registers.
+// workgroups then walk the batch as one stream of samples, 128 per step (see the stream
+// comment in the walk; not under blends with factors when colours vary along a segment); other
+// shapes walk the pairs one after another with one sample per lane, reading the pair's setup
+// from scalar registers.
 //
 // An item is walked twice: first its y-major pairs with the tile held transposed (pixel
 // (row y, column x) at x * T + y), then, after an in-place transpose, its x-major pairs with
@@ -1074,12 +1078,13 @@ constexpr uint32_t kEarlyClaimPairs = 8192;
 // (packed_fixed_bits); one with SCENE_HUES a word per hue; other scenes one channel per word in
 // four. RUNS: the kernel of a SCENE_RUNS frame, whose tiles go through the layers' lists one after
 // another with a 32-bit weight plane per run, and keep the pixels' channel sums in registers from
-// layer to layer. PACKED_ONLY: every scene of the frame has SCENE_PACKED, so the LDS tile holds two planes
-// only (half the LDS: two 512-thread workgroups share a compute unit at T = 64), or three in the
+// layer to layer. PACKED_ONLY: every scene of the frame has SCENE_PACKED, so the LDS tile holds two
+// planes only (half the LDS: two 512-thread workgroups share a compute unit at T = 64), or three in the
 // 1024-thread kernel, which serves up to three hues.
 enum WalkMode { WALK_COLOR, WALK_VERTEX_COLORS, WALK_VERTEX_STREAM, WALK_HUES, WALK_RUNS };
 template <int T, bool PACKED_ONLY, int BLOCK, bool RUNS>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void tile_accum_kernel(const SceneDesc* __restrict__ descs,
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
+void tile_accum_kernel(const SceneDesc* __restrict__ descs,
                                                           const uint32_t* __restrict__ pairs,
                                                           const WorkItem* __restrict__ items,
                                                           const uint32_t* __restrict__ row_start,
@@ -1106,8 +1111,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4))) void
   __shared__ uint32_t s_run[RUNS ? kRunPlanes : 1][4];  // the runs' colours (run_color)
   constexpr int kWaves = BLOCK / 64;
   // Sample-stream walk (two-channel frames, T = 64, one workgroup per compute unit; with a colour
-  // per vertex under the default blend, whose channel values need no factors): each wave lays the samples of its 64 pairs end to end and walks that stream
-  // 64 samples per step, every lane busy, instead of one pair per step. Per wave: a record per
+  // per vertex under the default blend, whose channel values need no factors): each wave lays the
+  // samples of its 64 pairs end to end and walks that stream two samples to a lane, 128 per step,
+  // every lane busy, instead of one pair per step. Per wave: a record per
   // pair with samples plus an empty one (two uint4 each) and a start bit per stream position.
   __shared__ HueScale s_hue[kHueKernel ? kMaxHues : 1];
   constexpr int kRecs = 66, kMaskWords = 64;
