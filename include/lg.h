@@ -313,7 +313,7 @@ int lg_accumulate(lg_ctx* ctx, const lg_segments* segs, lg_image* img);
 /* lg_accumulate without device allocation. No counterpart in the reference: it is for callers
  * that cannot allocate device memory (serving loops with a fixed footprint, harnesses that
  * forbid hipMalloc). The same kernels and the same result bits as lg_accumulate, with their
- * scratch in one static device array of about 63 MB (60.3 MiB) per device (kept until the
+ * scratch in one static device array of about 64 MB (60.6 MiB) per device (kept until the
  * process ends): an image of at most 4096 x 4096 pixels (2048 x 2048 with 32-pixel tiles), at
  * most 8,388,608 segment-tile pairs and at most 128 tiles split over several work items per
  * call. Beyond a limit it returns LG_E_CAPACITY and deposits nothing. Calls on one device share
@@ -381,7 +381,7 @@ int lg_batch_render(lg_ctx* ctx, uint32_t n, lg_scene* const* scenes, const lg_p
  * these are the knobs of the persistent GPU work lists, read by the autotuner. Apart from
  * `tile` none of them changes results: images are the same bits for every setting. */
 typedef struct lg_tuning {
-  uint32_t rays_per_item;  /* rays per trace work item, at most, [64, 2^20]; default 256 */
+  uint32_t rays_per_item;  /* rays per trace work item, at most, [64, 2^20]; default 1024 */
   uint32_t min_piece;      /* smallest tile work item in segment-tile pairs, >= 64; default 2048 */
   uint32_t max_piece;      /* largest tile work item, >= min_piece; default 32768; work items
                               hold at most 32768 pairs whatever the setting (the fixed point

@@ -152,7 +152,7 @@ struct lg_ctx {
   // 101, 60k lines with vertex colours 319 / 316 / 362); a cap of 8192 splits tiles for nothing
   // where the share is larger (8192 / 32768: 1M-ray frame 720 / 622, 1.6M segments at 4096x4096
   // 4350 / 3730, 20 uneven scenes 736 / 678).
-  lg_tuning tune{256u, 2048u, 32768u, 4u, 8u, 64u, 2u, 1024u};
+  lg_tuning tune{1024u, 2048u, 32768u, 4u, 8u, 64u, 2u, 1024u};
   std::vector<lg::StageRec> pending;  // events of the current call
   std::vector<hipEvent_t> event_pool;
   std::vector<lg_stage_time> last_times;

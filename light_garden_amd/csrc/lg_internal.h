@@ -356,16 +356,21 @@ constexpr int kMaxGen = kPathBits;
 // after another, 12 ns each over the whole chip, so the words that persistent workgroups count on
 // have lines of their own: a workgroup waits for its claim, and behind other words' adds it waits
 // for those too.
-// Rays of a trace item when a launch has `total`: at most the tuning's (`rpi`), fewer, down to 64,
-// when there would be fewer items than the grid has workgroups. A workgroup waits for its
-// slowest wave at every append, and a launch for its slowest workgroup, so few rays are done sooner by
-// workgroups of one wave. (us of trace launches, items of 256 rays and so: 20000 rays, 4
-// objects 94 and 86; 12000 rays, 3 objects 97 and 79; 75011 rays, 23 objects 213 and 214. Sharing
-// the rays of an item out over its four waves gave no more: every further wave fetches the
-// kernel's code through its own compute unit's cache.)
-__host__ __device__ inline uint32_t trace_item_rays(uint64_t total, uint32_t rpi, uint32_t groups) {
-  const uint64_t waves = (total + 64ull * groups - 1) / (64ull * groups);  // per item
-  const uint64_t m = waves > 1 ? 64 * waves : 64;
+// Rays of a trace item when a launch of n_scenes has `total`: a workgroup's share of them, at
+// least 64 and at most the tuning's (`rpi`). A workgroup waits for its slowest wave at every
+// append, and a launch for its slowest workgroup, so few rays are done sooner by workgroups of one
+// wave. (us of trace launches, items of 256 rays and so: 20000 rays, 4 objects 94 and 86; 12000
+// rays, 3 objects 97 and 79; 75011 rays, 23 objects 213 and 214. Sharing the rays of an item out
+// over its four waves gave no more: every further wave fetches the kernel's code through its own
+// compute unit's cache.) Between two items lies a chain of trips to memory (the cursor, the item's
+// scene, its tables), so many rays are done sooner in one item to a workgroup than in several (1M
+// rays, 64 objects: items of 256 576 us, 512 484, 1024 469), unless they are of several scenes,
+// where whole shares leave the workgroups of the cheap ones idle: those get two items, of at least 512
+// rays (800k rays in 20 scenes: items of 256 714 us, 512 621, whole shares of 832 680).
+__host__ __device__ inline uint32_t trace_item_rays(uint64_t total, uint32_t rpi, uint32_t groups, int n_scenes) {
+  const uint64_t waves = (total + 64ull * groups - 1) / (64ull * groups);  // per share
+  uint64_t m = waves > 1 ? 64 * waves : 64;
+  if (n_scenes > 1 && m > 512) m = m > 1024 ? (waves + 1) / 2 * 64 : 512;
   return m < rpi ? (uint32_t)m : rpi;
 }
 

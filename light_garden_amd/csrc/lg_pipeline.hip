@@ -432,7 +432,8 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
   uint64_t rays = 0;
   for (const Entry& e : E)
     if (trace && e.params.max_bounce) rays += e.scene->n_primary;
-  const uint32_t rpi = trace_item_rays(rays, ctx->tune.rays_per_item, (uint32_t)ctx->n_cu * ctx->tune.trace_waves);
+  const uint32_t rpi =
+      trace_item_rays(rays, ctx->tune.rays_per_item, (uint32_t)ctx->n_cu * ctx->tune.trace_waves, L.n);
   for (int i = 0; i < entries; i++) {
     const Entry& e = E[i];
     SceneDesc& D = hd[i];

@@ -3,9 +3,10 @@
 // Replaces Tracer::trace_all / Tracer::trace (src/light_garden/tracer.rs:276-330,
 // 360-493) and the collision2d ray/shape arithmetic it calls. The reference walks each
 // primary ray's bounce tree breadth-first on a rayon worker; here one kernel launch is one
-// generation of ALL rays: each lane owns one live ray, tests it against every scene record
-// held in LDS (records are uniform across the wave, so the object loop never diverges),
-// shades the nearest hit, and appends its segment and surviving children with one global
+// to three generations of ALL rays: each lane owns one live ray and culls the scene's objects
+// by their boxes, read as wave-uniform scalars, to a bit mask; the candidates are then tested
+// lane by lane (scenes of few objects test every record, wave-uniformly). A lane shades its
+// nearest hit, and appends its segment and surviving children with one global
 // atomic per workgroup (wave64 ballot + mbcnt prefix, then a cross-wave LDS prefix).
 // Children that the cutoff (tracer.rs:378-384) would skip are never queued, which is the
 // same as queueing and skipping them.
@@ -1111,7 +1112,7 @@ __device__ __forceinline__ void build_items_block(const SceneDesc* __restrict__ 
     if (c) atomicAdd(&s_rays, (unsigned long long)c);
   }
   __syncthreads();
-  const uint32_t rpi = trace_item_rays(s_rays, max_rpi, gridDim.x);
+  const uint32_t rpi = trace_item_rays(s_rays, max_rpi, gridDim.x, n_scenes);
   for (int base = 0; base < n_scenes; base += BLOCK) {
     const int sid = base + threadIdx.x;
     const uint32_t n_it = (uint32_t)((scene_rays(sid) + rpi - 1) / rpi);
