@@ -364,9 +364,10 @@ constexpr int kMaxGen = kPathBits;
 // over its four waves gave no more: every further wave fetches the kernel's code through its own
 // compute unit's cache.) Between two items lies a chain of trips to memory (the cursor, the item's
 // scene, its tables), so many rays are done sooner in one item to a workgroup than in several (1M
-// rays, 64 objects: items of 256 576 us, 512 484, 1024 469), unless they are of several scenes,
-// where whole shares leave the workgroups of the cheap ones idle: those get two items, of at least 512
-// rays (800k rays in 20 scenes: items of 256 714 us, 512 621, whole shares of 832 680).
+// rays, 64 objects: items of 256 576 us, 512 484, 1024 469), unless they are of several scenes:
+// their shares are halves, as the launch has twice the workgroups (trace_groups), and halved
+// again down to 512 rays where they are larger, since the items' costs differ (1.4M rays in 20
+// scenes, items of 256 714 us, 512 621, whole shares 748, so 527).
 __host__ __device__ inline uint32_t trace_item_rays(uint64_t total, uint32_t rpi, uint32_t groups, int n_scenes) {
   const uint64_t waves = (total + 64ull * groups - 1) / (64ull * groups);  // per share
   uint64_t m = waves > 1 ? 64 * waves : 64;

@@ -26,9 +26,9 @@ def frame(scenes, **tuning):
     return [(np.sort(s.download()[3]), i.accum().copy()) for s, i in zip(segs, imgs)]
 
 
-# a share of 512 rays a workgroup and just above (two scenes: items of 512), of 1024 and just
-# above (items of half a share), for 1024 workgroups of 4 to each of 256 compute units
-@pytest.mark.parametrize("total", [512 * 1024, 512 * 1024 + 1, 1024 * 1024, 1024 * 1024 + 1, 1600 * 1024 + 77])
+# 2048 workgroups (eight to each of 256 compute units, two scenes): a share of 256 rays and just
+# above, of 512 and just above (items of 512), just above 1024 (items of half a share)
+@pytest.mark.parametrize("total", [256 * 2048, 256 * 2048 + 1, 512 * 2048, 512 * 2048 + 1, 1024 * 2048 + 77])
 def test_frame_items_equal_small_items(total):
     few = 30007
     scenes = [configs.large_single(num_rays=total - few, seed=2, width=256),
