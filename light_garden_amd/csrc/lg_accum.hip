@@ -605,12 +605,19 @@ __global__ __launch_bounds__(1024) void plan_items_kernel(const SceneDesc* __res
     if (k.items > k.full) atomicAdd(&s_cls[k.cls_rem], 1u);
   }
   __syncthreads();
-  if (threadIdx.x < 32) {  // first slot of each size class, largest class first
-    uint32_t base = 0;
-    for (int c = 31; c > (int)threadIdx.x; c--) base += s_cls[c];
-    s_cur[threadIdx.x] = base;
+  // First slot of each size class, largest class first. (A lane that added up the larger classes by
+  // itself read the LDS 31 times in a row: 1.3 us of every frame's 11 to 8 us of this kernel.)
+  if (threadIdx.x < 32) {
+    const uint32_t n_own = s_cls[threadIdx.x];
+    uint32_t upto = n_own;  // of this class and the larger ones
+#pragma unroll
+    for (int d = 1; d < 32; d <<= 1) {
+      const uint32_t y = __shfl_down(upto, d, 32);
+      if ((int)threadIdx.x + d < 32) upto += y;
+    }
+    s_cur[threadIdx.x] = upto - n_own;
     if (threadIdx.x == 0) {
-      const uint32_t n_items = base + s_cls[0];
+      const uint32_t n_items = upto;
       row_start[2 * n_tiles * nl] = (uint32_t)total;
       ctl->total_pairs = total;
       ctl->n_work = n_items < L.items_cap ? n_items : L.items_cap;
