@@ -668,10 +668,23 @@ int compile_scene(lg_scene* sc, hipStream_t st) {
   return LG_OK;
 }
 
+void seg_forget(lg_segments* s) {
+  s->count = 0;
+  s->n_rays = 0;
+  s->has_pos64 = false;
+  s->one_color = true;
+  s->max_abs = 0.0f;
+  s->nonneg = true;
+  s->hues = SceneHues{};
+  s->runs = SegRuns{};
+}
+
 int seg_ensure(lg_segments* s, uint64_t cap, bool need64) {
   int rc;
   if (cap > kMaxSegments) return fail(LG_E_OOM, "segments: at most 2^31 - 1 in one buffer");
   if (cap > s->cap || !s->pos.p) {
+    seg_forget(s);
+    s->cap = 0;  // (of the smallest of the buffers, should one of them fail)
     if ((rc = s->pos.ensure(cap * sizeof(float4)))) return rc;
     if ((rc = s->col0.ensure(cap * sizeof(float4)))) return rc;
     if ((rc = s->key.ensure(cap * sizeof(uint64_t)))) return rc;
@@ -972,31 +985,29 @@ int lg_segments_upload(lg_segments* s, const float* pos, const float* color0, co
   hipStream_t st = s->ctx->stream;
   int rc = seg_ensure(s, std::max<uint64_t>(n, 1), false);
   if (rc) return rc;
-  s->max_abs = 0.0f;
-  s->nonneg = true;
-  s->hues = SceneHues{};
-  s->runs = SegRuns{};
-  s->n_rays = 0;
+  seg_forget(s);
   // a color1 equal to color0 bit for bit is no per-vertex colour: the accumulation then takes
   // the one-colour walk, which deposits the same bits
-  s->one_color = !color1 || !n || std::memcmp(color0, color1, n * 16) == 0;
+  const bool one_color = !color1 || !n || std::memcmp(color0, color1, n * 16) == 0;
+  ColorBounds b;
+  SegRuns runs;
   if (n) {
     LG_HIP(hipMemcpyAsync(s->pos.p, pos, n * 16, hipMemcpyHostToDevice, st));
     LG_HIP(hipMemcpyAsync(s->col0.p, color0, n * 16, hipMemcpyHostToDevice, st));
-    if (!s->one_color) LG_HIP(hipMemcpyAsync(s->col1.p, color1, n * 16, hipMemcpyHostToDevice, st));
+    if (!one_color) LG_HIP(hipMemcpyAsync(s->col1.p, color1, n * 16, hipMemcpyHostToDevice, st));
     LG_HIP(launch_iota_u64(s->key.as<uint64_t>(), n, st));
-    ColorBounds b;
     b.add(color0, 4 * n);
     if (color1) b.add(color1, 4 * n);
-    s->max_abs = b.max_abs();
-    s->nonneg = b.nonneg();
-    if (s->one_color)
-      for (uint64_t i = 0; i < n && s->runs.add(i, color0 + 4 * i); i++) {
+    if (one_color)
+      for (uint64_t i = 0; i < n && runs.add(i, color0 + 4 * i); i++) {
       }
     LG_HIP(hipStreamSynchronize(st));
   }
   s->count = n;
-  s->has_pos64 = false;
+  s->one_color = one_color;
+  s->max_abs = b.max_abs();
+  s->nonneg = b.nonneg();
+  s->runs = runs;
   return LG_OK;
 }
 

@@ -245,6 +245,10 @@ struct Entry {
 };
 
 int compile_scene(lg_scene* sc, hipStream_t st);
+// Whatever is going to overwrite a buffer's segments (or move them: seg_ensure) forgets them first and
+// publishes the new ones when they are complete, so that a call that fails in between leaves an empty
+// buffer and not the old counts over other contents.
+void seg_forget(lg_segments* s);
 int seg_ensure(lg_segments* s, uint64_t cap, bool need64);
 AccumView make_view(const lg_view& v, int tile);
 int check_params(const lg_params* p);

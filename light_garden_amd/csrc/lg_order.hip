@@ -53,24 +53,32 @@ struct alignas(16) Record64 {
   float4 col;
 };
 
-// count[ray] = segments of the ray; place[i] = how many of them were counted before segment i.
+// count[ray] = segments of the ray; place[i] = how many of them were counted before segment i. A
+// buffer whose keys name a ray that it does not have goes to the host too: *by_host ends the
+// kernels that follow before they index by a ray.
 __global__ __launch_bounds__(kOrderBlock) void order_count_kernel(const uint64_t* __restrict__ key, uint32_t n,
-                                                                  uint32_t* count, uint32_t* __restrict__ place,
-                                                                  uint32_t* too_long) {
+                                                                  uint32_t n_rays, uint32_t* count,
+                                                                  uint32_t* __restrict__ place, uint32_t* by_host) {
   const uint32_t i = blockIdx.x * kOrderBlock + threadIdx.x;
   if (i >= n) return;
-  const uint32_t a = atomicAdd(&count[key[i] >> kPathBits], 1u);
+  const uint64_t ray = key[i] >> kPathBits;
+  if (ray >= n_rays) {
+    *by_host = 1u;
+    return;
+  }
+  const uint32_t a = atomicAdd(&count[ray], 1u);
   place[i] = a;
-  if (a == kMaxRankedPerRay) *too_long = 1u;
+  if (a == kMaxRankedPerRay) *by_host = 1u;
 }
 
 // The paths grouped by ray, in arrival order.
 __global__ __launch_bounds__(kOrderBlock) void order_group_kernel(const uint64_t* __restrict__ key, uint32_t n,
                                                                   const uint32_t* __restrict__ start,
                                                                   const uint32_t* __restrict__ place,
-                                                                  uint32_t* __restrict__ path) {
+                                                                  uint32_t* __restrict__ path,
+                                                                  const uint32_t* __restrict__ by_host) {
   const uint32_t i = blockIdx.x * kOrderBlock + threadIdx.x;
-  if (i >= n) return;
+  if (i >= n || *by_host) return;
   const uint64_t k = key[i];
   path[start[k >> kPathBits] + place[i]] = (uint32_t)(k & ((1ull << kPathBits) - 1ull));
 }
@@ -83,9 +91,9 @@ __global__ __launch_bounds__(kOrderBlock) void order_write_kernel(const uint64_t
                                                                   const float4* __restrict__ pos,
                                                                   const double* __restrict__ pos64,
                                                                   const float4* __restrict__ col, R* __restrict__ out,
-                                                                  const uint32_t* __restrict__ too_long) {
+                                                                  const uint32_t* __restrict__ by_host) {
   const uint32_t i = blockIdx.x * kOrderBlock + threadIdx.x;
-  if (i >= n || *too_long) return;
+  if (i >= n || *by_host) return;
   const uint64_t k = key[i];
   const uint32_t mine = (uint32_t)(k & ((1ull << kPathBits) - 1ull));
   const uint32_t b = start[k >> kPathBits], e = start[(k >> kPathBits) + 1];
@@ -173,7 +181,7 @@ static int order_on_device(lg_segments* s, OrderScratch& S, double* xy, float* r
   const uint64_t stage_records = std::min(n, kChunkRecords);
   int rc;
   *done = false;
-  // count: a word per ray, the end, and the too-long flag
+  // count: a word per ray, the end, and the flag of a buffer for the host
   if ((rc = S.count.ensure((n_rays + 2) * 4)) || (rc = S.start.ensure((n_rays + 1) * 4)) ||
       (rc = S.scan.ensure(scan_scratch_elems(n_rays + 1) * 4)) || (rc = S.place.ensure(n * 4)) ||
       (rc = S.path.ensure(n * 4)) || (rc = S.records.ensure(n * sizeof(R))) ||
@@ -182,22 +190,22 @@ static int order_on_device(lg_segments* s, OrderScratch& S, double* xy, float* r
   if (n > kChunkRecords && (rc = S.stage[1].ensure(stage_records * sizeof(R)))) return rc;
   for (hipEvent_t& e : S.landed)
     if (!e) LG_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  uint32_t* const too_long = S.count.as<uint32_t>() + n_rays + 1;
+  uint32_t* const by_host = S.count.as<uint32_t>() + n_rays + 1;
   const uint64_t* key = s->key.as<const uint64_t>();
   R* const records = S.records.as<R>();
   const dim3 grid((unsigned)((n + kOrderBlock - 1) / kOrderBlock)), block(kOrderBlock);
   LG_HIP(launch_fill_u32(S.count.as<uint32_t>(), n_rays + 2, 0u, st));
-  hipLaunchKernelGGL(order_count_kernel, grid, block, 0, st, key, (uint32_t)n, S.count.as<uint32_t>(),
-                     S.place.as<uint32_t>(), too_long);
+  hipLaunchKernelGGL(order_count_kernel, grid, block, 0, st, key, (uint32_t)n, (uint32_t)n_rays,
+                     S.count.as<uint32_t>(), S.place.as<uint32_t>(), by_host);
   LG_HIP(hipGetLastError());
   LG_HIP(launch_scan_exclusive(S.count.as<const uint32_t>(), S.start.as<uint32_t>(), n_rays + 1,
                                S.scan.as<uint32_t>(), st, nullptr));
   hipLaunchKernelGGL(order_group_kernel, grid, block, 0, st, key, (uint32_t)n, S.start.as<const uint32_t>(),
-                     S.place.as<const uint32_t>(), S.path.as<uint32_t>());
+                     S.place.as<const uint32_t>(), S.path.as<uint32_t>(), by_host);
   LG_HIP(hipGetLastError());
   hipLaunchKernelGGL(order_write_kernel<R>, grid, block, 0, st, key, (uint32_t)n, S.start.as<const uint32_t>(),
                      S.path.as<const uint32_t>(), s->pos.as<const float4>(), s->pos64.as<const double>(),
-                     s->col0.as<const float4>(), records, too_long);
+                     s->col0.as<const float4>(), records, by_host);
   LG_HIP(hipGetLastError());
   auto copy = [&](uint64_t chunk) -> int {
     const uint64_t b = chunk * kChunkRecords, m = std::min(kChunkRecords, n - b);
@@ -205,7 +213,7 @@ static int order_on_device(lg_segments* s, OrderScratch& S, double* xy, float* r
     LG_HIP(hipEventRecord(S.landed[chunk & 1], st));
     return LG_OK;
   };
-  LG_HIP(hipMemcpyAsync(S.flag.p, too_long, 4, hipMemcpyDeviceToHost, st));
+  LG_HIP(hipMemcpyAsync(S.flag.p, by_host, 4, hipMemcpyDeviceToHost, st));
   if ((rc = copy(0))) return rc;
   for (uint64_t c = 0; c * kChunkRecords < n; c++) {
     if ((c + 1) * kChunkRecords < n && (rc = copy(c + 1))) return rc;

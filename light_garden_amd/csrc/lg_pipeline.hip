@@ -327,21 +327,12 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
   L.layers = L.runs ? run_layers(E[0].segs->runs) : 1;
   const int entries = (int)E.size();
   const int n = L.n = L.runs ? L.layers : entries;
-  // ---- capacities ----
+  // ---- limits (what they refuse has changed no buffer) ----
   L.max_bounce = 0;
   L.cap_recs = L.cap_objs = L.cap_verts = 1;
   for (const Entry& e : E) {
     if (trace) {
-      lg_scene* sc = e.scene;
-      uint64_t qn = std::max<uint64_t>(sc->q_cap, std::min<uint64_t>(2 * sc->n_primary, 0xffffffffull));
-      qn = std::max<uint64_t>(qn, 1);
-      if ((rc = sc->q0.ensure(qn * sizeof(QRay<double>)))) return rc;
-      if ((rc = sc->q1.ensure(qn * sizeof(QRay<double>)))) return rc;
-      sc->q_cap = qn;
-      uint64_t need = std::max<uint64_t>(sc->seg_hint + sc->seg_hint / 8,
-                                         sc->n_primary * std::min<uint32_t>(e.params.max_bounce, 4u) + 1024);
-      need = std::max<uint64_t>(need, e.segs->cap);
-      if ((rc = seg_ensure(e.segs, need, L.fp64))) return rc;
+      const lg_scene* sc = e.scene;
       L.max_bounce = std::max(L.max_bounce, e.params.max_bounce);
       L.cap_recs = std::max(L.cap_recs, sc->n_recs);
       L.cap_objs = std::max(L.cap_objs, sc->n_objs);
@@ -389,6 +380,22 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
   // n_s * bin_target / total + 1 of them and the batch fewer than bin_target + n
   if (accum) L.n_counts = 2 * (uint64_t)L.max_tiles * (L.bin_target + (uint64_t)n);
   if (L.n_counts > 0xffffffffull) return fail(LG_E_UNSUPPORTED, "batch too large for one frame");
+  // ---- queues and segments ----
+  for (const Entry& e : E) {
+    if (trace) {
+      lg_scene* sc = e.scene;
+      uint64_t qn = std::max<uint64_t>(sc->q_cap, std::min<uint64_t>(2 * sc->n_primary, 0xffffffffull));
+      qn = std::max<uint64_t>(qn, 1);
+      if ((rc = sc->q0.ensure(qn * sizeof(QRay<double>)))) return rc;
+      if ((rc = sc->q1.ensure(qn * sizeof(QRay<double>)))) return rc;
+      sc->q_cap = qn;
+      uint64_t need = std::max<uint64_t>(sc->seg_hint + sc->seg_hint / 8,
+                                         sc->n_primary * std::min<uint32_t>(e.params.max_bounce, 4u) + 1024);
+      need = std::max<uint64_t>(need, e.segs->cap);
+      if ((rc = seg_ensure(e.segs, need, L.fp64))) return rc;
+      seg_forget(e.segs);
+    }
+  }
   // ---- scratch ----
   // pieces hold at least min_piece pairs, so a frame without pair overflow has fewer than
   // n_tiles + pairs_cap / min_piece items
@@ -654,9 +661,7 @@ static int batch_finish(lg_ctx* ctx, Pipeline& P, bool profile, Batch& B, bool* 
       e.segs->has_pos64 = L.fp64;
       e.segs->max_abs = e.scene->light_max;
       e.segs->nonneg = e.scene->light_nonneg;
-      e.segs->one_color = true;
       e.segs->hues = scene_hues(e.scene);
-      e.segs->runs = SegRuns{};
       e.segs->n_rays = e.scene->n_primary;
       e.scene->seg_hint = std::max(e.scene->seg_hint, segs);
     }

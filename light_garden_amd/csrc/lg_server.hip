@@ -67,15 +67,14 @@ int copy_segments(lg_segments* dst, const lg_segments* src) {
   int rc;
   if (dst->ctx != src->ctx) return fail(LG_E_INVALID, "request: segments of another context");
   if ((rc = seg_ensure(dst, std::max<uint64_t>(src->count, 1), false))) return rc;
+  seg_forget(dst);
   const size_t n = src->count;
   if (n) {
     LG_HIP(hipMemcpy(dst->pos.p, src->pos.p, n * sizeof(float4), hipMemcpyDeviceToDevice));
     LG_HIP(hipMemcpy(dst->col0.p, src->col0.p, n * sizeof(float4), hipMemcpyDeviceToDevice));
     LG_HIP(hipMemcpy(dst->key.p, src->key.p, n * sizeof(uint64_t), hipMemcpyDeviceToDevice));
   }
-  dst->one_color = true;  // a traced segment has one colour for both ends (col0)
-  dst->count = n;
-  dst->has_pos64 = false;
+  dst->count = n;  // (one_color: a traced segment has one colour for both ends, col0)
   dst->max_abs = src->max_abs;
   dst->nonneg = src->nonneg;
   dst->hues = src->hues;

@@ -564,6 +564,7 @@ int lg_string_mod_draw(lg_ctx* ctx, uint32_t n, const lg_string_mod* mods, lg_se
   }
   if (total >= (1ull << 32)) return fail(LG_E_INVALID, "string mod: 2^32 or more segments in one call");
   if ((rc = lg::seg_ensure(out, std::max<uint64_t>(total, 1), false))) return rc;
+  lg::seg_forget(out);
   uint32_t max_bits = 0;
   if (total) {
     // The curves' points are made once per curve; the StringMods that have one take them from its
@@ -635,9 +636,7 @@ int lg_string_mod_draw(lg_ctx* ctx, uint32_t n, const lg_string_mod* mods, lg_se
   out->count = total;
   out->max_abs = max_abs;
   out->nonneg = nonneg;
-  out->hues = lg::SceneHues{};
-  out->runs = in_runs ? runs : lg::SegRuns{};
-  out->n_rays = 0;
+  if (in_runs) out->runs = runs;
   // without modulo colours both ends of every segment take their StringMod's colour
   // (get_color, string_mod.rs:124-150): col1 is then neither written nor read
   out->one_color = mrc.empty();
