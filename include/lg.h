@@ -388,8 +388,9 @@ typedef struct lg_tuning {
                               of two channels per LDS word is sized for that) */
   uint32_t trace_waves;    /* trace workgroups per compute unit, [1, 16]; default 4 */
   uint32_t bvh_min_objects; /* scenes with at least this many objects cull by their objects'
-                               bounding boxes, others test every object; 0xffffffff: never;
-                               default 8 */
+                               bounding boxes, others test every object (as FP32 traces
+                               do of scenes with an object or a light beyond 64 units from
+                               the origin); 0xffffffff: never; default 8 */
   uint32_t tile;           /* screen tile edge of the accumulation, 32 or 64 pixels; default 64.
                               Unlike the other knobs it moves sample positions by FP32
                               rounding and the two-channel fixed point's scale with the tile's

@@ -386,11 +386,14 @@ static uint32_t spread_bits(uint32_t v) {  // 16 bits -> even bit positions
   return v;
 }
 
-// Object boxes padded by 1e-5 (1 + |coordinates|), far more than the FP32 culling pass's
-// error and than the rounding of an FP64 inside test: a point outside an object's padded box
-// is neither hit by a culled ray nor contained.
+// Object boxes padded by 1e-5 (1 + |coordinates|) + 2e-6 reach, far more than the FP32 culling
+// pass's error and than the rounding of an FP64 inside test: a point outside an object's padded box
+// is neither hit by a culled ray nor contained. *reach: the largest |coordinate| that a ray
+// starts from, at a light or on an object; both the box test and the FP32 hits are off by some
+// 2^-21 of the ray's origin (5e-7), whatever the object's own coordinates.
 static std::vector<Box2> object_boxes(const std::vector<Rec<double>>& recs, const std::vector<double>& verts,
-                                      const std::vector<int32_t>& obj_rec) {
+                                      const std::vector<int32_t>& obj_rec, const std::vector<lg_light>& lights,
+                                      double* reach) {
   const int n = (int)obj_rec.size();
   std::vector<Box2> boxes(n);
   for (int o = 0; o < n; o++) {
@@ -402,15 +405,27 @@ static std::vector<Box2> object_boxes(const std::vector<Rec<double>>& recs, cons
     } else {
       b = rec_box(recs[top], verts);
     }
-    const double mag = std::max(std::max(std::fabs(b.lo[0]), std::fabs(b.lo[1])),
-                                std::max(std::fabs(b.hi[0]), std::fabs(b.hi[1])));
-    const double pad = 1e-5 * (1.0 + mag);
+    boxes[o] = b;
+  }
+  auto magnitude = [](const Box2& b) {
+    return std::max(std::max(std::fabs(b.lo[0]), std::fabs(b.lo[1])), std::max(std::fabs(b.hi[0]), std::fabs(b.hi[1])));
+  };
+  double r = 0.0;
+  for (const Box2& b : boxes) r = std::max(r, magnitude(b));
+  for (const lg_light& l : lights) {
+    Box2 b = empty_box();
+    b.add(l.position[0], l.position[1]);
+    if (l.kind == LG_LIGHT_DIRECTIONAL) b.add(l.direction[0], l.direction[1]);
+    if (std::isfinite(magnitude(b))) r = std::max(r, magnitude(b));  // (others are refused later)
+  }
+  for (Box2& b : boxes) {
+    const double pad = 1e-5 * (1.0 + magnitude(b)) + 2e-6 * r;
     b.lo[0] -= pad;
     b.lo[1] -= pad;
     b.hi[0] += pad;
     b.hi[1] += pad;
-    boxes[o] = b;
   }
+  *reach = r;
   return boxes;
 }
 
@@ -579,7 +594,8 @@ int compile_scene(lg_scene* sc, hipStream_t st) {
   at.tree_rec = pack.add(tree_rec);
   at.verts32 = pack.add(verts32);
   at.verts64 = pack.add(verts);
-  const std::vector<Box2> boxes = object_boxes(recs, verts, obj_rec);
+  double reach = 0.0;
+  const std::vector<Box2> boxes = object_boxes(recs, verts, obj_rec, sc->lights, &reach);
   std::vector<float4> box32(boxes.size());
   for (size_t o = 0; o < boxes.size(); o++) box32[o] = box_f32(boxes[o]);
   at.obj_box = pack.add(box32);
@@ -647,6 +663,7 @@ int compile_scene(lg_scene* sc, hipStream_t st) {
   sc->at = at;
   sc->n_trees = (int)tree_rec.size();
   sc->n_blocks = (int)cull.blocks.size();
+  sc->reach = reach;
   std::memcpy(sc->medium_map, medium_map, sizeof(medium_map));
   sc->n_primary = base;
   float lmax = 0.0f;

@@ -196,6 +196,7 @@ struct lg_scene {
     return reinterpret_cast<const U*>(tables.as<char>() + off);
   }
   int n_blocks = 0;
+  double reach = 0.0;         // largest |coordinate| that a ray starts from
   float medium_map[4] = {};
   int n_trees = 0;
   lg::DevBuf q0, q1;          // ray queues (QRay<double>)

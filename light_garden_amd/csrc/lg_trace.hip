@@ -749,8 +749,9 @@ struct CullView {
 // 99 us so: by boxes from lg_tuning.bvh_min_objects (8) objects.
 //
 // Every object that can hit within the window is a candidate (boxes are padded beyond the FP32
-// error of the test), so the winner, and any runner-up that the FP64 refinement looks at (within
-// 1e-5 (1 + t)), are those of the full walk: `consider` does not depend on the order.
+// error of the test and of the hits, for the scene's farthest ray origins: object_boxes), so the
+// winner, and any runner-up that the FP64 refinement looks at (within 1e-5 (1 + t)), are those of
+// the full walk: `consider` does not depend on the order.
 template <typename T, typename RS>
 __device__ __forceinline__ void walk_boxes(const RayT<T>& r, RS recs, const Rec<double>* recs64, const T* verts,
                                            const CullView& C, Nearest<T>& nb) {
