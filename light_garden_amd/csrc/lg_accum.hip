@@ -926,26 +926,36 @@ __device__ __forceinline__ void hue_add(double (&p)[4], const HueScale& h, unsig
 __device__ __forceinline__ bool slot_words(uint32_t n) { return n < kPackedPiece; }
 
 // Run weights (SCENE_RUNS). A run's segments have one colour, so a tile sums one number per pixel
-// and run: the weights of the deposits, each sample's 2^G cut into round(fr 2^G) at pixel jl + 1
-// and the rest at jl, as 32-bit words (a pair deposits at most once into a pixel, so n pairs keep a
-// word below n 2^G <= 2^32 - 1). The colours come in when a layer's sums are converted: channel c of
-// run f adds weight times C = round(value 2^K_c), exact 64-bit products, so neither the split of a
+// and run: the weights of the deposits, each sample's Q cut into round(fr Q) at pixel jl + 1 and the
+// rest at jl, as 32-bit words (a pair deposits at most once into a pixel, so n pairs keep a word
+// below n Q <= 2^32 - 1). The colours come in when a layer's sums are converted: channel c of run f
+// adds weight times C = round(value 2^K_c), exact 64-bit products, so neither the split of a
 // tile's list into items nor the order of anything changes a bit. C <= 2^30, less where the
 // tile's pairs would pass 2^62 in total. A deposit costs two 32-bit adds where two-channel words
 // take four of 64 bits, no colour is loaded, and instruction issue instead of the LDS is what bounds the
-// walk (1.6M segments in 16 runs at 4096x4096, 78M pairs: 3727 us by colours, 2110 us so).
-// Finer than the colours' fixed point: a weight has the levels the brightest channel had, and
-// no colour is rounded to them.
+// walk (1.6M segments in 16 runs at 4096x4096, 78M pairs: 3727 us by colours, 2168 us so). Q has all
+// the levels that the word has room for, no fewer than the brightest channel by colours, and no
+// colour is rounded to them. (Q a power of two, a field of the place's bits cut out: 2122 us, but
+// up to half the levels of a channel. Error of 16 x 20000 lines against FP64, rel L1: 7.6e-7 by
+// colours, 2.1e-7 with powers of two, 1.6e-7 so.)
 constexpr int kFxBits = 22;  // of a sample's place below the pixel; |slope| 2^22 is a 24-bit number
-__device__ __forceinline__ int weight_bits(uint32_t n) {
-  const int G = 31 - __clz((int)(0xFFFFFFFFu / (n > 1u ? n : 1u)));
-  return G < kFxBits ? G : kFxBits;
+__device__ __forceinline__ uint32_t run_weight(uint32_t n) {
+  const uint32_t Q = 0xFFFFFFFFu / (n > 1u ? n : 1u);
+  return Q < (1u << kFxBits) ? Q : 1u << kFxBits;
+}
+// round(fr Q), to nearest even, of the place M: with the fraction as the mantissa of 1 + fr / 2 and
+// the integer 2 Q as the bits of a denormal float (2 Q <= 2^23, which the bits hold as well), the
+// FMA's one rounding is to a multiple of 2^-149 (see mul_frac).
+__device__ __forceinline__ uint32_t cut_weight(int M, uint32_t Q) {
+  const uint32_t one_half_fr = ((uint32_t)M & ((1u << kFxBits) - 1u)) | 0x3f800000u;
+  const float q2 = __builtin_bit_cast(float, 2u * Q);
+  return __builtin_bit_cast(uint32_t, __builtin_fmaf(__builtin_bit_cast(float, one_half_fr), q2, -q2));
 }
 // K of channel c in a tile of n pairs.
 __device__ __forceinline__ int run_color_bits(const SceneDesc& D, int c, uint32_t n) {
   const double bound = (double)D.color_max * (double)D.factor_max[c];
   if (!(bound > 0.0) || !(bound < 1e300)) return 0;
-  const uint32_t over = n / kPackedPiece;  // n 2^G <= 2^32 (over + 1)
+  const uint32_t over = n / kPackedPiece;  // n Q <= 2^32 (over + 1)
   return 30 - (over ? 32 - __clz((int)over) : 0) - 1 - floor_log2_ratio(bound, 1.0);
 }
 __device__ __forceinline__ uint32_t run_color(float v, int K) {
@@ -1196,8 +1206,7 @@ void tile_accum_kernel(const SceneDesc* __restrict__ descs,
     const uint32_t n_layers = RUNS ? D.row_stride : 1u;
     const uint32_t* const tile_rows = row_start + 2u * n_layers * W.tile;
     int K[4] = {0, 0, 0, 0};
-    const int wG = RUNS ? weight_bits(W.tile_pairs) : 0;
-    const uint32_t wq = 1u << wG;  // a sample's weight
+    const uint32_t wq = RUNS ? run_weight(W.tile_pairs) : 0u;  // a sample's weight
     unsigned long long acc[RUNS ? T * T / BLOCK : 1][4] = {};
     if constexpr (RUNS) {
       const uint32_t nt = tile_rows[2u * n_layers] - tile_rows[0];
@@ -1378,8 +1387,7 @@ void tile_accum_kernel(const SceneDesc* __restrict__ descs,
               // (far outside end points leave FP64 pixels too coarse for two evaluations to agree; the
               // sample range, and so the rows that the walk may touch, follows m_first)
               mc = __builtin_fabs(mc - ml) < 0.25 ? mc : ml;
-              // (a weight rounds to nearest, with the carry into jl, by half a unit added here)
-              fx_m = (int)__builtin_rint(mc * (double)(1 << kFxBits)) + ((1 << (kFxBits - wG)) >> 1);
+              fx_m = (int)__builtin_rint(mc * (double)(1 << kFxBits));
               fx_s = (int)__builtin_rint(sl * (double)(1 << kFxBits));
               const uint32_t s = e_cur & kPairIndex;
               cq2 = ((s >= run1) + (s >= run2) + (s >= run3) + (s >= run4) + (s >= run5)) * kStride;  // its plane
@@ -1440,8 +1448,8 @@ void tile_accum_kernel(const SceneDesc* __restrict__ descs,
           // per vertex {q0_c, s_first, ds} in the second part and the first colour and the difference in
           // two more; with hues {off_c, m_first, slope, 8 off_c and the plane}, {s, a a, last position
           // with a second sample, delta_c}. With runs the line is in fixed point, 22 bits below the
-          // pixel: m = M + S position, both modulo 2^32 and exact, its pixel M >> 22 and the weight
-          // the G bits below; {M at position 0, S, 4 off_c and the plane, last position with a
+          // pixel: m = M + S position, both modulo 2^32 and exact, its pixel M >> 22 and the fraction
+          // of its weight the bits below; {M at position 0, S, 4 off_c and the plane, last position with a
           // second sample}, {S delta_c, 4 delta_c}. Record P (after the last pair) is empty, so the
           // positions past the end of the stream need no mask. Stream word i holds a bit per position
           // 64 i .. 64 i + 63 that starts a record; lane l of step s finds its record as the
@@ -1553,15 +1561,13 @@ void tile_accum_kernel(const SceneDesc* __restrict__ descs,
             };
             // Step st at stream positions p = 64 st + lane: the sample's column is off + p, its
             // entry in plane 0 jl * T + column.
-            uint32_t w_bits = (uint32_t)wG;  // in a lane register: the field extract takes one scalar only
-            if constexpr (kRuns) asm volatile("" : "+v"(w_bits));
             auto deposit_step = [&](int st, const StepRec& R) {
               if constexpr (kRuns) {
                 const int p = lane + (st << 6);
                 auto put = [&](int M, uint32_t b) {
                   const int jl = M >> kFxBits;
                   uint32_t* const t = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(tile32) + (((uint32_t)jl << 8) + b));
-                  const uint32_t r = __builtin_amdgcn_ubfe((uint32_t)M, (uint32_t)(kFxBits - wG), w_bits);
+                  const uint32_t r = cut_weight(M, wq);
                   atomicAdd(t, wq - r);
                   atomicAdd(t + T, r);
                 };
@@ -1844,7 +1850,7 @@ void tile_accum_kernel(const SceneDesc* __restrict__ descs,
       unsigned long long* fx = split_fx + (size_t)W.slot * kSlotU64;
       double un[4];
 #pragma unroll
-      for (int c = 0; c < 4; c++) un[c] = __builtin_ldexp(1.0, -(wG + K[c]));
+      for (int c = 0; c < 4; c++) un[c] = __builtin_ldexp(1.0 / (double)wq, -K[c]);
 #pragma unroll
       for (int i = 0; i < T * T / BLOCK; i++) {
         const int k = i * BLOCK + (int)threadIdx.x;
@@ -1985,9 +1991,9 @@ __global__ __launch_bounds__(kMergeBlock) void tile_merge_kernel(const SceneDesc
     if (!hues) {
 #pragma unroll
       for (int c = 0; c < 4; c++)
-        un[c] = __builtin_ldexp(1.0, runs ? -(weight_bits(np) + run_color_bits(D, c, nt))
-                                     : (D.flags & SCENE_PACKED) ? -packed_fixed_bits(D, c, np)
-                                                                : -(scene_fixed_bits(D, c) + kWBits));
+        un[c] = runs ? __builtin_ldexp(1.0 / (double)run_weight(np), -run_color_bits(D, c, nt))
+                     : __builtin_ldexp(1.0, (D.flags & SCENE_PACKED) ? -packed_fixed_bits(D, c, np)
+                                                                     : -(scene_fixed_bits(D, c) + kWBits));
     }
     const int n_fields = hues ? 2 * D.n_hues : 4;
     const bool whole = (D.flags & SCENE_FRESH_IMAGE) != 0;  // the frame clears and resolves here
