@@ -14,6 +14,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <memory>
 #include <numeric>
 #include <thread>
 #include <vector>
@@ -23,8 +24,9 @@
 namespace lg {
 
 // Segments of one ray that are ranked by comparing (the work is the sum of their squares); a
-// buffer with a longer ray is ordered on the host.
-constexpr uint32_t kMaxRankedPerRay = 2048;
+// buffer with a longer ray is ordered on the host. (Ordered vertices, ms, by the device and by the host:
+// 655k segments, the longest ray 16381: 7.3 and 14.2; 2.6M, 65491: 40 and 73; 1.0M, 261625: 46 and 29.)
+constexpr uint32_t kMaxRankedPerRay = 65536;
 constexpr int kOrderBlock = 256;
 // Records per copy to the host, and from how many on its threads share them.
 constexpr uint64_t kChunkRecords = 1u << 17;
@@ -98,6 +100,7 @@ __global__ __launch_bounds__(kOrderBlock) void order_write_kernel(const uint64_t
   const uint32_t mine = (uint32_t)(k & ((1ull << kPathBits) - 1ull));
   const uint32_t b = start[k >> kPathBits], e = start[(k >> kPathBits) + 1];
   uint32_t rank = 0;
+#pragma unroll 8
   for (uint32_t j = b; j < e; j++) rank += path[j] < mine ? 1u : 0u;
   R r;
   if constexpr (sizeof(R) == sizeof(Record64)) {
@@ -126,50 +129,76 @@ static void expand(const R* rec, uint64_t n, double* xy, float* rgba) {
   }
 }
 
-// expand, shared by a few threads from kShareRecords on (the host writes 64 bytes per record into
-// fresh pages: one thread keeps up with neither the link nor the memory).
-template <typename R>
-static void expand_shared(const R* rec, uint64_t n, double* xy, float* rgba) {
+// part(begin, end) over n records, shared by a few threads from kShareRecords on (the host writes
+// 64 bytes per record into fresh pages: one thread keeps up with neither the link nor the memory).
+template <typename F>
+static void share(uint64_t n, F&& part) {
   const uint64_t parts = std::min<uint64_t>(kHostThreads, n / kShareRecords + 1);
   const uint64_t per = (n + parts - 1) / parts;
   std::thread th[kHostThreads];
   uint64_t begun = 1;  // part 0 is this thread's
   for (; begun < parts; begun++) {
-    const uint64_t b = begun * per, e = std::min(n, b + per);
+    const uint64_t b = std::min(n, begun * per), e = std::min(n, b + per);
     try {
-      th[begun] = std::thread([=] { expand(rec + b, e - b, xy + 4 * b, rgba + 8 * b); });
+      th[begun] = std::thread([&part, b, e] { part(b, e); });
     } catch (...) {
       break;  // no more threads: the rest is this thread's
     }
   }
-  expand(rec, std::min(n, per), xy, rgba);
-  if (begun < parts) {
-    const uint64_t b = begun * per;
-    expand(rec + b, n - b, xy + 4 * b, rgba + 8 * b);
-  }
+  part(0, std::min(n, per));
+  if (begun < parts) part(std::min(n, begun * per), n);
   for (uint64_t p = 1; p < begun; p++) th[p].join();
+}
+
+// The indices of the keys in ascending order: a radix sort, 11 bits to a pass, over the bits that any
+// key has. Keys in order already (uploads, StringMods) take the first pass over them only.
+static std::vector<uint32_t> key_order(std::vector<uint64_t> key) {
+  const uint64_t n = key.size();
+  std::vector<uint32_t> order(n);
+  std::iota(order.begin(), order.end(), 0u);
+  if (std::is_sorted(key.begin(), key.end())) return order;
+  uint64_t bits = 0;
+  for (uint64_t k : key) bits |= k;
+  std::vector<uint64_t> key2(n);
+  std::vector<uint32_t> order2(n);
+  constexpr int kDigit = 11;
+  for (int shift = 0; shift < 64 && bits >> shift; shift += kDigit) {
+    auto digit = [&](uint64_t k) { return (uint32_t)(k >> shift) & ((1u << kDigit) - 1u); };
+    std::vector<uint32_t> at((1u << kDigit) + 1, 0u);
+    for (uint64_t k : key) at[digit(k) + 1]++;
+    for (uint32_t d = 0; d < 1u << kDigit; d++) at[d + 1] += at[d];
+    for (uint64_t i = 0; i < n; i++) {
+      const uint32_t to = at[digit(key[i])]++;
+      key2[to] = key[i];
+      order2[to] = order[i];
+    }
+    key.swap(key2);
+    order.swap(order2);
+  }
+  return order;
 }
 
 // The buffer ordered by the host: any buffer, whatever its keys.
 static int order_on_host(lg_segments* s, double* xy, float* rgba) {
   const uint64_t n = s->count;
-  std::vector<float> pos(4 * n), c0(4 * n), c1(4 * n);
-  std::vector<double> pos64;
-  std::vector<uint64_t> key(n), order(n);
+  auto room = [](bool wanted, uint64_t m) { return std::unique_ptr<float[]>(wanted ? new float[m] : nullptr); };
+  const auto pos = room(!s->has_pos64, 4 * n), c0 = room(true, 4 * n), c1 = room(!s->one_color, 4 * n);
+  const std::unique_ptr<double[]> pos64(s->has_pos64 ? new double[4 * n] : nullptr);
+  std::vector<uint64_t> key(n);
   int rc;
-  if ((rc = lg_segments_download(s, pos.data(), c0.data(), c1.data(), key.data(), n, nullptr))) return rc;
-  if (s->has_pos64) {
-    pos64.resize(4 * n);
-    if ((rc = lg_segments_download_pos64(s, pos64.data(), n, nullptr))) return rc;
-  }
-  std::iota(order.begin(), order.end(), 0ull);
-  std::sort(order.begin(), order.end(), [&](uint64_t a, uint64_t b) { return key[a] < key[b]; });
-  for (uint64_t i = 0; i < n; i++) {
-    const uint64_t k = order[i];
-    for (int c = 0; c < 4; c++) xy[4 * i + c] = pos64.empty() ? (double)pos[4 * k + c] : pos64[4 * k + c];
-    std::memcpy(rgba + 8 * i, &c0[4 * k], 16);
-    std::memcpy(rgba + 8 * i + 4, &c1[4 * k], 16);
-  }
+  if ((rc = lg_segments_download(s, pos.get(), c0.get(), c1.get(), key.data(), n, nullptr))) return rc;
+  if (pos64 && (rc = lg_segments_download_pos64(s, pos64.get(), n, nullptr))) return rc;
+  const std::vector<uint32_t> order = key_order(std::move(key));
+  const float *const p = pos.get(), *const a = c0.get(), *const b = c1 ? c1.get() : c0.get();
+  const double* const p64 = pos64.get();
+  share(n, [&](uint64_t i, uint64_t e) {
+    for (; i < e; i++) {
+      const uint64_t k = order[i];
+      for (int c = 0; c < 4; c++) xy[4 * i + c] = p64 ? p64[4 * k + c] : (double)p[4 * k + c];
+      std::memcpy(rgba + 8 * i, a + 4 * k, 16);
+      std::memcpy(rgba + 8 * i + 4, b + 4 * k, 16);
+    }
+  });
   return LG_OK;
 }
 
@@ -223,7 +252,8 @@ static int order_on_device(lg_segments* s, OrderScratch& S, double* xy, float* r
       return LG_OK;
     }
     const uint64_t b = c * kChunkRecords, m = std::min(kChunkRecords, n - b);
-    expand_shared(S.stage[c & 1].as<const R>(), m, xy + 4 * b, rgba + 8 * b);
+    const R* const rec = S.stage[c & 1].as<const R>();
+    share(m, [=](uint64_t i, uint64_t e) { expand(rec + i, e - i, xy + 4 * (b + i), rgba + 8 * (b + i)); });
   }
   *done = true;
   return LG_OK;
