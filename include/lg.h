@@ -235,7 +235,8 @@ int lg_segments_download_pos64(lg_segments* segs, double* pos64, uint64_t cap, u
 /* The buffer's vertex pairs in ascending key order, which for traced segments is trace_all's
  * order: xy gets 2 doubles and rgba 4 floats per vertex, 2 vertices per segment (FP64 end points
  * of an LG_TRACE_FP64 trace, else the stored FP32 ones). LG_E_CAPACITY with *n_vertices set to the
- * needed count when cap_vertices is too small. */
+ * needed count when cap_vertices is too small. The call's device scratch, 40 to 56 bytes per segment
+ * and 8 per ray, stays with the context up to 64 MiB, and some 12 MB of pinned host memory. */
 int lg_segments_download_vertices(lg_segments* segs, double* xy, float* rgba, uint64_t cap_vertices,
                                   uint64_t* n_vertices);
 
@@ -359,7 +360,8 @@ typedef struct lg_string_mod {          /* StringMod (string_mod.rs:3-15)       
 /* LightGarden::draw in Mode::StringMod (mod.rs:681-689): the segments of every StringMod's
  * draw() (string_mod.rs:152-158), concatenated in order, into `out` (device; created with
  * LG_SEG_VERTEX_COLORS; replaces its contents). A nested StringMod draws over the crossing
- * points of its outer lines. Points in FP64, stored as FP32 vertices; key = emission index.
+ * points of its outer lines. Points in FP64, stored as FP32 vertices; key = emission index. A table
+ * of the curves' points (16 bytes each) stays with the context up to 64 MiB.
  * LG_E_INVALID for an unknown mode/curve, a modulo colour with modulo 0 (the reference divides
  * by it), more than LG_MAX_MOD_COLORS colours or a nested outer above LG_MAX_CROSSING_LINES. */
 int lg_string_mod_draw(lg_ctx* ctx, uint32_t n, const lg_string_mod* mods, lg_segments* out);

@@ -46,6 +46,12 @@ struct OrderScratch {
 
 void OrderScratchDeleter::operator()(OrderScratch* s) const { delete s; }
 
+static size_t scratch_bytes(const OrderScratch& s) {
+  size_t b = 0;
+  for (const DevBuf* d : {&s.count, &s.start, &s.scan, &s.place, &s.path, &s.records}) b += d->bytes;
+  return b;
+}
+
 // One segment as the host reads it: 32 bytes, 48 with FP64 end points.
 struct Record32 {
   float4 pos, col;
@@ -178,7 +184,7 @@ static std::vector<uint32_t> key_order(std::vector<uint64_t> key) {
   return order;
 }
 
-// The buffer ordered by the host: any buffer, whatever its keys.
+// The buffer ordered by the host: any buffer, whatever its keys, and without device memory.
 static int order_on_host(lg_segments* s, double* xy, float* rgba) {
   const uint64_t n = s->count;
   auto room = [](bool wanted, uint64_t m) { return std::unique_ptr<float[]>(wanted ? new float[m] : nullptr); };
@@ -281,6 +287,10 @@ int lg_segments_download_vertices(lg_segments* s, double* xy, float* rgba, uint6
     bool done = false;
     const int rc = s->has_pos64 ? order_on_device<Record64>(s, *ctx->order, xy, rgba, &done)
                                 : order_on_device<Record32>(s, *ctx->order, xy, rgba, &done);
+    if (rc || scratch_bytes(*ctx->order) > kKeptScratch) {
+      (void)hipStreamSynchronize(ctx->stream);
+      ctx->order.reset();
+    }
     if (rc || done) return rc;
   }
   return order_on_host(s, xy, rgba);

@@ -590,7 +590,7 @@ int lg_string_mod_draw(lg_ctx* ctx, uint32_t n, const lg_string_mod* mods, lg_se
   uint32_t max_bits = 0;
   if (total) {
     // The curves' points are made once per curve; the StringMods that have one take them from its
-    // table (up to kMaxTable points: the scratch is kept).
+    // table (up to kMaxTable points).
     std::vector<SmDev> curves;
     std::vector<uint64_t> first;
     std::vector<int> curve_of(descs.size(), -1);
@@ -653,6 +653,7 @@ int lg_string_mod_draw(lg_ctx* ctx, uint32_t n, const lg_string_mod* mods, lg_se
     if (dev_max) LG_HIP(hipMemcpyAsync(stage, dev_max, sizeof(unsigned int), hipMemcpyDeviceToHost, st));
     LG_HIP(hipStreamSynchronize(st));
     if (dev_max) std::memcpy(&max_bits, stage, sizeof(max_bits));
+    if (S.points.bytes > lg::kKeptScratch) S.points.reset();
   } else {
     LG_HIP(hipStreamSynchronize(st));
   }

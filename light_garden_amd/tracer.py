@@ -454,6 +454,8 @@ def encode_table(ctx: Context) -> np.ndarray:
 class Tracer:
     """The reference's Tracer: owns objects and lights; traces on the GPU."""
 
+    KEPT_SEGMENTS = 1 << 20  # 40 MiB of device memory, 72 with FP64 end points
+
     def __init__(self, ctx: Optional[Context] = None, canvas_bounds=(-1.0, 1.0, -1.0, 1.0)):
         self.ctx = ctx or Context(0)
         self.objects: List[Object] = []
@@ -555,10 +557,17 @@ class Tracer:
     def trace_all(self):
         """Tracer::trace_all (tracer.rs:276): vertex pairs in the reference's order, as
         (xy float64 (2S, 2), rgba float32 (2S, 4)). One trace into a buffer that the tracer
-        keeps; the library orders it (light, ray, depth, parent, reflected before refracted)."""
+        keeps up to KEPT_SEGMENTS segments; the library orders it (light, ray, depth, parent,
+        reflected before refracted)."""
         if self._trace_segs is None or not self._trace_segs.handle:
             self._trace_segs = Segments(self.ctx)
-        return self.trace(self._trace_segs).vertices()
+        try:
+            return self.trace(self._trace_segs).vertices()
+        finally:
+            # (a trace makes room for four segments per ray)
+            rays = sum(int(light.num_rays) for light in self.lights)
+            if max(self._trace_segs.count(), 4 * rays) > self.KEPT_SEGMENTS:
+                self._trace_segs.close()
 
     def render(self, segs: Segments, img: Image):
         """One frame: clear, trace, accumulate, resolve (LightGarden::draw + Renderer::render)."""
