@@ -236,7 +236,8 @@ int lg_segments_download_pos64(lg_segments* segs, double* pos64, uint64_t cap, u
  * order: xy gets 2 doubles and rgba 4 floats per vertex, 2 vertices per segment (FP64 end points
  * of an LG_TRACE_FP64 trace, else the stored FP32 ones). LG_E_CAPACITY with *n_vertices set to the
  * needed count when cap_vertices is too small. The call's device scratch, 40 to 56 bytes per segment
- * and 8 per ray, stays with the context up to 64 MiB, and some 12 MB of pinned host memory. */
+ * and 8 per ray, stays with the context up to 64 MiB, and some 12 MB of pinned host memory; without
+ * room for it the host orders the buffer. */
 int lg_segments_download_vertices(lg_segments* segs, double* xy, float* rgba, uint64_t cap_vertices,
                                   uint64_t* n_vertices);
 

@@ -15,6 +15,7 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
+#include <new>
 #include <numeric>
 #include <thread>
 #include <vector>
@@ -291,9 +292,16 @@ int lg_segments_download_vertices(lg_segments* s, double* xy, float* rgba, uint6
       (void)hipStreamSynchronize(ctx->stream);
       ctx->order.reset();
     }
-    if (rc || done) return rc;
+    if (rc == LG_E_OOM)
+      (void)hipGetLastError();  // (no room for the scratch: nothing was launched)
+    else if (rc || done)
+      return rc;
   }
-  return order_on_host(s, xy, rgba);
+  try {
+    return order_on_host(s, xy, rgba);
+  } catch (const std::bad_alloc&) {
+    return fail(LG_E_OOM, "vertices: host memory");
+  }
 }
 
 }  // extern "C"
