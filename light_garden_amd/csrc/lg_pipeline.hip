@@ -327,8 +327,9 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
   int rc;
   Layout& L = B.L;
   // Segments in runs of one colour, every deposit non-negative: the tiles sum weights (not with
-  // 32-pixel tiles, whose kernels do not have that walk)
-  L.runs = accum && !trace && E.size() == 1 && use_runs(*E[0].segs) && ctx->tune.tile == 64 &&
+  // 32-pixel tiles, whose kernels do not have that walk, nor where the flush is to clear and
+  // resolve the image, which that of the weights does not)
+  L.runs = accum && !trace && !(stages & ST_FRESH) && E.size() == 1 && use_runs(*E[0].segs) && ctx->tune.tile == 64 &&
            scene_packed(ctx, *E[0].segs, *E[0].img);
   L.layers = L.runs ? run_layers(E[0].segs->runs) : 1;
   const int entries = (int)E.size();
