@@ -694,6 +694,7 @@ void seg_forget(lg_segments* s) {
   s->nonneg = true;
   s->hues = SceneHues{};
   s->runs = SegRuns{};
+  s->extent[0] = s->extent[1] = 0.0;
 }
 
 int seg_ensure(lg_segments* s, uint64_t cap, bool need64) {
@@ -1038,6 +1039,11 @@ int lg_segments_upload(lg_segments* s, const float* pos, const float* color0, co
   s->max_abs = b.max_abs();
   s->nonneg = b.nonneg();
   s->runs = runs;
+  if (runs.n) {
+    float4 samples[kExtentSamples];
+    for (int k = 0; k < kExtentSamples; k++) std::memcpy(&samples[k], pos + 4 * extent_sample(k, n), sizeof(float4));
+    set_extent(*s, samples);
+  }
   return LG_OK;
 }
 

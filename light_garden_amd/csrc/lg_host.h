@@ -221,6 +221,7 @@ struct lg_segments {
   bool one_color = true;
   lg::SceneHues hues;         // traced segments: the colours of their lights
   lg::SegRuns runs;           // segments of one colour each: their runs of equal colours, if few
+  double extent[2] = {0.0, 0.0};  // with runs: mean |dx| and |dy| of a sample of the segments
   uint64_t n_rays = 0;        // traced segments: the scene's rays (keys hold their index); else 0
   lg::DevBuf pos, col0, col1, key, pos64;
   bool has_pos64 = false;
@@ -267,9 +268,17 @@ void blend_factor_bounds(uint32_t code, float m, const float k[4], float out[4])
 // form in a frame's descriptor.
 SceneHues scene_hues(const lg_scene* sc);
 void set_hues(SceneDesc& D, const SceneHues& h);
-// Whether an accumulation goes by runs; the layers of such a frame, and the descriptor of one of them from the whole
-// scene's. All layers of a frame have the same tiles.
-bool use_runs(const lg_segments& s);
+// The mean extent of a buffer's segments comes from kExtentSamples of them, the same wherever they
+// came from: sample k of n segments, and the mean from the samples' end points.
+constexpr int kExtentSamples = 64;
+__host__ __device__ inline uint64_t extent_sample(int k, uint64_t n) {
+  const uint64_t spread = (uint64_t)(k + 1) * 0x9E3779B97F4A7C15ull;  // (evenly, and in step with no pattern)
+  return ((spread >> 32) * n) >> 32;  // (n < 2^32)
+}
+void set_extent(lg_segments& s, const float4* samples);
+// Whether an accumulation into the view goes by runs; the layers of such a frame, and the descriptor of one of them
+// from the whole scene's. All layers of a frame have the same tiles.
+bool use_runs(const lg_segments& s, const lg_view& view, int n_cu);
 int run_layers(const SegRuns& r);
 SceneDesc run_layer(const SceneDesc& D, const SegRuns& r, int layer, int n_layers);
 // Whether every value colour * factor is >= 0 for colour channels in [0, m].

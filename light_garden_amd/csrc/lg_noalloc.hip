@@ -135,7 +135,7 @@ int lg_accumulate_noalloc(lg_ctx* ctx, const lg_segments* segs, lg_image* img) {
   const bool hues = packed && segs->hues.n && D.blend_code == kBlendDefault && tile == 64;
   if (hues) set_hues(D, segs->hues);
   D.row_stride = 1u;
-  const bool runs = packed && use_runs(*segs) && tile == 64;
+  const bool runs = packed && tile == 64 && use_runs(*segs, img->view, ctx->n_cu);
   const int layers = runs ? run_layers(segs->runs) : 1;
   const uint32_t min_piece = std::max(kNaMinPiece, std::min(ctx->tune.min_piece, kPackedPiece));
   const uint32_t max_piece = std::max(min_piece, std::min(ctx->tune.max_piece, kPackedPiece));

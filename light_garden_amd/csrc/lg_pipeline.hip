@@ -175,8 +175,40 @@ void set_hues(SceneDesc& D, const SceneHues& h) {
   }
 }
 
-// Runs of a few segments are not worth a plane each: they average a batch of 64 pairs at least.
-bool use_runs(const lg_segments& s) { return s.runs.n > 0 && s.count >= 64ull * (uint64_t)s.runs.n; }
+void set_extent(lg_segments& s, const float4* samples) {
+  s.extent[0] = s.extent[1] = 0.0;
+  int n = 0;
+  for (int k = 0; k < kExtentSamples; k++) {
+    const double dx = std::fabs((double)samples[k].z - samples[k].x), dy = std::fabs((double)samples[k].w - samples[k].y);
+    if (!std::isfinite(dx) || !std::isfinite(dy)) continue;
+    s.extent[0] += dx;
+    s.extent[1] += dy;
+    n++;
+  }
+  for (double& e : s.extent) e = n ? e / n : 0.0;
+}
+
+// Summing weights saves 0.4 ps per sample of the frame where the whole chip walks them (more where
+// tiles and pieces are fewer than its workgroups). It costs each of a workgroup's tiles some 6 us for
+// every layer after the first (its planes, phases and barriers) and 0.25 us for every plane, of which
+// the channels' walk has about three. The samples are estimated from the segments' mean extent, a
+// tile's piece as 88000 of them. (Accumulation, us, by weights and by channels. 4096x4096, 24 runs:
+// 409600 StringMod lines 1143 and 1282, 102400 759 and 451; 1.6M lines of 400 px 1423 and 1131, in
+// 12 runs 1033 and 1136; 25000 lines of 4 px in 7 runs 304 and 230, in one 208 and 229. 2048x2048,
+// 24 runs: 409600 StringMod lines 510 and 668, 102400 278 and 249. 1920x1080, 100000 lines of 4 px
+// in 24 runs 128 and 79, in 6 84 and 80; 400000 of 400 px in 12 runs 292 and 298. 256x256, 7 runs:
+// 25600 StringMod lines 74 and 82, 1600 65 and 59.)
+bool use_runs(const lg_segments& s, const lg_view& view, int n_cu) {
+  if (s.runs.n == 0) return false;
+  const uint64_t tiles = (uint64_t)((view.width + 63) / 64) * ((view.height + 63) / 64);
+  const double rounds = (double)((tiles + n_cu - 1) / n_cu);
+  const double cost = rounds * (6.0 * (run_layers(s.runs) - 1) + 0.25 * (s.runs.n - 3));
+  const double px = std::max(std::min(s.extent[0] / (view.right - view.left), 1.0) * view.width,
+                             std::min(s.extent[1] / (view.top - view.bottom), 1.0) * view.height);
+  const double samples = (double)s.count * px;
+  const double groups = std::min(std::max((double)tiles, samples / 88000.0), (double)n_cu);
+  return 4e-7 * samples * n_cu / groups >= cost;
+}
 
 int run_layers(const SegRuns& r) { return (r.n + kRunPlanes - 1) / kRunPlanes; }
 
@@ -329,8 +361,8 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
   // Segments in runs of one colour, every deposit non-negative: the tiles sum weights (not with
   // 32-pixel tiles, whose kernels do not have that walk, nor where the flush is to clear and
   // resolve the image, which that of the weights does not)
-  L.runs = accum && !trace && !(stages & ST_FRESH) && E.size() == 1 && use_runs(*E[0].segs) && ctx->tune.tile == 64 &&
-           scene_packed(ctx, *E[0].segs, *E[0].img);
+  L.runs = accum && !trace && !(stages & ST_FRESH) && E.size() == 1 && ctx->tune.tile == 64 &&
+           use_runs(*E[0].segs, E[0].img->view, ctx->n_cu) && scene_packed(ctx, *E[0].segs, *E[0].img);
   L.layers = L.runs ? run_layers(E[0].segs->runs) : 1;
   const int entries = (int)E.size();
   const int n = L.n = L.runs ? L.layers : entries;

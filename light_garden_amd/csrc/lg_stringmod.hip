@@ -404,6 +404,11 @@ __global__ void __launch_bounds__(1024) sm_scan_rows_kernel(const uint32_t* __re
   if (threadIdx.x == 1023) *total = part[1023];
 }
 
+// The end points of a sample of the segments (set_extent), into host memory.
+__global__ void sm_extent_kernel(const float4* __restrict__ pos, uint64_t n, float4* samples) {
+  samples[threadIdx.x] = pos[lg::extent_sample((int)threadIdx.x, n)];
+}
+
 __global__ void sm_zero_u32_kernel(unsigned int* p) { *p = 0u; }
 
 int check_mod(const lg_string_mod& m, bool nested) {
@@ -617,7 +622,7 @@ int lg_string_mod_draw(lg_ctx* ctx, uint32_t n, const lg_string_mod* mods, lg_se
     const size_t db = descs.size() * sizeof(SmDev), cb = curves.size() * sizeof(SmDev), fb = first.size() * 8;
     const size_t mb = mrc.size() * sizeof(lg_mod_rem_color);
     if ((rc = S.descs.ensure(db + cb + fb + mb)) || (rc = S.maxbits.ensure(16)) ||
-        (rc = S.stage.ensure(std::max<size_t>(db + cb + fb + mb, 64))))
+        (rc = S.stage.ensure(std::max<size_t>(db + cb + fb + mb, 64 + lg::kExtentSamples * sizeof(float4)))))
       return rc;
     char* stage = S.stage.as<char>();
     std::memcpy(stage, descs.data(), db);
@@ -651,8 +656,17 @@ int lg_string_mod_draw(lg_ctx* ctx, uint32_t n, const lg_string_mod* mods, lg_se
     LG_HIP(hipGetLastError());
     // the staging buffer is free again once the stream has come this far
     if (dev_max) LG_HIP(hipMemcpyAsync(stage, dev_max, sizeof(unsigned int), hipMemcpyDeviceToHost, st));
+    // (up to three runs are summed as weights whatever the extent: use_runs)
+    float4* const samples = reinterpret_cast<float4*>(stage + 64);
+    const bool sampled = in_runs && runs.n > 3;
+    if (sampled) {
+      hipLaunchKernelGGL(sm_extent_kernel, dim3(1), dim3(lg::kExtentSamples), 0, st, out->pos.as<const float4>(), total,
+                         samples);
+      LG_HIP(hipGetLastError());
+    }
     LG_HIP(hipStreamSynchronize(st));
     if (dev_max) std::memcpy(&max_bits, stage, sizeof(max_bits));
+    if (sampled) lg::set_extent(*out, samples);
     if (S.points.bytes > lg::kKeptScratch) S.points.reset();
   } else {
     LG_HIP(hipStreamSynchronize(st));

@@ -19,8 +19,8 @@ def at_every(k, n_runs):
     return [k * i for i in range(1, n_runs)]
 
 
-@pytest.mark.parametrize("n,changes", [(1700, [255]), (1700, [256]), (1700, [257, 258]), (1700, [1, 511, 512, 513, 1699]), (1700, []),
-                                       (257, [256]), (2400, at_every(100, 24)), (2500, at_every(100, 25))],
+@pytest.mark.parametrize("n,changes", [(1700, [255]), (1700, [256]), (1700, [257, 258]), (30000, [1, 511, 512, 513, 1699]), (1700, []),
+                                       (257, [256]), (500000, at_every(1000, 24)), (2500, at_every(100, 25))],
                          ids=lambda v: str(len(v)) if isinstance(v, list) else str(v))
 def test_runs_around_stretches(ctx, orc, n, changes):
     rng = np.random.default_rng(n + len(changes))
