@@ -361,8 +361,7 @@ typedef struct lg_string_mod {          /* StringMod (string_mod.rs:3-15)       
 /* LightGarden::draw in Mode::StringMod (mod.rs:681-689): the segments of every StringMod's
  * draw() (string_mod.rs:152-158), concatenated in order, into `out` (device; created with
  * LG_SEG_VERTEX_COLORS; replaces its contents). A nested StringMod draws over the crossing
- * points of its outer lines. Points in FP64, stored as FP32 vertices; key = emission index. A table
- * of the curves' points (16 bytes each) stays with the context up to 64 MiB.
+ * points of its outer lines. Points in FP64, stored as FP32 vertices; key = emission index.
  * LG_E_INVALID for an unknown mode/curve, a modulo colour with modulo 0 (the reference divides
  * by it), more than LG_MAX_MOD_COLORS colours or a nested outer above LG_MAX_CROSSING_LINES. */
 int lg_string_mod_draw(lg_ctx* ctx, uint32_t n, const lg_string_mod* mods, lg_segments* out);

@@ -68,8 +68,8 @@ struct SmScratchDeleter {
   void operator()(SmScratch* p) const;
 };
 
-// Scratch of a call that its context keeps for the next one, at most (each of the string mods' point
-// table and the ordered downloads' device buffers): more is given back when the call ends.
+// Device scratch of an ordered download that its context keeps for the next one, at most: more is
+// given back when the call ends.
 constexpr size_t kKeptScratch = 64u << 20;
 struct OrderScratch;  // ordered downloads (lg_order.hip)
 struct OrderScratchDeleter {

@@ -20,7 +20,6 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
-#include <unordered_map>
 #include <vector>
 
 #include "lg_host.h"
@@ -41,11 +40,11 @@ struct SmDev {          // one StringMod as the generator reads it
   uint32_t mrc_off, n_mrc;
   uint64_t seg_base;    // first output segment of this StringMod
   uint64_t n_points;    // points indexed: modulo (own curve) or the crossing count (nested)
-  const double2* pts;   // NULL: the curve's own points; else a table of them or the crossing points
+  const double2* pts;   // NULL: the curve's own points; else the crossing points
 };
 
 struct SmScratch {
-  DevBuf descs, points, lines, chunk_counts, masks, row_counts, row_off, total, maxbits;
+  DevBuf descs, lines, chunk_counts, masks, row_counts, row_off, total, maxbits;
   std::vector<DevBuf*> crossings;  // crossing points of the i-th nested StringMod of a call (kept, grown)
   PinnedBuf stage;
   ~SmScratch() {
@@ -166,26 +165,11 @@ __device__ inline float absmax4(float4 c) {
   return fmaxf(fmaxf(fabsf(c.x), fabsf(c.y)), fmaxf(fabsf(c.z), fabsf(c.w)));
 }
 
-// The points of the curves of a call, each curve's from its pts on: one thread per point. Curves
-// that StringMods of the call share are there once (first: their first points, total: all).
-// (A segment's two points computed by the thread that writes it made every point twice for every StringMod: 16
-// StringMods over 100000 points 291 us, 23 us so; 3 over 20011 points with modulo colours 18 us, 14.)
-__global__ void __launch_bounds__(kBlock) sm_points_kernel(const SmDev* __restrict__ descs,
-                                                           const uint64_t* __restrict__ first, int n_curves,
-                                                           uint64_t total, double2* __restrict__ points) {
-  const uint64_t g = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (g >= total) return;
-  int lo = 0, hi = n_curves - 1;  // last curve with first <= g
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (first[mid] <= g) lo = mid;
-    else hi = mid - 1;
-  }
-  points[g] = curve_point(descs[lo], g - first[lo]);
-}
-
 // One thread per output segment of every StringMod of the call; col1 may be NULL (no modulo
-// colours: both ends have the StringMod's colour).
+// colours: both ends have the StringMod's colour). Each thread computes its two points: a table of
+// them, shared by the StringMods of a curve, costs a launch and 16-byte gathers (draws, us, with a
+// table and without: 1 StringMod over 4096 points 21 and 17; 16 over 100000 of a circle 39 and 37, of as
+// many circles 66 and 37, of one hypotrochoid 40 and 54; 16 over 20000 with modulo colours 44 and 40).
 __global__ void __launch_bounds__(kBlock) sm_segments_kernel(const SmDev* __restrict__ descs, int n_descs,
                                                              const lg_mod_rem_color* __restrict__ mrc,
                                                              uint64_t n_segs, float4* __restrict__ pos,
@@ -442,37 +426,6 @@ SmDev make_dev(const lg_string_mod& m, uint32_t mrc_off) {
   return d;
 }
 
-// Draws of fewer segments leave every thread its own points; tables hold at most this many.
-constexpr uint64_t kMinTable = 4096, kMaxTable = 1ull << 24;
-
-// Whether two StringMods have the same points.
-bool same_curve(const SmDev& a, const SmDev& b) {
-  return a.modulo == b.modulo && a.turns == b.turns && a.curve == b.curve &&
-         std::memcmp(a.cu, b.cu, sizeof(a.cu)) == 0 && std::memcmp(a.cf, b.cf, sizeof(a.cf)) == 0 &&
-         std::memcmp(&a.scale, &b.scale, sizeof(a.scale)) == 0;
-}
-
-// StringMods by their curves: a call may hold thousands (calls of 3000 and 24000 distinct curves: 1.6 and
-// 200 ms with a search through the curves so far for each, 0.25 and 3.7 ms so).
-struct CurveHash {
-  size_t operator()(const SmDev* d) const {
-    uint64_t w[8] = {d->modulo, d->turns, d->curve, d->cu[0], d->cu[1], d->cu[2]}, h = 0;
-    uint64_t f[3];
-    std::memcpy(f, d->cf, sizeof(d->cf));
-    std::memcpy(f + 2, &d->scale, sizeof(d->scale));
-    w[6] = f[0] ^ (f[1] << 1);
-    w[7] = f[2];
-    for (uint64_t x : w) {
-      h = (h ^ x) * 0x9E3779B97F4A7C15ull;
-      h ^= h >> 32;
-    }
-    return (size_t)h;
-  }
-};
-struct CurveEqual {
-  bool operator()(const SmDev* a, const SmDev* b) const { return same_curve(*a, *b); }
-};
-
 lg::SmScratch& scratch(lg_ctx* ctx) {
   if (!ctx->sm) ctx->sm.reset(new lg::SmScratch());
   return *ctx->sm;
@@ -594,42 +547,16 @@ int lg_string_mod_draw(lg_ctx* ctx, uint32_t n, const lg_string_mod* mods, lg_se
   lg::seg_forget(out);
   uint32_t max_bits = 0;
   if (total) {
-    // The curves' points are made once per curve; the StringMods that have one take them from its
-    // table (up to kMaxTable points).
-    std::vector<SmDev> curves;
-    std::vector<uint64_t> first;
-    std::vector<int> curve_of(descs.size(), -1);
-    std::unordered_map<const SmDev*, int, CurveHash, CurveEqual> known;
-    uint64_t n_points = 0;
-    for (size_t i = 0; i < descs.size() && total >= kMinTable; i++) {
-      if (descs[i].pts || descs[i].modulo > kMaxTable) continue;
-      const auto k = known.find(&descs[i]);
-      if (k != known.end()) {
-        curve_of[i] = k->second;
-        continue;
-      }
-      if (n_points + descs[i].modulo > kMaxTable) continue;
-      curve_of[i] = (int)curves.size();
-      known.emplace(&descs[i], curve_of[i]);
-      curves.push_back(descs[i]);
-      first.push_back(n_points);
-      n_points += descs[i].modulo;
-    }
-    if (n_points && (rc = S.points.ensure(n_points * sizeof(double2)))) return rc;
-    for (size_t i = 0; i < descs.size(); i++)
-      if (curve_of[i] >= 0) descs[i].pts = S.points.as<const double2>() + first[curve_of[i]];
-    // one upload: descs | curves | first | modulo colours
-    const size_t db = descs.size() * sizeof(SmDev), cb = curves.size() * sizeof(SmDev), fb = first.size() * 8;
+    // one upload: descs | modulo colours
+    const size_t db = descs.size() * sizeof(SmDev);
     const size_t mb = mrc.size() * sizeof(lg_mod_rem_color);
-    if ((rc = S.descs.ensure(db + cb + fb + mb)) || (rc = S.maxbits.ensure(16)) ||
-        (rc = S.stage.ensure(std::max<size_t>(db + cb + fb + mb, 64 + lg::kExtentSamples * sizeof(float4)))))
+    if ((rc = S.descs.ensure(db + mb)) || (rc = S.maxbits.ensure(16)) ||
+        (rc = S.stage.ensure(std::max<size_t>(db + mb, 64 + lg::kExtentSamples * sizeof(float4)))))
       return rc;
     char* stage = S.stage.as<char>();
     std::memcpy(stage, descs.data(), db);
-    if (cb) std::memcpy(stage + db, curves.data(), cb);
-    if (fb) std::memcpy(stage + db + cb, first.data(), fb);
-    if (mb) std::memcpy(stage + db + cb + fb, mrc.data(), mb);
-    LG_HIP(hipMemcpyAsync(S.descs.p, stage, db + cb + fb + mb, hipMemcpyHostToDevice, st));
+    if (mb) std::memcpy(stage + db, mrc.data(), mb);
+    LG_HIP(hipMemcpyAsync(S.descs.p, stage, db + mb, hipMemcpyHostToDevice, st));
     const char* dev = S.descs.as<const char>();
     // without modulo colours the largest |colour channel| is known here
     unsigned int* const dev_max = mrc.empty() ? nullptr : S.maxbits.as<unsigned int>();
@@ -643,13 +570,9 @@ int lg_string_mod_draw(lg_ctx* ctx, uint32_t n, const lg_string_mod* mods, lg_se
     if (dev_max) hipLaunchKernelGGL(sm_zero_u32_kernel, dim3(1), dim3(1), 0, st, dev_max);
     {
       lg::StageScope sc(ctx, "sm_generate", total);
-      if (n_points)
-        hipLaunchKernelGGL(sm_points_kernel, dim3((unsigned)((n_points + kBlock - 1) / kBlock)), dim3(kBlock), 0, st,
-                           reinterpret_cast<const SmDev*>(dev + db), reinterpret_cast<const uint64_t*>(dev + db + cb),
-                           (int)curves.size(), n_points, S.points.as<double2>());
       hipLaunchKernelGGL(sm_segments_kernel, dim3((unsigned)((total + kBlock - 1) / kBlock)), dim3(kBlock), 0, st,
                          reinterpret_cast<const SmDev*>(dev), (int)descs.size(),
-                         reinterpret_cast<const lg_mod_rem_color*>(dev + db + cb + fb), total,
+                         reinterpret_cast<const lg_mod_rem_color*>(dev + db), total,
                          out->pos.as<float4>(), out->col0.as<float4>(),
                          mrc.empty() ? nullptr : out->col1.as<float4>(), out->key.as<uint64_t>(), dev_max);
     }
@@ -667,7 +590,6 @@ int lg_string_mod_draw(lg_ctx* ctx, uint32_t n, const lg_string_mod* mods, lg_se
     LG_HIP(hipStreamSynchronize(st));
     if (dev_max) std::memcpy(&max_bits, stage, sizeof(max_bits));
     if (sampled) lg::set_extent(*out, samples);
-    if (S.points.bytes > lg::kKeptScratch) S.points.reset();
   } else {
     LG_HIP(hipStreamSynchronize(st));
   }

@@ -1,6 +1,6 @@
-"""Device memory that calls keep between them is bounded: after trace_all of a large scene and after a
-StringMod of many points the device has all but the kept scratch's bound (64 MiB each) back, and the
-calls give the same results as before."""
+"""Device memory that calls keep between them is bounded: after trace_all of a large scene the device
+has all but the kept scratch's bound (64 MiB) back, after a StringMod of many points all of it, and
+the calls give the same results as before."""
 import numpy as np
 import pytest
 import torch
@@ -42,7 +42,7 @@ def test_trace_all_gives_its_memory_back(ctx):
     tr.close()
 
 
-def test_string_mods_give_their_table_back(ctx):
+def test_string_mods_keep_no_points(ctx):
     torch.zeros(1, device="cuda")
     m = 6_000_000
     segs = lg.Segments(ctx, capacity=m, vertex_colors=True)
@@ -53,7 +53,7 @@ def test_string_mods_give_their_table_back(ctx):
     assert string_mod.draw(ctx, [lg.StringMod(modulo=m, num=2, scale=0.9, color=[0.01] * 4)], segs) == m
     kept = before - free()
     print("a draw of %d points keeps %.1f MiB" % (m, kept / MIB))
-    assert kept <= SLACK  # (the table: 92 MiB, above what is kept)
+    assert kept <= SLACK  # (the points: 92 MiB)
     string_mod.draw(ctx, small, segs)
     np.testing.assert_array_equal(segs.download()[0], want)
     segs.close()

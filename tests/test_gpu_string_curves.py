@@ -1,7 +1,6 @@
-"""One call over many StringMods, which share point tables where their curves are equal: the
-segments of each equal the StringMod drawn alone, bit for bit, with curves that differ in one parameter
-each and come back later in the call; and the call's time grows with the number of distinct curves,
-not with its square."""
+"""One call over many StringMods: the segments of each equal the StringMod drawn alone, bit for bit,
+with curves that differ in one parameter each and come back later in the call; the call's time grows
+with the number of StringMods, not with its square, and is the same whether they share a curve."""
 import ctypes as C
 import time
 
@@ -30,7 +29,7 @@ def test_shared_curves_equal_single_draws(ctx):
     segs, one = lg.Segments(ctx, vertex_colors=True), lg.Segments(ctx, vertex_colors=True)
     string_mod.draw(ctx, mods, segs)
     pos, c0, c1, _ = segs.download()
-    assert len(pos) >= 4096  # (tables are made from there on)
+    assert len(pos) >= 4096
     at = 0
     for m in mods:
         n = string_mod.draw(ctx, [m], one)
@@ -61,3 +60,22 @@ def test_time_grows_with_the_curves(ctx):
     few, many = call(3000), call(24000)
     print("3000 curves %.2f ms, 24000 curves %.2f ms" % (1e3 * few, 1e3 * many))
     assert many < 16 * few + 2e-3  # eight times the work
+
+
+def test_curves_need_not_be_shared(ctx):
+    segs = lg.Segments(ctx, capacity=1_700_000, vertex_colors=True)
+    best = {}
+    calls = {}
+    for name, step in (("shared", 0), ("own", 1)):
+        arr, keep = (abi.LgStringMod * 16)(), []
+        for i in range(16):
+            arr[i], k = lg.StringMod(modulo=100000 + step * i, num=2 + i, scale=0.9, color=[0.001] * 4).to_abi()
+            keep.append(k)
+        calls[name] = (arr, keep)
+    for _ in range(60):
+        for name, (arr, _) in calls.items():
+            t = time.perf_counter()
+            abi.call("lg_string_mod_draw", ctx.handle, 16, arr, segs.handle)
+            best[name] = min(best.get(name, 1.0), time.perf_counter() - t)
+    print("16 x 100000 points: one curve %.1f us, 16 curves %.1f us" % (1e6 * best["shared"], 1e6 * best["own"]))
+    assert best["own"] < 1.25 * best["shared"]
