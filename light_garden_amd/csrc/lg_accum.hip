@@ -863,11 +863,14 @@ __device__ __forceinline__ int scene_fixed_bits(const SceneDesc& D, int c) {
 // and no carry crosses into the other field. Every item of a tile takes G from n = min(pairs
 // of the tile, kPackedPiece) (no item holds more), so the items' sums add up in the merge slot
 // and the launch tuning changes no bit.
-constexpr double kPackLevels = 4194304.0;  // 2^22
+constexpr uint32_t kPackLevels = 1u << 22;
+__device__ __forceinline__ uint32_t packed_levels(uint32_t n) {
+  const uint32_t q = 0xFFFFFFFFu / (n > 1u ? n : 1u);  // floor((2^32 - 1) / n)
+  return q < kPackLevels ? q : kPackLevels;
+}
 __device__ __forceinline__ int packed_fixed_bits(double bound, uint32_t n) {
   if (!(bound > 0.0) || !(bound < 1e300)) return 0;
-  const uint32_t q = 0xFFFFFFFFu / (n > 1u ? n : 1u);  // floor((2^32 - 1) / n)
-  const double lim = (double)q < kPackLevels ? (double)q : kPackLevels;
+  const double lim = (double)packed_levels(n);
   // the largest G with bound * 2^G <= lim - 1/2: v <= bound, rounded once in FP32, keeps
   // v * 2^G + 1/2 below lim + 1
   return clamp_fixed_bits(floor_log2_ratio(lim - 0.5, bound));
@@ -896,7 +899,8 @@ struct HueScale {
 __device__ __forceinline__ HueScale hue_scale(const SceneDesc& D, int f, uint32_t n) {
   HueScale h{};
   if (f < D.n_hues) {
-    const int gs = packed_fixed_bits((double)D.hue_bound[f][0], n), ga = packed_fixed_bits((double)D.hue_bound[f][1], n);
+    const double a = (double)D.hue_bound[f][1];
+    const int gs = packed_fixed_bits((double)D.hue_bound[f][0], n), ga = packed_fixed_bits(a * a, n);
     h.us = __builtin_ldexp(1.0, -gs);
     h.ua = __builtin_ldexp(1.0, -ga);
     h.ss = __builtin_ldexpf(1.0f, gs);
@@ -960,7 +964,7 @@ __device__ __forceinline__ int run_color_bits(const SceneDesc& D, int c, uint32_
 }
 __device__ __forceinline__ uint32_t run_color(float v, int K) {
   const double x = __builtin_ldexp((double)v, K);
-  return x > 0.0 && x < 4294967295.0 ? (uint32_t)__builtin_rint(x) : 0u;
+  return x > 0.0 ? (uint32_t)__builtin_rint(x < 1073741824.0 ? x : 1073741824.0) : 0u;  // (2^30: an overflown product)
 }
 
 // One packed channel value of a sample: cq = round(max(v, 0) * 2^G), the low bits of one FMA against
@@ -968,6 +972,12 @@ __device__ __forceinline__ uint32_t run_color(float v, int K) {
 constexpr float kMagic = 8388608.0f;  // 2^23
 __device__ __forceinline__ uint32_t pack_q(float v, float scale) {
   return __builtin_bit_cast(uint32_t, __builtin_fmaf(__builtin_fmaxf(v, 0.0f), scale, kMagic)) & 0x7FFFFFu;
+}
+// Of a product of two numbers, which may be infinite in FP32 where the bound, in FP64, is finite: then
+// all the levels (top: 2^23 + packed_levels), so that the pixel's sum overflows and not vanishes.
+__device__ __forceinline__ uint32_t pack_q(float v, float scale, float top) {
+  const float x = __builtin_fminf(__builtin_fmaf(__builtin_fmaxf(v, 0.0f), scale, kMagic), top);
+  return __builtin_bit_cast(uint32_t, x) & 0x7FFFFFu;
 }
 
 // round(f * q) for 0 <= f < 1 and an integer q < 2^23, as one multiplication: the integer's bits
@@ -1224,6 +1234,7 @@ void tile_accum_kernel(const SceneDesc* __restrict__ descs,
     }
     const float cs0 = __builtin_ldexpf(1.0f, G[0]), cs1 = __builtin_ldexpf(1.0f, G[1]);
     const float cs2 = __builtin_ldexpf(1.0f, G[2]), cs3 = __builtin_ldexpf(1.0f, G[3]);
+    const float q_top = kMagic + (float)packed_levels(W.tile_pairs);
     const uint32_t bc = __builtin_amdgcn_readfirstlane(D.blend_code);
     const uint32_t bc0 = bc & 15u, bc1 = (bc >> 4) & 15u, bc2 = (bc >> 8) & 15u, bc3 = (bc >> 12) & 15u;
     const float bk0 = D.blend_k[0], bk1 = D.blend_k[1], bk2 = D.blend_k[2], bk3 = D.blend_k[3];
@@ -1401,19 +1412,19 @@ void tile_accum_kernel(const SceneDesc* __restrict__ descs,
               const int hch = h.ch;
               const float val = hch == 0 ? ca.x : hch == 1 ? ca.y : ca.z;
               cq0 = (int)pack_q(val, h.ss);
-              cq1 = (int)pack_q(ca.w * ca.w, h.sa);
+              cq1 = (int)pack_q(ca.w * ca.w, h.sa, q_top);
               cq2 = f * kStride;  // its plane
             } else if (two_ch) {
               if (bc == kBlendDefault) {  // (the same values, without the factors' branches)
                 cq0 = (int)pack_q(ca.x, cs0);
                 cq1 = (int)pack_q(ca.y, cs1);
                 cq2 = (int)pack_q(ca.z, cs2);
-                cq3 = (int)pack_q(ca.w * ca.w, cs3);
+                cq3 = (int)pack_q(ca.w * ca.w, cs3, q_top);
               } else {
-                cq0 = (int)pack_q(blend_value(bc0, ca.x, ca.w, bk0), cs0);
-                cq1 = (int)pack_q(blend_value(bc1, ca.y, ca.w, bk1), cs1);
-                cq2 = (int)pack_q(blend_value(bc2, ca.z, ca.w, bk2), cs2);
-                cq3 = (int)pack_q(blend_value(bc3, ca.w, ca.w, bk3), cs3);
+                cq0 = (int)pack_q(blend_value(bc0, ca.x, ca.w, bk0), cs0, q_top);
+                cq1 = (int)pack_q(blend_value(bc1, ca.y, ca.w, bk1), cs1, q_top);
+                cq2 = (int)pack_q(blend_value(bc2, ca.z, ca.w, bk2), cs2, q_top);
+                cq3 = (int)pack_q(blend_value(bc3, ca.w, ca.w, bk3), cs3, q_top);
               }
             } else {
               cq0 = fx(blend_value(bc0, ca.x, ca.w, bk0), cs0);
@@ -1610,7 +1621,7 @@ void tile_accum_kernel(const SceneDesc* __restrict__ descs,
                   const float al = __builtin_fmaf(sp, d.w, a.w);
                   deposit2<T, kStride>(t, m, pack_q(__builtin_fmaf(sp, d.x, a.x), cs0),
                                        pack_q(__builtin_fmaf(sp, d.y, a.y), cs1),
-                                       pack_q(__builtin_fmaf(sp, d.z, a.z), cs2), pack_q(al * al, cs3));
+                                       pack_q(__builtin_fmaf(sp, d.z, a.z), cs2), pack_q(al * al, cs3, q_top));
                 } else {
                   deposit2<T, kStride>(t, m, r1.x, r1.y, r1.z, r1.w);
                 }
@@ -1715,10 +1726,10 @@ void tile_accum_kernel(const SceneDesc* __restrict__ descs,
               const float d0 = bcast_f(dc.x, j), d1 = bcast_f(dc.y, j), d2 = bcast_f(dc.z, j), d3 = bcast_f(dc.w, j);
               const float sp = __builtin_fmaf(lane_f, jds, jsa);
               const float al = __builtin_fmaf(sp, d3, a3);
-              q0 = pack_q(blend_value(bc0, __builtin_fmaf(sp, d0, a0), al, bk0), cs0);
-              q1 = pack_q(blend_value(bc1, __builtin_fmaf(sp, d1, a1), al, bk1), cs1);
-              q2 = pack_q(blend_value(bc2, __builtin_fmaf(sp, d2, a2), al, bk2), cs2);
-              q3 = pack_q(blend_value(bc3, al, al, bk3), cs3);
+              q0 = pack_q(blend_value(bc0, __builtin_fmaf(sp, d0, a0), al, bk0), cs0, q_top);
+              q1 = pack_q(blend_value(bc1, __builtin_fmaf(sp, d1, a1), al, bk1), cs1, q_top);
+              q2 = pack_q(blend_value(bc2, __builtin_fmaf(sp, d2, a2), al, bk2), cs2, q_top);
+              q3 = pack_q(blend_value(bc3, al, al, bk3), cs3, q_top);
             }
             if (in) deposit2<T, kStride>(tile + e0, m, q0, q1, q2, q3);
             continue;

@@ -325,8 +325,9 @@ struct SceneDesc {
   uint32_t blend_code;
   float blend_k[4];
   float factor_max[4];
-  // SCENE_HUES: per hue the light's brightest RGB channel, the bounds of what a segment of it
-  // deposits there and in alpha (a * a), and the RGB channels over the brightest
+  // SCENE_HUES: per hue the light's brightest RGB channel, the bound of what a segment of it
+  // deposits there and its alpha (whose square a segment deposits), and the RGB channels over the
+  // brightest
   int32_t n_hues;
   int32_t hue_ch[kMaxHues];
   uint64_t hue_ray[kMaxHues];

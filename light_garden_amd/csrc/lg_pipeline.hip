@@ -170,7 +170,7 @@ void set_hues(SceneDesc& D, const SceneHues& h) {
     D.hue_ch[f] = p;
     D.hue_ray[f] = h.first_ray[f];
     D.hue_bound[f][0] = c[p];
-    D.hue_bound[f][1] = c[3] * c[3];
+    D.hue_bound[f][1] = c[3];
     for (int k = 0; k < 3; k++) D.hue_ratio[f][k] = c[p] > 0.0f ? (double)c[k] / (double)c[p] : 0.0;
   }
 }
