@@ -183,7 +183,8 @@ __device__ __forceinline__ uint32_t scene_chunk(uint32_t chunk, uint32_t groups,
 // chunk_pre[s] = first chunk of scene s, cbase[s] = first entry of scene s's [chunk][tile][axis]
 // matrix (2 x tiles x its chunk count). Frames of up to kBinScenes scenes have a wave of every
 // workgroup of the count pass make it (bin_kernel): a launch less, which at 5 us was a twentieth
-// of the smallest frames (20000 rays 185 -> 182 us a frame). For more scenes, one block of 1024:
+// of the smallest frames (20000 rays 185 -> 182 us a frame). For more scenes build_chunks_kernel
+// does, one block of 1024.
 constexpr int kBinScenes = 64;
 struct BinPlan {
   uint32_t chunk_min, target, groups;
@@ -2202,10 +2203,11 @@ hipError_t launch_work_items(const SceneDesc* descs, const uint32_t* tile_scene,
 }
 
 // The tile kernel of a frame: tile edge 64 or 32; `packed_only` when every scene of the frame
-// keeps two channels per LDS word. Workgroups per compute unit follow from the LDS tile: 64 with
-// four planes 139.3 KB (one 1024-thread workgroup), with two 69.6 KB (one of 1024 or, with
-// block = 512, two of 512), 32 with four 36.9 KB and with two 18.4 KB (four of 256); the
-// persistent grid fills every compute unit.
+// keeps two channels per LDS word. Workgroups per compute unit follow from the LDS: 64 with four
+// planes 139.3 KB (one 1024-thread workgroup); 64 packed, with 1024 threads three planes and the
+// streams' records and masks, 146.4 KB (one; so the kernel of runs too), with block = 512 two planes,
+// 69.6 KB (two); 32 with four planes 36.9 KB and with two 18.4 KB (four of 256). The persistent
+// grid fills every compute unit.
 hipError_t launch_tile_accum(const SceneDesc* descs, const uint32_t* pairs, const WorkItem* items,
                              const uint32_t* row_start, unsigned long long* split_fx, BatchCtl* ctl, int tile,
                              bool packed_only, int block, bool runs, bool count_work, int n_cu, hipStream_t st) {

@@ -353,10 +353,6 @@ constexpr uint32_t kBlendDefault = BC_ONE | (BC_ONE << 4) | (BC_ONE << 8) | (BC_
 
 constexpr int kMaxGen = kPathBits;
 
-// Device-side control block of one batched frame. Atomic adds to one line of memory are served one
-// after another, 12 ns each over the whole chip, so the words that persistent workgroups count on
-// have lines of their own: a workgroup waits for its claim, and behind other words' adds it waits
-// for those too.
 // Rays of a trace item when a launch of n_scenes has `total`: a workgroup's share of them, at
 // least 64 and at most the tuning's (`rpi`). A workgroup waits for its slowest wave at every
 // append, and a launch for its slowest workgroup, so few rays are done sooner by workgroups of one
@@ -376,6 +372,10 @@ __host__ __device__ inline uint32_t trace_item_rays(uint64_t total, uint32_t rpi
   return m < rpi ? (uint32_t)m : rpi;
 }
 
+// Device-side control block of one batched frame. Atomic adds to one line of memory are served one
+// after another, 12 ns each over the whole chip, so the words that persistent workgroups count on
+// have lines of their own: a workgroup waits for its claim, and behind other words' adds it waits
+// for those too.
 struct BatchCtl {
   uint32_t n_items_gen[kMaxGen];   // trace items per generation
   uint32_t item_rays[kMaxGen];     // rays of an item, per generation

@@ -1,7 +1,7 @@
 // lg_noalloc.hip — lg_accumulate_noalloc: lg_accumulate without any device allocation.
 //
-// lg_accumulate sizes its frame scratch (bin count matrix, pair list, tile work items, merge
-// slots, control block) on demand and grows it with hipMalloc when a frame overflows. Callers
+// lg_accumulate sizes its frame scratch (the bin chunks' places, row totals, pair list, tile work items,
+// merge slots, control block) on demand and grows it with hipMalloc when a frame overflows. Callers
 // that may not allocate (a serving loop with a fixed footprint, a harness that forbids
 // allocation) call this variant instead: the same kernels in the same order, with every
 // scratch buffer carved out of one file-scope device array, `scratch`, of fixed size. Its
