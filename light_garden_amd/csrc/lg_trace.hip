@@ -745,8 +745,9 @@ struct CullView {
 // bounces: trace launches 894 us over every object, 716 us through a hierarchy of boxes, 553 us
 // so (573 with the kind read from each lane's record: branches over execution masks); 75011 rays,
 // 23 objects, 8 bounces: 263, 256 and 200 us; FP64, 40009 rays, 12 objects, 6
-// bounces: 110 and 97 us (records in LDS). With 4 objects (20000 rays): 93 us over every object,
-// 99 us so: by boxes from lg_tuning.bvh_min_objects (8) objects.
+// bounces: 110 and 97 us (records in LDS). Few objects are tested as soon as their boxes (trace calls of
+// 20000 rays, 6 bounces, us, over every object and by boxes: 4 objects 77 and 78, 6 93 and 92, 8 101
+// and 95, 12 111 and 100): by boxes from lg_tuning.bvh_min_objects (8) objects.
 //
 // Every object that can hit within the window is a candidate (boxes are padded beyond the FP32
 // error of the test and of the hits, for the scene's farthest ray origins: object_boxes), so the
