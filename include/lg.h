@@ -387,7 +387,9 @@ typedef struct lg_tuning {
   uint32_t min_piece;      /* smallest tile work item in segment-tile pairs, >= 64; default 2048 */
   uint32_t max_piece;      /* largest tile work item, >= min_piece; default 32768; work items
                               hold at most 32768 pairs whatever the setting (the fixed point
-                              of two channels per LDS word is sized for that) */
+                              of two channels per LDS word is sized for that), and at most
+                              max(min_piece, 8192) where the tile walk goes pair by pair
+                              (32-pixel tiles, one channel per LDS word, tile_block 512) */
   uint32_t trace_waves;    /* trace workgroups per compute unit, [1, 16]; default 4 */
   uint32_t bvh_min_objects; /* scenes with at least this many objects cull by their objects'
                                bounding boxes, others test every object (as FP32 traces

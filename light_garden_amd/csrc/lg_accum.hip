@@ -2208,26 +2208,31 @@ hipError_t launch_work_items(const SceneDesc* descs, const uint32_t* tile_scene,
 // streams' records and masks, 146.4 KB (one; so the kernel of runs too), with block = 512 two planes,
 // 69.6 KB (two); 32 with four planes 36.9 KB and with two 18.4 KB (four of 256). The persistent
 // grid fills every compute unit.
+int tile_groups_per_cu(int tile, bool packed_only, int block, bool runs) {
+  return tile == 32 ? 4 : packed_only && block == 512 && !runs ? 2 : 1;
+}
+
 hipError_t launch_tile_accum(const SceneDesc* descs, const uint32_t* pairs, const WorkItem* items,
                              const uint32_t* row_start, unsigned long long* split_fx, BatchCtl* ctl, int tile,
                              bool packed_only, int block, bool runs, bool count_work, int n_cu, hipStream_t st) {
-#define LG_TILE_LAUNCH(T, P, B, PER_CU, ...)                                                                     \
-  hipLaunchKernelGGL((tile_accum_kernel<T, P, B, bool(__VA_ARGS__ + 0)>), dim3(n_cu * (PER_CU)), dim3(B), 0, st, \
+  const int grid = n_cu * tile_groups_per_cu(tile, packed_only, block, runs);
+#define LG_TILE_LAUNCH(T, P, B, ...)                                                                   \
+  hipLaunchKernelGGL((tile_accum_kernel<T, P, B, bool(__VA_ARGS__ + 0)>), dim3(grid), dim3(B), 0, st, \
                      descs, pairs, items, row_start, split_fx, ctl, count_work ? 1u : 0u)
   if (runs) {
-    LG_TILE_LAUNCH(64, true, 1024, 1, 1);
+    LG_TILE_LAUNCH(64, true, 1024, 1);
   } else if (tile == 64) {
     if (packed_only && block == 512)
-      LG_TILE_LAUNCH(64, true, 512, 2);
+      LG_TILE_LAUNCH(64, true, 512);
     else if (packed_only)
-      LG_TILE_LAUNCH(64, true, 1024, 1);
+      LG_TILE_LAUNCH(64, true, 1024);
     else
-      LG_TILE_LAUNCH(64, false, 1024, 1);
+      LG_TILE_LAUNCH(64, false, 1024);
   } else {
     if (packed_only)
-      LG_TILE_LAUNCH(32, true, 256, 4);
+      LG_TILE_LAUNCH(32, true, 256);
     else
-      LG_TILE_LAUNCH(32, false, 256, 4);
+      LG_TILE_LAUNCH(32, false, 256);
   }
 #undef LG_TILE_LAUNCH
   return hipGetLastError();

@@ -120,6 +120,8 @@ hipError_t launch_work_items(const SceneDesc* descs, const uint32_t* tile_scene,
                              WorkItem* items, uint32_t items_cap, uint32_t* split_tiles, uint32_t split_cap,
                              uint64_t pairs_cap, uint32_t min_piece, uint32_t max_piece, uint32_t grid,
                              bool whole_images, hipStream_t st);
+// Workgroups of the tile kernel per compute unit (launch_tile_accum).
+int tile_groups_per_cu(int tile, bool packed_only, int block, bool runs);
 hipError_t launch_tile_accum(const SceneDesc* descs, const uint32_t* pairs, const WorkItem* items,
                              const uint32_t* row_start, unsigned long long* split_fx, BatchCtl* ctl, int tile,
                              bool packed_only, int block, bool runs, bool count_work, int n_cu, hipStream_t st);

@@ -143,6 +143,7 @@ struct Layout {
   bool packed_only = false;          // every accumulated scene keeps two channels per LDS word
   bool hues = false;                 // some scene's deposits are one LDS word (SCENE_HUES)
   bool runs = false;                 // the frame's tiles sum weights of runs (SCENE_RUNS)
+  bool streams = false;              // every accumulated scene is walked as streams of samples
   uint64_t n_counts = 0;             // capacity of the per-frame [chunk][tile][axis] matrix
   uint32_t bin_target = 0;           // bin chunks per frame
   std::vector<int> tile_base;
@@ -237,6 +238,30 @@ static bool scene_packed(const lg_ctx* ctx, const lg_segments& segs, const lg_im
          blend_nonneg(img.blend_code, segs.max_abs, img.blend.constant);
 }
 
+// The pieces that the tiles' lists are cut into, and the share that they are measured by. Where the
+// walk goes by streams a piece is half a workgroup's even share of the pairs, within the tuning's
+// limits. Pair by pair each one takes longer, so the piece that ends last costs more than a merge:
+// a quarter of the share, and at most 8192 pairs. (Accumulation, us, with pieces of half a compute
+// unit's share up to 32768 pairs / with these: 32-pixel tiles, colours per vertex, 770k string-mod
+// lines at 36x2111 5102 / 3513, 1.6M at 1024x1024 6843 / 5620; one channel per word, 770k lines at
+// 36x2111 2136 / 1962, 800k at 640x480 1274 / 1168.)
+struct TilePieces {
+  uint32_t groups, min_piece, max_piece;
+};
+constexpr uint32_t kPairWalkPiece = 8192;
+static int frame_block(const lg_ctx* ctx, const Layout& L) { return L.hues ? 1024 : (int)ctx->tune.tile_block; }
+static TilePieces tile_pieces(const lg_ctx* ctx, const Layout& L) {
+  TilePieces p;
+  p.groups = (uint32_t)(ctx->n_cu * tile_groups_per_cu(L.tile, L.packed_only, frame_block(ctx, L), L.runs));
+  p.min_piece = std::min(ctx->tune.min_piece, kPackedPiece);
+  p.max_piece = std::min(ctx->tune.max_piece, kPackedPiece);
+  if (!L.streams) {
+    p.groups *= 2;
+    p.max_piece = std::max(p.min_piece, std::min(p.max_piece, kPairWalkPiece));
+  }
+  return p;
+}
+
 // Stage events only where the caller asked for them (the synchronous entry points on the
 // context's own stream).
 struct Scope {
@@ -281,11 +306,11 @@ static int enqueue(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, const
     }
     {
       Scope s(ctx, profile, "bin_scan", 2 * (uint64_t)L.n_tiles);
+      const TilePieces tp = tile_pieces(ctx, L);
       LG_HIP(launch_work_items(d_descs, P.tile_scene.as<uint32_t>(), L.n_tiles, L.layers, P.row_count.as<uint32_t>(),
                                P.row_start.as<uint32_t>(), P.scan_scratch.as<uint32_t>(), d_ctl,
                                P.items.as<WorkItem>(), P.items_cap, P.split_tiles.as<uint32_t>(), P.split_cap,
-                               P.pairs_cap, std::min(ctx->tune.min_piece, kPackedPiece),
-                               std::min(ctx->tune.max_piece, kPackedPiece), (uint32_t)ctx->n_cu, whole, st));
+                               P.pairs_cap, tp.min_piece, tp.max_piece, tp.groups, whole, st));
     }
     {
       Scope s(ctx, profile, "bin_fill", 0);
@@ -297,7 +322,7 @@ static int enqueue(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, const
       Scope s(ctx, profile, "tile_accum", 0);
       LG_HIP(launch_tile_accum(d_descs, P.pairs.as<uint32_t>(), P.items.as<WorkItem>(), P.row_start.as<uint32_t>(),
                                P.split_fx.as<unsigned long long>(), d_ctl, L.tile, L.packed_only,
-                               L.hues ? 1024 : (int)ctx->tune.tile_block, L.runs, profile, ctx->n_cu, st));
+                               frame_block(ctx, L), L.runs, profile, ctx->n_cu, st));
     }
     {
       Scope s(ctx, profile, "tile_merge", 0);
@@ -580,6 +605,10 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
       for (int k = 0; k < t; k++) h_tile_scene[L.tile_base[i] + k] = (uint32_t)i;
     }
   }
+  // colours per vertex go pair by pair under every blend but the default
+  L.streams = accum && L.tile == 64 && L.packed_only && (L.runs || frame_block(ctx, L) == 1024);
+  for (const Entry& e : E)
+    if (accum && !trace && !e.segs->one_color && e.img->blend_code != kBlendDefault) L.streams = false;
   if (L.runs) {
     const SceneDesc whole = hd[0];
     for (int l = 0; l < n; l++) hd[l] = run_layer(whole, E[0].segs->runs, l, n);
@@ -595,7 +624,8 @@ static int batch_launch(lg_ctx* ctx, Pipeline& P, hipStream_t st, bool profile, 
                                  (uint64_t)L.max_tiles, L.n_counts, L.bin_target, P.pairs_cap, P.items_cap,
                                  P.split_cap, ctx->tune.rays_per_item, ctx->tune.min_piece, ctx->tune.max_piece,
                                  ctx->tune.trace_waves, ctx->tune.bvh_min_objects,
-                                 (uint64_t)L.tile, (uint64_t)L.packed_only, (uint64_t)L.hues, (uint64_t)L.runs, L.chunk,
+                                 (uint64_t)L.tile, (uint64_t)L.packed_only, (uint64_t)L.hues, (uint64_t)L.runs,
+                                 (uint64_t)L.streams, L.chunk,
                                  ctx->tune.tile_block};
   for (DevBuf* b : {&P.frame_in, &P.item_pre, &P.chunk_pre, &P.cbase, &P.places, &P.scan_scratch, &P.row_start,
                     &P.pairs, &P.items, &P.split_tiles, &P.split_fx})
